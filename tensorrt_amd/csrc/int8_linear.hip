@@ -24,7 +24,9 @@
 #include "host_utils.hpp"
 #include "trtamd_encoder_ops.h"
 
-#include <cstdlib>
+#include <algorithm>
+#include <cmath>
+#include <limits>
 #include <type_traits>
 
 namespace trtamd
@@ -1108,6 +1110,203 @@ __device__ __forceinline__ void linear_piece64(
     }
 }
 
+// One tile of BM = WM*MT*32 channels x BN = WN*NT*32 tokens with the stages brought in by direct-to-LDS loads, for
+// launches that do not fill the chip with 256 x 256 tiles.  The LDS layout of a stage, its swizzles and its load units
+// are those of linear_tile_run_dma; a ring of RING stages, stage k + RING - 1 requested while stage k is multiplied and
+// one barrier per stage.  Rows behind the last one are read as the last one (their results are not stored), so any
+// T and N are taken; K a multiple of 64 bytes.  Operands both interleaved (IL) or both linear.
+template <bool IL, bool IL_OUT, int EPI, int WM, int WN, int MT, int NT, int RING>
+__device__ __forceinline__ void linear_tile_dma(
+    LinearArgs const& p, int const n0, int const t0, uint8_t* __restrict__ lds, float* sScale)
+{
+    constexpr int NWAVES = WM * WN;
+    constexpr int BM = WM * MT * 32;
+    constexpr int BN = WN * NT * 32;
+    constexpr int AF = (BM / 32) * 2;
+    constexpr int BF = (BN / 32) * 2;
+    static_assert(AF % NWAVES == 0 && BF % NWAVES == 0, "load units divide evenly among the waves");
+    static_assert(BM <= kBigTile, "scale vectors");
+    constexpr int LA = AF / NWAVES;
+    constexpr int LB = BF / NWAVES;
+    constexpr int kLoads = LA + LB;
+    constexpr int STAGE = (AF + BF) * 1024;
+
+    int const lane = threadIdx.x & 63;
+    int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int const wm = wave / WN;
+    int const wn = wave % WN;
+    uint32_t const ldsBase = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) lds;
+    uint32_t const scaleBase = (uint32_t) (size_t) (__attribute__((address_space(3))) float*) sScale;
+
+    auto unit_offset = [&](int u, int row0, int R) -> uint32_t {
+        int const rb = u >> 1, sel = u & 1;
+        if constexpr (IL)
+        {
+            int const r = lane >> 1;
+            uint32_t const half = (uint32_t) ((lane & 1) ^ ((r >> 3) & 1));
+            return ((uint32_t) sel * (uint32_t) R + (uint32_t) min(row0 + rb * 32 + r, R - 1)) * 32u + half * 16u;
+        }
+        else
+        {
+            int const rr = lane >> 2;
+            uint32_t const chunk = (uint32_t) ((lane & 3) ^ (rr >> 2));
+            return (uint32_t) min(row0 + rb * 32 + sel * 16 + rr, R - 1) * (uint32_t) p.K + chunk * 16u;
+        }
+    };
+    uint32_t offA[LA], offB[LB];
+#pragma unroll
+    for (int q = 0; q < LA; ++q)
+    {
+        offA[q] = unit_offset(q * NWAVES + wave, n0, p.N);
+    }
+#pragma unroll
+    for (int q = 0; q < LB; ++q)
+    {
+        offB[q] = unit_offset(q * NWAVES + wave, t0, p.T);
+    }
+    uint32_t const stepA = IL ? 2u * (uint32_t) p.N * 32u : 64u;
+    uint32_t const stepB = IL ? 2u * (uint32_t) p.T * 32u : 64u;
+    int const nk = p.K / 64;
+    auto fetch = [&](int kt, int slot) {
+        uint32_t const dst = ldsBase + (uint32_t) slot * STAGE;
+#pragma unroll
+        for (int q = 0; q < LA; ++q)
+        {
+            load_to_lds16_sbase(p.w + (uint64_t) kt * stepA, offA[q], dst + (uint32_t) (q * NWAVES + wave) * 1024u);
+        }
+#pragma unroll
+        for (int q = 0; q < LB; ++q)
+        {
+            load_to_lds16_sbase(p.a + (uint64_t) kt * stepB, offB[q], dst + (uint32_t) (AF + q * NWAVES + wave) * 1024u);
+        }
+    };
+    AccT<EPI> acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+    {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+        {
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+            {
+                acc[i][j][v] = 0;
+            }
+        }
+    }
+    int readOff[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+    {
+        if constexpr (IL)
+        {
+            readOff[ks] = ks * 1024 + frag_offset(lane & 31, lane >> 5);
+        }
+        else
+        {
+            int const fr = lane & 31, rr = fr & 15;
+            readOff[ks] = (fr >> 4) * 1024 + rr * 64 + (((ks * 2 + (lane >> 5)) ^ (rr >> 2)) << 4);
+        }
+    }
+    auto multiply = [&](int slot) {
+        uint8_t const* base = lds + slot * STAGE;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+        {
+            i32x4 fa[MT], fb[NT];
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+            {
+                fa[i] = *reinterpret_cast<i32x4 const*>(base + (wm * MT + i) * 2048 + readOff[ks]);
+            }
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+            {
+                fb[j] = *reinterpret_cast<i32x4 const*>(base + AF * 1024 + (wn * NT + j) * 2048 + readOff[ks]);
+            }
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+            {
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                {
+                    acc[i][j] = mma<EPI>(fa[i], fb[j], acc[i][j]);
+                }
+            }
+        }
+    };
+    // requested first, so the wait for stage 0 covers them
+    if (wave < 2 && lane < BM / 4)
+    {
+        float const* src = (wave == 0 ? p.alpha : p.beta) + min(n0 + lane * 4, p.N - 4);
+        load_to_lds16(src, scaleBase + (uint32_t) (wave * kBigTile) * 4u);
+    }
+#pragma unroll
+    for (int s = 0; s < RING - 1; ++s)
+    {
+        if (s < nk)
+        {
+            fetch(s, s);
+        }
+    }
+    int slot = 0, k = 0;
+    for (; k + RING - 1 < nk; ++k)
+    {
+        wait_vmcnt<(RING - 2) * kLoads>(); // this wavefront's part of stage k has landed
+        __syncthreads();                   // everybody's has, and nobody reads stage k - 1 any more
+        fetch(k + RING - 1, slot == 0 ? RING - 1 : slot - 1);
+        multiply(slot);
+        slot = slot == RING - 1 ? 0 : slot + 1;
+    }
+    int const rest = nk - k; // at most RING - 1 stages, all requested
+    auto last = [&](auto behindTag) {
+        constexpr int behind = decltype(behindTag)::value;
+        if (behind < rest)
+        {
+            wait_vmcnt<behind * kLoads>();
+            __syncthreads();
+            multiply(slot);
+            slot = slot == RING - 1 ? 0 : slot + 1;
+        }
+    };
+    static_assert(RING >= 2 && RING <= 4, "unrolled tail");
+    if constexpr (RING >= 4)
+    {
+        last(std::integral_constant<int, 2>{});
+    }
+    if constexpr (RING >= 3)
+    {
+        last(std::integral_constant<int, 1>{});
+    }
+    last(std::integral_constant<int, 0>{});
+
+    bool const full = t0 + BN <= p.T; // uniform
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+    {
+        int const cl = (wm * MT + i) * 32;
+        if (n0 + cl >= p.N)
+        {
+            break;
+        }
+        BlockScales const sc = load_block_scales<EPI>(sScale + cl, sScale + kBigTile + cl);
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+        {
+            int const tb = t0 + (wn * NT + j) * 32;
+            constexpr bool through = IL_OUT && (EPI == kAFFINE || EPI == kGELU);
+            if (full)
+            {
+                store_block_scaled<IL_OUT, EPI, true, through>(p, acc[i][j], n0 + cl, tb, sc);
+            }
+            else
+            {
+                store_block_scaled<IL_OUT, EPI, false, through>(p, acc[i][j], n0 + cl, tb, sc);
+            }
+        }
+    }
+}
+
 // The persistent tile plan with direct-to-LDS loads for the 256 x 256 tiles.
 template <bool IL, bool IL_OUT, int EPI>
 __global__ __launch_bounds__(512) void int8_linear_dma_kernel(LinearArgs const p)
@@ -1141,12 +1340,471 @@ __global__ __launch_bounds__(512) void int8_linear_dma_kernel(LinearArgs const p
             }
         }
         uint32_t const nbm = (uint32_t) ((p.N + kSmall - 1) / kSmall);
-        auto origin = [&](int, int& n0, int& t0) {
-            n0 = (int) (tile % nbm) * kSmall;
-            t0 = p.tokMain * kBig + (int) (tile / nbm) * kSmall;
-        };
-        linear_tile_run<2, 4, 2, 1, IL, IL, IL_OUT, EPI>(p, 1, origin, lds, sScale);
+        linear_tile_dma<IL, IL_OUT, EPI, 2, 4, 2, 1, 4>(p, (int) (tile % nbm) * kSmall,
+            p.tokMain * kBig + (int) (tile / nbm) * kSmall, lds, sScale);
     }
+}
+
+template <bool IL, bool IL_OUT, int EPI, int WM, int WN, int MT, int NT, int RING, int PER_SIMD>
+__global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(LinearArgs const p)
+{
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[RING * (WM * MT + WN * NT) * 2 * 1024];
+    __shared__ __attribute__((aligned(16))) float sScale[2 * kBigTile];
+    // panel numbering as for the large tiles (see int8_linear_kernel)
+    uint32_t const pw = (uint32_t) p.panel;
+    uint32_t const perPanel = (uint32_t) p.tokMain * pw;
+    uint32_t const tile = xcd_remap(blockIdx.x, gridDim.x);
+    uint32_t const pan = tile / perPanel, rem = tile % perPanel;
+    linear_tile_dma<IL, IL_OUT, EPI, WM, WN, MT, NT, RING>(
+        p, (int) (pan * pw + rem % pw) * (WM * MT * 32), (int) (rem / pw) * (WN * NT * 32), lds, sScale);
+}
+
+// The results of one lane for four consecutive channels (c .. c+3) of one token, packed and stored.
+template <bool IL_OUT, int EPI, typename Acc4>
+__device__ __forceinline__ void store_quad(LinearArgs const& p, Acc4 const& acc, int const c, int const t)
+{
+    f32x4 const al = *reinterpret_cast<f32x4 const*>(p.alpha + c);
+    f32x4 const be = *reinterpret_cast<f32x4 const*>(p.beta + c);
+    if (t >= p.T)
+    {
+        return;
+    }
+    if constexpr (EPI >= kF16_AFFINE)
+    {
+        f16x4 h;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+        {
+            float const y = fmaf(acc[e], al[e], be[e]);
+            h[e] = (f16) (EPI == kF16_GELU ? gelu_erf(y) : y);
+        }
+        *reinterpret_cast<f16x4*>(static_cast<f16*>(p.out) + (size_t) t * p.N + c) = h;
+    }
+    else
+    {
+        uint32_t w = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+        {
+            if constexpr (EPI == kGELU)
+            {
+                float const y = fmaf((float) acc[e], al[e], be[e]);
+                w = __builtin_amdgcn_cvt_pk_u8_f32(fmaf(gelu_erf(y), p.qOut, 128.f), e, w);
+            }
+            else
+            {
+                w = __builtin_amdgcn_cvt_pk_u8_f32(fmaf((float) acc[e], al[e], be[e] + 128.f), e, w);
+            }
+        }
+        size_t const o = IL_OUT ? ((size_t) (c >> 5) * p.T + t) * 32 + (c & 31) : (size_t) t * p.N + c;
+        *reinterpret_cast<uint32_t*>(static_cast<int8_t*>(p.out) + o) = w ^ 0x80808080u;
+    }
+}
+
+// A piece of CB x TB blocks of 32 channels x 32 tokens by one workgroup whose eight wavefronts split k, for launches
+// with too few tokens to fill the chip with tiles that walk k one stage after the other: bound by the latency of one trip
+// to memory and by what one CU can read (64 bytes a clock), not by the matrix cores.  Interleaved operands, as in
+// linear_piece64: a fragment is 1 KB of consecutive memory and goes straight into the operand registers, DEPTH k-slabs
+// in flight per wavefront, no LDS stage and no barrier before the eight partial accumulators meet in LDS; every wavefront
+// then adds up and stores quarters of blocks.  40 tokens x 4096 -> 1024: 19.1 us in 128 x 128 tiles, 4.7 us in 32 x 32
+// pieces; K any multiple of 32 bytes, N and T any.
+template <bool IL_OUT, int EPI, int CB, int TB, int DEPTH, int PER_SIMD>
+__global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(LinearArgs const p)
+{
+    constexpr int NW = 8;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[NW * CB * TB * 4096];
+    int const lane = threadIdx.x & 63;
+    int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int const row = lane & 31, half = lane >> 5;
+    uint32_t const nbm = (uint32_t) ceil_div(p.N, 32 * CB);
+    int const n0 = (int) (blockIdx.x % nbm) * (32 * CB), t0 = (int) (blockIdx.x / nbm) * (32 * TB);
+    uint32_t offA[CB], offB[TB];
+#pragma unroll
+    for (int b = 0; b < CB; ++b)
+    {
+        uint32_t const r = (uint32_t) min(n0 + 32 * b + row, p.N - 1);
+        offA[b] = r * 32u + (uint32_t) half * 16u;
+    }
+#pragma unroll
+    for (int b = 0; b < TB; ++b)
+    {
+        uint32_t const r = (uint32_t) min(t0 + 32 * b + row, p.T - 1);
+        offB[b] = r * 32u + (uint32_t) half * 16u;
+    }
+    uint32_t const slabA = (uint32_t) p.N * 32u, slabB = (uint32_t) p.T * 32u;
+    int const slabs = p.K / 32;
+    int const per = ceil_div(slabs, NW), first = wave * per;
+    int const steps = max(0, min(per, slabs - first)); // consecutive k-slabs of this wavefront
+    i32x4 fa[DEPTH][CB], fb[DEPTH][TB];
+    auto fetch = [&](int slot, int step) {
+        uint32_t const ks = (uint32_t) min(first + step, slabs - 1);
+#pragma unroll
+        for (int b = 0; b < CB; ++b)
+        {
+            fa[slot][b] = *reinterpret_cast<i32x4 const*>(p.w + (size_t) ks * slabA + offA[b]);
+        }
+#pragma unroll
+        for (int b = 0; b < TB; ++b)
+        {
+            fb[slot][b] = *reinterpret_cast<i32x4 const*>(p.a + (size_t) ks * slabB + offB[b]);
+        }
+    };
+    AccT<EPI> acc[CB][TB];
+#pragma unroll
+    for (int i = 0; i < CB; ++i)
+    {
+#pragma unroll
+        for (int j = 0; j < TB; ++j)
+        {
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+            {
+                acc[i][j][v] = 0;
+            }
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+    {
+        fetch(d, d);
+    }
+    for (int s0 = 0; s0 < steps; s0 += DEPTH)
+    {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d)
+        {
+            if (s0 + d < steps)
+            {
+#pragma unroll
+                for (int i = 0; i < CB; ++i)
+                {
+#pragma unroll
+                    for (int j = 0; j < TB; ++j)
+                    {
+                        acc[i][j] = mma<EPI>(fa[d][i], fb[d][j], acc[i][j]);
+                    }
+                }
+                if (s0 + d + DEPTH < steps)
+                {
+                    fetch(d, s0 + d + DEPTH);
+                }
+            }
+        }
+    }
+    using Acc4 = std::conditional_t<(EPI >= kF16_AFFINE), f32x4, i32x4>;
+    // partial accumulators: [wavefront][block][four registers][lane], 16 bytes per lane and access
+    Acc4* const part = reinterpret_cast<Acc4*>(lds);
+#pragma unroll
+    for (int i = 0; i < CB; ++i)
+    {
+#pragma unroll
+        for (int j = 0; j < TB; ++j)
+        {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+            {
+                part[((wave * CB * TB + (i * TB + j)) * 4 + q) * 64 + lane]
+                    = Acc4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+            }
+        }
+    }
+    __syncthreads();
+    for (int u = wave; u < CB * TB * 4; u += NW)
+    {
+        Acc4 t = part[u * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < NW; ++w)
+        {
+            t += part[(w * CB * TB * 4 + u) * 64 + lane];
+        }
+        int const b = u >> 2, q = u & 3, cb = n0 + (b / TB) * 32, tb = t0 + (b % TB) * 32;
+        if (cb < p.N)
+        {
+            store_quad<IL_OUT, EPI>(p, t, cb + 8 * q + 4 * half, tb + row);
+        }
+    }
+}
+
+// The same pieces for linear operands, where the 32 rows of a fragment are 32 separate lines (read straight into
+// registers, 40 tokens x 3072 -> 768 in FP16 take 16 us): every wavefront brings its own k range in through a ring of
+// direct-to-LDS loads of its own (units, swizzle and fragment reads of the linear tiles; 7.2 us), so there is still no
+// barrier before the partial accumulators meet.  K a multiple of 64 bytes.
+template <bool IL_OUT, int EPI, int CB, int TB, int RING, int PER_SIMD>
+__global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearArgs const p)
+{
+    constexpr int NW = 8;
+    constexpr int kLoads = (CB + TB) * 2;
+    constexpr int STAGE = kLoads * 1024;
+    static_assert(CB * TB * 4096 <= RING * STAGE, "the partial accumulators go where the wavefront's stages were");
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[NW * RING * STAGE];
+    int const lane = threadIdx.x & 63;
+    int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int const row = lane & 31, half = lane >> 5;
+    uint32_t const nbm = (uint32_t) ceil_div(p.N, 32 * CB);
+    int const n0 = (int) (blockIdx.x % nbm) * (32 * CB), t0 = (int) (blockIdx.x / nbm) * (32 * TB);
+    uint8_t* const own = lds + wave * (RING * STAGE);
+    uint32_t const ownBase = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) own;
+    int const rr = lane >> 2;
+    uint32_t const chunk = (uint32_t) ((lane & 3) ^ (rr >> 2)) * 16u;
+    uint32_t off[kLoads];
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u)
+    {
+        int const r = (u >> 1) * 32 + (u & 1) * 16 + rr;
+        int const g = u < 2 * CB ? min(n0 + r, p.N - 1) : min(t0 + r - 32 * CB, p.T - 1);
+        off[u] = (uint32_t) g * (uint32_t) p.K + chunk;
+    }
+    int const nk = p.K / 64;
+    int const per = ceil_div(nk, NW), first = wave * per;
+    int const steps = max(0, min(per, nk - first));
+    auto fetch = [&](int step, int slot) {
+        uint64_t const k = (uint64_t) (first + step) * 64u;
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u)
+        {
+            load_to_lds16_sbase((u < 2 * CB ? p.w : p.a) + k, off[u], ownBase + (uint32_t) (slot * STAGE + u * 1024));
+        }
+    };
+    AccT<EPI> acc[CB][TB];
+#pragma unroll
+    for (int i = 0; i < CB; ++i)
+    {
+#pragma unroll
+        for (int j = 0; j < TB; ++j)
+        {
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+            {
+                acc[i][j][v] = 0;
+            }
+        }
+    }
+    auto multiply = [&](int slot) {
+        uint8_t const* base = own + slot * STAGE;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+        {
+            int const fr = row & 15;
+            int const o = (row >> 4) * 1024 + fr * 64 + (((ks * 2 + half) ^ (fr >> 2)) << 4);
+            i32x4 fa[CB], fb[TB];
+#pragma unroll
+            for (int i = 0; i < CB; ++i)
+            {
+                fa[i] = *reinterpret_cast<i32x4 const*>(base + i * 2048 + o);
+            }
+#pragma unroll
+            for (int j = 0; j < TB; ++j)
+            {
+                fb[j] = *reinterpret_cast<i32x4 const*>(base + (CB + j) * 2048 + o);
+            }
+#pragma unroll
+            for (int i = 0; i < CB; ++i)
+            {
+#pragma unroll
+                for (int j = 0; j < TB; ++j)
+                {
+                    acc[i][j] = mma<EPI>(fa[i], fb[j], acc[i][j]);
+                }
+            }
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < RING - 1; ++s)
+    {
+        if (s < steps)
+        {
+            fetch(s, s);
+        }
+    }
+    int slot = 0, k = 0;
+    for (; k + RING - 1 < steps; ++k)
+    {
+        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): stage k - 1 has been read before its slot is requested again
+        fetch(k + RING - 1, slot == 0 ? RING - 1 : slot - 1);
+        wait_vmcnt<(RING - 1) * kLoads>();
+        asm volatile("" ::: "memory");
+        multiply(slot);
+        slot = slot == RING - 1 ? 0 : slot + 1;
+    }
+    int const rest = steps - k;
+    auto last = [&](auto behindTag) {
+        constexpr int behind = decltype(behindTag)::value;
+        if (behind < rest)
+        {
+            wait_vmcnt<behind * kLoads>();
+            asm volatile("" ::: "memory");
+            multiply(slot);
+            slot = slot == RING - 1 ? 0 : slot + 1;
+        }
+    };
+    static_assert(RING >= 2 && RING <= 4, "unrolled tail");
+    if constexpr (RING >= 4)
+    {
+        last(std::integral_constant<int, 2>{});
+    }
+    if constexpr (RING >= 3)
+    {
+        last(std::integral_constant<int, 1>{});
+    }
+    last(std::integral_constant<int, 0>{});
+    using Acc4 = std::conditional_t<(EPI >= kF16_AFFINE), f32x4, i32x4>;
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+#pragma unroll
+    for (int i = 0; i < CB; ++i)
+    {
+#pragma unroll
+        for (int j = 0; j < TB; ++j)
+        {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+            {
+                reinterpret_cast<Acc4*>(own)[((i * TB + j) * 4 + q) * 64 + lane]
+                    = Acc4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+            }
+        }
+    }
+    __syncthreads();
+    for (int u = wave; u < CB * TB * 4; u += NW)
+    {
+        Acc4 t = reinterpret_cast<Acc4 const*>(lds)[u * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < NW; ++w)
+        {
+            t += reinterpret_cast<Acc4 const*>(lds + w * (RING * STAGE))[u * 64 + lane];
+        }
+        int const b = u >> 2, q = u & 3, cb = n0 + (b / TB) * 32, tb = t0 + (b % TB) * 32;
+        if (cb < p.N)
+        {
+            store_quad<IL_OUT, EPI>(p, t, cb + 8 * q + 4 * half, tb + row);
+        }
+    }
+}
+
+// Which kernel a launch with operands of one layout takes: the one with the lowest estimate of
+//
+//   launch + share(x) * (tile + gelu + stage * K / 64)                    [us]
+//
+// where x is the number of tiles per CU.  Up to `resident` tiles run on a CU at once and share it, each further one
+// costing `share` of a tile's time on its own; beyond that the CU works through them at that rate, with `tail` of a
+// tile lost at the end.  Small tiles fill the chip where the problem has few of them, large ones move fewer bytes per
+// multiplication where it has many, and the pieces cut the chain of stages by eight where neither fills it.
+//
+// The constants are a fit to launches of 16 to 33289 tokens on the four layers of a 1024-channel INT8 and of a
+// 768-channel FP16 encoder (graph replays, weights from memory): every row within 5-8 %, and the choice on average
+// 1.8 % (interleaved) and 0.4 % (linear) slower than the fastest of all kernels at each of the 128 points, 12 % at
+// worst.  Before, every launch short of half a round of large tiles went in 128 x 128 tiles staged through registers:
+// 40 tokens x (1024 -> 3072 / 4096 -> 1024) INT8 7.2 / 19.1 -> 3.7 / 4.7 us, 600 tokens 7.4 / 19.0 -> 5.2 / 7.9 us,
+// 5300 tokens 20.5 / 43.0 -> 20.9 / 27.1 us; FP16 40 tokens x (768 -> 2304 / 3072 -> 768) 9.7 / 29.9 -> 4.0 / 7.2 us,
+// 9100 tokens x 3072 -> 768 80.0 -> 54.4 us.
+struct TileCost
+{
+    int channels, tokens, resident;
+    float launch, tile, stage, gelu, share, tail;
+};
+enum LinearPlan
+{
+    kLargeTiles = 0, // whole rounds of 256 x 256 tiles by persistent workgroups and smaller ones for the rest
+    kTile128x256,
+    kTile128x128,
+    kTile64x128,
+    kTile64x64,
+    kPiece64x64,
+    kPiece32x64,
+    kPiece32x32,
+    kLinearPlans
+};
+// [0]: linear operands, [1]: interleaved ones.  No channels: the layout has no such kernel.
+constexpr TileCost kTileCosts[2][kLinearPlans] = {
+    {{256, 256, 1, 0.0f, 8.32f, 0.75f, 0.33f, 0.f, 0.f}, {128, 256, 2, 0.42f, 3.40f, 0.44f, 0.79f, 1.05f, 0.78f},
+        {128, 128, 2, 0.47f, 2.02f, 0.31f, 0.38f, 0.82f, 0.75f}, {64, 128, 3, 2.06f, 0.86f, 0.189f, 0.20f, 1.00f, 0.68f},
+        {64, 64, 4, 2.19f, 0.40f, 0.136f, 0.13f, 0.83f, 0.60f}, {}, {32, 64, 1, 2.90f, 0.21f, 0.071f, 0.21f, 0.f, 1.42f},
+        {32, 32, 1, 2.09f, 0.55f, 0.054f, 0.19f, 0.f, 0.77f}},
+    {{256, 256, 1, 0.13f, 4.82f, 0.70f, 3.35f, 0.f, 0.f}, {128, 256, 2, 1.11f, 1.82f, 0.39f, 1.52f, 0.77f, 0.89f},
+        {128, 128, 3, 2.16f, 0.75f, 0.23f, 0.73f, 0.74f, 0.98f}, {64, 128, 3, 2.11f, 0.37f, 0.159f, 0.33f, 0.74f, 0.78f},
+        {64, 64, 4, 2.24f, 0.23f, 0.114f, 0.19f, 0.62f, 0.66f}, {64, 64, 1, 2.69f, 0.45f, 0.074f, 0.32f, 0.f, 1.40f},
+        {32, 64, 2, 2.40f, 0.19f, 0.053f, 0.11f, 1.07f, 0.99f}, {32, 32, 4, 2.11f, 0.90f, 0.029f, 0.30f, 0.92f, 0.77f}}};
+
+inline float tile_time(TileCost const& c, LinearArgs const& a, bool gelu)
+{
+    float const x = (float) ceil_div(a.N, c.channels) * (float) ceil_div(a.T, c.tokens) / (float) num_cus();
+    float const full = 1.f + c.share * (float) (c.resident - 1);
+    float const units = x <= (float) c.resident ? 1.f + c.share * (std::max(1.f, std::ceil(x)) - 1.f)
+                                                : full / (float) c.resident * (x + c.tail);
+    return c.launch + units * (c.tile + (gelu ? c.gelu : 0.f) + c.stage * (float) (a.K / 64));
+}
+
+// The same for the large tiles: whole rounds, then what is left (as pieces next to nothing, as 128 x 128 tiles in
+// proportion to how many there are).
+inline float large_tiles_time(TileCost const& c, bool il, LinearArgs const& a, int64_t smallTiles, bool pieces, bool gelu)
+{
+    float const stages = (float) (a.K / 64);
+    float const rest = smallTiles == 0 ? 0.f
+        : pieces                       ? 0.3f
+                                       : (float) smallTiles / (float) num_cus()
+                * (il ? 1.25f + 0.47f * stages : 0.66f * stages);
+    return c.launch + (float) ceil_div(a.mainTiles, num_cus()) * (c.tile + (gelu ? c.gelu : 0.f) + c.stage * stages) + rest;
+}
+
+template <bool IL, bool IL_OUT, int EPI>
+int launch_plan(hipStream_t stream, LinearArgs a, int plan)
+{
+    TileCost const& c = kTileCosts[IL][plan];
+    int64_t const nbm = ceil_div(a.N, c.channels), grid = nbm * ceil_div(a.T, c.tokens);
+    if (grid >= (int64_t) 1 << 31)
+    {
+        return set_error(TRTAMD_STATUS_NOT_SUPPORTED, "int8_linear: too many tiles");
+    }
+    // panels of at most 2 MB of weights: half of an XCD's L2
+    a.tokMain = ceil_div(a.T, c.tokens);
+    a.panel = 1;
+    for (int w = 1; w <= nbm && (int64_t) w * c.channels * a.K <= 2 << 20; ++w)
+    {
+        if (nbm % w == 0)
+        {
+            a.panel = w;
+        }
+    }
+    auto run = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, dim3((uint32_t) grid), dim3(threads), 0, stream, a);
+        return check_launch("int8_linear");
+    };
+    switch (plan)
+    {
+    case kTile128x256: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 4, 2, 2, 3, 4>, 512);
+    case kTile128x128:
+        // four wavefronts and three workgroups per CU; linear operands gain from eight and a deeper ring
+        if constexpr (IL)
+        {
+            return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 2, 3, 3>, 256);
+        }
+        else
+        {
+            return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 4, 2, 1, 4, 4>, 512);
+        }
+    case kTile64x128: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 2, 4, 3>, 256);
+    case kTile64x64: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 1, 4, 4>, 256);
+    default: break;
+    }
+    if constexpr (IL)
+    {
+        switch (plan)
+        {
+        case kPiece64x64: return run(linear_piece_kernel<IL_OUT, EPI, 2, 2, 4, 2>, 512);
+        case kPiece32x64: return run(linear_piece_kernel<IL_OUT, EPI, 1, 2, 4, 4>, 512);
+        case kPiece32x32: return run(linear_piece_kernel<IL_OUT, EPI, 1, 1, 8, 4>, 512);
+        default: break;
+        }
+    }
+    else
+    {
+        switch (plan)
+        {
+        case kPiece32x64: return run(linear_piece_dma_kernel<IL_OUT, EPI, 1, 2, 3, 2>, 512);
+        case kPiece32x32: return run(linear_piece_dma_kernel<IL_OUT, EPI, 1, 1, 4, 2>, 512);
+        default: break;
+        }
+    }
+    return set_error(TRTAMD_STATUS_BAD_PARAM, "int8_linear: no such plan for this layout: %d", plan);
 }
 
 template <bool IL_W, bool IL_IN, bool IL_OUT, int EPI>
@@ -1182,35 +1840,61 @@ int launch_shape(hipStream_t stream, LinearArgs a)
         return set_error(TRTAMD_STATUS_NOT_SUPPORTED, "int8_linear: too many tiles");
     }
     int const persistent = tuning(Tuning::kLinearPersistent);
+    int const direct = tuning(Tuning::kLinearDirect);
+    if constexpr (IL_W == IL_IN && (EPI == kAFFINE || EPI == kGELU || EPI == kF16_AFFINE || EPI == kF16_GELU))
+    {
+        if (persistent && direct)
+        {
+            constexpr bool gelu = EPI == kGELU || EPI == kF16_GELU;
+            // few 128 x 128 tiles behind the large ones (no more than TRTAMD_LINEAR_PIECES per cent of the CUs busy with
+            // a long k loop each): the same tokens as 64 x 64 pieces whose wavefronts split k (linear_piece64)
+            int64_t const smallTiles = grid - a.mainTiles;
+            if constexpr (IL_W && (EPI == kAFFINE || EPI == kGELU))
+            {
+                a.pieces = restTokens > 0 && smallTiles * 100 <= (int64_t) tuning(Tuning::kLinearPieces) * cus;
+            }
+            bool const large = a.N % kBig == 0 && a.K % 256 == 0 && a.mainTiles > 0;
+            int plan = tuning(Tuning::kLinearPlan);
+            if (plan < 0 || plan >= kLinearPlans || kTileCosts[IL_W][plan].channels == 0 || (plan == kLargeTiles && !large))
+            {
+                // the smaller tiles read more bytes per multiplication; a network's pass runs at the chip's power limit and
+                // pays for that in the clock of the kernels around it: they have to win by more than 8 % (the pass of 128
+                // sequences as two halves against large tiles only: +1.1 % without the margin, +0.3 +- 0.5 % with it)
+                constexpr float kMargin = 1.f / 1.08f;
+                float best = large
+                    ? kMargin * large_tiles_time(kTileCosts[IL_W][kLargeTiles], IL_W, a, smallTiles, a.pieces != 0, gelu)
+                    : std::numeric_limits<float>::max();
+                plan = kLargeTiles;
+                for (int q = kTile128x256; q < kLinearPlans; ++q)
+                {
+                    if (kTileCosts[IL_W][q].channels == 0)
+                    {
+                        continue;
+                    }
+                    float const t = tile_time(kTileCosts[IL_W][q], a, gelu);
+                    if (t < best)
+                    {
+                        best = t;
+                        plan = q;
+                    }
+                }
+            }
+            if (plan != kLargeTiles)
+            {
+                return launch_plan<IL_W, IL_OUT, EPI>(stream, a, plan);
+            }
+            a.persist = a.mainTiles < cus ? a.mainTiles : cus;
+            int64_t const behind = a.pieces ? (int64_t) (a.N / 64) * ceil_div(restTokens, 64) : smallTiles;
+            hipLaunchKernelGGL((int8_linear_dma_kernel<IL_W, IL_OUT, EPI>), dim3((uint32_t) (a.persist + behind)), dim3(512), 0,
+                stream, a);
+            return check_launch("int8_linear_dma_kernel");
+        }
+    }
     if (persistent && a.K % 128 == 0)
     {
         a.persist = a.mainTiles < cus ? a.mainTiles : cus;
-        int64_t const pgrid = grid - a.mainTiles + a.persist;
-        int const direct = tuning(Tuning::kLinearDirect);
-        if constexpr (IL_W == IL_IN && (EPI == kAFFINE || EPI == kGELU || EPI == kF16_AFFINE || EPI == kF16_GELU))
-        {
-            if (direct && a.N % kBig == 0 && a.K % 256 == 0 && a.mainTiles > 0)
-            {
-                int64_t dgrid = pgrid;
-                if constexpr (IL_W && (EPI == kAFFINE || EPI == kGELU))
-                {
-                    // few 128 x 128 tiles behind the large ones (no more than TRTAMD_LINEAR_PIECES per cent of the CUs
-                    // busy with a long k loop each): the same tokens as 64 x 64 pieces whose wavefronts split k
-                    // (linear_piece64)
-                    int64_t const smallTiles = grid - a.mainTiles;
-                    if (restTokens > 0 && smallTiles * 100 <= (int64_t) tuning(Tuning::kLinearPieces) * cus)
-                    {
-                        a.pieces = 1;
-                        dgrid = (int64_t) a.persist + (int64_t) (a.N / 64) * ceil_div(restTokens, 64);
-                    }
-                }
-                hipLaunchKernelGGL((int8_linear_dma_kernel<IL_W, IL_OUT, EPI>), dim3((uint32_t) dgrid), dim3(512), 0, stream,
-                    a);
-                return check_launch("int8_linear_dma_kernel");
-            }
-        }
-        hipLaunchKernelGGL((int8_linear_persistent_kernel<IL_W, IL_IN, IL_OUT, EPI>), dim3((uint32_t) pgrid), dim3(512), 0,
-            stream, a);
+        hipLaunchKernelGGL((int8_linear_persistent_kernel<IL_W, IL_IN, IL_OUT, EPI>),
+            dim3((uint32_t) (grid - a.mainTiles + a.persist)), dim3(512), 0, stream, a);
         return check_launch("int8_linear_persistent_kernel");
     }
     hipLaunchKernelGGL((int8_linear_kernel<IL_W, IL_IN, IL_OUT, EPI>), dim3((uint32_t) grid), dim3(512), 0, stream, a);

@@ -12,7 +12,7 @@ import oracle
 from helpers import (assert_fp_close, assert_int8_close, attention_f64, dev, dev_empty, half2_bits, host,
                      int8_attention_parity, ptr, quantize_amax, rng, stream, sync)
 from tensorrt_amd import capi
-from test_gpu_linear import interleave, problem, run_gpu
+from test_gpu_linear import interleave, problem, run_fp16, run_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -83,6 +83,35 @@ def test_linear_variants(name, value, il):
         ref = oracle.int8_linear(a, w, al, be, oepi, out_scale=scale, out_interleaved=il)
         assert_int8_close(got, ref, what=f"{name}={value} epilogue {epi}", max_frac_off=frac)
         assert np.array_equal(got, default), f"{name}={value}: bytes differ from the default kernel choice"
+
+
+@pytest.mark.parametrize("plan", range(1, 8))
+@pytest.mark.parametrize("T,K,N", [(1, 64, 32), (33, 192, 96), (130, 448, 160), (259, 768, 288)])
+def test_linear_plans(plan, T, K, N):
+    """Every tile shape of the linear layers at the edges of its tiles (one token, one past a block, channels and k that
+    are no multiple of a tile; k shorter than the ring of stages), both layouts, INT8 and FP16: the oracle's bar, and
+    INT8 bytes equal to the register-staged kernel's."""
+    a, w, alpha, beta = problem(95 + T, T, K, N)
+    for il in (True, False):
+        for epi, oepi, frac, q in ((capi.LINEAR_AFFINE, oracle.LINEAR_AFFINE, 1e-3, 1.0),
+                                   (capi.LINEAR_GELU, oracle.LINEAR_GELU, 2e-3, float(np.float32(127.0 / 4.0)))):
+            al, be = (alpha, beta) if q == 1.0 else ((alpha * 0.06).astype(np.float32), (beta * 0.02).astype(np.float32))
+            with tuning("TRTAMD_LINEAR_DIRECT", 0):
+                want = run_gpu(a, w, al, be, epi, out_scale=q, a_il=il, out_il=il, w_il=il)
+            with tuning("TRTAMD_LINEAR_PLAN", plan):
+                got = run_gpu(a, w, al, be, epi, out_scale=q, a_il=il, out_il=il, w_il=il)
+            ref = oracle.int8_linear(a, w, al, be, oepi, out_scale=q, out_interleaved=il)
+            # one value of a small output is more than the allowed share
+            assert_int8_close(got, ref, what=f"plan {plan} epilogue {epi}", max_frac_off=max(frac, 1.5 / got.size))
+            assert np.array_equal(got, want)
+    r = rng(96 + T)
+    x = r.standard_normal((T, K)).astype(np.float16)
+    w = (0.05 * r.standard_normal((N, K))).astype(np.float16)
+    for gelu in (0, 1):
+        with tuning("TRTAMD_LINEAR_PLAN", plan):
+            got = run_fp16(x, w, np.ones(N, np.float32), beta * 0.1, bool(gelu))
+        ref = oracle.fp16_linear(x, w, np.ones(N, np.float32), beta * 0.1, gelu=bool(gelu))
+        assert_fp_close(got, ref, what=f"plan {plan} FP16")
 
 
 FMHA_SETTINGS = [("TRTAMD_FMHA_GENERIC", 1), ("TRTAMD_FMHA_QSPLIT", 1), ("TRTAMD_FMHA_QSPLIT", 2),
