@@ -11,6 +11,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 ROOT = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(ROOT, "csrc")
@@ -19,6 +20,7 @@ LIB_DIR = os.path.join(ROOT, "lib")
 LIB_NAME = "libtrtamd_bert_plugins.so"
 MICROBENCH_LIB_NAME = "libtrtamd_microbench.so"   # instruction-rate probes for bench.py; not part of the plugin library
 ABLATION_LIB_NAME = "libtrtamd_ablation.so"       # the plugin library with the attention MFMAs left out (timing only)
+PLUGIN_CALL_NAME = "_plugin_call.so"              # CPython module: the plugins' runtime calls (plugin.py)
 OBJ_DIR = os.path.join(CSRC, "_obj")
 
 ARCH = "gfx950"
@@ -73,8 +75,26 @@ def build_library(jobs: int | None = None, verbose: bool = False) -> str:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     os.replace(tmp, out)
+    build_plugin_call(verbose)
     if verbose:
         print(f"built {out} from {len(srcs)} sources")
+    return out
+
+
+def build_plugin_call(verbose: bool = False) -> str:
+    """The CPython module behind Plugin.enqueue and on_shape_change (csrc/python/plugin_call.cpp): host code only."""
+    os.makedirs(LIB_DIR, exist_ok=True)
+    src = os.path.join(CSRC, "python", "plugin_call.cpp")
+    out = os.path.join(LIB_DIR, PLUGIN_CALL_NAME)
+    tmp = out + ".tmp"
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-I{INCLUDE}",
+           f"-I{sysconfig.get_paths()['include']}", src, "-o", tmp]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on {src}:\n{res.stderr}")
+    os.replace(tmp, out)
+    if verbose:
+        print(f"built {out}")
     return out
 
 

@@ -137,6 +137,7 @@ PluginTensorDesc toDesc(trtamd_tensor_desc const& t)
 std::vector<PluginTensorDesc> toDescs(trtamd_tensor_desc const* t, int32_t n)
 {
     std::vector<PluginTensorDesc> v;
+    v.reserve(static_cast<size_t>(n > 0 ? n : 0));
     for (int32_t i = 0; i < n; ++i)
     {
         v.push_back(toDesc(t[i]));

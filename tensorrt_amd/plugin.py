@@ -10,12 +10,15 @@ from __future__ import annotations
 
 import ctypes as C
 import enum
+import importlib.machinery
+import importlib.util
+import os
 from dataclasses import dataclass, field
 from typing import Iterable, Sequence
 
 import numpy as np
 
-from . import load_library
+from . import LibraryNotBuilt, library_path, load_library
 
 MAX_DIMS = 8
 
@@ -184,6 +187,16 @@ def _library():
         fn.restype = res
         fn.argtypes = args
     lib._trtamd_plugin_symbols = list(sigs)
+    # the calls made once per layer and pass go through a CPython module that reads the descriptions itself
+    path = os.path.join(os.path.dirname(library_path()), "_plugin_call.so")
+    if not os.path.exists(path):
+        raise LibraryNotBuilt(f"{path} is missing: run `python -m tensorrt_amd.build`")
+    loader = importlib.machinery.ExtensionFileLoader("_plugin_call", path)
+    lib._trtamd_call = importlib.util.module_from_spec(importlib.util.spec_from_loader("_plugin_call", loader))
+    loader.exec_module(lib._trtamd_call)
+    address = lambda name: C.cast(getattr(lib, name), C.c_void_p).value
+    lib._trtamd_addresses = {n: address(n) for n in ("trtamd_plugin_on_shape_change", "trtamd_plugin_enqueue",
+                                                     "trtamd_legacy_enqueue")}
     _lib = lib
     return lib
 
@@ -221,6 +234,9 @@ class Plugin:
     def __init__(self, handle: int):
         self._h = handle
         self._lib = _library()
+        self._call = self._lib._trtamd_call
+        self._on_shape_change = self._lib._trtamd_addresses["trtamd_plugin_on_shape_change"]
+        self._enqueue = self._lib._trtamd_addresses["trtamd_plugin_enqueue"]
 
     def __del__(self):
         if getattr(self, "_h", None):
@@ -284,18 +300,11 @@ class Plugin:
 
     # IPluginV3OneRuntime
     def on_shape_change(self, inputs: Sequence[TensorDesc], outputs: Sequence[TensorDesc]) -> int:
-        ci, ni = _descs(inputs)
-        co, no = _descs(outputs)
-        return self._lib.trtamd_plugin_on_shape_change(self._h, ci, ni, co, no)
+        return self._call.on_shape_change(self._on_shape_change, self._h, inputs, outputs)
 
     def enqueue(self, input_desc: Sequence[TensorDesc], output_desc: Sequence[TensorDesc], inputs: Sequence[int],
                 outputs: Sequence[int], workspace: int = 0, stream: int = 0) -> int:
-        ci, ni = _descs(input_desc)
-        co, no = _descs(output_desc)
-        pin = (C.c_void_p * max(len(inputs), 1))(*[C.c_void_p(int(p)) for p in inputs])
-        pout = (C.c_void_p * max(len(outputs), 1))(*[C.c_void_p(int(p)) for p in outputs])
-        return self._lib.trtamd_plugin_enqueue(self._h, ci, ni, co, no, pin, pout, C.c_void_p(int(workspace)),
-                                               C.c_void_p(int(stream)))
+        return self._call.enqueue(self._enqueue, self._h, input_desc, output_desc, inputs, outputs, workspace, stream)
 
     def get_fields_to_serialize(self) -> list[PluginField] | None:
         ptr = C.POINTER(_CField)()
@@ -382,12 +391,8 @@ class LegacyPlugin:
 
     def enqueue(self, input_desc: Sequence[TensorDesc], output_desc: Sequence[TensorDesc], inputs: Sequence[int],
                 outputs: Sequence[int], workspace: int = 0, stream: int = 0) -> int:
-        ci, ni = _descs(input_desc)
-        co, no = _descs(output_desc)
-        pin = (C.c_void_p * max(len(inputs), 1))(*[C.c_void_p(int(p)) for p in inputs])
-        pout = (C.c_void_p * max(len(outputs), 1))(*[C.c_void_p(int(p)) for p in outputs])
-        return self._lib.trtamd_legacy_enqueue(self._h, ci, ni, co, no, pin, pout, C.c_void_p(int(workspace)),
-                                               C.c_void_p(int(stream)))
+        return self._lib._trtamd_call.enqueue(self._lib._trtamd_addresses["trtamd_legacy_enqueue"], self._h, input_desc,
+                                              output_desc, inputs, outputs, workspace, stream)
 
 
 class LegacyPluginCreator:
