@@ -6,6 +6,8 @@
 // plugin/embLayerNormPlugin/embLayerNormVarSeqlenPlugin.cpp (:40-712, creators :716-830).
 #include "plugin_base.h"
 
+#include "../emb_mask.hpp"
+
 namespace trtamd
 {
 namespace plugin
@@ -233,35 +235,19 @@ protected:
         auto const* ids = static_cast<int32_t const*>(inputs[0]);
         auto const* segs = static_cast<int32_t const*>(inputs[1]);
         auto const* mask = static_cast<int32_t const*>(inputs[2]);
-        int32_t status;
-        if (mType == DataType::kFLOAT)
-        {
-            status = trtamd_emb_layer_norm_fp32(stream, mW.ld, B, S, ids, segs, mW.betaDev.as<float>(),
-                mW.gammaDev.as<float>(), mW.wordDev.as<float>(), mW.posDev.as<float>(), mW.tokDev.as<float>(),
-                mW.wordVocab, mW.tokVocab, static_cast<float*>(outputs[0]));
-        }
-        else if (mType == DataType::kHALF)
-        {
-            status = trtamd_emb_layer_norm_fp16(stream, mW.ld, B, S, ids, segs, mW.betaDev.as<float>(),
-                mW.gammaDev.as<float>(), mW.wordDev.as<uint16_t>(), mW.posDev.as<uint16_t>(),
-                mW.tokDev.as<uint16_t>(), mW.wordVocab, mW.tokVocab, static_cast<uint16_t*>(outputs[0]));
-        }
-        else
+        if (mType != DataType::kFLOAT && mType != DataType::kHALF)
         {
             logMessage(ILogger::Severity::kERROR,
                 "Unsupported type error, expected [kHALF,kFLOAT], but received "
                     + std::to_string(static_cast<int32_t>(mType)));
             return kSTATUS_NOT_SUPPORTED;
         }
-        if (status != 0)
-        {
-            return status;
-        }
         // packed mask when the attention plugin downstream runs a fused kernel at this S, else the
         // index of the first masked position per sequence
-        if (mUseFullMask || getMHAMaskPackedSize(mSM, mMhaType, S) != kUnfusedMaskSize)
+        uint32_t warpsM = 0, warpsN = 0;
+        bool const packed = mUseFullMask || getMHAMaskPackedSize(mSM, mMhaType, S) != kUnfusedMaskSize;
+        if (packed)
         {
-            uint32_t warpsM = 0, warpsN = 0;
             if (S == 64 || S == 96 || S == 128)
             {
                 warpsM = 2;
@@ -272,10 +258,19 @@ protected:
                 warpsM = 1;
                 warpsN = 8;
             }
-            return trtamd_convert_mask(static_cast<uint32_t>(S), static_cast<uint32_t>(B), warpsM, warpsN, 1, mask,
-                static_cast<uint32_t*>(outputs[1]), stream);
         }
-        return trtamd_compute_mask_idx(stream, S, B, mask, static_cast<int32_t*>(outputs[1]));
+        if (packed && warpsM == 0)
+        {
+            // a full mask was asked for at a length that has none: the embedding runs, the mask is refused
+            int32_t const status = embed(stream, B, S, ids, segs, outputs[0]);
+            return status != 0 ? status
+                               : trtamd_convert_mask(static_cast<uint32_t>(S), static_cast<uint32_t>(B), 0, 0, 1, mask,
+                                   static_cast<uint32_t*>(outputs[1]), stream);
+        }
+        EmbMask const m{mask, outputs[1], warpsM, warpsN};
+        return emb_layer_norm_with_mask(stream, mType == DataType::kHALF ? 1 : 0, mW.ld, B, S, ids, segs,
+            mW.betaDev.as<float>(), mW.gammaDev.as<float>(), mW.wordDev.get(), mW.posDev.get(), mW.tokDev.get(),
+            mW.wordVocab, mW.tokVocab, outputs[0], m);
     }
 
     void doSerialize(FieldList& f) override
@@ -287,6 +282,20 @@ protected:
     }
 
 private:
+    int32_t embed(
+        hipStream_t stream, int32_t B, int32_t S, int32_t const* ids, int32_t const* segs, void* output) const
+    {
+        if (mType == DataType::kFLOAT)
+        {
+            return trtamd_emb_layer_norm_fp32(stream, mW.ld, B, S, ids, segs, mW.betaDev.as<float>(),
+                mW.gammaDev.as<float>(), mW.wordDev.as<float>(), mW.posDev.as<float>(), mW.tokDev.as<float>(),
+                mW.wordVocab, mW.tokVocab, static_cast<float*>(output));
+        }
+        return trtamd_emb_layer_norm_fp16(stream, mW.ld, B, S, ids, segs, mW.betaDev.as<float>(),
+            mW.gammaDev.as<float>(), mW.wordDev.as<uint16_t>(), mW.posDev.as<uint16_t>(), mW.tokDev.as<uint16_t>(),
+            mW.wordVocab, mW.tokVocab, static_cast<uint16_t*>(output));
+    }
+
     EmbeddingWeights mW;
     DataType mType;
     DataType mMhaType;
