@@ -103,6 +103,52 @@ TRTAMD_API int trtamd_encoder_reserve_contexts(trtamd_encoder_t encoder, int32_t
 TRTAMD_API int trtamd_encoder_enqueue_concurrent(trtamd_encoder_t encoder, trtamd_encoder_batch const* parts,
     int32_t count, trtamd_stream_t stream);
 
+/* ------------------------------------------------------------------------------------------
+ * The FP16 encoder (EmbLayerNorm v4 -> L x [ QKV GEMM, QKV-to-context v5 on cu_seqlens, projection GEMM, SkipLayerNorm v6
+ * with bias, feed-forward GEMM + GELU, feed-forward GEMM, SkipLayerNorm v6 ]).  One call enqueues one pass; the plugin
+ * objects (runtime phase, IPluginV3*), the device weights and the activation buffers are the caller's, and the call only
+ * launches.  A plugin object serves one pass at a time: it keeps per-shape state between onShapeChange and enqueue.
+ * tensorrt_amd/encoder_fp16.py is the builder side.
+ * ------------------------------------------------------------------------------------------ */
+typedef struct trtamd_fp16_encoder_linear
+{
+    trtamd_half_t const* w; /* device [N][K] */
+    float const* alpha;     /* device [N] */
+    float const* beta;      /* device [N] */
+} trtamd_fp16_encoder_linear;
+
+typedef struct trtamd_fp16_encoder_layer
+{
+    trtamd_fp16_encoder_linear qkv, proj, ffn1, ffn2; /* rows of qkv ordered [head][q|k|v][64] */
+    void* attention;                                  /* IPluginV3 objects */
+    void* ln1;
+    void* ln2;
+} trtamd_fp16_encoder_layer;
+
+typedef struct trtamd_fp16_encoder_config
+{
+    int32_t hidden, ffn, layers;
+    int32_t max_seqlen; /* extent of the "maximum sequence length" inputs: up to 512 */
+    void* embedding;    /* IPluginV3 object */
+} trtamd_fp16_encoder_config;
+
+typedef struct trtamd_fp16_encoder_batch
+{
+    int32_t const* ids;         /* device [tokens] */
+    int32_t const* segment_ids; /* device [tokens] */
+    int32_t const* cu_seqlens;  /* device [batch + 1] */
+    int32_t batch, tokens;
+    int32_t const* mask;    /* device [1], not read by the cu_seqlens attention */
+    int32_t const* longest; /* device [max_seqlen], of which only the extent counts */
+    /* activations, device binary16: x (the result), ctx, ao, h, f [tokens][hidden]; qkv [tokens][3*hidden];
+     * m [tokens][ffn]; emb2: the embedding plugin's second output, device int32 [1] */
+    trtamd_half_t *x, *qkv, *ctx, *ao, *h, *m, *f;
+    int32_t* emb2;
+} trtamd_fp16_encoder_batch;
+
+TRTAMD_API int trtamd_fp16_encoder_enqueue(trtamd_fp16_encoder_config const* config, trtamd_fp16_encoder_layer const* layers,
+    trtamd_fp16_encoder_batch const* batch, trtamd_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -79,6 +79,26 @@ class EncoderBatch(C.Structure):
                 ("workspace", c_p), ("out", c_p)]
 
 
+class Fp16EncoderLinear(C.Structure):
+    """struct trtamd_fp16_encoder_linear (include/trtamd_encoder_runtime.h), as are the three that follow."""
+    _fields_ = [("w", c_p), ("alpha", c_p), ("beta", c_p)]
+
+
+class Fp16EncoderLayer(C.Structure):
+    _fields_ = [("qkv", Fp16EncoderLinear), ("proj", Fp16EncoderLinear), ("ffn1", Fp16EncoderLinear),
+                ("ffn2", Fp16EncoderLinear), ("attention", c_p), ("ln1", c_p), ("ln2", c_p)]
+
+
+class Fp16EncoderConfig(C.Structure):
+    _fields_ = [("hidden", i32), ("ffn", i32), ("layers", i32), ("max_seqlen", i32), ("embedding", c_p)]
+
+
+class Fp16EncoderBatch(C.Structure):
+    _fields_ = [("ids", c_p), ("segment_ids", c_p), ("cu_seqlens", c_p), ("batch", i32), ("tokens", i32), ("mask", c_p),
+                ("longest", c_p), ("x", c_p), ("qkv", c_p), ("ctx", c_p), ("ao", c_p), ("h", c_p), ("m", c_p), ("f", c_p),
+                ("emb2", c_p)]
+
+
 _SIGS = {
     "trtamd_version": (C.c_int, []),
     "trtamd_last_error": (C.c_char_p, []),
@@ -129,6 +149,8 @@ _SIGS = {
     "trtamd_encoder_enqueue": (C.c_int, [c_p, c_p, c_p, c_p, i32, i32, c_p, c_p, c_p]),
     "trtamd_encoder_reserve_contexts": (C.c_int, [c_p, i32]),
     "trtamd_encoder_enqueue_concurrent": (C.c_int, [c_p, C.POINTER(EncoderBatch), i32, c_p]),
+    "trtamd_fp16_encoder_enqueue": (C.c_int, [C.POINTER(Fp16EncoderConfig), C.POINTER(Fp16EncoderLayer),
+                                              C.POINTER(Fp16EncoderBatch), c_p]),
     "trtamd_int8_linear_to_interleaved": (C.c_int, [c_p, i32, i32, c_p, c_p]),
     "trtamd_int8_interleaved_to_linear": (C.c_int, [c_p, i32, i32, c_p, c_p]),
     "trtamd_quantize_fp16_to_interleaved": (C.c_int, [c_p, i32, i32, c_p, f32, c_p]),
@@ -144,7 +166,8 @@ ENCODER_OPS_SYMBOLS = ["trtamd_int8_linear", "trtamd_fp16_linear", "trtamd_int8_
 # Entry points declared in include/trtamd_encoder_runtime.h.
 ENCODER_RUNTIME_SYMBOLS = ["trtamd_encoder_create", "trtamd_encoder_destroy", "trtamd_encoder_set_embedding",
                            "trtamd_encoder_set_layer", "trtamd_encoder_workspace_size", "trtamd_encoder_enqueue",
-                           "trtamd_encoder_reserve_contexts", "trtamd_encoder_enqueue_concurrent"]
+                           "trtamd_encoder_reserve_contexts", "trtamd_encoder_enqueue_concurrent",
+                           "trtamd_fp16_encoder_enqueue"]
 HEADER_SYMBOLS = [k for k in _SIGS if k not in TEST_HOOK_SYMBOLS and k not in ENCODER_OPS_SYMBOLS
                   and k not in ENCODER_RUNTIME_SYMBOLS]
 

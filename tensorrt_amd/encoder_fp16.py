@@ -11,8 +11,8 @@
         residual + LN     CustomSkipLayerNormPluginDynamic v6, with bias
 
 All tensors are linear: activations [T, C] over the packed tokens, weights [N][K] (QKV rows ordered
-[head][q|k|v][64], plugin/bertQKVToContextPlugin/README.md:27-30).  torch is the allocator; every operation is a call
-into libtrtamd_bert_plugins.so.
+[head][q|k|v][64], plugin/bertQKVToContextPlugin/README.md:27-30).  torch is the allocator; a pass is one call into
+libtrtamd_bert_plugins.so (trtamd_fp16_encoder_enqueue), or one per operation where the intermediate tensors are captured.
 """
 from __future__ import annotations
 
@@ -44,6 +44,38 @@ class Fp16Linear:
         p.T, p.K, p.N = T, self.K, self.N
         p.epilogue = capi.LINEAR_GELU if self.gelu else capi.LINEAR_AFFINE
         return p
+
+
+class _Staging:
+    """Pinned host memory through which a pass's small inputs go to the GPU without waiting for it: a copy from pageable
+    memory returns only when the stream has drained, which puts the host work of every pass behind the GPU work of the
+    one before.  Four buffers take turns; one is written again only when the copy out of it has happened."""
+    SLOTS = 4
+
+    def __init__(self, torch):
+        self.torch, self.slots, self.next = torch, [None] * self.SLOTS, 0
+
+    def upload(self, arrays):
+        """One int32 device tensor with the arrays behind each other, and where each starts (at multiples of 16 bytes)."""
+        torch = self.torch
+        starts, n = [], 0
+        for a in arrays:
+            starts.append(n)
+            n += (len(a) + 3) // 4 * 4
+        i = self.next
+        self.next = (i + 1) % self.SLOTS
+        slot = self.slots[i]
+        if slot is not None:
+            slot[2].synchronize()
+        if slot is None or slot[0].numel() < n:
+            pinned = torch.empty((max(1024, 1 << (n - 1).bit_length()),), dtype=torch.int32, pin_memory=True)
+            slot = self.slots[i] = (pinned, pinned.numpy(), torch.cuda.Event())
+        for a, start in zip(arrays, starts):
+            slot[1][start:start + len(a)] = a
+        dev = torch.empty((n,), dtype=torch.int32, device="cuda")
+        dev.copy_(slot[0][:n], non_blocking=True)
+        slot[2].record()
+        return dev, starts
 
 
 class Fp16BertEncoder:
@@ -108,6 +140,21 @@ class Fp16BertEncoder:
             self.layers.append(L)
         self.T = self.B = 0
         self.buf = {}
+        self._staging = _Staging(torch)
+        self._native = self._native_structs()
+
+    def _native_structs(self):
+        """The network as trtamd_fp16_encoder_enqueue takes it; the objects pointed to live as long as the encoder."""
+        cfg = self.cfg
+        config = capi.Fp16EncoderConfig(hidden=cfg.hidden, ffn=cfg.ffn, layers=cfg.layers, max_seqlen=cfg.max_seqlen,
+                                        embedding=self.emb_plugin.handle)
+        layers = (capi.Fp16EncoderLayer * max(cfg.layers, 1))()
+        for d, L in zip(layers, self.layers):
+            for name in ("qkv", "proj", "ffn1", "ffn2"):
+                lin = L[name]
+                setattr(d, name, capi.Fp16EncoderLinear(lin.w.data_ptr(), lin.alpha.data_ptr(), lin.beta.data_ptr()))
+            d.attention, d.ln1, d.ln2 = L["attention"].handle, L["ln1"].handle, L["ln2"].handle
+        return config, layers, capi.Fp16EncoderBatch()
 
     def _bind(self, ids: np.ndarray, segs: np.ndarray, cu: np.ndarray):
         torch, cfg = self.torch, self.cfg
@@ -122,9 +169,19 @@ class Fp16BertEncoder:
                             mask=torch.zeros((1,), dtype=torch.int32, device="cuda"),
                             dummy=torch.zeros((cfg.max_seqlen,), dtype=torch.int32, device="cuda"))
             self.T, self.B = T, B
-        self.buf["ids"] = torch.from_numpy(np.ascontiguousarray(ids, np.int32)).cuda()
-        self.buf["segs"] = torch.from_numpy(np.ascontiguousarray(segs, np.int32)).cuda()
-        self.buf["cu"] = torch.from_numpy(np.ascontiguousarray(cu, np.int32)).cuda()
+            b, q = self.buf, self._native[2]
+            q.tokens, q.batch = T, B
+            q.mask, q.longest, q.emb2 = b["mask"].data_ptr(), b["dummy"].data_ptr(), b["emb2"].data_ptr()
+            for k in ("x", "qkv", "ctx", "ao", "h", "m", "f"):
+                setattr(q, k, b[k].data_ptr())
+        arrays = (ids, segs, cu)
+        dev, starts = self._staging.upload(arrays)
+        if torch.cuda.current_stream().cuda_stream != self.stream:
+            torch.cuda.current_stream().synchronize()  # the pass runs on the stream the encoder was built on
+        for k, a, start in zip(("ids", "segs", "cu"), arrays, starts):
+            self.buf[k] = dev[start:start + len(a)]
+        q = self._native[2]
+        q.ids, q.segment_ids, q.cu_seqlens = (dev.data_ptr() + 4 * start for start in starts)
 
     def _check(self, st, what):
         if st != 0:
@@ -172,10 +229,13 @@ class Fp16BertEncoder:
         if ids is not None:
             self._bind(ids, segs, cu)
         b = self.buf
+        if capture is None:
+            config, layers, batch = self._native
+            self.api.check(self.api.fp16_encoder_enqueue(C.byref(config), layers, C.byref(batch), self.stream))
+            return b["x"]
 
         def keep(key, t):
-            if capture is not None:
-                capture[key] = t.detach().cpu().numpy().copy()
+            capture[key] = t.detach().cpu().numpy().copy()
 
         self._embed()
         keep("emb", b["x"])

@@ -243,6 +243,11 @@ class Plugin:
             self._lib.trtamd_plugin_destroy(self._h)
             self._h = None
 
+    @property
+    def handle(self) -> int:
+        """The IPluginV3 object, for C functions that take one."""
+        return self._h
+
     # IPluginV3
     def clone(self) -> "Plugin | None":
         h = self._lib.trtamd_plugin_clone(self._h)
