@@ -166,10 +166,8 @@ __device__ __forceinline__ void mask_workgroup(MaskJob const& job, uint32_t cons
 // TPW consecutive token slots per wavefront.  gamma and beta are fetched once per wavefront (converted to T and
 // back, as the reference does per element) instead of once per token: at TPW = 1 they are two thirds of the
 // bytes a token pulls through the vector cache.
-// A short launch is bound by its chain of trips to memory, so that nothing waits that need not: the ids are requested
-// first, the position row, gamma and beta while they are on their way, and gamma and beta are converted only when the
-// row has been gathered (B = 32, S = 128, 768 channels FP16 with the mask output: 9.5 -> 6.0 us back to back, of which
-// the mask as a launch of its own was 4.2 us).
+// With the plugin's mask output, whose workgroups come first (MaskJob): B = 32, S = 128, 768 channels FP16 takes 6.0 us
+// where the embedding and the mask as two launches took 9.5.
 template <typename T, int NV, int MODE, int TPW>
 __global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B, int const S,
     int32_t const* __restrict__ inputIds, int32_t const* __restrict__ tokenIds, int32_t const* __restrict__ cuSeqlens,
@@ -191,26 +189,25 @@ __global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B
         (int) ((int64_t) (blockIdx.x - (MODE == kFIXED ? job.blocks : 0u)) * kWavesPerBlock + (threadIdx.x >> 6)));
     int const nvec = ld / VPT;
 
-    f32x4 g4[NV][VPT / 4], b4[NV][VPT / 4];
-    auto load_scales = [&] {
+    // gamma/beta take the output type first: `const R g(gamma[i])`, common.cuh:275-276
+    float gk[NV][VPT], bk[NV][VPT];
 #pragma unroll
-        for (int j = 0; j < NV; ++j)
+    for (int j = 0; j < NV; ++j)
+    {
+        int const vi = lane + kWaveSize * j;
+        bool const ok = vi < nvec;
+#pragma unroll
+        for (int q = 0; q < VPT / 4; ++q)
         {
-            int const vi = lane + kWaveSize * j;
-            bool const ok = vi < nvec;
+            f32x4 const g4 = ok ? *reinterpret_cast<f32x4 const*>(gamma + vi * VPT + q * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+            f32x4 const b4 = ok ? *reinterpret_cast<f32x4 const*>(beta + vi * VPT + q * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int q = 0; q < VPT / 4; ++q)
+            for (int e = 0; e < 4; ++e)
             {
-                g4[j][q] = ok ? *reinterpret_cast<f32x4 const*>(gamma + vi * VPT + q * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
-                b4[j][q] = ok ? *reinterpret_cast<f32x4 const*>(beta + vi * VPT + q * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+                gk[j][q * 4 + e] = (float) (T) g4[e];
+                bk[j][q * 4 + e] = (float) (T) b4[e];
             }
         }
-    };
-    // gamma/beta take the output type first: `const R g(gamma[i])`, common.cuh:275-276
-    auto through_t = [](float x) { return (float) (T) x; };
-    if constexpr (TPW > 1)
-    {
-        load_scales();
     }
 
 #pragma unroll 1
@@ -222,21 +219,11 @@ __global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B
         {
             continue;
         }
-        int const anyWord = inputIds[tokenIdx], anyTok = tokenIds[tokenIdx];
-        Vec16<T> w[NV], t[NV], p[NV];
-#pragma unroll
-        for (int j = 0; j < NV; ++j)
-        {
-            int const vi = lane + kWaveSize * j;
-            p[j].u = vi < nvec ? *reinterpret_cast<u32x4 const*>(posEmb + (int64_t) pos * ld + vi * VPT) : u32x4{0, 0, 0, 0};
-        }
-        if constexpr (TPW == 1)
-        {
-            load_scales();
-        }
-        int const wordId = __builtin_amdgcn_readfirstlane(anyWord);
-        int const tokId = __builtin_amdgcn_readfirstlane(anyTok);
+        int const wordId = __builtin_amdgcn_readfirstlane(inputIds[tokenIdx]);
+        int const tokId = __builtin_amdgcn_readfirstlane(tokenIds[tokenIdx]);
         bool const inRange = wordId >= 0 && wordId < wordSize && tokId >= 0 && tokId < tokSize;
+
+        Vec16<T> w[NV], t[NV], p[NV];
 #pragma unroll
         for (int j = 0; j < NV; ++j)
         {
@@ -244,14 +231,7 @@ __global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B
             bool const ok = vi < nvec && inRange;
             w[j].u = ok ? *reinterpret_cast<u32x4 const*>(wordEmb + (int64_t) wordId * ld + vi * VPT) : u32x4{0, 0, 0, 0};
             t[j].u = ok ? *reinterpret_cast<u32x4 const*>(tokEmb + (int64_t) tokId * ld + vi * VPT) : u32x4{0, 0, 0, 0};
-        }
-        if (!inRange)
-        {
-#pragma unroll
-            for (int j = 0; j < NV; ++j)
-            {
-                p[j].u = u32x4{0, 0, 0, 0};
-            }
+            p[j].u = ok ? *reinterpret_cast<u32x4 const*>(posEmb + (int64_t) pos * ld + vi * VPT) : u32x4{0, 0, 0, 0};
         }
 
         float v[NV][VPT];
@@ -305,7 +285,7 @@ __global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B
 #pragma unroll
                 for (int k = 0; k < VPT; ++k)
                 {
-                    y.e[k] = (T) (through_t(g4[j][k / 4][k % 4]) * (v[j][k] - mu) * rsigma + through_t(b4[j][k / 4][k % 4]));
+                    y.e[k] = (T) (gk[j][k] * (v[j][k] - mu) * rsigma + bk[j][k]);
                 }
                 store_through_l2(output + tokenIdx * ld + (int64_t) vi * VPT, y.u);
             }
