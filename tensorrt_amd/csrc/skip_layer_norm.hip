@@ -230,13 +230,24 @@ int skip_layer_norm(hipStream_t stream, int32_t ld, int64_t n, T const* in, T co
     bool const vec_ok = ld % VPT == 0 && ld > 32 && aligned16(in) && aligned16(skip) && aligned16(out)
         && aligned16(beta) && aligned16(gamma) && (!bias || aligned16(bias));
     int const nv = vec_ok ? ceil_div(ld / VPT, kWaveSize) : 0;
+    // One row per wavefront: a short launch then has the most wavefronts to wait for memory in parallel and the shortest
+    // chain in each (FP16, 400 rows: 384 channels 4.3 -> 2.9 us against four rows per wavefront, 768 channels 3.8 -> 3.0 us
+    // against two), and a long one is as fast within 1-2 % either way.  Two rows are kept where they are the faster:
+    // FP16 rows of two vectors per lane beyond 8192 rows (65664 x 768: 55.2 against 56.2 us).
     if (vec_ok && nv == 1)
     {
-        return launch_rows<T, 1, 4>(stream, ld, rows, in, skip, beta, gamma, bias, out, eps);
+        return launch_rows<T, 1, 1>(stream, ld, rows, in, skip, beta, gamma, bias, out, eps);
     }
     if (vec_ok && nv == 2)
     {
-        return launch_rows<T, 2, 2>(stream, ld, rows, in, skip, beta, gamma, bias, out, eps);
+        if constexpr (sizeof(T) == 2)
+        {
+            if (rows > 8192)
+            {
+                return launch_rows<T, 2, 2>(stream, ld, rows, in, skip, beta, gamma, bias, out, eps);
+            }
+        }
+        return launch_rows<T, 2, 1>(stream, ld, rows, in, skip, beta, gamma, bias, out, eps);
     }
     if (vec_ok && nv <= 4)
     {
@@ -707,6 +718,115 @@ __global__ __launch_bounds__(W * kWaveSize) void skipln_interleaved_kernel(int c
     }
 }
 
+// The same for few tokens: one wavefront per token, lane = (channel group, half) as in the tail above, so that a handful
+// of tokens spreads over as many CUs and nothing is exchanged between wavefronts.  (The 32-token blocks put 48 tokens on
+// two CUs, which then take longer over the arithmetic than over the loads.)
+template <int G, bool PRELN>
+__global__ __launch_bounds__(kBlock) void skipln_interleaved_token_kernel(int const total, int8_t const* __restrict__ in,
+    int8_t const* __restrict__ skip, f16 const* __restrict__ beta, f16 const* __restrict__ gamma, int8_t* __restrict__ out,
+    int8_t* __restrict__ preln, float const dqIn, float const dqSkip, float const qScale, float const qSkipScale,
+    float const eps, float const prelnMin)
+{
+    constexpr int LD = G * 32;
+    constexpr int NE = (G + 31) / 32; // loads per tensor and lane: 32 channel groups x 2 halves each
+    int const lane = threadIdx.x & (kWaveSize - 1);
+    int const hf = lane & 1;
+    int const token = (int) blockIdx.x * kWavesPerBlock + (int) (threadIdx.x >> 6);
+    if (token >= total)
+    {
+        return;
+    }
+    int64_t const groupStride = (int64_t) total * 32;
+    u32x4 xi[NE], xs[NE];
+    f16x8 g[NE][2], b[NE][2];
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+    {
+        int const grp = e * 32 + (lane >> 1);
+        bool const live = grp < G;
+        int64_t const off = (int64_t) grp * groupStride + (int64_t) token * 32 + hf * 16;
+        xi[e] = live ? *reinterpret_cast<u32x4 const*>(in + off) : u32x4{0, 0, 0, 0};
+        xs[e] = live ? *reinterpret_cast<u32x4 const*>(skip + off) : u32x4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+    {
+        int const grp = e * 32 + (lane >> 1);
+        int const ch = grp < G ? grp * 32 + hf * 16 : 0;
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+        {
+            g[e][q] = *reinterpret_cast<f16x8 const*>(gamma + ch + 8 * q);
+            b[e][q] = *reinterpret_cast<f16x8 const*>(beta + ch + 8 * q);
+        }
+    }
+    int sIn = 0, sSk = 0, sII = 0, sIS = 0, sSS = 0;
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+    {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+        {
+            sIn = __builtin_amdgcn_sdot4((int) xi[e][q], 0x01010101, sIn, false);
+            sSk = __builtin_amdgcn_sdot4((int) xs[e][q], 0x01010101, sSk, false);
+            sII = __builtin_amdgcn_sdot4((int) xi[e][q], (int) xi[e][q], sII, false);
+            sIS = __builtin_amdgcn_sdot4((int) xi[e][q], (int) xs[e][q], sIS, false);
+            sSS = __builtin_amdgcn_sdot4((int) xs[e][q], (int) xs[e][q], sSS, false);
+        }
+    }
+    sIn = wave_sum_i32(sIn);
+    sSk = wave_sum_i32(sSk);
+    sII = wave_sum_i32(sII);
+    sIS = wave_sum_i32(sIS);
+    sSS = wave_sum_i32(sSS);
+    double const dIn = (double) dqIn, dSk = (double) dqSkip;
+    double const mean = (dIn * sIn + dSk * sSk) * (1.0 / LD);
+    double const ex2 = (dIn * dIn * sII + 2.0 * dIn * dSk * sIS + dSk * dSk * sSS) * (1.0 / LD);
+    float const rsigma = rsqrtf(fmaxf((float) (ex2 - mean * mean), 0.f) + eps);
+    float const a1 = dqIn * rsigma;
+    float const a2 = dqSkip * rsigma;
+    float const c1 = (float) (-mean * (double) rsigma);
+    float const p1 = dqIn * qSkipScale;
+    float const p2 = dqSkip * qSkipScale;
+    float const prelnLo = prelnMin + 128.f;
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+    {
+        int const grp = e * 32 + (lane >> 1);
+        u32x4 o, po;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+        {
+            uint32_t yw = 0, pw = 0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+            {
+                float const fa = i8_to_f32(xi[e][q], k);
+                float const fs = i8_to_f32(xs[e][q], k);
+                float const gq = (float) g[e][q >> 1][(q & 1) * 4 + k] * qScale;
+                float const bq = (float) b[e][q >> 1][(q & 1) * 4 + k] * qScale + 128.f;
+                float const nrm = fmaf(fa, a1, fmaf(fs, a2, c1));
+                yw = __builtin_amdgcn_cvt_pk_u8_f32(fmaf(gq, nrm, bq), k, yw);
+                if (PRELN)
+                {
+                    pw = __builtin_amdgcn_cvt_pk_u8_f32(fmaxf(fmaf(fa, p1, fmaf(fs, p2, 128.f)), prelnLo), k, pw);
+                }
+            }
+            o[q] = yw ^ 0x80808080u;
+            po[q] = pw ^ 0x80808080u;
+        }
+        if (grp < G)
+        {
+            int64_t const off = (int64_t) grp * groupStride + (int64_t) token * 32 + hf * 16;
+            *reinterpret_cast<u32x4*>(out + off) = o;
+            if (PRELN)
+            {
+                *reinterpret_cast<u32x4*>(preln + off) = po;
+            }
+        }
+    }
+}
+
 // Workgroups of this kernel that the current device holds at once (asked once per process and kernel; 0 when it
 // cannot be asked).
 template <int G, int W, int TOK, bool PRELN, bool TAIL>
@@ -732,6 +852,17 @@ int launch_interleaved_as(hipStream_t stream, int32_t total, int8_t const* in, i
     f16 const* gamma, int8_t* out, int8_t* preln, float dqIn, float dqSkip, float qScale, float qSkipScale, float eps,
     float prelnMin)
 {
+    // One wavefront per token up to the 4 MB per tensor where the blocks of 32 tokens, whose loads are whole lines, have
+    // caught up (us per launch, blocks / tokens, 1024 channels: 48 tokens 4.4 / 2.3, 1000 tokens 4.6 / 2.6, 3000 tokens
+    // 4.6 / 3.7, 4000 tokens 4.8 / 4.3, 5500 tokens 4.9 / 5.8).
+    constexpr int64_t kFewBytes = 4 << 20;
+    if ((int64_t) total * (G * 32) <= kFewBytes && aligned16(gamma) && aligned16(beta))
+    {
+        hipLaunchKernelGGL((skipln_interleaved_token_kernel<G, PRELN>), dim3((unsigned) ceil_div(total, kWavesPerBlock)),
+            dim3(kBlock), 0, stream, total, in, skip, beta, gamma, out, preln, dqIn, dqSkip, qScale, qSkipScale, eps,
+            prelnMin);
+        return check_launch("skipln_interleaved_token_kernel");
+    }
     // One workgroup per block of TOK tokens.  When that is a few workgroups more than the chip holds at once, the
     // stragglers of a second round cost 1.4-1.7 us whatever their number (33280 tokens x 1024 channels: 18.7 us where
     // 32736 tokens take 17.0), so when one token more per workgroup lets a single round cover the tensor the launch is

@@ -189,6 +189,15 @@ def test_skipln_interleaved_one_round_with_tail(api, variant, large, ld, total):
     test_skipln_interleaved(api, variant, large, ld, total)
 
 
+@pytest.mark.parametrize("variant,large,ld,total", [
+    # either side of the 4 MB per tensor up to which a wavefront takes one token, and a last workgroup of one wavefront
+    (0, True, 1024, 4096), (0, True, 1024, 4097), (1, False, 1536, 2730), (1, False, 1536, 2731), (1, False, 4096, 1021),
+    (1, False, 4096, 1025), (1, True, 768, 5461), (0, False, 768, 5), (1, False, 3072, 1),
+])
+def test_skipln_interleaved_few_tokens(api, variant, large, ld, total):
+    test_skipln_interleaved(api, variant, large, ld, total)
+
+
 def test_skipln_interleaved_tail_launch_replays_from_a_graph(api):
     """The one-round launch (its workgroup count comes from an occupancy query, its extra tokens travel through LDS)
     recorded in a graph: every replay gives the eager bytes."""
