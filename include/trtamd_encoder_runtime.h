@@ -123,6 +123,11 @@ typedef struct trtamd_fp16_encoder_layer
     void* attention;                                  /* IPluginV3 objects */
     void* ln1;
     void* ln2;
+    /* the parameters of ln2 again, device binary16 [hidden]: for batches of few tokens, where the normalisation adds up
+     * partial sums of ffn2 */
+    trtamd_half_t const* ln2_gamma;
+    trtamd_half_t const* ln2_beta;
+    trtamd_half_t const* ln2_bias;
 } trtamd_fp16_encoder_layer;
 
 typedef struct trtamd_fp16_encoder_config
@@ -144,6 +149,8 @@ typedef struct trtamd_fp16_encoder_batch
      * m [tokens][ffn]; emb2: the embedding plugin's second output, device int32 [1] */
     trtamd_half_t *x, *qkv, *ctx, *ao, *h, *m, *f;
     int32_t* emb2;
+    float* partial; /* device scratch for batches of few tokens, 16-byte aligned; NULL or too small: done without */
+    size_t partial_bytes; /* 2 MiB serve every such batch */
 } trtamd_fp16_encoder_batch;
 
 TRTAMD_API int trtamd_fp16_encoder_enqueue(trtamd_fp16_encoder_config const* config, trtamd_fp16_encoder_layer const* layers,

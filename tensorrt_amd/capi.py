@@ -86,7 +86,8 @@ class Fp16EncoderLinear(C.Structure):
 
 class Fp16EncoderLayer(C.Structure):
     _fields_ = [("qkv", Fp16EncoderLinear), ("proj", Fp16EncoderLinear), ("ffn1", Fp16EncoderLinear),
-                ("ffn2", Fp16EncoderLinear), ("attention", c_p), ("ln1", c_p), ("ln2", c_p)]
+                ("ffn2", Fp16EncoderLinear), ("attention", c_p), ("ln1", c_p), ("ln2", c_p), ("ln2_gamma", c_p),
+                ("ln2_beta", c_p), ("ln2_bias", c_p)]
 
 
 class Fp16EncoderConfig(C.Structure):
@@ -96,7 +97,7 @@ class Fp16EncoderConfig(C.Structure):
 class Fp16EncoderBatch(C.Structure):
     _fields_ = [("ids", c_p), ("segment_ids", c_p), ("cu_seqlens", c_p), ("batch", i32), ("tokens", i32), ("mask", c_p),
                 ("longest", c_p), ("x", c_p), ("qkv", c_p), ("ctx", c_p), ("ao", c_p), ("h", c_p), ("m", c_p), ("f", c_p),
-                ("emb2", c_p)]
+                ("emb2", c_p), ("partial", c_p), ("partial_bytes", C.c_size_t)]
 
 
 _SIGS = {

@@ -22,6 +22,7 @@
 // load unit 1 KB of contiguous memory.
 #include "device_utils.hpp"
 #include "host_utils.hpp"
+#include "network_ops.hpp"
 #include "trtamd_encoder_ops.h"
 
 #include <algorithm>
@@ -44,7 +45,8 @@ enum Epilogue
     kHALF = TRTAMD_LINEAR_AFFINE_FP16,
     // FP16 operands (trtamd_fp16_linear): the same kernels with v_mfma_f32_32x32x16_f16 and binary32 accumulators
     kF16_AFFINE = 4,
-    kF16_GELU = 5
+    kF16_GELU = 5,
+    kF16_RAW = 6 // the binary32 accumulators (partial sums of fp16_linear_partial)
 };
 
 // INT8 operands accumulate in INT32, FP16 operands in binary32.  Either way a lane feeds 16 bytes of a row per
@@ -80,6 +82,8 @@ struct LinearArgs
     int panel;     // channel tiles per panel of the tile numbering (divides the number of channel tiles)
     int persist;   // persistent kernel: workgroups that loop over the 256 x 256 tiles
     int pieces;    // direct-to-LDS kernel: the tokens behind the large tiles go in 64 x 64 pieces (see linear_piece64)
+    int parts;     // pieces: workgroups that share the k range of a piece, each with an output of its own
+    WeightPrefetch prefetch; // by the workgroups behind mainTiles of the tile and piece kernels
 };
 
 // gelu(y) = y * Phi(y) = max(y, 0) - |y| * Phi(-|y|).  log2(Phi(-a)) is smooth and nearly quadratic, so
@@ -1110,6 +1114,71 @@ __device__ __forceinline__ void linear_piece64(
     }
 }
 
+// The results of one lane for four consecutive channels (c .. c+3) of one token, packed and stored.
+template <bool IL_OUT, int EPI, typename Acc4>
+__device__ __forceinline__ void store_quad(LinearArgs const& p, Acc4 const& acc, int const c, int const t, int const part)
+{
+    if constexpr (EPI == kRAW || EPI == kF16_RAW)
+    {
+        if (t < p.T)
+        {
+            static_cast<Acc4*>(p.out)[(((size_t) part * p.T + t) * p.N + c) >> 2] = acc;
+        }
+        return;
+    }
+    f32x4 const al = *reinterpret_cast<f32x4 const*>(p.alpha + c);
+    f32x4 const be = *reinterpret_cast<f32x4 const*>(p.beta + c);
+    if (t >= p.T)
+    {
+        return;
+    }
+    if constexpr (EPI >= kF16_AFFINE)
+    {
+        f16x4 h;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+        {
+            float const y = fmaf(acc[e], al[e], be[e]);
+            h[e] = (f16) (EPI == kF16_GELU ? gelu_erf(y) : y);
+        }
+        *reinterpret_cast<f16x4*>(static_cast<f16*>(p.out) + (size_t) t * p.N + c) = h;
+    }
+    else
+    {
+        uint32_t w = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+        {
+            if constexpr (EPI == kGELU)
+            {
+                float const y = fmaf((float) acc[e], al[e], be[e]);
+                w = __builtin_amdgcn_cvt_pk_u8_f32(fmaf(gelu_erf(y), p.qOut, 128.f), e, w);
+            }
+            else
+            {
+                w = __builtin_amdgcn_cvt_pk_u8_f32(fmaf((float) acc[e], al[e], be[e] + 128.f), e, w);
+            }
+        }
+        size_t const o = IL_OUT ? ((size_t) (c >> 5) * p.T + t) * 32 + (c & 31) : (size_t) t * p.N + c;
+        *reinterpret_cast<uint32_t*>(static_cast<int8_t*>(p.out) + o) = w ^ 0x80808080u;
+    }
+}
+
+// The last `rest` stages of a ring, MOST + 1 of them at most: f is called for each with the number of stages requested
+// behind it as a constant (what its wait may leave in flight).
+template <int MOST, typename F>
+__device__ __forceinline__ void for_each_behind(int const rest, F&& f)
+{
+    if (MOST < rest)
+    {
+        f(std::integral_constant<int, MOST>{});
+    }
+    if constexpr (MOST > 0)
+    {
+        for_each_behind<MOST - 1>(rest, f);
+    }
+}
+
 // One tile of BM = WM*MT*32 channels x BN = WN*NT*32 tokens with the stages brought in by direct-to-LDS loads, for
 // launches that do not fill the chip with 256 x 256 tiles.  The LDS layout of a stage, its swizzles and its load units
 // are those of linear_tile_run_dma; a ring of RING stages, stage k + RING - 1 requested while stage k is multiplied and
@@ -1258,27 +1327,13 @@ __device__ __forceinline__ void linear_tile_dma(
         multiply(slot);
         slot = slot == RING - 1 ? 0 : slot + 1;
     }
-    int const rest = nk - k; // at most RING - 1 stages, all requested
-    auto last = [&](auto behindTag) {
-        constexpr int behind = decltype(behindTag)::value;
-        if (behind < rest)
-        {
-            wait_vmcnt<behind * kLoads>();
-            __syncthreads();
-            multiply(slot);
-            slot = slot == RING - 1 ? 0 : slot + 1;
-        }
-    };
-    static_assert(RING >= 2 && RING <= 4, "unrolled tail");
-    if constexpr (RING >= 4)
-    {
-        last(std::integral_constant<int, 2>{});
-    }
-    if constexpr (RING >= 3)
-    {
-        last(std::integral_constant<int, 1>{});
-    }
-    last(std::integral_constant<int, 0>{});
+    // at most RING - 1 stages, all requested
+    for_each_behind<RING - 2>(nk - k, [&](auto behind) {
+        wait_vmcnt<decltype(behind)::value * kLoads>();
+        __syncthreads();
+        multiply(slot);
+        slot = slot == RING - 1 ? 0 : slot + 1;
+    });
 
     bool const full = t0 + BN <= p.T; // uniform
 #pragma unroll
@@ -1345,60 +1400,49 @@ __global__ __launch_bounds__(512) void int8_linear_dma_kernel(LinearArgs const p
     }
 }
 
+// The workgroups behind the tiles of a launch: each wavefront requests 4 KB of the weights in p.prefetch, on the XCD
+// whose L2 the launch that uses them will look in (ids are dealt to the 8 XCDs in turn), waits for them and drops them.
+constexpr int kPrefetchLoads = 4; // per wavefront, 1 KB each
+
+__device__ __forceinline__ void prefetch_weights(LinearArgs const& p)
+{
+    int const lane = threadIdx.x & 63;
+    uint32_t const waves = blockDim.x >> 6;
+    uint32_t const xcd = blockIdx.x & 7u, rank = (blockIdx.x - (uint32_t) p.mainTiles) >> 3;
+    uint32_t const perXcd = p.prefetch.units / 8u;
+    uint32_t const first = (rank * waves + (threadIdx.x >> 6)) * kPrefetchLoads;
+    i32x4 v[kPrefetchLoads];
+#pragma unroll
+    for (int i = 0; i < kPrefetchLoads; ++i)
+    {
+        uint32_t const u = min(first + (uint32_t) i, perXcd - 1u);
+        uint64_t const unit = (uint64_t) u * 8u + xcd;
+        v[i] = *reinterpret_cast<i32x4 const*>(static_cast<uint8_t const*>(p.prefetch.data) + unit * 1024u + (uint32_t) lane * 16u);
+    }
+#pragma unroll
+    for (int i = 0; i < kPrefetchLoads; ++i)
+    {
+        asm volatile("" ::"v"(v[i]));
+    }
+}
+
 template <bool IL, bool IL_OUT, int EPI, int WM, int WN, int MT, int NT, int RING, int PER_SIMD>
 __global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(LinearArgs const p)
 {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[RING * (WM * MT + WN * NT) * 2 * 1024];
     __shared__ __attribute__((aligned(16))) float sScale[2 * kBigTile];
+    if ((int) blockIdx.x >= p.mainTiles)
+    {
+        prefetch_weights(p);
+        return;
+    }
     // panel numbering as for the large tiles (see int8_linear_kernel)
     uint32_t const pw = (uint32_t) p.panel;
     uint32_t const perPanel = (uint32_t) p.tokMain * pw;
-    uint32_t const tile = xcd_remap(blockIdx.x, gridDim.x);
+    uint32_t const tile = xcd_remap(blockIdx.x, (uint32_t) p.mainTiles);
     uint32_t const pan = tile / perPanel, rem = tile % perPanel;
     linear_tile_dma<IL, IL_OUT, EPI, WM, WN, MT, NT, RING>(
         p, (int) (pan * pw + rem % pw) * (WM * MT * 32), (int) (rem / pw) * (WN * NT * 32), lds, sScale);
-}
-
-// The results of one lane for four consecutive channels (c .. c+3) of one token, packed and stored.
-template <bool IL_OUT, int EPI, typename Acc4>
-__device__ __forceinline__ void store_quad(LinearArgs const& p, Acc4 const& acc, int const c, int const t)
-{
-    f32x4 const al = *reinterpret_cast<f32x4 const*>(p.alpha + c);
-    f32x4 const be = *reinterpret_cast<f32x4 const*>(p.beta + c);
-    if (t >= p.T)
-    {
-        return;
-    }
-    if constexpr (EPI >= kF16_AFFINE)
-    {
-        f16x4 h;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-        {
-            float const y = fmaf(acc[e], al[e], be[e]);
-            h[e] = (f16) (EPI == kF16_GELU ? gelu_erf(y) : y);
-        }
-        *reinterpret_cast<f16x4*>(static_cast<f16*>(p.out) + (size_t) t * p.N + c) = h;
-    }
-    else
-    {
-        uint32_t w = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-        {
-            if constexpr (EPI == kGELU)
-            {
-                float const y = fmaf((float) acc[e], al[e], be[e]);
-                w = __builtin_amdgcn_cvt_pk_u8_f32(fmaf(gelu_erf(y), p.qOut, 128.f), e, w);
-            }
-            else
-            {
-                w = __builtin_amdgcn_cvt_pk_u8_f32(fmaf((float) acc[e], al[e], be[e] + 128.f), e, w);
-            }
-        }
-        size_t const o = IL_OUT ? ((size_t) (c >> 5) * p.T + t) * 32 + (c & 31) : (size_t) t * p.N + c;
-        *reinterpret_cast<uint32_t*>(static_cast<int8_t*>(p.out) + o) = w ^ 0x80808080u;
-    }
 }
 
 // A piece of CB x TB blocks of 32 channels x 32 tokens by one workgroup whose eight wavefronts split k, for launches
@@ -1416,8 +1460,14 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(LinearArgs 
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int const row = lane & 31, half = lane >> 5;
+    if ((int) blockIdx.x >= p.mainTiles)
+    {
+        prefetch_weights(p);
+        return;
+    }
     uint32_t const nbm = (uint32_t) ceil_div(p.N, 32 * CB);
-    int const n0 = (int) (blockIdx.x % nbm) * (32 * CB), t0 = (int) (blockIdx.x / nbm) * (32 * TB);
+    int const n0 = (int) (blockIdx.x % nbm) * (32 * CB);
+    int const kpart = (int) (blockIdx.x / nbm) / p.tokMain, t0 = (int) (blockIdx.x / nbm) % p.tokMain * (32 * TB);
     uint32_t offA[CB], offB[TB];
 #pragma unroll
     for (int b = 0; b < CB; ++b)
@@ -1432,9 +1482,11 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(LinearArgs 
         offB[b] = r * 32u + (uint32_t) half * 16u;
     }
     uint32_t const slabA = (uint32_t) p.N * 32u, slabB = (uint32_t) p.T * 32u;
-    int const slabs = p.K / 32;
-    int const per = ceil_div(slabs, NW), first = wave * per;
-    int const steps = max(0, min(per, slabs - first)); // consecutive k-slabs of this wavefront
+    // this workgroup's k-slabs, and the consecutive ones of this wavefront
+    int const perPart = ceil_div(p.K / 32, p.parts);
+    int const slabs = min(p.K / 32, (kpart + 1) * perPart);
+    int const per = ceil_div(perPart, NW), first = kpart * perPart + wave * per;
+    int const steps = max(0, min(per, slabs - first));
     i32x4 fa[DEPTH][CB], fb[DEPTH][TB];
     auto fetch = [&](int slot, int step) {
         uint32_t const ks = (uint32_t) min(first + step, slabs - 1);
@@ -1520,7 +1572,7 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(LinearArgs 
         int const b = u >> 2, q = u & 3, cb = n0 + (b / TB) * 32, tb = t0 + (b % TB) * 32;
         if (cb < p.N)
         {
-            store_quad<IL_OUT, EPI>(p, t, cb + 8 * q + 4 * half, tb + row);
+            store_quad<IL_OUT, EPI>(p, t, cb + 8 * q + 4 * half, tb + row, kpart);
         }
     }
 }
@@ -1540,8 +1592,14 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int const row = lane & 31, half = lane >> 5;
+    if ((int) blockIdx.x >= p.mainTiles)
+    {
+        prefetch_weights(p);
+        return;
+    }
     uint32_t const nbm = (uint32_t) ceil_div(p.N, 32 * CB);
-    int const n0 = (int) (blockIdx.x % nbm) * (32 * CB), t0 = (int) (blockIdx.x / nbm) * (32 * TB);
+    int const n0 = (int) (blockIdx.x % nbm) * (32 * CB);
+    int const kpart = (int) (blockIdx.x / nbm) / p.tokMain, t0 = (int) (blockIdx.x / nbm) % p.tokMain * (32 * TB);
     uint8_t* const own = lds + wave * (RING * STAGE);
     uint32_t const ownBase = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) own;
     int const rr = lane >> 2;
@@ -1554,8 +1612,9 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
         int const g = u < 2 * CB ? min(n0 + r, p.N - 1) : min(t0 + r - 32 * CB, p.T - 1);
         off[u] = (uint32_t) g * (uint32_t) p.K + chunk;
     }
-    int const nk = p.K / 64;
-    int const per = ceil_div(nk, NW), first = wave * per;
+    int const perPart = ceil_div(p.K / 64, p.parts); // stages of this workgroup
+    int const nk = min(p.K / 64, (kpart + 1) * perPart);
+    int const per = ceil_div(perPart, NW), first = kpart * perPart + wave * per;
     int const steps = max(0, min(per, nk - first));
     auto fetch = [&](int step, int slot) {
         uint64_t const k = (uint64_t) (first + step) * 64u;
@@ -1626,27 +1685,12 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
         multiply(slot);
         slot = slot == RING - 1 ? 0 : slot + 1;
     }
-    int const rest = steps - k;
-    auto last = [&](auto behindTag) {
-        constexpr int behind = decltype(behindTag)::value;
-        if (behind < rest)
-        {
-            wait_vmcnt<behind * kLoads>();
-            asm volatile("" ::: "memory");
-            multiply(slot);
-            slot = slot == RING - 1 ? 0 : slot + 1;
-        }
-    };
-    static_assert(RING >= 2 && RING <= 4, "unrolled tail");
-    if constexpr (RING >= 4)
-    {
-        last(std::integral_constant<int, 2>{});
-    }
-    if constexpr (RING >= 3)
-    {
-        last(std::integral_constant<int, 1>{});
-    }
-    last(std::integral_constant<int, 0>{});
+    for_each_behind<RING - 2>(steps - k, [&](auto behind) {
+        wait_vmcnt<decltype(behind)::value * kLoads>();
+        asm volatile("" ::: "memory");
+        multiply(slot);
+        slot = slot == RING - 1 ? 0 : slot + 1;
+    });
     using Acc4 = std::conditional_t<(EPI >= kF16_AFFINE), f32x4, i32x4>;
     __builtin_amdgcn_s_waitcnt(0xC07F);
 #pragma unroll
@@ -1675,31 +1719,39 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
         int const b = u >> 2, q = u & 3, cb = n0 + (b / TB) * 32, tb = t0 + (b % TB) * 32;
         if (cb < p.N)
         {
-            store_quad<IL_OUT, EPI>(p, t, cb + 8 * q + 4 * half, tb + row);
+            store_quad<IL_OUT, EPI>(p, t, cb + 8 * q + 4 * half, tb + row, kpart);
         }
     }
 }
 
 // Which kernel a launch with operands of one layout takes: the one with the lowest estimate of
 //
-//   launch + share(x) * (tile + gelu + stage * K / 64)                    [us]
+//   launch + units(x) * (tile + gelu + stage * K / 64)                    [us]
 //
-// where x is the number of tiles per CU.  Up to `resident` tiles run on a CU at once and share it, each further one
-// costing `share` of a tile's time on its own; beyond that the CU works through them at that rate, with `tail` of a
-// tile lost at the end.  Small tiles fill the chip where the problem has few of them, large ones move fewer bytes per
-// multiplication where it has many, and the pieces cut the chain of stages by eight where neither fills it.
+// where x is the number of tiles per CU.  Up to `resident` tiles run on a CU at once and share it, each behind the first
+// costing `share` of a tile's time on its own; the ones beyond that wait their turn at `turn` each.  The CUs with the
+// most tiles decide how long the launch takes as far as `whole` says (1: entirely, 0: an even spread).  Small tiles fill the
+// chip where the problem has few of them, large ones move fewer bytes per multiplication where it has many, and the pieces
+// cut the chain of stages by eight where neither fills it.
 //
-// The constants are a fit to launches of 16 to 33289 tokens on the four layers of a 1024-channel INT8 and of a
-// 768-channel FP16 encoder (graph replays, weights from memory): every row within 5-8 %, and the choice on average
-// 1.8 % (interleaved) and 0.4 % (linear) slower than the fastest of all kernels at each of the 128 points, 12 % at
-// worst.  Before, every launch short of half a round of large tiles went in 128 x 128 tiles staged through registers:
-// 40 tokens x (1024 -> 3072 / 4096 -> 1024) INT8 7.2 / 19.1 -> 3.7 / 4.7 us, 600 tokens 7.4 / 19.0 -> 5.2 / 7.9 us,
-// 5300 tokens 20.5 / 43.0 -> 20.9 / 27.1 us; FP16 40 tokens x (768 -> 2304 / 3072 -> 768) 9.7 / 29.9 -> 4.0 / 7.2 us,
-// 9100 tokens x 3072 -> 768 80.0 -> 54.4 us.
+// The constants are a fit to launches of 16 to 33289 tokens on the four layers of a 1024-channel INT8 encoder (graph
+// replays, every launch with weights that are in no cache) and of a 768-channel FP16 one (weights in the last-level
+// cache): every row within 3-9 %, and the choice on average 0.6 % (interleaved) and 0.4 % (linear) slower than the fastest
+// of all kernels at each of the 128 points, 17 % at worst.  Before, every launch short of half a round of large tiles went
+// in 128 x 128 tiles staged through registers (weights in the last-level cache): 40 tokens x (1024 -> 3072 /
+// 4096 -> 1024) INT8 7.2 / 19.1 -> 3.7 / 4.7 us, 600 tokens 7.4 / 19.0 -> 5.2 / 7.9 us, 5300 tokens 20.5 / 43.0 -> 20.9 /
+// 27.1 us; FP16 40 tokens x (768 -> 2304 / 3072 -> 768) 9.7 / 29.9 -> 4.0 / 7.2 us, 9100 tokens x 3072 -> 768 80.0 ->
+// 54.4 us.
+// Deep rings: where one workgroup per CU is all there is, a tile is bound by the trips to memory of its own stages, and
+// the LDS of the workgroups that do not come is better used for more of them (interleaved, weights from memory, 600 tokens
+// x 4096 -> 1024 in 64 x 64 tiles: 12.9 us with three stages ahead, 9.5 us with seven; 128 x 128 tiles, 1900 tokens 20.8
+// us with two, 17.4 us with three); with two and more per CU they are slower.  Sharing the k range of such a tile between
+// groups of wavefronts instead (two or four groups, rings of their own) measured 9.9-10.4 us on the first of these and
+// lost elsewhere.  Linear operands gain 1-5 % from them and go without.
 struct TileCost
 {
     int channels, tokens, resident;
-    float launch, tile, stage, gelu, share, tail;
+    float launch, tile, stage, gelu, share, turn, whole;
 };
 enum LinearPlan
 {
@@ -1708,41 +1760,57 @@ enum LinearPlan
     kTile128x128,
     kTile64x128,
     kTile64x64,
-    kPiece64x64,
+    kTile128x128Deep, // the same tiles with a deeper ring of stages and fewer workgroups per CU
+    kTile64x128Deep,
+    kTile64x64Deep,
     kPiece32x64,
     kPiece32x32,
     kLinearPlans
 };
 // [0]: linear operands, [1]: interleaved ones.  No channels: the layout has no such kernel.
 constexpr TileCost kTileCosts[2][kLinearPlans] = {
-    {{256, 256, 1, 0.0f, 8.32f, 0.75f, 0.33f, 0.f, 0.f}, {128, 256, 2, 0.42f, 3.40f, 0.44f, 0.79f, 1.05f, 0.78f},
-        {128, 128, 2, 0.47f, 2.02f, 0.31f, 0.38f, 0.82f, 0.75f}, {64, 128, 3, 2.06f, 0.86f, 0.189f, 0.20f, 1.00f, 0.68f},
-        {64, 64, 4, 2.19f, 0.40f, 0.136f, 0.13f, 0.83f, 0.60f}, {}, {32, 64, 1, 2.90f, 0.21f, 0.071f, 0.21f, 0.f, 1.42f},
-        {32, 32, 1, 2.09f, 0.55f, 0.054f, 0.19f, 0.f, 0.77f}},
-    {{256, 256, 1, 0.13f, 4.82f, 0.70f, 3.35f, 0.f, 0.f}, {128, 256, 2, 1.11f, 1.82f, 0.39f, 1.52f, 0.77f, 0.89f},
-        {128, 128, 3, 2.16f, 0.75f, 0.23f, 0.73f, 0.74f, 0.98f}, {64, 128, 3, 2.11f, 0.37f, 0.159f, 0.33f, 0.74f, 0.78f},
-        {64, 64, 4, 2.24f, 0.23f, 0.114f, 0.19f, 0.62f, 0.66f}, {64, 64, 1, 2.69f, 0.45f, 0.074f, 0.32f, 0.f, 1.40f},
-        {32, 64, 2, 2.40f, 0.19f, 0.053f, 0.11f, 1.07f, 0.99f}, {32, 32, 4, 2.11f, 0.90f, 0.029f, 0.30f, 0.92f, 0.77f}}};
+    {{256, 256, 1, 0.00f, 8.31f, 0.750f, 0.33f, 0.f, 0.f, 0.f}, {128, 256, 2, 2.06f, 2.05f, 0.430f, 0.64f, 1.50f, 1.22f, 0.62f},
+        {128, 128, 2, 1.93f, 1.06f, 0.292f, 0.41f, 1.30f, 1.10f, 0.53f}, {64, 128, 3, 2.49f, 0.32f, 0.188f, 0.21f, 1.27f, 1.14f, 0.52f},
+        {64, 64, 4, 2.29f, 0.30f, 0.138f, 0.13f, 0.94f, 0.89f, 0.47f}, {}, {}, {},
+        {32, 64, 1, 2.88f, 0.30f, 0.071f, 0.05f, 0.57f, 1.91f, 0.80f}, {32, 32, 1, 2.38f, 0.34f, 0.053f, 0.13f, 1.48f, 1.49f, 0.68f}},
+    {{256, 256, 1, 0.00f, 3.12f, 0.780f, 2.97f, 0.f, 0.f, 0.f}, {128, 256, 2, 2.72f, 0.81f, 0.391f, 1.33f, 1.25f, 1.12f, 0.54f},
+        {128, 128, 3, 3.06f, 0.45f, 0.276f, 0.67f, 0.85f, 0.86f, 0.30f}, {64, 128, 3, 2.96f, 0.26f, 0.169f, 0.32f, 0.90f, 0.85f, 0.26f},
+        {64, 64, 4, 3.19f, 0.04f, 0.141f, 0.24f, 0.60f, 0.66f, 0.00f}, {128, 128, 2, 3.04f, 0.62f, 0.221f, 0.66f, 1.29f, 1.06f, 0.44f},
+        {64, 128, 2, 2.54f, 0.60f, 0.150f, 0.32f, 1.22f, 0.93f, 0.35f}, {64, 64, 2, 2.46f, 0.54f, 0.100f, 0.35f, 0.93f, 0.91f, 0.46f},
+        {32, 64, 2, 3.19f, 0.17f, 0.068f, 0.04f, 0.90f, 1.19f, 0.67f}, {32, 32, 4, 2.69f, 1.21f, 0.042f, 0.16f, 0.67f, 1.19f, 0.64f}}};
 
 inline float tile_time(TileCost const& c, LinearArgs const& a, bool gelu)
 {
     float const x = (float) ceil_div(a.N, c.channels) * (float) ceil_div(a.T, c.tokens) / (float) num_cus();
-    float const full = 1.f + c.share * (float) (c.resident - 1);
-    float const units = x <= (float) c.resident ? 1.f + c.share * (std::max(1.f, std::ceil(x)) - 1.f)
-                                                : full / (float) c.resident * (x + c.tail);
+    float units = 1.f;
+    if (x > 1.f)
+    {
+        float const y = c.whole * std::ceil(x) + (1.f - c.whole) * x, r = (float) c.resident;
+        units += c.share * (std::min(y, r) - 1.f) + c.turn * std::max(0.f, y - r);
+    }
     return c.launch + units * (c.tile + (gelu ? c.gelu : 0.f) + c.stage * (float) (a.K / 64));
 }
 
-// The same for the large tiles: whole rounds, then what is left (as pieces next to nothing, as 128 x 128 tiles in
-// proportion to how many there are).
-inline float large_tiles_time(TileCost const& c, bool il, LinearArgs const& a, int64_t smallTiles, bool pieces, bool gelu)
+// The same for the large tiles: whole rounds, and what is left behind them, as 64 x 64 pieces or as 128 x 128 tiles.
+inline float large_tiles_time(TileCost const& c, bool il, LinearArgs const& a, int64_t smallTiles, bool gelu)
 {
-    float const stages = (float) (a.K / 64);
-    float const rest = smallTiles == 0 ? 0.f
-        : pieces                       ? 0.3f
-                                       : (float) smallTiles / (float) num_cus()
-                * (il ? 1.25f + 0.47f * stages : 0.66f * stages);
-    return c.launch + (float) ceil_div(a.mainTiles, num_cus()) * (c.tile + (gelu ? c.gelu : 0.f) + c.stage * stages) + rest;
+    float const stages = (float) (a.K / 64), cus = (float) num_cus();
+    float const rounds = (float) ceil_div(a.mainTiles, num_cus());
+    if (!il)
+    {
+        return c.launch + rounds * (c.tile + (gelu ? c.gelu : 0.f) + c.stage * stages) + (float) smallTiles / cus * 0.66f * stages;
+    }
+    float const fill = (float) a.mainTiles / (rounds * cus); // a part of the chip is less in its own way
+    float rest = 0.f;
+    if (a.pieces)
+    {
+        rest = (float) (a.N / 64) * (float) ceil_div(a.T - a.tokMain * kBig, 64) / cus * 5.57f;
+    }
+    else if (smallTiles)
+    {
+        rest = std::ceil((float) smallTiles / cus) * (0.83f + (gelu ? 0.25f * c.gelu : 0.f) + 0.38f * stages);
+    }
+    return c.launch + rounds * (c.tile + (gelu ? c.gelu : 0.f) + c.stage * (0.75f + 0.25f * fill) * stages) + rest;
 }
 
 template <bool IL, bool IL_OUT, int EPI>
@@ -1764,10 +1832,34 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
             a.panel = w;
         }
     }
+    a.parts = std::max(a.parts, 1);
+    a.mainTiles = (int) grid * a.parts;
     auto run = [&](auto kernel, int threads) {
-        hipLaunchKernelGGL(kernel, dim3((uint32_t) grid), dim3(threads), 0, stream, a);
+        uint32_t behind = 0;
+        // only beside a launch that leaves CUs idle
+        if (a.prefetch.data && a.mainTiles <= num_cus())
+        {
+            behind = 8u * ceil_div(a.prefetch.units / 8u, (uint32_t) (threads / 64 * kPrefetchLoads));
+        }
+        hipLaunchKernelGGL(kernel, dim3((uint32_t) a.mainTiles + behind), dim3(threads), 0, stream, a);
         return check_launch("int8_linear");
     };
+    if constexpr (EPI == kRAW || EPI == kF16_RAW)
+    {
+        // partial sums: only the pieces of 32 channels share k between workgroups
+        bool const wide = plan == kPiece32x64;
+        if constexpr (IL)
+        {
+            return wide ? run(linear_piece_kernel<false, EPI, 1, 2, 4, 4>, 512) : run(linear_piece_kernel<false, EPI, 1, 1, 8, 4>, 512);
+        }
+        else
+        {
+            return wide ? run(linear_piece_dma_kernel<false, EPI, 1, 2, 3, 2>, 512)
+                        : run(linear_piece_dma_kernel<false, EPI, 1, 1, 4, 2>, 512);
+        }
+    }
+    else
+    {
     switch (plan)
     {
     case kTile128x256: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 4, 2, 2, 3, 4>, 512);
@@ -1789,7 +1881,9 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
     {
         switch (plan)
         {
-        case kPiece64x64: return run(linear_piece_kernel<IL_OUT, EPI, 2, 2, 4, 2>, 512);
+        case kTile128x128Deep: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 2, 4, 2>, 256);
+        case kTile64x128Deep: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 2, 6, 2>, 256);
+        case kTile64x64Deep: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 1, 8, 2>, 256);
         case kPiece32x64: return run(linear_piece_kernel<IL_OUT, EPI, 1, 2, 4, 4>, 512);
         case kPiece32x32: return run(linear_piece_kernel<IL_OUT, EPI, 1, 1, 8, 4>, 512);
         default: break;
@@ -1805,6 +1899,69 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
         }
     }
     return set_error(TRTAMD_STATUS_BAD_PARAM, "int8_linear: no such plan for this layout: %d", plan);
+    }
+}
+
+// The plan of a launch with operands of one layout and tokMain / mainTiles / pieces set up for the large tiles.
+template <bool IL>
+int choose_plan(LinearArgs const& a, int64_t smallTiles, bool gelu)
+{
+    bool const large = a.N % kBig == 0 && a.K % 256 == 0 && a.mainTiles > 0;
+    int plan = tuning(Tuning::kLinearPlan);
+    if (plan >= 0 && plan < kLinearPlans && kTileCosts[IL][plan].channels != 0 && (plan != kLargeTiles || large))
+    {
+        return plan;
+    }
+    // the smaller tiles read more bytes per multiplication; a network's pass runs at the chip's power limit and
+    // pays for that in the clock of the kernels around it: they have to win by more than 8 % (the pass of 128
+    // sequences as two halves against large tiles only: +1.1 % without the margin, +0.3 +- 0.5 % with it)
+    constexpr float kMargin = 1.f / 1.08f;
+    float best = large ? kMargin * large_tiles_time(kTileCosts[IL][kLargeTiles], IL, a, smallTiles, gelu)
+                       : std::numeric_limits<float>::max();
+    plan = kLargeTiles;
+    for (int q = kTile128x256; q < kLinearPlans; ++q)
+    {
+        if (kTileCosts[IL][q].channels == 0)
+        {
+            continue;
+        }
+        float const t = tile_time(kTileCosts[IL][q], a, gelu);
+        if (t < best)
+        {
+            best = t;
+            plan = q;
+        }
+    }
+    return plan;
+}
+
+// The plan of a launch too short for large tiles, for callers that want to know ahead (-1: one that may have them).
+template <bool IL>
+int small_plan(LinearArgs a, bool gelu)
+{
+    if ((int64_t) ceil_div(a.N, kBig) * (a.T / kBig) > 0 || !tuning(Tuning::kLinearPersistent) || !tuning(Tuning::kLinearDirect))
+    {
+        return -1;
+    }
+    a.mainTiles = 0;
+    return choose_plan<IL>(a, 0, gelu);
+}
+
+bool is_piece(int plan)
+{
+    return plan == kPiece32x64 || plan == kPiece32x32;
+}
+
+// Parts of a layer whose launch is `plan`: as many as bring its workgroups to one per CU, and no less than 1 KB of k for
+// each (two k-slabs per wavefront).
+int parts_of(int plan, LinearArgs const& a)
+{
+    if (plan != kPiece32x64 && plan != kPiece32x32)
+    {
+        return 1;
+    }
+    int const grid = ceil_div(a.N, 32) * ceil_div(a.T, plan == kPiece32x64 ? 64 : 32);
+    return std::max(1, std::min({kMaxLinearParts, num_cus() / grid, a.K / 1024}));
 }
 
 template <bool IL_W, bool IL_IN, bool IL_OUT, int EPI>
@@ -1853,32 +2010,7 @@ int launch_shape(hipStream_t stream, LinearArgs a)
             {
                 a.pieces = restTokens > 0 && smallTiles * 100 <= (int64_t) tuning(Tuning::kLinearPieces) * cus;
             }
-            bool const large = a.N % kBig == 0 && a.K % 256 == 0 && a.mainTiles > 0;
-            int plan = tuning(Tuning::kLinearPlan);
-            if (plan < 0 || plan >= kLinearPlans || kTileCosts[IL_W][plan].channels == 0 || (plan == kLargeTiles && !large))
-            {
-                // the smaller tiles read more bytes per multiplication; a network's pass runs at the chip's power limit and
-                // pays for that in the clock of the kernels around it: they have to win by more than 8 % (the pass of 128
-                // sequences as two halves against large tiles only: +1.1 % without the margin, +0.3 +- 0.5 % with it)
-                constexpr float kMargin = 1.f / 1.08f;
-                float best = large
-                    ? kMargin * large_tiles_time(kTileCosts[IL_W][kLargeTiles], IL_W, a, smallTiles, a.pieces != 0, gelu)
-                    : std::numeric_limits<float>::max();
-                plan = kLargeTiles;
-                for (int q = kTile128x256; q < kLinearPlans; ++q)
-                {
-                    if (kTileCosts[IL_W][q].channels == 0)
-                    {
-                        continue;
-                    }
-                    float const t = tile_time(kTileCosts[IL_W][q], a, gelu);
-                    if (t < best)
-                    {
-                        best = t;
-                        plan = q;
-                    }
-                }
-            }
+            int const plan = choose_plan<IL_W>(a, smallTiles, gelu);
             if (plan != kLargeTiles)
             {
                 return launch_plan<IL_W, IL_OUT, EPI>(stream, a, plan);
@@ -1921,9 +2053,45 @@ int launch_out(hipStream_t stream, LinearArgs const& a, int epilogue, bool ilOut
 } // namespace
 } // namespace trtamd
 
-extern "C" int trtamd_int8_linear(trtamd_stream_t stream, trtamd_int8_linear_params const* p)
+namespace trtamd
 {
-    using namespace trtamd;
+namespace
+{
+
+LinearArgs args_of(trtamd_int8_linear_params const& p)
+{
+    LinearArgs a{};
+    a.a = p.a;
+    a.w = p.w;
+    a.alpha = p.alpha;
+    a.beta = p.beta;
+    a.out = p.out;
+    a.T = p.T;
+    a.K = p.K;
+    a.N = p.N;
+    a.qOut = p.out_scale;
+    a.panel = 1;
+    return a;
+}
+
+LinearArgs args_of(trtamd_fp16_linear_params const& p)
+{
+    LinearArgs a{};
+    a.a = reinterpret_cast<int8_t const*>(p.a);
+    a.w = reinterpret_cast<int8_t const*>(p.w);
+    a.alpha = p.alpha;
+    a.beta = p.beta;
+    a.out = p.out;
+    a.T = p.T;
+    a.K = 2 * p.K;
+    a.N = p.N;
+    a.qOut = 1.f;
+    a.panel = 1;
+    return a;
+}
+
+int run_int8(trtamd_stream_t stream, trtamd_int8_linear_params const* p, WeightPrefetch const& prefetch)
+{
     if (p == nullptr || p->a == nullptr || p->w == nullptr || p->out == nullptr)
     {
         return set_error(TRTAMD_STATUS_BAD_PARAM, "int8_linear: null pointer");
@@ -1955,7 +2123,8 @@ extern "C" int trtamd_int8_linear(trtamd_stream_t stream, trtamd_int8_linear_par
     {
         return TRTAMD_STATUS_SUCCESS;
     }
-    LinearArgs a{p->a, p->w, p->alpha, p->beta, p->out, p->T, p->K, p->N, p->out_scale, 0, 0, 1, 0};
+    LinearArgs a = args_of(*p);
+    a.prefetch = prefetch;
     bool const ilOut = p->out_interleaved != 0;
     hipStream_t const st = as_stream(stream);
     if (p->w_interleaved)
@@ -1967,9 +2136,8 @@ extern "C" int trtamd_int8_linear(trtamd_stream_t stream, trtamd_int8_linear_par
                             : launch_out<false, false>(st, a, p->epilogue, ilOut);
 }
 
-extern "C" int trtamd_fp16_linear(trtamd_stream_t stream, trtamd_fp16_linear_params const* p)
+int run_fp16(trtamd_stream_t stream, trtamd_fp16_linear_params const* p)
 {
-    using namespace trtamd;
     if (p == nullptr || p->a == nullptr || p->w == nullptr || p->out == nullptr || p->alpha == nullptr
         || p->beta == nullptr)
     {
@@ -1996,9 +2164,79 @@ extern "C" int trtamd_fp16_linear(trtamd_stream_t stream, trtamd_fp16_linear_par
     {
         return TRTAMD_STATUS_SUCCESS;
     }
-    LinearArgs a{reinterpret_cast<int8_t const*>(p->a), reinterpret_cast<int8_t const*>(p->w), p->alpha, p->beta, p->out,
-        p->T, 2 * p->K, p->N, 1.f, 0, 0, 1, 0};
+    LinearArgs const a = args_of(*p);
     hipStream_t const st = as_stream(stream);
     return p->epilogue == TRTAMD_LINEAR_GELU ? launch_shape<false, false, false, kF16_GELU>(st, a)
                                              : launch_shape<false, false, false, kF16_AFFINE>(st, a);
+}
+
+// Whether operands are what the partial launches take (the public calls check the rest).
+bool interleaved(trtamd_int8_linear_params const& p)
+{
+    return p.a_interleaved && p.w_interleaved && (p.epilogue == TRTAMD_LINEAR_AFFINE || p.epilogue == TRTAMD_LINEAR_GELU);
+}
+
+} // namespace
+
+WeightPrefetch prefetch_of(trtamd_int8_linear_params const& next)
+{
+    // N: the channel blocks have to come round to the same XCD in every k-slab
+    if (!interleaved(next) || next.N % 256 != 0
+        || !is_piece(small_plan<true>(args_of(next), next.epilogue == TRTAMD_LINEAR_GELU)))
+    {
+        return {nullptr, 0};
+    }
+    return {next.w, (uint32_t) ((int64_t) next.N * next.K / 1024)};
+}
+
+int int8_linear(trtamd_stream_t stream, trtamd_int8_linear_params const& p, WeightPrefetch const& prefetch)
+{
+    return run_int8(stream, &p, prefetch);
+}
+
+int linear_parts(trtamd_int8_linear_params const& p)
+{
+    return interleaved(p) && p.epilogue == TRTAMD_LINEAR_AFFINE ? parts_of(small_plan<true>(args_of(p), false), args_of(p)) : 1;
+}
+
+int linear_parts(trtamd_fp16_linear_params const& p)
+{
+    return p.epilogue == TRTAMD_LINEAR_AFFINE ? parts_of(small_plan<false>(args_of(p), false), args_of(p)) : 1;
+}
+
+size_t linear_partial_bytes()
+{
+    return (size_t) num_cus() * 32 * 64 * sizeof(int32_t);
+}
+
+int int8_linear_partial(trtamd_stream_t stream, trtamd_int8_linear_params const& p, int parts, int32_t* partial,
+    WeightPrefetch const& prefetch)
+{
+    LinearArgs a = args_of(p);
+    int const plan = small_plan<true>(a, false);
+    a.out = partial;
+    a.parts = parts;
+    a.prefetch = prefetch;
+    return launch_plan<true, false, kRAW>(as_stream(stream), a, plan);
+}
+
+int fp16_linear_partial(trtamd_stream_t stream, trtamd_fp16_linear_params const& p, int parts, float* partial)
+{
+    LinearArgs a = args_of(p);
+    int const plan = small_plan<false>(a, false);
+    a.out = partial;
+    a.parts = parts;
+    return launch_plan<false, false, kF16_RAW>(as_stream(stream), a, plan);
+}
+
+} // namespace trtamd
+
+extern "C" int trtamd_int8_linear(trtamd_stream_t stream, trtamd_int8_linear_params const* p)
+{
+    return trtamd::run_int8(stream, p, {nullptr, 0});
+}
+
+extern "C" int trtamd_fp16_linear(trtamd_stream_t stream, trtamd_fp16_linear_params const* p)
+{
+    return trtamd::run_fp16(stream, p);
 }

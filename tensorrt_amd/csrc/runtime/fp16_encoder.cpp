@@ -5,6 +5,7 @@
 #include "trtamd_encoder_runtime.h"
 
 #include "../host_utils.hpp"
+#include "../network_ops.hpp"
 
 #include <string>
 
@@ -75,7 +76,7 @@ int enqueue(trtamd_fp16_encoder_config const& c, trtamd_fp16_encoder_layer const
         void* outputs[2] = {b.x, b.emb2};
         run(c.embedding, "embeddings", in, 4, out, 2, inputs, outputs, stream);
     }
-    auto linear = [&](trtamd_fp16_encoder_linear const& l, void const* a, void* out, int32_t K, int32_t N, int32_t epilogue) {
+    auto params = [&](trtamd_fp16_encoder_linear const& l, void const* a, void* out, int32_t K, int32_t N, int32_t epilogue) {
         trtamd_fp16_linear_params p{};
         p.a = static_cast<trtamd_half_t const*>(a);
         p.w = l.w;
@@ -86,6 +87,9 @@ int enqueue(trtamd_fp16_encoder_config const& c, trtamd_fp16_encoder_layer const
         p.K = K;
         p.N = N;
         p.epilogue = epilogue;
+        return p;
+    };
+    auto linear = [&](trtamd_fp16_linear_params const& p) {
         checkKernelStatus(trtamd_fp16_linear(stream, &p), "linear layer");
     };
     auto skipln = [&](void* plugin, void const* x, void const* skip, void* out) {
@@ -93,21 +97,40 @@ int enqueue(trtamd_fp16_encoder_config const& c, trtamd_fp16_encoder_layer const
         void const* inputs[2] = {x, skip};
         run(plugin, "skipLayerNorm", in, 2, &row, 1, inputs, &out, stream);
     };
+    // Few tokens: the second feed-forward layer, whose k loop is the longest, shares it between workgroups, and the
+    // normalisation behind it adds up the sums.
+    int parts = 1;
+    if (c.layers > 0 && c.hidden % 8 == 0 && c.hidden > 32 && c.hidden <= 1024 && layers[0].ln2_gamma && layers[0].ln2_beta
+        && layers[0].ln2_bias && b.partial && b.partial_bytes >= linear_partial_bytes())
+    {
+        parts = linear_parts(params(layers[0].ffn2, b.m, b.f, c.ffn, c.hidden, TRTAMD_LINEAR_AFFINE));
+    }
     for (int32_t i = 0; i < c.layers; ++i)
     {
         trtamd_fp16_encoder_layer const& L = layers[i];
-        linear(L.qkv, b.x, b.qkv, c.hidden, 3 * c.hidden, TRTAMD_LINEAR_AFFINE);
+        linear(params(L.qkv, b.x, b.qkv, c.hidden, 3 * c.hidden, TRTAMD_LINEAR_AFFINE));
         {
             PluginTensorDesc const in[4] = {qkvAct, tOne, tCu, tLongest};
             void const* inputs[4] = {b.qkv, b.mask, b.cu_seqlens, b.longest};
             void* outputs[1] = {b.ctx};
             run(L.attention, "attention", in, 4, &act, 1, inputs, outputs, stream);
         }
-        linear(L.proj, b.ctx, b.ao, c.hidden, c.hidden, TRTAMD_LINEAR_AFFINE);
+        linear(params(L.proj, b.ctx, b.ao, c.hidden, c.hidden, TRTAMD_LINEAR_AFFINE));
         skipln(L.ln1, b.ao, b.x, b.h);
-        linear(L.ffn1, b.h, b.m, c.hidden, c.ffn, TRTAMD_LINEAR_GELU);
-        linear(L.ffn2, b.m, b.f, c.ffn, c.hidden, TRTAMD_LINEAR_AFFINE);
-        skipln(L.ln2, b.f, b.h, b.x);
+        linear(params(L.ffn1, b.h, b.m, c.hidden, c.ffn, TRTAMD_LINEAR_GELU));
+        auto const f2 = params(L.ffn2, b.m, b.f, c.ffn, c.hidden, TRTAMD_LINEAR_AFFINE);
+        if (parts > 1)
+        {
+            checkKernelStatus(fp16_linear_partial(stream, f2, parts, b.partial), "linear layer");
+            checkKernelStatus(skip_layer_norm_fp16_from_partial(stream, c.hidden, tokens, b.partial, parts, f2.alpha, f2.beta, b.h,
+                                  L.ln2_beta, L.ln2_gamma, b.x, L.ln2_bias),
+                "skipLayerNorm");
+        }
+        else
+        {
+            linear(f2);
+            skipln(L.ln2, b.f, b.h, b.x);
+        }
     }
     return TRTAMD_STATUS_SUCCESS;
 }

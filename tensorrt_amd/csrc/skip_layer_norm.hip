@@ -11,6 +11,7 @@
 // plugin/skipLayerNormPlugin/skipLayerNormInt8InterleavedKernelMTron.cu of the reference.
 #include "device_utils.hpp"
 #include "host_utils.hpp"
+#include "network_ops.hpp"
 
 #include <cstdlib>
 
@@ -269,6 +270,117 @@ int skip_layer_norm(hipStream_t stream, int32_t ld, int64_t n, T const* in, T co
             gamma, bias, out, eps);
     }
     return check_launch("skipln_generic_kernel");
+}
+
+// The output of an affine linear layer as the partial sums of its accumulators (network_ops.hpp).
+template <typename Acc>
+struct PartialSums
+{
+    Acc const* sums; // [parts][rows][ld]
+    int parts;
+    float const* alpha;
+    float const* beta;
+};
+
+// The same rows (binary16, one per wavefront) behind a linear layer that left partial sums: its output is formed here as
+// that layer's epilogue forms it, f16(fmaf(sum, alpha, beta)), and never stored.  ld a multiple of 8, at most 1024.
+template <int NV>
+__global__ __launch_bounds__(kBlock) void skipln_rows_partial_kernel(int const ld, int const rows,
+    PartialSums<float> const sums, f16 const* __restrict__ skip, f16 const* __restrict__ beta, f16 const* __restrict__ gamma,
+    f16 const* __restrict__ bias, f16* __restrict__ out, float const eps)
+{
+    int const lane = threadIdx.x & (kWaveSize - 1);
+    int const row = (int) blockIdx.x * kWavesPerBlock + (int) (threadIdx.x >> 6);
+    if (row >= rows)
+    {
+        return;
+    }
+    int const nvec = ld / 8;
+    f32x4 x[NV][2];
+    Vec16<f16> xs[NV], g[NV], b[NV], bs[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+    {
+        int const vi = lane + kWaveSize * j;
+        bool const ok = vi < nvec;
+        int const c = ok ? vi * 8 : 0;
+        f32x4 v[kMaxLinearParts][2];
+#pragma unroll
+        for (int s = 0; s < kMaxLinearParts; ++s)
+        {
+            float const* src = sums.sums + ((int64_t) min(s, sums.parts - 1) * rows + row) * ld + c;
+            v[s][0] = *reinterpret_cast<f32x4 const*>(src);
+            v[s][1] = *reinterpret_cast<f32x4 const*>(src + 4);
+        }
+        xs[j].u = ok ? *reinterpret_cast<u32x4 const*>(skip + (int64_t) row * ld + c) : u32x4{0, 0, 0, 0};
+        g[j].u = ok ? *reinterpret_cast<u32x4 const*>(gamma + c) : u32x4{0, 0, 0, 0};
+        b[j].u = ok ? *reinterpret_cast<u32x4 const*>(beta + c) : u32x4{0, 0, 0, 0};
+        bs[j].u = ok ? *reinterpret_cast<u32x4 const*>(bias + c) : u32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+        {
+            x[j][h] = v[0][h];
+#pragma unroll
+            for (int s = 1; s < kMaxLinearParts; ++s)
+            {
+                x[j][h] += s < sums.parts ? v[s][h] : f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+            f32x4 const al = *reinterpret_cast<f32x4 const*>(sums.alpha + c + 4 * h);
+            f32x4 const be = *reinterpret_cast<f32x4 const*>(sums.beta + c + 4 * h);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+            {
+                x[j][h][e] = ok ? fmaf(x[j][h][e], al[e], be[e]) : 0.f;
+            }
+        }
+    }
+    float v[NV][8];
+    float sum = 0.f, cnt = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+    {
+        bool const ok = lane + kWaveSize * j < nvec;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+        {
+            f16 const t = ((f16) x[j][k >> 2][k & 3] + xs[j].e[k]) + bs[j].e[k];
+            v[j][k] = (float) t;
+            sum += ok ? v[j][k] : 0.f;
+        }
+        cnt += ok ? 8.f : 0.f;
+    }
+    Welford w;
+    w.n = cnt;
+    w.mean = cnt > 0.f ? sum / cnt : 0.f;
+    w.m2 = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+    {
+        bool const ok = lane + kWaveSize * j < nvec;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+        {
+            float const dlt = v[j][k] - w.mean;
+            w.m2 += ok ? dlt * dlt : 0.f;
+        }
+    }
+    w = group_welford<kWaveSize>(w);
+    float const rsigma = rsqrtf(w.m2 * (1.f / (float) ld) + eps);
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+    {
+        int const vi = lane + kWaveSize * j;
+        if (vi < nvec)
+        {
+            Vec16<f16> y;
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+            {
+                y.e[k] = (f16) ((float) g[j].e[k] * (v[j][k] - w.mean) * rsigma + (float) b[j].e[k]);
+            }
+            store_through_l2(out + (int64_t) row * ld + vi * 8, y.u);
+        }
+    }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -827,6 +939,89 @@ __global__ __launch_bounds__(kBlock) void skipln_interleaved_token_kernel(int co
     }
 }
 
+// The same behind an affine INT8 layer that left the partial sums of its accumulators: its output is formed here as that
+// layer's epilogue forms it and never stored.  A workgroup per token and a thread per four channels, so that the sums of
+// all parts, 16 bytes per thread each, are one trip to memory; with a wavefront per token and 16 channels per lane as above
+// the launch took 4.7 us at 32 tokens and four parts.
+template <int G>
+__global__ __launch_bounds__(G * 8) void skipln_interleaved_sums_kernel(int const total, PartialSums<int32_t> const sums,
+    int8_t const* __restrict__ skip, f16 const* __restrict__ beta, f16 const* __restrict__ gamma, int8_t* __restrict__ out,
+    float const dqIn, float const dqSkip, float const qScale, float const eps)
+{
+    constexpr int LD = G * 32, WAVES = G / 8;
+    __shared__ int sStat[WAVES][5];
+    int const token = (int) blockIdx.x;
+    int const wave = (int) (threadIdx.x >> 6);
+    int const ch = (int) threadIdx.x * 4;
+    int64_t const off = ((int64_t) (ch >> 5) * total + token) * 32 + (ch & 31);
+    i32x4 v[kMaxLinearParts];
+#pragma unroll
+    for (int s = 0; s < kMaxLinearParts; ++s)
+    {
+        // a part that does not exist re-reads the last one
+        v[s] = *reinterpret_cast<i32x4 const*>(sums.sums + ((int64_t) min(s, sums.parts - 1) * total + token) * LD + ch);
+    }
+    uint32_t const xs = *reinterpret_cast<uint32_t const*>(skip + off);
+    f32x4 const al = *reinterpret_cast<f32x4 const*>(sums.alpha + ch);
+    f32x4 const be = *reinterpret_cast<f32x4 const*>(sums.beta + ch);
+    f16x4 const g = *reinterpret_cast<f16x4 const*>(gamma + ch);
+    f16x4 const b = *reinterpret_cast<f16x4 const*>(beta + ch);
+    i32x4 acc = v[0];
+#pragma unroll
+    for (int s = 1; s < kMaxLinearParts; ++s)
+    {
+        acc += s < sums.parts ? v[s] : i32x4{0, 0, 0, 0};
+    }
+    uint32_t xi = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+    {
+        xi = __builtin_amdgcn_cvt_pk_u8_f32(fmaf((float) acc[e], al[e], be[e] + 128.f), e, xi);
+    }
+    xi ^= 0x80808080u;
+    int sIn = wave_sum_i32(__builtin_amdgcn_sdot4((int) xi, 0x01010101, 0, false));
+    int sSk = wave_sum_i32(__builtin_amdgcn_sdot4((int) xs, 0x01010101, 0, false));
+    int sII = wave_sum_i32(__builtin_amdgcn_sdot4((int) xi, (int) xi, 0, false));
+    int sIS = wave_sum_i32(__builtin_amdgcn_sdot4((int) xi, (int) xs, 0, false));
+    int sSS = wave_sum_i32(__builtin_amdgcn_sdot4((int) xs, (int) xs, 0, false));
+    if ((threadIdx.x & (kWaveSize - 1)) == 0)
+    {
+        sStat[wave][0] = sIn;
+        sStat[wave][1] = sSk;
+        sStat[wave][2] = sII;
+        sStat[wave][3] = sIS;
+        sStat[wave][4] = sSS;
+    }
+    __syncthreads();
+    sIn = sSk = sII = sIS = sSS = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+    {
+        sIn += sStat[w][0];
+        sSk += sStat[w][1];
+        sII += sStat[w][2];
+        sIS += sStat[w][3];
+        sSS += sStat[w][4];
+    }
+    double const dIn = (double) dqIn, dSk = (double) dqSkip;
+    double const mean = (dIn * sIn + dSk * sSk) * (1.0 / LD);
+    double const ex2 = (dIn * dIn * sII + 2.0 * dIn * dSk * sIS + dSk * dSk * sSS) * (1.0 / LD);
+    float const rsigma = rsqrtf(fmaxf((float) (ex2 - mean * mean), 0.f) + eps);
+    float const a1 = dqIn * rsigma;
+    float const a2 = dqSkip * rsigma;
+    float const c1 = (float) (-mean * (double) rsigma);
+    uint32_t yw = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+    {
+        float const gq = (float) g[k] * qScale;
+        float const bq = (float) b[k] * qScale + 128.f;
+        float const nrm = fmaf(i8_to_f32(xi, k), a1, fmaf(i8_to_f32(xs, k), a2, c1));
+        yw = __builtin_amdgcn_cvt_pk_u8_f32(fmaf(gq, nrm, bq), k, yw);
+    }
+    *reinterpret_cast<uint32_t*>(out + off) = yw ^ 0x80808080u;
+}
+
 // Workgroups of this kernel that the current device holds at once (asked once per process and kernel; 0 when it
 // cannot be asked).
 template <int G, int W, int TOK, bool PRELN, bool TAIL>
@@ -858,9 +1053,9 @@ int launch_interleaved_as(hipStream_t stream, int32_t total, int8_t const* in, i
     constexpr int64_t kFewBytes = 4 << 20;
     if ((int64_t) total * (G * 32) <= kFewBytes && aligned16(gamma) && aligned16(beta))
     {
-        hipLaunchKernelGGL((skipln_interleaved_token_kernel<G, PRELN>), dim3((unsigned) ceil_div(total, kWavesPerBlock)),
-            dim3(kBlock), 0, stream, total, in, skip, beta, gamma, out, preln, dqIn, dqSkip, qScale, qSkipScale, eps,
-            prelnMin);
+        hipLaunchKernelGGL((skipln_interleaved_token_kernel<G, PRELN>),
+            dim3((unsigned) ceil_div(total, kWavesPerBlock)), dim3(kBlock), 0, stream, total, in, skip, beta, gamma, out, preln,
+            dqIn, dqSkip, qScale, qSkipScale, eps, prelnMin);
         return check_launch("skipln_interleaved_token_kernel");
     }
     // One workgroup per block of TOK tokens.  When that is a few workgroups more than the chip holds at once, the
@@ -947,6 +1142,45 @@ int skipln_interleaved(hipStream_t stream, bool large, bool mtron, int32_t ld, i
 }
 
 } // namespace
+
+int skipln_interleaved_from_partial(trtamd_stream_t stream, bool large, int32_t ld, int32_t total, int32_t const* partial,
+    int parts, float const* alpha, float const* beta, int8_t const* skip, trtamd_half_t const* lnBeta,
+    trtamd_half_t const* lnGamma, int8_t* output, float dqScaleIn, float dqScaleSkip, float qScale)
+{
+    if ((ld != 768 && ld != 1024) || total <= 0 || parts < 1 || parts > kMaxLinearParts || !aligned16(lnBeta) || !aligned16(lnGamma))
+    {
+        return set_error(TRTAMD_STATUS_NOT_SUPPORTED, "SkipLayerNorm from partial sums: unsupported problem");
+    }
+    PartialSums<int32_t> const sums{partial, parts, alpha, beta};
+    float const eps = large ? 1.1920928955078125e-07f : 0.0009765625f;
+    auto const launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned) total), dim3((unsigned) ld / 4), 0, as_stream(stream), total, sums, skip,
+            reinterpret_cast<f16 const*>(lnBeta), reinterpret_cast<f16 const*>(lnGamma), output, dqScaleIn, dqScaleSkip, qScale,
+            eps);
+        return check_launch("skipln_interleaved_sums_kernel");
+    };
+    return ld == 768 ? launch(skipln_interleaved_sums_kernel<24>) : launch(skipln_interleaved_sums_kernel<32>);
+}
+
+int skip_layer_norm_fp16_from_partial(trtamd_stream_t stream, int32_t ld, int32_t rows, float const* partial, int parts,
+    float const* alpha, float const* beta, trtamd_half_t const* skip, trtamd_half_t const* lnBeta,
+    trtamd_half_t const* lnGamma, trtamd_half_t* output, trtamd_half_t const* bias)
+{
+    if (ld % 8 != 0 || ld > 1024 || rows <= 0 || parts < 1 || parts > kMaxLinearParts || !bias)
+    {
+        return set_error(TRTAMD_STATUS_NOT_SUPPORTED, "SkipLayerNorm from partial sums: unsupported problem");
+    }
+    PartialSums<float> const sums{partial, parts, alpha, beta};
+    float const eps = (ld == 768 || ld == 1024) ? 0.0009765625f : 0.f; // as skip_layer_norm
+    auto const half = [](trtamd_half_t const* x) { return reinterpret_cast<f16 const*>(x); };
+    auto const launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned) ceil_div(rows, kWavesPerBlock)), dim3(kBlock), 0, as_stream(stream), ld, rows,
+            sums, half(skip), half(lnBeta), half(lnGamma), half(bias), reinterpret_cast<f16*>(output), eps);
+        return check_launch("skipln_rows_partial_kernel");
+    };
+    return ld <= 512 ? launch(skipln_rows_partial_kernel<1>) : launch(skipln_rows_partial_kernel<2>);
+}
+
 } // namespace trtamd
 
 using namespace trtamd;

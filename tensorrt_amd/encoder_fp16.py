@@ -154,7 +154,11 @@ class Fp16BertEncoder:
                 lin = L[name]
                 setattr(d, name, capi.Fp16EncoderLinear(lin.w.data_ptr(), lin.alpha.data_ptr(), lin.beta.data_ptr()))
             d.attention, d.ln1, d.ln2 = L["attention"].handle, L["ln1"].handle, L["ln2"].handle
-        return config, layers, capi.Fp16EncoderBatch()
+            for name in ("ln2_gamma", "ln2_beta", "ln2_bias"):
+                L[name + "_dev"] = self.torch.from_numpy(L[name].astype(np.float16)).cuda()
+                setattr(d, name, L[name + "_dev"].data_ptr())
+        self._partial = self.torch.empty((2 << 20,), dtype=self.torch.uint8, device="cuda")
+        return config, layers, capi.Fp16EncoderBatch(partial=self._partial.data_ptr(), partial_bytes=2 << 20)
 
     def _bind(self, ids: np.ndarray, segs: np.ndarray, cu: np.ndarray):
         torch, cfg = self.torch, self.cfg

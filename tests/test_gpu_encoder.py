@@ -171,6 +171,25 @@ def test_native_runner_matches_the_python_chain(setup):
     enc.enqueue(ids, segs, cu)   # leave the fixture's buffers as the other tests expect them
 
 
+@pytest.mark.parametrize("lens", [[1], [31], [32], [33], [40, 24], [64, 1], [97], [128, 2], [257, 1, 3]])
+def test_native_runner_with_few_tokens(setup, lens):
+    """Batches of few tokens take launches of their own in the runner (the second feed-forward layer as partial sums that
+    the normalisation adds up, weights fetched ahead): the bytes of the chain of single operations, on both sides of the
+    token counts where the pieces and the number of parts change."""
+    import torch
+    cfg, enc, ids, segs, cu, cap, out = setup
+    r = rng(31 + sum(lens))
+    c = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    t = int(c[-1])
+    i, s = r.integers(0, cfg.vocab, t).astype(np.int32), r.integers(0, 2, t).astype(np.int32)
+    want = enc.enqueue(i, s, c).cpu().numpy()
+    for _ in range(2):
+        got = enc.enqueue_native(i, s, c)
+        torch.cuda.synchronize()
+        assert np.array_equal(got.cpu().numpy(), want)
+    enc.enqueue(ids, segs, cu)   # leave the fixture's buffers as the other tests expect them
+
+
 def test_native_runner_replays_from_a_captured_graph(setup):
     """enqueue launches kernels only (no allocation, copy, memset or synchronisation), so a caller can record it
     into a graph.  Every replay is checked, with eager work on the same buffers between the replays."""

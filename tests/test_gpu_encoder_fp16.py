@@ -70,3 +70,20 @@ def test_output_is_finite_and_repeatable(setup):
     again = enc.enqueue()
     torch.cuda.synchronize()
     assert np.array_equal(again.cpu().numpy().view(np.uint16), out.view(np.uint16))
+
+
+@pytest.mark.parametrize("lens", [[1], [31], [33], [64, 1], [97], [128, 2], [257, 1, 3]])
+def test_few_tokens_against_single_operations(setup, lens):
+    """The native pass with few tokens (partial sums of the second feed-forward layer, added up in the normalisation)
+    against the same network one operation at a time: the order of binary32 sums is all that differs."""
+    import torch
+    cfg, enc, ids, segs, cu, cap, out = setup
+    r = rng(41 + sum(lens))
+    c = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    t = int(c[-1])
+    i, s = r.integers(0, cfg.vocab, t).astype(np.int32), r.integers(0, 2, t).astype(np.int32)
+    want = enc.enqueue(i, s, c, capture={}).cpu().numpy()
+    got = enc.enqueue(i, s, c)
+    torch.cuda.synchronize()
+    assert_fp_close(got.cpu().numpy(), want, atol=1e-2, what="native pass")   # a few binary16 steps of values up to ~4
+    enc.enqueue(ids, segs, cu)

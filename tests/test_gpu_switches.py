@@ -85,7 +85,7 @@ def test_linear_variants(name, value, il):
         assert np.array_equal(got, default), f"{name}={value}: bytes differ from the default kernel choice"
 
 
-@pytest.mark.parametrize("plan", range(1, 8))
+@pytest.mark.parametrize("plan", range(1, 10))
 @pytest.mark.parametrize("T,K,N", [(1, 64, 32), (33, 192, 96), (130, 448, 160), (259, 768, 288)])
 def test_linear_plans(plan, T, K, N):
     """Every tile shape of the linear layers at the edges of its tiles (one token, one past a block, channels and k that
