@@ -1041,7 +1041,9 @@ __global__ __launch_bounds__(kBlock, 2) void attention_two_pass_kernel(int const
     Frag ringK[D][NP];
 
     // ---- first pass: row maximum and sum of exponentials -------------------------------------------------------
-    float mx = -3.0e38f, sum = 0.f;
+    // a lane that meets no valid key keeps this maximum, which is above the score of a masked key: at an equal one the
+    // fma below would leave the rounding error of the product, some 1e30, and its exponential can be infinite
+    float mx = -2.9e38f, sum = 0.f;
 #pragma unroll
     for (int u = 0; u < D; ++u)
     {
