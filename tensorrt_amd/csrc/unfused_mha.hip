@@ -8,6 +8,7 @@
 // zeroPadding2d (plugin/bertQKVToContextPlugin/zeroPadding2d.cu) of the reference.
 #include "device_utils.hpp"
 #include "host_utils.hpp"
+#include "unfused_mha.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -478,8 +479,8 @@ int can_vectorise(T const* base, GemmOperand const& o)
 }
 
 // ------------------------------------------------------------------------------------------
-// The same attention in one launch, for sequences whose scores fit in registers (S <= 512, head size <= 128): no
-// score matrix goes to memory.  A workgroup of four wavefronts owns 64 queries of one (batch, head), a wavefront 16
+// The same attention in one launch, for sequences whose scores fit in registers (S <= 512, head size <= 128) and that
+// attention_split_keys (binary32) does not take: no score matrix goes to memory.  A workgroup of four wavefronts owns 64 queries of one (batch, head), a wavefront 16
 // of them with ALL their keys, so the row maximum and sum need no exchange between wavefronts.  The matrix products
 // are computed transposed, S^T = K Q^T and O^T = V^T P^T, with the 16 x 16 MFMA tiles: a lane then holds, for its
 // one query, four consecutive keys per tile — the softmax reductions run inside the lane (plus two lane exchanges),
@@ -1243,6 +1244,15 @@ int launch_attention_in_registers(hipStream_t stream, int32_t S, int32_t B, int3
     // 16-byte reads of a row's pieces: every row of Q, K and V starts at a multiple of d elements from the base
     int const vecIn = d % V == 0 && (reinterpret_cast<uintptr_t>(qkv) & 15u) == 0;
     int const vecOut = d % 4 == 0 && (reinterpret_cast<uintptr_t>(output) & (4 * sizeof(T) - 1)) == 0;
+    if constexpr (sizeof(T) == 4)
+    {
+        // 1.8 times as fast in the mean over S = 20 .. 1000, one sequence up to 8192 tokens, head sizes 32 .. 80 (0.94 to 6
+        // times; the slower end is S = 64 without a mask in a full grid, where the strips below have no idle rows)
+        if (attention_split_keys_takes(S, B, N, d, qkv, output))
+        {
+            return attention_split_keys(stream, S, B, N, d, qkv, maskIdx, output);
+        }
+    }
     float const w = 1.f / sqrtf((float) d);
     dim3 const grid((unsigned) groups), block(kBlock);
     int const tiles = ceil_div(S, 16);

@@ -315,7 +315,7 @@ def config_rows(api, torch, steps: int = 100, seed: int = 1, cpu: bool = True, l
                note="every query row of the S x B tensor is computed; ops count valid lengths only")
 
     # ---- unfused attention (FP32, other head sizes, S > 512) ------------------------------------------
-    # head sizes up to 128: one launch, a query's scores in registers up to S = 512 and two passes over the keys beyond
+    # head sizes up to 128: one launch, a query's scores in registers up to S = 512 (FP32: 1024) and two passes over the keys beyond
     # (larger head sizes: two MFMA GEMMs around a softmax with the S x S scores in the workspace)
     for dt, tname, type_id, peak in ((np.float16, "fp16", 1, PEAK_F16), (np.float32, "fp32", 0, PEAK_F32_MFMA)):
         for S, B, N, d in ((128, 32, 12, 64), (384, 32, 12, 64), (1024, 4, 12, 64)):
@@ -325,9 +325,10 @@ def config_rows(api, torch, steps: int = 100, seed: int = 1, cpu: bool = True, l
             ws = torch.empty((api.unfused_mha_workspace_size(type_id, S, B, N),), dtype=torch.uint8, device="cuda")
             t = timeit(lambda: api.check(api.unfused_mha(stream, type_id, S, B, N, d, qkv.data_ptr(), 0,
                                                          out.data_ptr(), ws.data_ptr())))
-            one = S <= 512
+            one = S <= 512 or dt == np.float32
             report("C3 shape, unfused path",
-                   "QKV-to-context v4 (attention_in_registers_kernel)" if one
+                   "QKV-to-context v4 (attention_split_keys_kernel)" if dt == np.float32
+                   else "QKV-to-context v4 (attention_in_registers_kernel)" if one
                    else "QKV-to-context v4 (attention_two_pass_kernel)", tname,
                    f"S={S} B={B} N={N} d={d}, all keys", t, ops=4.0 * d * N * B * S * S, peak_ops=peak,
                    note="one launch, scores in registers" if one else "one launch, two passes over the keys")

@@ -180,6 +180,19 @@ def test_unfused_mha_batch_without_valid_keys(api, dt, S):
     ref = oracle.mha_unfused_fixed(qkv, S, B, N, d, np.array([0, S, S // 2], np.int32))
     assert_fp_close(got, ref, what="vs oracle", **(dict(atol=2e-5, rtol=1e-4) if dt == np.float32 else {}))
 
+@pytest.mark.parametrize("d", [32, 48, 64, 80, 96, 112, 128])
+@pytest.mark.parametrize("S", [15, 16, 17, 63, 65, 256, 257, 512, 513, 1024, 1025])
+def test_fp32_keys_split_between_wavefronts(api, S, d):
+    """The edges of the tiles of 16 queries and keys (the last one starts 16 rows before the end), of the scores a
+    wavefront keeps (256 and 512 keys) and of the lengths that the kernel takes, for each head size that it takes."""
+    B, N = 5, 2
+    r = rng(870 + S + d)
+    qkv = r.standard_normal((S, B, 3 * N * d)).astype(np.float32)
+    lens = np.array([S, 0, 1, min(S, 17), S - 1], np.int32)
+    got = _run_unfused(api, np.float32, S, B, N, d, qkv, lens)
+    assert not got[:, 1].any()
+    assert_fp_close(got, oracle.mha_unfused_fixed(qkv, S, B, N, d, lens), atol=2e-5, rtol=1e-4, what="vs oracle")
+
 
 def test_unfused_mha_unaligned_operands(api):
     """Operands that start 2 bytes off a 16-byte boundary take the element-wise loads and stores."""
