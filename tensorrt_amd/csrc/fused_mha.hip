@@ -28,6 +28,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 #include <mutex>
 #include <vector>
 
@@ -38,7 +39,8 @@ namespace
 
 constexpr int kQPerWave = 16;
 constexpr int kWavesI8 = 4;
-constexpr int kWavesF16 = 8; // FP16 K/V take twice the LDS, so one (larger) workgroup per CU
+constexpr int kWavesF16 = 8;  // FP16 K/V take twice the LDS, so one (larger) workgroup per CU
+constexpr int kWavesF16T = 4; // where K and V take turns in LDS
 constexpr int kHeadSize = 64;
 constexpr int kMagicBits = 0x4B400000;         // bit pattern of 12582912.f = 1.5 * 2^23
 constexpr float kMagic = 12582912.f;
@@ -1337,7 +1339,8 @@ __global__ __launch_bounds__(kWavesF16* kWaveSize) void fmha_f16_kernel(FmhaArgs
 }
 
 // ------------------------------------------------------------------------------------------
-// FP16, prefix-valid keys: same specialisation on the number of 64-key blocks as the INT8 kernel.
+// FP16, prefix-valid keys, many units of more than 384: same specialisation on the number of 64-key blocks as the INT8
+// kernel.  K and V of a unit are staged once for all of its queries, at one workgroup of eight wavefronts per CU.
 // ------------------------------------------------------------------------------------------
 
 template <int KT>
@@ -1639,6 +1642,311 @@ __global__ __launch_bounds__(kWavesF16* kWaveSize) void fmha_f16_prefix_kernel(F
 }
 
 // ------------------------------------------------------------------------------------------
+// FP16, prefix-valid keys, up to 384 of them (or few units): the same specialisation, but K and V take turns in LDS, one
+// block of V in the place of each block of K as soon as every wavefront has multiplied it.  48 KB for 384 keys instead of
+// 96 KB: three workgroups of four wavefronts share a CU, so that one computes while another waits for its sequence, its K
+// or its V, and a unit's queries are shared out 64 at a time over as many workgroups.  What bounds either kernel is that
+// wait; with one workgroup per CU nothing covered it.  All of Q, K and V come by direct-to-LDS loads, whose number in
+// flight the waits below count; a wavefront requests 16 rows of every block.  12 heads, sequences of a third of the length
+// to the length, before and after: 32 x 128 keys 12.9 -> 5.8 us, 128 x 256 42.8 -> 35.7 us, 32 x 384 20.7 -> 20.1 us,
+// 128 x 384 71.5 -> 64.8 us.
+// ------------------------------------------------------------------------------------------
+constexpr int kQueriesF16 = kWavesF16T * kQPerWave;
+
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void for_each_block(F&& f)
+{
+    if constexpr (I < N)
+    {
+        f(std::integral_constant<int, I>{});
+        for_each_block<N, I + 1>(f);
+    }
+}
+
+template <int NKB, bool DEBUG>
+__device__ __forceinline__ void attend_f16_turns(
+    FmhaArgs const& a, SeqInfo const& sq, int const b, int const n, int const q0, uint8_t* const lds)
+{
+    constexpr int kRow = Lds<2>::kRow;
+    constexpr int kBlock = 64 * kRow;
+    constexpr int NT = NKB * 4;
+    int const lane = threadIdx.x & (kWaveSize - 1);
+    int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int const lq = lane & 15;
+    int const g = lane >> 4;
+    uint32_t const ldsBase = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) lds;
+    uint8_t const* const unit = static_cast<uint8_t const*>(a.qkv) + sq.seqBaseIn + (int64_t) n * 3 * kRow;
+    uint32_t const stride = (uint32_t) a.tokStrideIn;
+
+    // 16 rows of matrix `mat` from `row` on (unless complete, those at or behind `limit` as the last one) into the LDS
+    // rows from `to` on
+    int const r8 = lane >> 3;
+    uint32_t const chunk = (uint32_t) (((lane & 7) ^ r8) * 16); // the swizzle of swz<2>, on the source side
+    uint32_t const whole = (uint32_t) r8 * stride + chunk;
+    auto request = [&](int mat, int row, int limit, int to, bool complete) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+        {
+            int const first = complete ? row + 8 * i : min(row + 8 * i, limit - 1);
+            uint32_t off = whole;
+            if (!complete && first + 8 > limit)
+            {
+                off = (uint32_t) min(r8, limit - 1 - first) * stride + chunk;
+            }
+            load_to_lds16_sbase(unit + (int64_t) first * a.tokStrideIn + mat * kRow, off, ldsBase + (to + 8 * i) * kRow);
+        }
+    };
+    auto request_block = [&](int mat, int kb) { request(mat, kb * 64 + wave * 16, sq.nk, kb * 64 + wave * 16, kb < NKB - 1); };
+
+    int const qw = q0 + wave * kQPerWave; // this wavefront's first query
+    bool const active = qw < sq.nq;       // if not, it only brings in its rows
+    // Q passes through the place of this wavefront's rows of the last block
+    int const qRow = (NKB - 1) * 64 + wave * 16;
+    request(0, qw, sq.nq, qRow, false);
+#pragma unroll
+    for (int kb = 0; kb < NKB - 1; ++kb)
+    {
+        request_block(1, kb);
+    }
+    wait_vmcnt<2 * (NKB - 1)>();
+    f16x8 qreg[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+    {
+        qreg[h] = *reinterpret_cast<f16x8 const*>(lds + (qRow + lq) * kRow + swz<2>(lq, h * 4 + g) * 16);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(qreg[0]), "+v"(qreg[1])::"memory"); // read before it is overwritten
+    request_block(1, NKB - 1);
+
+    int const lastKeys = sq.nk - (NKB - 1) * 64;
+    int const lastHalves = (lastKeys + 31) >> 5;   // 32-key halves of the last block that hold keys
+    int const lastRel = lastKeys - 4 * g;          // key 16u + j of this lane group exists iff 16u + j < lastRel
+
+    // ---- S^T = K Q^T (binary32 accumulation); absent keys start from -infinity
+    f32x4 acc[NT];
+    auto scores = [&](auto block) {
+        constexpr int kb = decltype(block)::value;
+        // in flight behind block kb: the later blocks of K and V of the blocks before kb - 1
+        wait_vmcnt<2 * (NKB - 1 - kb + (kb > 0 ? kb - 1 : 0))>();
+        __syncthreads(); // everybody's rows of block kb have landed, and everybody has read block kb - 1
+        if constexpr (kb > 0)
+        {
+            request_block(2, kb - 1);
+        }
+        if (active)
+        {
+#pragma unroll
+            for (int t = kb * 4; t < kb * 4 + 4; ++t)
+            {
+                int const key = t * 16 + lq;
+                f32x4 sd = {0.f, 0.f, 0.f, 0.f};
+                if (kb == NKB - 1 && 16 * (t & 3) + 16 > lastKeys) // uniform: a tile that is not all there
+                {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                    {
+                        sd[j] = (16 * (t & 3) + j) < lastRel ? 0.f : -__builtin_inff();
+                    }
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                {
+                    f16x8 const kreg = *reinterpret_cast<f16x8 const*>(lds + key * kRow + swz<2>(key, h * 4 + g) * 16);
+                    sd = attention_mfma_f16(kreg, qreg[h], sd);
+                }
+                acc[t] = sd;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for_each_block<NKB>(scores);
+    __syncthreads();
+    request_block(2, NKB - 1);
+
+    int const q = qw + lq;
+    bool const qValid = q < sq.nq;
+    if (DEBUG && a.dbgAcc1 && qValid)
+    {
+        for (int t = 0; t < NT; ++t)
+        {
+            for (int j = 0; j < 4; ++j)
+            {
+                int const key = t * 16 + g * 4 + j;
+                if (key < sq.nk)
+                {
+                    a.dbgAcc1[(((int64_t) b * a.N + n) * a.S + q) * a.S + key] = __float_as_int(acc[t][j]);
+                }
+            }
+        }
+    }
+
+    // ---- row max
+    float negK0 = 0.f;
+    __builtin_amdgcn_sched_barrier(0);
+    if (active)
+    {
+        float mxA = -__builtin_inff(), mxB = -__builtin_inff();
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+        {
+            mxA = fmaxf(fmaxf(mxA, acc[t][0]), acc[t][1]);
+            mxB = fmaxf(fmaxf(mxB, acc[t][2]), acc[t][3]);
+        }
+        float mx = fmaxf(mxA, mxB);
+        mx = reduce_step<16>(mx, [](float x, float y) { return fmaxf(x, y); });
+        mx = reduce_step<32>(mx, [](float x, float y) { return fmaxf(x, y); });
+        negK0 = -mx * a.c; // nk >= 1: the maximum is finite
+    }
+
+    // ---- p = 2^((s - max) * c) rounded to binary16; O^T = V^T P^T; row sum by a tile of ones
+    f16x8 ones;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+    {
+        ones[i] = (f16) 1.f;
+    }
+    f32x4 oacc[4];
+    f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+    {
+        oacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    auto weigh = [&](auto block) {
+        constexpr int kb = decltype(block)::value;
+        wait_vmcnt<DEBUG ? 0 : 2 * (NKB - 1 - kb)>();
+        __syncthreads();
+        if (!active)
+        {
+            return;
+        }
+#pragma unroll
+        for (int hb = 0; hb < 2; ++hb)
+        {
+            if (kb == NKB - 1 && hb >= lastHalves)
+            {
+                continue; // no key in this half
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            f16x8 preg;
+#pragma unroll
+            for (int w = 0; w < 2; ++w)
+            {
+                int const t = kb * 4 + hb * 2 + w;
+                float pr[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                {
+                    pr[j] = __builtin_amdgcn_exp2f(fmaf(acc[t][j], a.c, negK0));
+                }
+                f16x2 const p01 = __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(pr[0], pr[1]));
+                f16x2 const p23 = __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(pr[2], pr[3]));
+                preg[w * 4 + 0] = p01[0];
+                preg[w * 4 + 1] = p01[1];
+                preg[w * 4 + 2] = p23[0];
+                preg[w * 4 + 3] = p23[1];
+            }
+            int const vrow = kb * 64 + hb * 32 + 4 * g + (lq >> 2);
+            uint8_t const* vbase = lds + vrow * kRow + 8 * (lq & 1);
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt)
+            {
+                int const sc = swz<2>(vrow, 2 * dt + ((lq >> 1) & 1)) * 16;
+                i16x4 const v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*) (vbase + sc));
+                i16x4 const v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*) (vbase + 16 * kRow + sc));
+                typedef short i16x8 __attribute__((ext_vector_type(8)));
+                i16x8 const both = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+                oacc[dt] = attention_mfma_f16(__builtin_bit_cast(f16x8, both), preg, oacc[dt]);
+            }
+            sacc = attention_mfma_f16(ones, preg, sacc);
+        }
+    };
+    for_each_block<NKB>(weigh);
+
+    // Lane (g, query) holds 8 bytes of each 32-byte quarter dt of the query's 128-byte row; a 4 x 4 transpose over
+    // the four rows of 16 lanes (v_permlane32_swap, v_permlane16_swap, once for each dword) leaves it with the
+    // whole quarter dt = g, which goes out as two 16-byte stores.
+    if (active)
+    {
+        float const rinv = 1.f / sacc[0];
+        uint32_t lo[4], hi[4];
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+        {
+            f16x4 y;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            {
+                y[j] = (f16) (oacc[dt][j] * rinv);
+            }
+            u32x2 const w = __builtin_bit_cast(u32x2, y);
+            lo[dt] = w[0];
+            hi[dt] = w[1];
+        }
+        rows_transpose(lo);
+        rows_transpose(hi);
+        if (qValid)
+        {
+            uint8_t* dst = static_cast<uint8_t*>(a.out);
+            int64_t const off = sq.seqBaseOut + (int64_t) q * a.tokStrideOut + ((int64_t) n * kHeadSize + g * 16) * 2;
+            u32x4 const first = {lo[0], hi[0], lo[1], hi[1]};
+            u32x4 const second = {lo[2], hi[2], lo[3], hi[3]};
+            *reinterpret_cast<u32x4*>(dst + off) = first;
+            *reinterpret_cast<u32x4*>(dst + off + 16) = second;
+        }
+    }
+}
+
+template <int KT, bool DEBUG>
+__global__ __launch_bounds__(kWavesF16T* kWaveSize)
+    __attribute__((amdgpu_waves_per_eu(KT <= 4 ? 4 : KT <= 6 ? 3 : 2))) void fmha_f16_turns_kernel(FmhaArgs const a)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    __shared__ PickLds sPick;
+    UnitPart const up = unit_of_workgroup(blockIdx.x, gridDim.x, a.qSplit);
+    int const n = __builtin_amdgcn_readfirstlane(up.unit % a.N);
+    int const q0 = __builtin_amdgcn_readfirstlane(up.part) * kQueriesF16;
+    int b;
+    SeqInfo sq = pick_sequence_info<kWavesF16T * kWaveSize>(a, up.unit / a.N, KT * 64, sPick, b);
+    // the same in every lane, which the compiler cannot see where they come from LDS: scalars keep the addresses scalar
+    b = __builtin_amdgcn_readfirstlane(b);
+    sq.nq = __builtin_amdgcn_readfirstlane(sq.nq);
+    sq.nk = __builtin_amdgcn_readfirstlane(sq.nk);
+    sq.firstTok = __builtin_amdgcn_readfirstlane((int) sq.firstTok);
+    if (a.cuSeqlens)
+    {
+        sq.seqBaseIn = sq.firstTok * a.tokStrideIn;
+        sq.seqBaseOut = sq.firstTok * a.tokStrideOut;
+    }
+    else
+    {
+        sq.seqBaseIn = b * a.seqStrideIn;
+        sq.seqBaseOut = b * a.seqStrideOut;
+    }
+    if (q0 >= sq.nq)
+    {
+        return;
+    }
+    switch ((sq.nk + 63) >> 6)
+    {
+#define TRTAMD_BLOCKS(NKB)                                                                                             \
+    case NKB:                                                                                                          \
+        if constexpr (KT >= NKB) attend_f16_turns<NKB, DEBUG>(a, sq, b, n, q0, smem);                                        \
+        break
+        TRTAMD_BLOCKS(1);
+        TRTAMD_BLOCKS(2);
+        TRTAMD_BLOCKS(3);
+        TRTAMD_BLOCKS(4);
+        TRTAMD_BLOCKS(5);
+        TRTAMD_BLOCKS(6);
+        TRTAMD_BLOCKS(7);
+        TRTAMD_BLOCKS(8);
+#undef TRTAMD_BLOCKS
+    default: break;
+    }
+}
+
+// ------------------------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------------------------
 
@@ -1740,26 +2048,30 @@ int run_i8(hipStream_t stream, FmhaArgs const& a, bool interleaved)
 }
 
 template <bool DEBUG>
-int run_f16(hipStream_t stream, FmhaArgs const& a)
+int run_f16(hipStream_t stream, FmhaArgs const& a, bool turns)
 {
     int const kt = pick_kt(a.S);
-    int const noFast = tuning(Tuning::kFmhaGeneric);
-    if (a.packedMask == nullptr && !noFast)
+    if (turns)
     {
-#define TRTAMD_F16P(KT)                                                                                                \
+#define TRTAMD_F16T(KT)                                                                                                \
     case KT:                                                                                                           \
-        return launch_fmha(fmha_f16_prefix_kernel<KT, DEBUG>, "fmha_f16_prefix", stream, a, Lds<2>::total(KT), kWavesF16)
+        return launch_fmha(                                                                                            \
+            fmha_f16_turns_kernel<KT, DEBUG>, "fmha_f16_turns", stream, a, Lds<2>::matBytes(KT), kWavesF16T)
         switch (kt)
         {
-            TRTAMD_F16P(1);
-            TRTAMD_F16P(2);
-            TRTAMD_F16P(3);
-            TRTAMD_F16P(4);
-            TRTAMD_F16P(6);
-            TRTAMD_F16P(8);
+            TRTAMD_F16T(1);
+            TRTAMD_F16T(2);
+            TRTAMD_F16T(3);
+            TRTAMD_F16T(4);
+            TRTAMD_F16T(6);
+            TRTAMD_F16T(8);
         default: break;
         }
-#undef TRTAMD_F16P
+#undef TRTAMD_F16T
+    }
+    if (a.packedMask == nullptr && kt == 8 && !tuning(Tuning::kFmhaGeneric))
+    {
+        return launch_fmha(fmha_f16_prefix_kernel<8, DEBUG>, "fmha_f16_prefix", stream, a, Lds<2>::total(8), kWavesF16);
     }
 #define TRTAMD_F16(KT)                                                                                                 \
     case KT: return launch_fmha(fmha_f16_kernel<KT, DEBUG>, "fmha_f16", stream, a, Lds<2>::total(KT), kWavesF16)
@@ -1789,8 +2101,13 @@ int prepare_kt()
     st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_i8_kernel<KT, true, false>), "fmha_i8_interleaved",
                       Lds<1>::total(KT));
     st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_i8_kernel<KT, false, false>), "fmha_i8", Lds<1>::total(KT));
-    st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_f16_prefix_kernel<KT, false>), "fmha_f16_prefix",
-                      Lds<2>::total(KT));
+    st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_f16_turns_kernel<KT, false>), "fmha_f16_turns",
+                      Lds<2>::matBytes(KT));
+    if constexpr (KT == 8)
+    {
+        st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_f16_prefix_kernel<KT, false>), "fmha_f16_prefix",
+                          Lds<2>::total(KT));
+    }
     st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_f16_kernel<KT, false>), "fmha_f16", Lds<2>::total(KT));
     return st;
 }
@@ -1864,6 +2181,14 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
     a.B = p->b;
     a.N = p->h;
     a.S = p->s;
+    int const kt = pick_kt(p->s);
+    // FP16, prefix-valid keys: K and V take turns in LDS, save where there are whole units of more than 384 keys for all of
+    // the 256 CUs.  The scores of 512 keys leave room for two wavefronts per SIMD in either kernel, and staging K and V for
+    // 64 queries at a time then costs more than the wait it hides (12 heads x 32 sequences of 171-512 keys: 33.8 us
+    // against 27.6; 12 x 16: 20.2 us against 23.5).
+    bool const turns = dataType == 1 && (p->cu_seqlens || !p->packed_mask_ptr) && !tuning(Tuning::kFmhaGeneric)
+        && (kt < 8 || (int64_t) p->b * p->h <= 256)
+        && p->qkv_stride_in_bytes < (1LL << 29); // eight tokens within a 32-bit offset
     {
         // Workgroups per (sequence, head).  Every extra workgroup stages K and V again, so a unit is only shared
         // while the launch would otherwise leave the chip partly idle or badly balanced.  INT8 (three workgroups per
@@ -1872,14 +2197,19 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         // 896 units: 29.1 against 28.1 us), and more of them only to reach one round (256 units: three, 12.6 us
         // against 13.1 with two and 17.4 with one; at most four).  FP16 (its K and V take most of a CU's LDS, one
         // workgroup per CU, and staging them is 40 % of a workgroup's time): only below 160 units (192 units of 192-384
-        // keys: 15.3 us alone, 17.5 us shared by two; 144 units: 14.9 against 12.9 us).
-        int const waves = dataType == 2 ? kWavesI8 : kWavesF16;
+        // keys: 15.3 us alone, 17.5 us shared by two; 144 units: 14.9 against 12.9 us).  Where K and V take turns, 64
+        // queries each.
+        int const waves = dataType == 2 ? kWavesI8 : turns ? kWavesF16T : kWavesF16;
         int const maxSplit = std::max(1, ceil_div(ceil_div(p->s, kQPerWave), waves));
         int64_t const heads = (int64_t) p->b * p->h;
         int split = 1;
         if (dataType == 2)
         {
             split = heads >= 896 ? 1 : (int) std::max<int64_t>(2, std::min<int64_t>(4, ceil_div<int64_t>(768, heads)));
+        }
+        else if (turns)
+        {
+            split = maxSplit;
         }
         else
         {
@@ -1891,7 +2221,7 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         a.qSplit = std::min(split, maxSplit);
         // tuning override: TRTAMD_FMHA_QSPLIT=<n> forces the number of workgroups per head
         int const forced = tuning(Tuning::kFmhaQsplit);
-        if (forced > 0)
+        if (forced > 0 && !turns)
         {
             a.qSplit = std::min(forced, maxSplit);
         }
@@ -1902,10 +2232,11 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         // The order in which sequences are served matters when workgroups run in several rounds (the long ones
         // first, so that the short ones fill the tail).  When every workgroup of the launch is resident at once it
         // changes nothing, and the workgroups skip the ranking (a trip to LDS and two barriers before their loads).
-        int const kt = pick_kt(p->s);
+        // Workgroups of 64 queries are short enough to even out by themselves (12 heads x 128 sequences of 67-200 keys:
+        // 29.1 us in natural order, 36.8 ranked).
         int64_t const lds = dataType == 2 ? Lds<1>::total(kt) : Lds<2>::total(kt);
         int64_t const perCu = std::max<int64_t>(1, std::min<int64_t>(dataType == 2 ? 3 : 2, (160 * 1024) / std::max<int64_t>(lds, 1)));
-        a.ranked = (int64_t) a.B * a.N * a.qSplit > perCu * 256 ? 1 : 0;
+        a.ranked = !turns && (int64_t) a.B * a.N * a.qSplit > perCu * 256 ? 1 : 0;
         // tuning override: TRTAMD_FMHA_RANKED=0 / 1 forces natural order / the longest-first order
         int const forcedRank = tuning(Tuning::kFmhaRanked);
         if (forcedRank >= 0)
@@ -2000,7 +2331,7 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
     a.c = s1 * kLog2e;
     a.scaleSoftmax = 1.f;
     a.scaleBmm2 = 1.f;
-    return dbgAcc1 ? run_f16<true>(stream, a) : run_f16<false>(stream, a);
+    return dbgAcc1 ? run_f16<true>(stream, a, turns) : run_f16<false>(stream, a, turns);
 }
 
 } // namespace

@@ -228,6 +228,41 @@ def test_fmha_fp16_packed(api, B, N, S, rule):
                 assert_fp_close(got[lo:hi, n * D:(n + 1) * D], o, what="FP16 packed vs float64")
 
 
+@pytest.mark.parametrize("B,N,S", [(9, 2, 64), (12, 1, 128), (12, 2, 192), (14, 1, 256), (14, 2, 384), (16, 1, 512),
+                                   # either side of the unit count from which K and V keep places of their own
+                                   (16, 16, 385), (17, 16, 385)])
+def test_fmha_fp16_packed_tile_edges(api, B, N, S):
+    """Lengths either side of the wavefront's 16 queries, the workgroup's 64 queries and the 64-key blocks."""
+    from tensorrt_amd import capi
+    edges = [1, 8, 15, 16, 17, 33, 63, 64, 65, 127, 128, 129, 191, 193, 256, 257, 320, 321, 384, 385, 449, 512]
+    lens = np.resize([n for n in edges if n <= S] + [S], B) if S < 512 else np.array(edges[-B:])
+    cu = _cu(lens)
+    T = int(cu[-1])
+    qkv = rng(28).standard_normal((T, 3 * N * D)).astype(np.float16)
+    d_qkv, d_cu, out = dev(qkv), dev(cu), dev_empty((T, N * D), np.float16, fill=0)
+    p = _params(capi, qkv_ptr=ptr(d_qkv), o_ptr=ptr(out), b=B, h=N, s=S, d=D, qkv_stride_in_bytes=2 * 3 * N * D,
+                o_stride_in_bytes=2 * N * D, scale_bmm1=half2_bits(0.125), cu_seqlens=ptr(d_cu))
+    api.check(api.fused_mha_run(stream(), 1, C.byref(p)))
+    sync()
+    assert_fp_close(host(out), oracle.mha_fused_f16_packed(qkv, cu, N, D), what="FP16 packed, tile edges")
+
+
+@pytest.mark.parametrize("S", [60, 200, 512])
+def test_fmha_fp16_fixed_without_mask(api, S):
+    """The fixed [S, B, N, 3, d] layout with every key valid."""
+    from tensorrt_amd import capi
+    B, N = 3, 2
+    qkv = rng(29).standard_normal((S, B, 3 * N * D)).astype(np.float16)
+    d_qkv, out = dev(qkv), dev_empty((S, B, N * D), np.float16, fill=0)
+    p = _params(capi, qkv_ptr=ptr(d_qkv), o_ptr=ptr(out), b=B, h=N, s=S, d=D, qkv_stride_in_bytes=2 * 3 * N * D * B,
+                o_stride_in_bytes=2 * N * D * B, scale_bmm1=half2_bits(0.125))
+    api.check(api.fused_mha_run(stream(), 1, C.byref(p)))
+    sync()
+    packed = np.ascontiguousarray(qkv.transpose(1, 0, 2)).reshape(B * S, -1)
+    ref = oracle.mha_fused_f16_packed(packed, _cu(np.full(B, S)), N, D)
+    assert_fp_close(host(out).transpose(1, 0, 2).reshape(B * S, -1), ref, what="FP16 fixed, no mask")
+
+
 def test_fmha_packing_invariance_and_special_cases(api):
     """Per-sequence results do not depend on what else is packed beside them; a length-1
     sequence returns V; identical keys give the plain average of V."""
