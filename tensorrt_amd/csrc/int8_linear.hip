@@ -83,7 +83,7 @@ struct LinearArgs
     int persist;   // persistent kernel: workgroups that loop over the 256 x 256 tiles
     int pieces;    // direct-to-LDS kernel: the tokens behind the large tiles go in 64 x 64 pieces (see linear_piece64)
     int parts;     // pieces: workgroups that share the k range of a piece, each with an output of its own
-    WeightPrefetch prefetch; // by the workgroups behind mainTiles of the tile and piece kernels
+    WeightPrefetch prefetch; // by the workgroups behind mainTiles of the interleaved tile and piece kernels
 };
 
 // gelu(y) = y * Phi(y) = max(y, 0) - |y| * Phi(-|y|).  log2(Phi(-a)) is smooth and nearly quadratic, so
@@ -1431,10 +1431,13 @@ __global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(Line
 {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[RING * (WM * MT + WN * NT) * 2 * 1024];
     __shared__ __attribute__((aligned(16))) float sScale[2 * kBigTile];
-    if ((int) blockIdx.x >= p.mainTiles)
+    if constexpr (IL)
     {
-        prefetch_weights(p);
-        return;
+        if ((int) blockIdx.x >= p.mainTiles)
+        {
+            prefetch_weights(p);
+            return;
+        }
     }
     // panel numbering as for the large tiles (see int8_linear_kernel)
     uint32_t const pw = (uint32_t) p.panel;
@@ -1592,11 +1595,6 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int const row = lane & 31, half = lane >> 5;
-    if ((int) blockIdx.x >= p.mainTiles)
-    {
-        prefetch_weights(p);
-        return;
-    }
     uint32_t const nbm = (uint32_t) ceil_div(p.N, 32 * CB);
     int const n0 = (int) (blockIdx.x % nbm) * (32 * CB);
     int const kpart = (int) (blockIdx.x / nbm) / p.tokMain, t0 = (int) (blockIdx.x / nbm) % p.tokMain * (32 * TB);
@@ -1813,6 +1811,19 @@ inline float large_tiles_time(TileCost const& c, bool il, LinearArgs const& a, i
     return c.launch + rounds * (c.tile + (gelu ? c.gelu : 0.f) + c.stage * (0.75f + 0.25f * fill) * stages) + rest;
 }
 
+// The workgroups of a.mainTiles tiles, with those that fetch a.prefetch behind them where the launch leaves CUs idle.
+template <typename Kernel>
+int launch_tiles(hipStream_t stream, LinearArgs const& a, Kernel kernel, int threads)
+{
+    uint32_t behind = 0;
+    if (a.prefetch.data && a.mainTiles <= num_cus())
+    {
+        behind = 8u * ceil_div(a.prefetch.units / 8u, (uint32_t) (threads / 64 * kPrefetchLoads));
+    }
+    hipLaunchKernelGGL(kernel, dim3((uint32_t) a.mainTiles + behind), dim3(threads), 0, stream, a);
+    return check_launch("int8_linear");
+}
+
 template <bool IL, bool IL_OUT, int EPI>
 int launch_plan(hipStream_t stream, LinearArgs a, int plan)
 {
@@ -1832,34 +1843,9 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
             a.panel = w;
         }
     }
-    a.parts = std::max(a.parts, 1);
-    a.mainTiles = (int) grid * a.parts;
-    auto run = [&](auto kernel, int threads) {
-        uint32_t behind = 0;
-        // only beside a launch that leaves CUs idle
-        if (a.prefetch.data && a.mainTiles <= num_cus())
-        {
-            behind = 8u * ceil_div(a.prefetch.units / 8u, (uint32_t) (threads / 64 * kPrefetchLoads));
-        }
-        hipLaunchKernelGGL(kernel, dim3((uint32_t) a.mainTiles + behind), dim3(threads), 0, stream, a);
-        return check_launch("int8_linear");
-    };
-    if constexpr (EPI == kRAW || EPI == kF16_RAW)
-    {
-        // partial sums: only the pieces of 32 channels share k between workgroups
-        bool const wide = plan == kPiece32x64;
-        if constexpr (IL)
-        {
-            return wide ? run(linear_piece_kernel<false, EPI, 1, 2, 4, 4>, 512) : run(linear_piece_kernel<false, EPI, 1, 1, 8, 4>, 512);
-        }
-        else
-        {
-            return wide ? run(linear_piece_dma_kernel<false, EPI, 1, 2, 3, 2>, 512)
-                        : run(linear_piece_dma_kernel<false, EPI, 1, 1, 4, 2>, 512);
-        }
-    }
-    else
-    {
+    a.parts = 1;
+    a.mainTiles = (int) grid;
+    auto run = [&](auto kernel, int threads) { return launch_tiles(stream, a, kernel, threads); };
     switch (plan)
     {
     case kTile128x256: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 4, 2, 2, 3, 4>, 512);
@@ -1899,6 +1885,24 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
         }
     }
     return set_error(TRTAMD_STATUS_BAD_PARAM, "int8_linear: no such plan for this layout: %d", plan);
+}
+
+// Partial sums of `parts` workgroups per piece, in pieces of 32 x 32.
+template <bool IL, int EPI>
+int launch_partial(hipStream_t stream, LinearArgs a, int parts, void* partial, WeightPrefetch const& prefetch = {nullptr, 0})
+{
+    a.out = partial;
+    a.parts = parts;
+    a.prefetch = prefetch;
+    a.tokMain = ceil_div(a.T, 32);
+    a.mainTiles = ceil_div(a.N, 32) * a.tokMain * parts;
+    if constexpr (IL)
+    {
+        return launch_tiles(stream, a, linear_piece_kernel<false, EPI, 1, 1, 8, 4>, 512);
+    }
+    else
+    {
+        return launch_tiles(stream, a, linear_piece_dma_kernel<false, EPI, 1, 1, 4, 2>, 512);
     }
 }
 
@@ -1953,14 +1957,15 @@ bool is_piece(int plan)
 }
 
 // Parts of a layer whose launch is `plan`: as many as bring its workgroups to one per CU, and no less than 1 KB of k for
-// each (two k-slabs per wavefront).
+// each (two k-slabs per wavefront).  The wider pieces are chosen where the smaller ones no longer fit on the CUs at once, so
+// there is nothing left to share them between.
 int parts_of(int plan, LinearArgs const& a)
 {
-    if (plan != kPiece32x64 && plan != kPiece32x32)
+    if (plan != kPiece32x32)
     {
         return 1;
     }
-    int const grid = ceil_div(a.N, 32) * ceil_div(a.T, plan == kPiece32x64 ? 64 : 32);
+    int const grid = ceil_div(a.N, 32) * ceil_div(a.T, 32);
     return std::max(1, std::min({kMaxLinearParts, num_cus() / grid, a.K / 1024}));
 }
 
@@ -2206,27 +2211,18 @@ int linear_parts(trtamd_fp16_linear_params const& p)
 
 size_t linear_partial_bytes()
 {
-    return (size_t) num_cus() * 32 * 64 * sizeof(int32_t);
+    return (size_t) num_cus() * 32 * 32 * sizeof(int32_t);
 }
 
 int int8_linear_partial(trtamd_stream_t stream, trtamd_int8_linear_params const& p, int parts, int32_t* partial,
     WeightPrefetch const& prefetch)
 {
-    LinearArgs a = args_of(p);
-    int const plan = small_plan<true>(a, false);
-    a.out = partial;
-    a.parts = parts;
-    a.prefetch = prefetch;
-    return launch_plan<true, false, kRAW>(as_stream(stream), a, plan);
+    return launch_partial<true, kRAW>(as_stream(stream), args_of(p), parts, partial, prefetch);
 }
 
 int fp16_linear_partial(trtamd_stream_t stream, trtamd_fp16_linear_params const& p, int parts, float* partial)
 {
-    LinearArgs a = args_of(p);
-    int const plan = small_plan<false>(a, false);
-    a.out = partial;
-    a.parts = parts;
-    return launch_plan<false, false, kF16_RAW>(as_stream(stream), a, plan);
+    return launch_partial<false, kF16_RAW>(as_stream(stream), args_of(p), parts, partial);
 }
 
 } // namespace trtamd

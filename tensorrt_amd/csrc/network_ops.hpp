@@ -30,7 +30,7 @@ int int8_linear(trtamd_stream_t stream, trtamd_int8_linear_params const& p, Weig
 constexpr int kMaxLinearParts = 4;
 int linear_parts(trtamd_int8_linear_params const& p);
 int linear_parts(trtamd_fp16_linear_params const& p);
-// Bytes that the partial sums of any such layer fit in: they come from one workgroup per CU at most, 32 x 64 of them each.
+// Bytes that the partial sums of any such layer fit in: they come from one workgroup per CU at most, 32 x 32 of them each.
 size_t linear_partial_bytes();
 int int8_linear_partial(trtamd_stream_t stream, trtamd_int8_linear_params const& p, int parts, int32_t* partial,
     WeightPrefetch const& prefetch);
