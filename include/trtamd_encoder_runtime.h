@@ -123,8 +123,8 @@ typedef struct trtamd_fp16_encoder_layer
     void* attention;                                  /* IPluginV3 objects */
     void* ln1;
     void* ln2;
-    /* the parameters of ln2 again, device binary16 [hidden]: for batches of few tokens, where the normalisation adds up
-     * partial sums of ffn2 */
+    /* the parameters of ln2 again, device binary16 [hidden], 16-byte aligned: for batches of few tokens, where the
+     * normalisation adds up partial sums of ffn2; missing in any layer: done without */
     trtamd_half_t const* ln2_gamma;
     trtamd_half_t const* ln2_beta;
     trtamd_half_t const* ln2_bias;
@@ -149,7 +149,7 @@ typedef struct trtamd_fp16_encoder_batch
      * m [tokens][ffn]; emb2: the embedding plugin's second output, device int32 [1] */
     trtamd_half_t *x, *qkv, *ctx, *ao, *h, *m, *f;
     int32_t* emb2;
-    float* partial; /* device scratch for batches of few tokens, 16-byte aligned; NULL or too small: done without */
+    float* partial; /* device scratch for batches of few tokens, 16-byte aligned; NULL, too small or misaligned: done without */
     size_t partial_bytes; /* 2 MiB serve every such batch */
 } trtamd_fp16_encoder_batch;
 

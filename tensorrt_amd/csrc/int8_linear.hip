@@ -1961,7 +1961,7 @@ bool is_piece(int plan)
 // there is nothing left to share them between.
 int parts_of(int plan, LinearArgs const& a)
 {
-    if (plan != kPiece32x32)
+    if (plan != kPiece32x32 || a.T <= 0)
     {
         return 1;
     }
@@ -2095,7 +2095,7 @@ LinearArgs args_of(trtamd_fp16_linear_params const& p)
     return a;
 }
 
-int run_int8(trtamd_stream_t stream, trtamd_int8_linear_params const* p, WeightPrefetch const& prefetch)
+int check_int8(trtamd_int8_linear_params const* p)
 {
     if (p == nullptr || p->a == nullptr || p->w == nullptr || p->out == nullptr)
     {
@@ -2124,6 +2124,16 @@ int run_int8(trtamd_stream_t stream, trtamd_int8_linear_params const* p, WeightP
     {
         return set_error(TRTAMD_STATUS_BAD_PARAM, "int8_linear: pointers must be 16-byte aligned");
     }
+    return TRTAMD_STATUS_SUCCESS;
+}
+
+int run_int8(trtamd_stream_t stream, trtamd_int8_linear_params const* p, WeightPrefetch const& prefetch)
+{
+    int const checked = check_int8(p);
+    if (checked != TRTAMD_STATUS_SUCCESS)
+    {
+        return checked;
+    }
     if (p->T == 0)
     {
         return TRTAMD_STATUS_SUCCESS;
@@ -2141,7 +2151,7 @@ int run_int8(trtamd_stream_t stream, trtamd_int8_linear_params const* p, WeightP
                             : launch_out<false, false>(st, a, p->epilogue, ilOut);
 }
 
-int run_fp16(trtamd_stream_t stream, trtamd_fp16_linear_params const* p)
+int check_fp16(trtamd_fp16_linear_params const* p)
 {
     if (p == nullptr || p->a == nullptr || p->w == nullptr || p->out == nullptr || p->alpha == nullptr
         || p->beta == nullptr)
@@ -2165,6 +2175,16 @@ int run_fp16(trtamd_stream_t stream, trtamd_fp16_linear_params const* p)
     {
         return set_error(TRTAMD_STATUS_BAD_PARAM, "fp16_linear: pointers must be 16-byte aligned");
     }
+    return TRTAMD_STATUS_SUCCESS;
+}
+
+int run_fp16(trtamd_stream_t stream, trtamd_fp16_linear_params const* p)
+{
+    int const checked = check_fp16(p);
+    if (checked != TRTAMD_STATUS_SUCCESS)
+    {
+        return checked;
+    }
     if (p->T == 0)
     {
         return TRTAMD_STATUS_SUCCESS;
@@ -2175,7 +2195,21 @@ int run_fp16(trtamd_stream_t stream, trtamd_fp16_linear_params const* p)
                                              : launch_shape<false, false, false, kF16_AFFINE>(st, a);
 }
 
-// Whether operands are what the partial launches take (the public calls check the rest).
+// What the partial launches ask beyond that: the sums fit in linear_partial_bytes().
+int check_partial(int32_t T, int32_t N, int parts, void const* partial)
+{
+    if (partial == nullptr || !aligned16(partial))
+    {
+        return set_error(TRTAMD_STATUS_BAD_PARAM, "linear layer: the buffer of partial sums must be 16-byte aligned");
+    }
+    if (T <= 0 || parts < 1 || parts > kMaxLinearParts || (int64_t) ceil_div(N, 32) * ceil_div(T, 32) * parts > num_cus())
+    {
+        return set_error(TRTAMD_STATUS_NOT_SUPPORTED, "linear layer: %d parts of T=%d N=%d do not fit the partial sums", parts, T, N);
+    }
+    return TRTAMD_STATUS_SUCCESS;
+}
+
+// Whether operands are what the partial launches take (the checks above see to the rest).
 bool interleaved(trtamd_int8_linear_params const& p)
 {
     return p.a_interleaved && p.w_interleaved && (p.epilogue == TRTAMD_LINEAR_AFFINE || p.epilogue == TRTAMD_LINEAR_GELU);
@@ -2217,12 +2251,21 @@ size_t linear_partial_bytes()
 int int8_linear_partial(trtamd_stream_t stream, trtamd_int8_linear_params const& p, int parts, int32_t* partial,
     WeightPrefetch const& prefetch)
 {
-    return launch_partial<true, kRAW>(as_stream(stream), args_of(p), parts, partial, prefetch);
+    int st = check_int8(&p);
+    st = st ? st : check_partial(p.T, p.N, parts, partial);
+    return st ? st : launch_partial<true, kRAW>(as_stream(stream), args_of(p), parts, partial, prefetch);
 }
 
 int fp16_linear_partial(trtamd_stream_t stream, trtamd_fp16_linear_params const& p, int parts, float* partial)
 {
-    return launch_partial<false, kF16_RAW>(as_stream(stream), args_of(p), parts, partial);
+    int st = check_fp16(&p);
+    st = st ? st : check_partial(p.T, p.N, parts, partial);
+    return st ? st : launch_partial<false, kF16_RAW>(as_stream(stream), args_of(p), parts, partial);
+}
+
+int fp16_linear_check(trtamd_fp16_linear_params const& p)
+{
+    return check_fp16(&p);
 }
 
 } // namespace trtamd

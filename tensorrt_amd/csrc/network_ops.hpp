@@ -32,9 +32,12 @@ int linear_parts(trtamd_int8_linear_params const& p);
 int linear_parts(trtamd_fp16_linear_params const& p);
 // Bytes that the partial sums of any such layer fit in: they come from one workgroup per CU at most, 32 x 32 of them each.
 size_t linear_partial_bytes();
+// `parts`: what linear_parts said.  The parameters are checked as the public calls check theirs.
 int int8_linear_partial(trtamd_stream_t stream, trtamd_int8_linear_params const& p, int parts, int32_t* partial,
     WeightPrefetch const& prefetch);
 int fp16_linear_partial(trtamd_stream_t stream, trtamd_fp16_linear_params const& p, int parts, float* partial);
+// The checks of trtamd_fp16_linear without its launch, for a pass that is refused before its first launch.
+int fp16_linear_check(trtamd_fp16_linear_params const& p);
 
 // trtamd_skipln_interleaved_{small,large}_hface with the input given as the partial sums of an affine INT8 layer (alpha,
 // beta as in trtamd_int8_linear_params): the same bytes as the layer's output through memory would give.

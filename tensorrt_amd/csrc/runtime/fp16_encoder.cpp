@@ -70,12 +70,6 @@ int enqueue(trtamd_fp16_encoder_config const& c, trtamd_fp16_encoder_layer const
     PluginTensorDesc const tIds = int32({T}), tCu = int32({B + 1}), tLongest = int32({c.max_seqlen}), tOne = int32({1});
     PluginTensorDesc const act = half({T, E, 1, 1}), qkvAct = half({T, 3 * E, 1, 1}), row = half({T, 1, E, 1, 1});
 
-    {
-        PluginTensorDesc const in[4] = {tIds, tIds, tCu, tLongest}, out[2] = {act, int32({})};
-        void const* inputs[4] = {b.ids, b.segment_ids, b.cu_seqlens, b.longest};
-        void* outputs[2] = {b.x, b.emb2};
-        run(c.embedding, "embeddings", in, 4, out, 2, inputs, outputs, stream);
-    }
     auto params = [&](trtamd_fp16_encoder_linear const& l, void const* a, void* out, int32_t K, int32_t N, int32_t epilogue) {
         trtamd_fp16_linear_params p{};
         p.a = static_cast<trtamd_half_t const*>(a);
@@ -89,6 +83,28 @@ int enqueue(trtamd_fp16_encoder_config const& c, trtamd_fp16_encoder_layer const
         p.epilogue = epilogue;
         return p;
     };
+    // Few tokens: the second feed-forward layer, whose k loop is the longest, shares it between workgroups, and the
+    // normalisation behind it adds up the sums, if what that takes beside the plugins is there.
+    int parts = 1;
+    if (c.layers > 0 && c.hidden % 8 == 0 && c.hidden > 32 && c.hidden <= 1024 && b.partial && aligned16(b.partial)
+        && b.partial_bytes >= linear_partial_bytes())
+    {
+        parts = linear_parts(params(layers[0].ffn2, b.m, b.f, c.ffn, c.hidden, TRTAMD_LINEAR_AFFINE));
+    }
+    // everything that can be refused is refused before the first launch
+    auto check = [&](trtamd_fp16_linear_params const& p) { checkKernelStatus(fp16_linear_check(p), "linear layer"); };
+    for (int32_t i = 0; i < c.layers; ++i)
+    {
+        trtamd_fp16_encoder_layer const& L = layers[i];
+        check(params(L.qkv, b.x, b.qkv, c.hidden, 3 * c.hidden, TRTAMD_LINEAR_AFFINE));
+        check(params(L.proj, b.ctx, b.ao, c.hidden, c.hidden, TRTAMD_LINEAR_AFFINE));
+        check(params(L.ffn1, b.h, b.m, c.hidden, c.ffn, TRTAMD_LINEAR_GELU));
+        check(params(L.ffn2, b.m, b.f, c.ffn, c.hidden, TRTAMD_LINEAR_AFFINE));
+        for (trtamd_half_t const* v : {L.ln2_gamma, L.ln2_beta, L.ln2_bias})
+        {
+            parts = v && aligned16(v) ? parts : 1;
+        }
+    }
     auto linear = [&](trtamd_fp16_linear_params const& p) {
         checkKernelStatus(trtamd_fp16_linear(stream, &p), "linear layer");
     };
@@ -97,13 +113,11 @@ int enqueue(trtamd_fp16_encoder_config const& c, trtamd_fp16_encoder_layer const
         void const* inputs[2] = {x, skip};
         run(plugin, "skipLayerNorm", in, 2, &row, 1, inputs, &out, stream);
     };
-    // Few tokens: the second feed-forward layer, whose k loop is the longest, shares it between workgroups, and the
-    // normalisation behind it adds up the sums.
-    int parts = 1;
-    if (c.layers > 0 && c.hidden % 8 == 0 && c.hidden > 32 && c.hidden <= 1024 && layers[0].ln2_gamma && layers[0].ln2_beta
-        && layers[0].ln2_bias && b.partial && b.partial_bytes >= linear_partial_bytes())
     {
-        parts = linear_parts(params(layers[0].ffn2, b.m, b.f, c.ffn, c.hidden, TRTAMD_LINEAR_AFFINE));
+        PluginTensorDesc const in[4] = {tIds, tIds, tCu, tLongest}, out[2] = {act, int32({})};
+        void const* inputs[4] = {b.ids, b.segment_ids, b.cu_seqlens, b.longest};
+        void* outputs[2] = {b.x, b.emb2};
+        run(c.embedding, "embeddings", in, 4, out, 2, inputs, outputs, stream);
     }
     for (int32_t i = 0; i < c.layers; ++i)
     {
