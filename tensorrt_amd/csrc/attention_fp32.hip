@@ -248,6 +248,25 @@ __global__ __launch_bounds__(kBlock, split_waves(KD, NT)) void attention_split_k
     {
         if (exists(u))
         {
+            int const before = 16 * (4 * (u - NT) + turn) - first_row(4 * (u - NT) + turn);
+            if (before > 0) // uniform: rows of the tile in front of this one, which count there; 0 times infinity is no 0
+            {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                {
+                    bool const own = 4 * g + i >= before;
+#pragma unroll
+                    for (int b = 0; b < kBlocks; ++b)
+                    {
+                        ring[u % D][4 * b + i] = own ? ring[u % D][4 * b + i] : f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
+#pragma unroll
+                    for (int dt = 4 * kBlocks; dt < KD; ++dt)
+                    {
+                        ring[u % D][dt][i] = own ? ring[u % D][dt][i] : 0.f;
+                    }
+                }
+            }
 #pragma unroll
             for (int dt = 0; dt < KD; ++dt)
             {

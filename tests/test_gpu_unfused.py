@@ -194,6 +194,25 @@ def test_fp32_keys_split_between_wavefronts(api, S, d):
     assert_fp_close(got, oracle.mha_unfused_fixed(qkv, S, B, N, d, lens), atol=2e-5, rtol=1e-4, what="vs oracle")
 
 
+@pytest.mark.parametrize("S,d", [(17, 64), (30, 48), (197, 64), (500, 80), (1001, 128)])
+def test_fp32_infinite_values_of_valid_keys(api, S, d):
+    """An infinite V of a key with a positive probability makes that dimension infinite and leaves the others alone, also
+    for the keys that the last tile of 16 rows reads a second time."""
+    B, N = 1, 1
+    r = rng(890 + S + d)
+    qkv = r.standard_normal((S, B, 3 * N * d)).astype(np.float32)
+    want = oracle.mha_unfused_fixed(qkv, S, B, N, d, None)
+    first = S // 16 * 16
+    keys = {0: first - 1, 1: first, 2: S - 1, 3: max(0, S - 16), d - 1: max(0, S - 10)}   # dimension: key
+    for dim, key in keys.items():
+        qkv[key, 0, 2 * d + dim] = np.inf
+        want[..., dim] = np.inf
+    got = _run_unfused(api, np.float32, S, B, N, d, qkv, None)
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and not np.isnan(got).any()
+    fine = np.isfinite(want)
+    assert_fp_close(got[fine], want[fine], atol=2e-5, rtol=1e-4, what="the other dimensions")
+
+
 def test_unfused_mha_unaligned_operands(api):
     """Operands that start 2 bytes off a 16-byte boundary take the element-wise loads and stores."""
     S, B, N, d = 90, 2, 2, 64
