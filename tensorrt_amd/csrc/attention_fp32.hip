@@ -38,6 +38,9 @@ namespace
 // ------------------------------------------------------------------------------------------
 constexpr int kBlock = 256;
 constexpr int kInFlight = 2; // tiles of K, then V, on their way to a wavefront
+// The weights of up to 1024 keys, each at most 1, on their way to the division by their sum: smaller by a power of two, so
+// that no value is rounded and a weighted sum of V does not overflow where the result is finite.
+constexpr float kDown = 1.f / 1024.f;
 
 // Wavefronts per SIMD that the registers are to leave room for, without spills.
 constexpr int split_waves(int const KD, int const NT)
@@ -223,7 +226,7 @@ __global__ __launch_bounds__(kBlock, split_waves(KD, NT)) void attention_split_k
             for (int i = 0; i < 4; ++i)
             {
                 float const e = __builtin_amdgcn_exp2f(fmaf(acc[u][i], wl2, nmx));
-                acc[u][i] = e;
+                acc[u][i] = e * kDown;
                 sum += e;
             }
         }
@@ -315,7 +318,7 @@ __global__ __launch_bounds__(kBlock, split_waves(KD, NT)) void attention_split_k
             sum += rowSum[v][q] * c;
             r += *reinterpret_cast<f32x4 const*>(lds[v] + q * kPitch + d0) * c;
         }
-        r *= valid > 0 ? 1.f / sum : 0.f;
+        r *= valid > 0 ? 1.f / (sum * kDown) : 0.f;
         int const query = first_row(up.part) + q;
         if (query >= 16 * up.part)
         {

@@ -213,6 +213,23 @@ def test_fp32_infinite_values_of_valid_keys(api, S, d):
     assert_fp_close(got[fine], want[fine], atol=2e-5, rtol=1e-4, what="the other dimensions")
 
 
+@pytest.mark.parametrize("S,d", [(16, 64), (197, 64), (512, 32), (1024, 128)])
+def test_fp32_values_near_the_largest(api, S, d):
+    """Weighted averages of values near the largest binary32 number are finite: what is multiplied with V sums to 1."""
+    B, N = 2, 2
+    r = rng(895 + S + d)
+    qkv = r.standard_normal((S, B, N, 3, d)).astype(np.float32)
+    qkv[:, :, :, 2] = r.uniform(2.0e38, 3.3e38, (S, B, N, d)) * np.sign(r.standard_normal((1, B, N, d)))
+    qkv = qkv.reshape(S, B, 3 * N * d)
+    lens = np.array([S, max(1, S // 2)], np.int32)
+    got = _run_unfused(api, np.float32, S, B, N, d, qkv, lens)
+    assert np.isfinite(got).all()
+    small = qkv.reshape(S, B, N, 3, d).copy()
+    small[:, :, :, 2] *= np.float32(2.0 ** -20)    # exact: the oracle's own sums stay in range
+    want = oracle.mha_unfused_fixed(small.reshape(S, B, 3 * N * d), S, B, N, d, lens)
+    assert_fp_close(got * np.float32(2.0 ** -20), want, atol=0, rtol=1e-4, what="vs oracle")
+
+
 def test_unfused_mha_unaligned_operands(api):
     """Operands that start 2 bytes off a 16-byte boundary take the element-wise loads and stores."""
     S, B, N, d = 90, 2, 2, 64
