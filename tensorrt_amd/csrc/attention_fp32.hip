@@ -191,8 +191,9 @@ __global__ __launch_bounds__(kBlock, split_waves(KD, NT)) void attention_split_k
     }
 
     // ---- softmax over this wavefront's keys: exp((x - max) w) as one fma per score, the way the reference's kernel
-    // forms it; a masked key gets the most negative score, whose exponential is exactly 0 -------------------------
-    float mx = -3.0e38f;
+    // forms it; a masked key gets minus infinity, whose exponential is 0 whatever the maximum (which stays finite, so that
+    // the fma does not subtract infinities where every valid score is one) -----------------------------------------
+    float mx = -3.402823466e38f;
 #pragma unroll
     for (int u = 0; u < NT; ++u)
     {
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(kBlock, split_waves(KD, NT)) void attention_split_k
                 for (int i = 0; i < 4; ++i)
                 {
                     int const key = first_row(tile) + 4 * g + i;
-                    x[i] = key >= 16 * tile && key < valid ? x[i] : -3.0e38f;
+                    x[i] = key >= 16 * tile && key < valid ? x[i] : -__builtin_inff();
                 }
                 acc[u] = x;
             }

@@ -230,6 +230,21 @@ def test_fp32_values_near_the_largest(api, S, d):
     assert_fp_close(got * np.float32(2.0 ** -20), want, atol=0, rtol=1e-4, what="vs oracle")
 
 
+@pytest.mark.parametrize("d", [32, 48, 64, 80, 96, 112, 128])
+def test_fp32_tile_whose_scores_are_all_minus_infinity(api, d):
+    """Where every valid key of a wavefront scores minus infinity its masked keys weigh nothing either: the result is that
+    of the other wavefronts' keys."""
+    S, B, N = 40, 2, 2
+    r = rng(897 + d)
+    qkv = r.standard_normal((S, B, N, 3, d)).astype(np.float32)
+    qkv[:, :, :, 0] = np.abs(qkv[:, :, :, 0]) + 1
+    qkv[32:, :, :, 1] = -3.0e38          # the ragged tile: 8 valid keys behind 8 rows that it reads a second time
+    lens = np.array([S, 35], np.int32)
+    got = _run_unfused(api, np.float32, S, B, N, d, qkv.reshape(S, B, 3 * N * d), lens)
+    want = oracle.mha_unfused_fixed(qkv.reshape(S, B, 3 * N * d), S, B, N, d, np.array([32, 32], np.int32))
+    assert_fp_close(got, want, atol=2e-5, rtol=1e-4, what="vs oracle on the other keys")
+
+
 def test_unfused_mha_unaligned_operands(api):
     """Operands that start 2 bytes off a 16-byte boundary take the element-wise loads and stores."""
     S, B, N, d = 90, 2, 2, 64
