@@ -1246,9 +1246,15 @@ int launch_attention_in_registers(hipStream_t stream, int32_t S, int32_t B, int3
     int const vecOut = d % 4 == 0 && (reinterpret_cast<uintptr_t>(output) & (4 * sizeof(T) - 1)) == 0;
     if constexpr (sizeof(T) == 4)
     {
-        // 1.8 times as fast in the mean over S = 20 .. 1000, one sequence up to 8192 tokens, head sizes 32 .. 80 (0.94 to 6
-        // times; the slower end is S = 64 without a mask in a full grid, where the strips below have no idle rows)
-        if (attention_split_keys_takes(S, B, N, d, qkv, output))
+        // 1.8 times as fast in the mean over S = 20 .. 1000, one sequence up to 8192 tokens, head sizes 32 .. 80.  The strips
+        // below win where none of their rows idles, without a mask, in one or two whole strips of whole blocks of 64
+        // dimensions, and there are enough units to fill the chip with them (us, strips / split keys, d = 64: S = 64 and
+        // 1024 units 17.5 / 19.3, 1536 23.1 / 25.2, 4096 51.6 / 60.6, but 256 units 6.9 / 6.3; S = 128 and 1536 units 66.5 /
+        // 73.8; S = 192 and 1024 units 97 / 95).  With a mask the split keys skip more of the masked ones: 65 % valid, S =
+        // 128, 1536 units 63.9 / 60.1.
+        bool const wholeStrips
+            = maskIdx == nullptr && (S == 64 || S == 128) && d % 64 == 0 && (int64_t) B * N >= 1024;
+        if (!wholeStrips && attention_split_keys_takes(S, B, N, d, qkv, output))
         {
             return attention_split_keys(stream, S, B, N, d, qkv, maskIdx, output);
         }

@@ -194,6 +194,18 @@ def test_fp32_keys_split_between_wavefronts(api, S, d):
     assert_fp_close(got, oracle.mha_unfused_fixed(qkv, S, B, N, d, lens), atol=2e-5, rtol=1e-4, what="vs oracle")
 
 
+@pytest.mark.parametrize("S,B,N,d", [(64, 128, 8, 64), (64, 93, 11, 64), (128, 128, 8, 128), (128, 93, 11, 128)])
+def test_fp32_whole_strips(api, S, B, N, d):
+    """Either side of the 1024 units from which unmasked sequences of 64 and 128 go in strips of 64 queries; with lengths
+    that mask nothing they go the other way, to the same result."""
+    r = rng(880 + S + d)
+    qkv = r.standard_normal((S, B, 3 * N * d)).astype(np.float32)
+    got = _run_unfused(api, np.float32, S, B, N, d, qkv, None)
+    assert_fp_close(got, oracle.mha_unfused_fixed(qkv, S, B, N, d, None), atol=2e-5, rtol=1e-4, what="vs oracle")
+    masked = _run_unfused(api, np.float32, S, B, N, d, qkv, np.full(B, S, np.int32))
+    assert_fp_close(got, masked, atol=2e-6, rtol=2e-5, what="vs lengths that mask nothing")
+
+
 @pytest.mark.parametrize("S,d", [(17, 64), (30, 48), (197, 64), (500, 80), (1001, 128)])
 def test_fp32_infinite_values_of_valid_keys(api, S, d):
     """An infinite V of a key with a positive probability makes that dimension infinite and leaves the others alone, also
