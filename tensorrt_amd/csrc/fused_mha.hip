@@ -1652,6 +1652,7 @@ __global__ __launch_bounds__(kWavesF16* kWaveSize) void fmha_f16_prefix_kernel(F
 // 128 x 384 71.5 -> 64.8 us.
 // ------------------------------------------------------------------------------------------
 constexpr int kQueriesF16 = kWavesF16T * kQPerWave;
+__device__ u32x4 const kZeroRow[8] = {}; // 64 binary16 zeros, in memory
 
 template <int N, int I = 0, typename F>
 __device__ __forceinline__ void for_each_block(F&& f)
@@ -1678,8 +1679,8 @@ __device__ __forceinline__ void attend_f16_turns(
     uint8_t const* const unit = static_cast<uint8_t const*>(a.qkv) + sq.seqBaseIn + (int64_t) n * 3 * kRow;
     uint32_t const stride = (uint32_t) a.tokStrideIn;
 
-    // 16 rows of matrix `mat` from `row` on (unless complete, those at or behind `limit` as the last one) into the LDS
-    // rows from `to` on
+    // 16 rows of matrix `mat` from `row` on into the LDS rows from `to` on; unless complete, those at or behind `limit` as
+    // the last one, or for V as zeros: 0, the weight of such a key, times an infinite V would not be 0
     int const r8 = lane >> 3;
     uint32_t const chunk = (uint32_t) (((lane & 7) ^ r8) * 16); // the swizzle of swz<2>, on the source side
     uint32_t const whole = (uint32_t) r8 * stride + chunk;
@@ -1688,12 +1689,19 @@ __device__ __forceinline__ void attend_f16_turns(
         for (int i = 0; i < 2; ++i)
         {
             int const first = complete ? row + 8 * i : min(row + 8 * i, limit - 1);
+            uint8_t const* const src = unit + (int64_t) first * a.tokStrideIn + mat * kRow;
+            uint32_t const dst = ldsBase + (to + 8 * i) * kRow;
             uint32_t off = whole;
-            if (!complete && first + 8 > limit)
+            if (!complete && row + 8 * i + 8 > limit)
             {
+                if (mat == 2)
+                {
+                    load_to_lds16(row + 8 * i + r8 < limit ? src + whole : reinterpret_cast<uint8_t const*>(kZeroRow) + chunk, dst);
+                    continue;
+                }
                 off = (uint32_t) min(r8, limit - 1 - first) * stride + chunk;
             }
-            load_to_lds16_sbase(unit + (int64_t) first * a.tokStrideIn + mat * kRow, off, ldsBase + (to + 8 * i) * kRow);
+            load_to_lds16_sbase(src, off, dst);
         }
     };
     auto request_block = [&](int mat, int kb) { request(mat, kb * 64 + wave * 16, sq.nk, kb * 64 + wave * 16, kb < NKB - 1); };

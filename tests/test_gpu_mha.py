@@ -247,6 +247,29 @@ def test_fmha_fp16_packed_tile_edges(api, B, N, S):
     assert_fp_close(host(out), oracle.mha_fused_f16_packed(qkv, cu, N, D), what="FP16 packed, tile edges")
 
 
+@pytest.mark.parametrize("S", [64, 128, 384, 512])
+def test_fmha_fp16_infinite_value_of_the_last_key(api, S):
+    """An infinite V of the last key makes that dimension infinite and leaves the others alone, whatever the rows behind it
+    in the last block of 64 keys hold."""
+    from tensorrt_amd import capi
+    N = 2
+    lens = np.array([n for n in (1, 7, 15, 17, 40, 63, 64, 65, 100, 129, 321, 385, 500) if n <= S])
+    cu = _cu(lens)
+    T = int(cu[-1])
+    qkv = rng(31).standard_normal((T, N, 3, D)).astype(np.float16)
+    want = oracle.mha_fused_f16_packed(qkv.reshape(T, -1), cu, N, D).astype(np.float32).reshape(T, N, D).copy()
+    qkv[cu[1:] - 1, :, 2, 5] = np.inf
+    want[:, :, 5] = np.inf
+    d_qkv, d_cu, out = dev(qkv), dev(cu), dev_empty((T, N * D), np.float16, fill=0)
+    p = _params(capi, qkv_ptr=ptr(d_qkv), o_ptr=ptr(out), b=len(lens), h=N, s=S, d=D, qkv_stride_in_bytes=2 * 3 * N * D,
+                o_stride_in_bytes=2 * N * D, scale_bmm1=half2_bits(0.125), cu_seqlens=ptr(d_cu))
+    api.check(api.fused_mha_run(stream(), 1, C.byref(p)))
+    sync()
+    got = host(out).astype(np.float32).reshape(T, N, D)
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and not np.isnan(got).any()
+    assert_fp_close(np.delete(got, 5, axis=2), np.delete(want, 5, axis=2), what="the other dimensions")
+
+
 @pytest.mark.parametrize("S", [60, 200, 512])
 def test_fmha_fp16_fixed_without_mask(api, S):
     """The fixed [S, B, N, 3, d] layout with every key valid."""
