@@ -2206,8 +2206,9 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         // against 13.1 with two and 17.4 with one; at most four).  FP16 (its K and V take most of a CU's LDS, one
         // workgroup per CU, and staging them is 40 % of a workgroup's time): only below 160 units (192 units of 192-384
         // keys: 15.3 us alone, 17.5 us shared by two; 144 units: 14.9 against 12.9 us).  Where K and V take turns, 64
-        // queries each.
-        int const waves = dataType == 2 ? kWavesI8 : turns ? kWavesF16T : kWavesF16;
+        // queries each, one for each block of 64 keys that the kernel has room for: a sequence longer than s that still fits
+        // is served whole, as by the kernels that walk the queries.
+        int const waves = dataType == 2 ? kWavesI8 : kWavesF16;
         int const maxSplit = std::max(1, ceil_div(ceil_div(p->s, kQPerWave), waves));
         int64_t const heads = (int64_t) p->b * p->h;
         int split = 1;
@@ -2217,7 +2218,7 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         }
         else if (turns)
         {
-            split = maxSplit;
+            split = kt;
         }
         else
         {
@@ -2226,7 +2227,7 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
                 split *= 2;
             }
         }
-        a.qSplit = std::min(split, maxSplit);
+        a.qSplit = turns ? split : std::min(split, maxSplit);
         // tuning override: TRTAMD_FMHA_QSPLIT=<n> forces the number of workgroups per head
         int const forced = tuning(Tuning::kFmhaQsplit);
         if (forced > 0 && !turns)

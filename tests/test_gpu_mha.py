@@ -247,6 +247,22 @@ def test_fmha_fp16_packed_tile_edges(api, B, N, S):
     assert_fp_close(host(out), oracle.mha_fused_f16_packed(qkv, cu, N, D), what="FP16 packed, tile edges")
 
 
+@pytest.mark.parametrize("s,longest", [(40, 64), (250, 256), (257, 384), (300, 384), (400, 512)])
+def test_fmha_fp16_sequences_longer_than_s(api, s, longest):
+    """s chooses the kernel; sequences up to the 64, 128, 192, 256, 384 or 512 keys that it holds are served whole."""
+    from tensorrt_amd import capi
+    N = 2
+    cu = _cu(np.array([longest, s, longest - 1, 3]))
+    T = int(cu[-1])
+    qkv = rng(32).standard_normal((T, 3 * N * D)).astype(np.float16)
+    d_qkv, d_cu, out = dev(qkv), dev(cu), dev_empty((T, N * D), np.float16, fill=0)
+    p = _params(capi, qkv_ptr=ptr(d_qkv), o_ptr=ptr(out), b=4, h=N, s=s, d=D, qkv_stride_in_bytes=2 * 3 * N * D,
+                o_stride_in_bytes=2 * N * D, scale_bmm1=half2_bits(0.125), cu_seqlens=ptr(d_cu))
+    api.check(api.fused_mha_run(stream(), 1, C.byref(p)))
+    sync()
+    assert_fp_close(host(out), oracle.mha_fused_f16_packed(qkv, cu, N, D), what="FP16 packed, longer than s")
+
+
 @pytest.mark.parametrize("S", [64, 128, 384, 512])
 def test_fmha_fp16_infinite_value_of_the_last_key(api, S):
     """An infinite V of the last key makes that dimension infinite and leaves the others alone, whatever the rows behind it
