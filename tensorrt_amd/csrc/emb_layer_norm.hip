@@ -440,6 +440,10 @@ int emb_layer_norm_with_mask(trtamd_stream_t stream, int32_t type, int32_t ld, i
             }
         }
     }
+    else if (S == 0 && B > 0 && !m.warpsM)
+    {
+        return trtamd_compute_mask_idx(stream, S, B, m.mask, static_cast<int32_t*>(m.out)); // nothing to embed
+    }
     hipStream_t const st = as_stream(stream);
     if (type == 0)
     {

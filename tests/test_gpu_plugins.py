@@ -193,6 +193,19 @@ def test_embln_v6_plugin(reg, S, mha_type, fp16):
         assert not got[want.size:].any()
 
 
+def test_embln_v6_plugin_of_empty_sequences(reg):
+    """Sequences of length 0 have nothing to embed and a first masked position of 0."""
+    r = rng(109)
+    ld, B, vocab = 256, 5, 50
+    c = reg.get_creator(EMBLN, "6")
+    p = through_runtime(c, c.create_plugin("emb", emb_fields(emb_weights(r, ld, vocab, 16), 1, [i32("mha_type_id", 1)])))
+    ins = [TensorDesc([0, B], DataType.INT32)] * 3
+    outs = [TensorDesc([0, B, ld, 1, 1], DataType.HALF), TensorDesc([B, 1], DataType.INT32)]
+    ids, emb, mout = dev_empty((4,), np.int32, fill=1), dev_empty((4,), np.float16, fill=0), dev_empty((B, 1), np.int32, fill=1)
+    run(p, ins, outs, [ids, ids, ids], [emb, mout])
+    assert not host(mout).any()
+
+
 @pytest.mark.parametrize("version", ["4", "5"])
 @pytest.mark.parametrize("fp16", [0, 1])
 def test_embln_varseqlen_plugin(reg, version, fp16):
