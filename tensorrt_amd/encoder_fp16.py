@@ -85,7 +85,9 @@ class Fp16BertEncoder:
         import torch
         self.torch, self.cfg = torch, cfg
         self.api = capi.api()
-        self.stream = torch.cuda.current_stream().cuda_stream
+        # every pass runs here, whatever stream is current when it is asked for; so do its allocations and copies
+        self._torch_stream = torch.cuda.current_stream()
+        self.stream = self._torch_stream.cuda_stream
         reg = get_plugin_registry()
         r = np.random.default_rng(cfg.seed)
         E, F = cfg.hidden, cfg.ffn
@@ -161,7 +163,11 @@ class Fp16BertEncoder:
         return config, layers, capi.Fp16EncoderBatch(partial=self._partial.data_ptr(), partial_bytes=2 << 20)
 
     def _bind(self, ids: np.ndarray, segs: np.ndarray, cu: np.ndarray):
-        torch, cfg = self.torch, self.cfg
+        torch = self.torch
+        if torch.cuda.current_stream().cuda_stream != self.stream:
+            with torch.cuda.stream(self._torch_stream):
+                return self._bind(ids, segs, cu)
+        cfg = self.cfg
         T, B = int(cu[-1]), len(cu) - 1
         if len(ids) != T or len(segs) != T:
             raise ValueError("ids and segment ids must hold one entry per packed token")
@@ -180,8 +186,6 @@ class Fp16BertEncoder:
                 setattr(q, k, b[k].data_ptr())
         arrays = (ids, segs, cu)
         dev, starts = self._staging.upload(arrays)
-        if torch.cuda.current_stream().cuda_stream != self.stream:
-            torch.cuda.current_stream().synchronize()  # the pass runs on the stream the encoder was built on
         for k, a, start in zip(("ids", "segs", "cu"), arrays, starts):
             self.buf[k] = dev[start:start + len(a)]
         q = self._native[2]
@@ -228,7 +232,8 @@ class Fp16BertEncoder:
 
     def enqueue(self, ids=None, segs=None, cu=None, capture: dict | None = None):
         """One forward pass over the packed batch; returns the FP16 [T, hidden] output tensor (device).
-        With ids=None the inputs of the previous call are reused.  `capture`, if given, receives host copies of
+        With ids=None the inputs of the previous call are reused.  The pass runs on the stream that was current when the
+        encoder was built; another stream has to wait for it before it reads the output.  `capture`, if given, receives host copies of
         every intermediate tensor under the names emb, l<i>.qkv, l<i>.ctx, l<i>.ao, l<i>.h, l<i>.m, l<i>.f, l<i>.out."""
         if ids is not None:
             self._bind(ids, segs, cu)

@@ -87,3 +87,31 @@ def test_few_tokens_against_single_operations(setup, lens):
     torch.cuda.synchronize()
     assert_fp_close(got.cpu().numpy(), want, atol=1e-2, what="native pass")   # a few binary16 steps of values up to ~4
     enc.enqueue(ids, segs, cu)
+
+
+def test_passes_asked_for_on_another_stream(setup):
+    """Passes of changing sizes asked for while another stream is current, one after the other without waiting: memory that
+    a pass reads or writes is not given to a later one before it is through with it."""
+    import torch
+    cfg, enc, ids, segs, cu, cap, out = setup
+    r = rng(43)
+    batches, want = [], []
+    for n in (300, 20, 300, 7, 129, 300, 20, 64):
+        c = np.array([0, n // 2, n], np.int32)
+        batches.append((r.integers(0, cfg.vocab, n).astype(np.int32), r.integers(0, 2, n).astype(np.int32), c))
+        want.append(enc.enqueue(*batches[-1]).cpu().numpy())
+    home, other = torch.cuda.current_stream(), torch.cuda.Stream()
+    got = []
+    with torch.cuda.stream(other):
+        for b in batches:
+            x = enc.enqueue(*b)
+            # what the caching allocator hands out on this stream is no memory of a pass in flight
+            junk = [torch.full((n, c), 7, dtype=torch.float16, device="cuda") for n in (300, 129, 64) for c in (768, 3072)]
+            junk += [torch.full((1 << k,), 7, dtype=torch.int32, device="cuda") for k in range(2, 11)]
+            with torch.cuda.stream(home):
+                got.append(x.clone())
+            del junk
+    torch.cuda.synchronize()
+    for g, w in zip(got, want):
+        assert np.array_equal(g.cpu().numpy().view(np.uint16), w.view(np.uint16))
+    enc.enqueue(ids, segs, cu)
