@@ -190,6 +190,33 @@ def test_native_runner_with_few_tokens(setup, lens):
     enc.enqueue(ids, segs, cu)   # leave the fixture's buffers as the other tests expect them
 
 
+@pytest.fixture(scope="module")
+def large_model():
+    """Two layers of the 1024-channel model, whose second feed-forward layer is shared by up to four workgroups."""
+    cfg = EncoderConfig(hidden=1024, heads=16, ffn=4096, layers=2, vocab=1000, max_pos=512, max_seqlen=384, seed=8)
+    enc = Int8BertEncoder(cfg)
+    r = rng(10)
+    cu = np.array([0, 100, 300], np.int32)
+    enc.calibrate(r.integers(0, cfg.vocab, 300).astype(np.int32), r.integers(0, 2, 300).astype(np.int32), cu)
+    return cfg, enc
+
+
+@pytest.mark.parametrize("lens", [[1], [32], [20, 13], [64], [65], [90, 6], [128], [129], [200, 55], [256]])
+def test_native_runner_with_few_tokens_of_1024_channels(large_model, lens):
+    """Four parts up to 64 tokens, two up to 128, then none."""
+    import torch
+    cfg, enc = large_model
+    r = rng(32 + sum(lens))
+    c = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    t = int(c[-1])
+    i, s = r.integers(0, cfg.vocab, t).astype(np.int32), r.integers(0, 2, t).astype(np.int32)
+    want = enc.enqueue(i, s, c).cpu().numpy()
+    for _ in range(2):
+        got = enc.enqueue_native(i, s, c)
+        torch.cuda.synchronize()
+        assert np.array_equal(got.cpu().numpy(), want)
+
+
 def test_native_runner_replays_from_a_captured_graph(setup):
     """enqueue launches kernels only (no allocation, copy, memset or synchronisation), so a caller can record it
     into a graph.  Every replay is checked, with eager work on the same buffers between the replays."""

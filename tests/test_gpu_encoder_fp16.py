@@ -89,6 +89,48 @@ def test_few_tokens_against_single_operations(setup, lens):
     enc.enqueue(ids, segs, cu)
 
 
+@pytest.fixture(scope="module")
+def one_layer():
+    """One-layer models: their intermediate buffers still hold that layer's values after a native pass."""
+    made = {}
+
+    def get(hidden, ffn):
+        if hidden not in made:
+            made[hidden] = Fp16BertEncoder(EncoderConfig(hidden=hidden, heads=hidden // 64, ffn=ffn, layers=1, vocab=500,
+                                                         max_pos=512, max_seqlen=384, seed=13))
+        return made[hidden]
+    return get
+
+
+@pytest.mark.parametrize("hidden,ffn", [(768, 3072), (1024, 4096), (512, 2048), (320, 2048)])
+@pytest.mark.parametrize("lens", [[1], [32], [20, 13], [64], [70, 26]])
+def test_normalisation_of_partial_sums(one_layer, hidden, ffn, lens):
+    """Few tokens: the partial sums of the second feed-forward layer add up to that layer's accumulators, and the
+    normalisation that reads them is the oracle's SkipLayerNorm of the layer's output."""
+    import torch
+    enc = one_layer(hidden, ffn)
+    r = rng(44 + sum(lens))
+    c = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    t = int(c[-1])
+    enc._partial.zero_()   # at most four parts: the sums of parts that do not exist are 0
+    out = enc.enqueue(r.integers(0, 500, t).astype(np.int32), r.integers(0, 2, t).astype(np.int32), c)
+    torch.cuda.synchronize()
+    sums = enc._partial.view(torch.float32)[:4 * t * hidden].cpu().numpy().reshape(4, t, hidden)
+    assert np.abs(sums[1]).max() > 0, "more than one part"
+    m, h = (enc.buf[k].cpu().numpy() for k in ("m", "h"))
+    L = enc.layers[0]
+    lin = L["ffn2"]
+    acc = m.astype(np.float64) @ lin.w_h.astype(np.float64).T
+    total = sums.astype(np.float64).sum(0)
+    # ffn products of binary32 accumulations in any order: |error| <= ffn * 2^-24 * sum |m w|, far below that in practice
+    bound = ffn * 2.0 ** -24 * (np.abs(m).astype(np.float64) @ np.abs(lin.w_h).astype(np.float64).T)
+    assert (np.abs(total - acc) <= bound + 1e-12).all()
+    f = oracle.fp16_linear(m, lin.w_h, lin.alpha_h, lin.bias_h)
+    half = lambda a: a.astype(np.float16)
+    want = oracle.skipln(f, h, half(L["ln2_beta"]), half(L["ln2_gamma"]), half(L["ln2_bias"]))
+    assert_fp_close(out.cpu().numpy(), want, what="SkipLayerNorm of partial sums")
+
+
 def test_passes_asked_for_on_another_stream(setup):
     """Passes of changing sizes asked for while another stream is current, one after the other without waiting: memory that
     a pass reads or writes is not given to a later one before it is through with it."""

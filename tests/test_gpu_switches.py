@@ -38,11 +38,16 @@ LINEAR_SETTINGS = [("TRTAMD_LINEAR_DIRECT", 0), ("TRTAMD_LINEAR_PERSISTENT", 0),
                    ("TRTAMD_LINEAR_PARTIAL_ROUND", 100)]
 
 
-def test_remainder_pieces_against_remainder_tiles():
-    """More than half a round of large tiles (so that they run, as a partial round) and 60 tokens behind them: by
-    default those go in 64 x 64 pieces whose wavefronts split k, with TRTAMD_LINEAR_PIECES=0 in 128 x 128 tiles; both
-    must give the oracle's accumulator-exact results and the same bytes."""
-    T, K, N = 133 * 256 + 60, 256, 512
+@pytest.mark.parametrize("T", [67 * 256 + 60, 133 * 256 + 60])
+def test_remainder_pieces_against_remainder_tiles(T):
+    """Large tiles as a partial round with 60 tokens behind them, and as a whole round with 1340: those go in 64 x 64
+    pieces whose wavefronts split k, with TRTAMD_LINEAR_PIECES=0 in 128 x 128 tiles; both must give the oracle's
+    accumulator-exact results and the same bytes."""
+    with tuning("TRTAMD_LINEAR_PLAN", 0):   # the cost model may prefer smaller tiles for all of it
+        _remainder_pieces_against_remainder_tiles(T, 256, 512)
+
+
+def _remainder_pieces_against_remainder_tiles(T, K, N):
     a, w, alpha, beta = problem(93, T, K, N)
     ref = oracle.int8_linear(a, w, alpha, beta, oracle.LINEAR_AFFINE, out_interleaved=True)
     pieces = run_gpu(a, w, alpha, beta, capi.LINEAR_AFFINE, a_il=True, out_il=True, w_il=True)
@@ -62,11 +67,16 @@ def test_remainder_pieces_against_remainder_tiles():
 
 @pytest.mark.parametrize("name,value", LINEAR_SETTINGS)
 @pytest.mark.parametrize("il", [True, False])
-def test_linear_variants(name, value, il):
-    """Shapes the direct-to-LDS kernel takes by default (N a multiple of 256, K of 256, a ragged token count with
-    whole 256-token tiles and a remainder): accumulators bit-exact, affine and GELU outputs to the oracle's bar and
-    equal to the default choice's bytes."""
-    T, K, N = 777, 1024, 512
+@pytest.mark.parametrize("T,K,N", [(777, 1024, 512), (70 * 256 + 9, 256, 512)])
+def test_linear_variants(T, K, N, name, value, il):
+    """Ragged token counts with whole 256-token tiles and a remainder, N and K multiples of 256: less than half a round of
+    large tiles (which run only with TRTAMD_LINEAR_PARTIAL_ROUND=0) and more (which run unless it is 100).  Accumulators
+    bit-exact, affine and GELU outputs to the oracle's bar and equal to the default setting's bytes."""
+    with tuning("TRTAMD_LINEAR_PLAN", 0):   # large tiles wherever the setting allows them
+        _linear_variants(T, K, N, name, value, il)
+
+
+def _linear_variants(T, K, N, name, value, il):
     a, w, alpha, beta = problem(91, T, K, N, full_range=True)
     with tuning(name, value):
         raw = run_gpu(a, w, None, None, capi.LINEAR_RAW_INT32, a_il=il, w_il=il)
@@ -85,8 +95,13 @@ def test_linear_variants(name, value, il):
         assert np.array_equal(got, default), f"{name}={value}: bytes differ from the default kernel choice"
 
 
-@pytest.mark.parametrize("plan", range(1, 10))
-@pytest.mark.parametrize("T,K,N", [(1, 64, 32), (33, 192, 96), (130, 448, 160), (259, 768, 288)])
+# large tiles: 132 of 256 CUs with one token behind them, 136 with 255, a round with 80 tiles' worth of smaller ones behind
+LARGE_TILE_SHAPES = [(33 * 256 + 1, 256, 1024), (34 * 256 + 255, 512, 1024), (84 * 256 + 33, 256, 1024)]
+
+
+@pytest.mark.parametrize("plan,T,K,N", [(plan, *shape) for plan in range(1, 10) for shape in
+                                        [(1, 64, 32), (33, 192, 96), (130, 448, 160), (259, 768, 288)]]
+                         + [(0, *shape) for shape in LARGE_TILE_SHAPES])
 def test_linear_plans(plan, T, K, N):
     """Every tile shape of the linear layers at the edges of its tiles (one token, one past a block, channels and k that
     are no multiple of a tile; k shorter than the ring of stages), both layouts, INT8 and FP16: the oracle's bar, and
@@ -134,12 +149,14 @@ def test_int8_attention_variants(name, value, interleaved):
         int8_attention_parity(qkv, cu, N, s1, ss, s2, interleaved, S=S, expect=default)
 
 
-@pytest.mark.parametrize("name,value", FMHA_SETTINGS)
-def test_fp16_attention_variants(name, value):
+# In FP16 only the kernel of many units of more than 384 keys shares a unit's queries by the launch size; where K and V take
+# turns in LDS a workgroup has 64 of them.
+@pytest.mark.parametrize("name,value,S,lens", [(n, v, 512, [512, 7, 385, 130] * 22) for n, v in FMHA_SETTINGS]
+                         + [(n, v, 384, [384, 7, 250, 130]) for n, v in FMHA_SETTINGS if n != "TRTAMD_FMHA_QSPLIT"])
+def test_fp16_attention_variants(name, value, S, lens):
     api = capi.api()
     r = rng(1300 + value)
-    B, N, S = 4, 3, 384
-    lens = np.array([384, 7, 250, 130])
+    B, N = len(lens), 3
     cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     T = int(cu[-1])
     qkv = (r.standard_normal((T, N, 3, 64)) * 0.7).astype(np.float16)
