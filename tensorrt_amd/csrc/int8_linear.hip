@@ -1732,14 +1732,19 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
 // chip where the problem has few of them, large ones move fewer bytes per multiplication where it has many, and the pieces
 // cut the chain of stages by eight where neither fills it.
 //
-// The constants are a fit to launches of 16 to 33289 tokens on the four layers of a 1024-channel INT8 encoder (graph
-// replays, every launch with weights that are in no cache) and of a 768-channel FP16 one (weights in the last-level
-// cache): every row within 3-9 %, and the choice on average 0.6 % (interleaved) and 0.4 % (linear) slower than the fastest
-// of all kernels at each of the 128 points, 17 % at worst.  Before, every launch short of half a round of large tiles went
-// in 128 x 128 tiles staged through registers (weights in the last-level cache): 40 tokens x (1024 -> 3072 /
-// 4096 -> 1024) INT8 7.2 / 19.1 -> 3.7 / 4.7 us, 600 tokens 7.4 / 19.0 -> 5.2 / 7.9 us, 5300 tokens 20.5 / 43.0 -> 20.9 /
-// 27.1 us; FP16 40 tokens x (768 -> 2304 / 3072 -> 768) 9.7 / 29.9 -> 4.0 / 7.2 us, 9100 tokens x 3072 -> 768 80.0 ->
-// 54.4 us.
+// The constants are fits.  Linear operands: to launches by themselves on the four layers of a 768-channel FP16 encoder
+// (graph replays, weights in the last-level cache).  Interleaved operands: to launches by themselves on those of a
+// 1024-channel INT8 encoder with weights from memory, and the ones that decide from 2500 tokens on (large tiles, 128 x 256,
+// 128 x 128, 64 x 128, 128 x 128 deep) to whole passes of that encoder with the plans of one or two of its layers changed at a
+// time: what a launch takes by itself does not say what it costs the ones around it.  At 9084 tokens 128 x 128 tiles are the
+// faster ones for either feed-forward layer by itself, and the pass is 2.5 % faster with large tiles for both.  Over 28
+// sizes of 3300 to 21000 tokens the pass takes 1.1 % less than with constants for launches by themselves, none takes more,
+// and the best of the measured combinations would take another 1.1 % less (4 % at most).  32 sequences of up to 256 tokens:
+// 2945 -> 2798 us.
+// Against 128 x 128 tiles staged through registers for every launch short of half a round of large tiles (single launches,
+// weights in the last-level cache): 40 tokens x (1024 -> 3072 / 4096 -> 1024) INT8 7.2 / 19.1 -> 3.7 / 4.7 us, 600 tokens
+// 7.4 / 19.0 -> 5.2 / 7.9 us, 5300 tokens 20.5 / 43.0 -> 20.9 / 27.1 us; FP16 40 tokens x (768 -> 2304 / 3072 -> 768) 9.7 /
+// 29.9 -> 4.0 / 7.2 us, 9100 tokens x 3072 -> 768 80.0 -> 54.4 us.
 // Deep rings: where one workgroup per CU is all there is, a tile is bound by the trips to memory of its own stages, and
 // the LDS of the workgroups that do not come is better used for more of them (interleaved, weights from memory, 600 tokens
 // x 4096 -> 1024 in 64 x 64 tiles: 12.9 us with three stages ahead, 9.5 us with seven; 128 x 128 tiles, 1900 tokens 20.8
@@ -1771,9 +1776,9 @@ constexpr TileCost kTileCosts[2][kLinearPlans] = {
         {128, 128, 2, 1.93f, 1.06f, 0.292f, 0.41f, 1.30f, 1.10f, 0.53f}, {64, 128, 3, 2.49f, 0.32f, 0.188f, 0.21f, 1.27f, 1.14f, 0.52f},
         {64, 64, 4, 2.29f, 0.30f, 0.138f, 0.13f, 0.94f, 0.89f, 0.47f}, {}, {}, {},
         {32, 64, 1, 2.88f, 0.30f, 0.071f, 0.05f, 0.57f, 1.91f, 0.80f}, {32, 32, 1, 2.38f, 0.34f, 0.053f, 0.13f, 1.48f, 1.49f, 0.68f}},
-    {{256, 256, 1, 0.00f, 3.12f, 0.780f, 2.97f, 0.f, 0.f, 0.f}, {128, 256, 2, 2.72f, 0.81f, 0.391f, 1.33f, 1.25f, 1.12f, 0.54f},
-        {128, 128, 3, 3.06f, 0.45f, 0.276f, 0.67f, 0.85f, 0.86f, 0.30f}, {64, 128, 3, 2.96f, 0.26f, 0.169f, 0.32f, 0.90f, 0.85f, 0.26f},
-        {64, 64, 4, 3.19f, 0.04f, 0.141f, 0.24f, 0.60f, 0.66f, 0.00f}, {128, 128, 2, 3.04f, 0.62f, 0.221f, 0.66f, 1.29f, 1.06f, 0.44f},
+    {{256, 256, 1, 0.00f, 3.72f, 0.513f, 4.84f, 0.f, 0.f, 0.f}, {128, 256, 2, 2.72f, 0.81f, 0.391f, 1.43f, 1.05f, 1.57f, 0.62f},
+        {128, 128, 3, 3.06f, 0.80f, 0.242f, 0.39f, 0.84f, 1.06f, 0.43f}, {64, 128, 3, 2.96f, 0.26f, 0.169f, 0.32f, 1.34f, 1.44f, 0.04f},
+        {64, 64, 4, 3.19f, 0.04f, 0.141f, 0.24f, 0.60f, 0.66f, 0.00f}, {128, 128, 2, 3.04f, 0.62f, 0.221f, 0.66f, 1.56f, 1.31f, 0.39f},
         {64, 128, 2, 2.54f, 0.60f, 0.150f, 0.32f, 1.22f, 0.93f, 0.35f}, {64, 64, 2, 2.46f, 0.54f, 0.100f, 0.35f, 0.93f, 0.91f, 0.46f},
         {32, 64, 2, 3.19f, 0.17f, 0.068f, 0.04f, 0.90f, 1.19f, 0.67f}, {32, 32, 4, 2.69f, 1.21f, 0.042f, 0.16f, 0.67f, 1.19f, 0.64f}}};
 
@@ -1798,17 +1803,16 @@ inline float large_tiles_time(TileCost const& c, bool il, LinearArgs const& a, i
     {
         return c.launch + rounds * (c.tile + (gelu ? c.gelu : 0.f) + c.stage * stages) + (float) smallTiles / cus * 0.66f * stages;
     }
-    float const fill = (float) a.mainTiles / (rounds * cus); // a part of the chip is less in its own way
     float rest = 0.f;
     if (a.pieces)
     {
-        rest = (float) (a.N / 64) * (float) ceil_div(a.T - a.tokMain * kBig, 64) / cus * 5.57f;
+        rest = (float) (a.N / 64) * (float) ceil_div(a.T - a.tokMain * kBig, 64) / cus * (6.48f + 0.206f * stages);
     }
     else if (smallTiles)
     {
-        rest = std::ceil((float) smallTiles / cus) * (0.83f + (gelu ? 0.25f * c.gelu : 0.f) + 0.38f * stages);
+        rest = std::ceil((float) smallTiles / cus) * (0.83f + (gelu ? 0.25f * c.gelu : 0.f) + 0.464f * stages);
     }
-    return c.launch + rounds * (c.tile + (gelu ? c.gelu : 0.f) + c.stage * (0.75f + 0.25f * fill) * stages) + rest;
+    return c.launch + rounds * (c.tile + (gelu ? c.gelu : 0.f) + c.stage * stages) + rest;
 }
 
 // The workgroups of a.mainTiles tiles, with those that fetch a.prefetch behind them where the launch leaves CUs idle.
@@ -1916,10 +1920,10 @@ int choose_plan(LinearArgs const& a, int64_t smallTiles, bool gelu)
     {
         return plan;
     }
-    // the smaller tiles read more bytes per multiplication; a network's pass runs at the chip's power limit and
-    // pays for that in the clock of the kernels around it: they have to win by more than 8 % (the pass of 128
-    // sequences as two halves against large tiles only: +1.1 % without the margin, +0.3 +- 0.5 % with it)
-    constexpr float kMargin = 1.f / 1.08f;
+    // Linear operands: the smaller tiles have to win by more than 8 %.  They read more bytes per multiplication, which a pass
+    // pays for in the launches around them too, and these constants are for launches by themselves (FP16 passes of 1000 to
+    // 25000 tokens without it: another choice at 5 of 17 sizes, 0.0 to 1.9 % slower; nowhere faster).
+    constexpr float kMargin = IL ? 1.f : 1.f / 1.08f;
     float best = large ? kMargin * large_tiles_time(kTileCosts[IL][kLargeTiles], IL, a, smallTiles, gelu)
                        : std::numeric_limits<float>::max();
     plan = kLargeTiles;
