@@ -58,7 +58,9 @@ TRTAMD_API int trtamd_int8_linear(trtamd_stream_t stream, trtamd_int8_linear_par
 /* FP16 linear layer for the FP16 encoder: out[t][n] = binary16(f(fmaf(acc, alpha[n], beta[n]))), acc = sum_k
  * a[t][k] * w[n][k] accumulated in binary32 on the FP16 matrix cores, f = identity (TRTAMD_LINEAR_AFFINE) or erf-GELU
  * (TRTAMD_LINEAR_GELU).  alpha = 1 and beta = bias give the usual fully-connected layer.  All tensors linear:
- * a [T][K], w [N][K], out [T][N]; K % 32 == 0, N % 32 == 0.  The open counterpart in the reference is the deprecated
+ * a [T][K], w [N][K], out [T][N]; K % 32 == 0, N % 32 == 0.  The order in which the K products are added (one after the
+ * other, or in eight sums that meet at the end) depends on T, K and N, so a row can come out a binary16 step apart in calls
+ * of different T; calls of the same sizes give the same bits.  The open counterpart in the reference is the deprecated
  * cuBLASLt GEMM plugin CustomFCPluginDynamic (plugin/fcPlugin/README.md:20-45, FP16 without bias or activation);
  * bias and GELU are what TensorRT's core fuses onto it. */
 typedef struct trtamd_fp16_linear_params

@@ -108,6 +108,11 @@ TRTAMD_API int trtamd_encoder_enqueue_concurrent(trtamd_encoder_t encoder, trtam
  * with bias, feed-forward GEMM + GELU, feed-forward GEMM, SkipLayerNorm v6 ]).  One call enqueues one pass; the plugin
  * objects (runtime phase, IPluginV3*), the device weights and the activation buffers are the caller's, and the call only
  * launches.  A plugin object serves one pass at a time: it keeps per-shape state between onShapeChange and enqueue.
+ * The linear layers add their products in an order that depends on `tokens` (trtamd_fp16_linear), and with few tokens the
+ * second feed-forward layer's are added in up to four parts, in the normalisation behind it.  Sums are binary32 in every
+ * order; a sequence by itself and the same sequence in a larger batch differ by such rounding (1.5e-3 relative after 12
+ * layers of 768 channels), as does a pass from the same operations called one by one.  The same batch sizes give the same
+ * bits.  (The INT8 pass above adds integers: its bytes do not depend on the batch around a sequence.)
  * tensorrt_amd/encoder_fp16.py is the builder side.
  * ------------------------------------------------------------------------------------------ */
 typedef struct trtamd_fp16_encoder_linear

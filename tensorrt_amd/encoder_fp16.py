@@ -234,7 +234,9 @@ class Fp16BertEncoder:
         """One forward pass over the packed batch; returns the FP16 [T, hidden] output tensor (device).
         With ids=None the inputs of the previous call are reused.  The pass runs on the stream that was current when the
         encoder was built; another stream has to wait for it before it reads the output.  `capture`, if given, receives host copies of
-        every intermediate tensor under the names emb, l<i>.qkv, l<i>.ctx, l<i>.ao, l<i>.h, l<i>.m, l<i>.f, l<i>.out."""
+        every intermediate tensor under the names emb, l<i>.qkv, l<i>.ctx, l<i>.ao, l<i>.h, l<i>.m, l<i>.f, l<i>.out; the
+        operations then run one by one, and with few tokens the second feed-forward layer's sums are added in another order
+        than in the native pass (include/trtamd_encoder_runtime.h)."""
         if ids is not None:
             self._bind(ids, segs, cu)
         b = self.buf
