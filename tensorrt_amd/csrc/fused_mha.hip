@@ -1648,8 +1648,9 @@ __global__ __launch_bounds__(kWavesF16* kWaveSize) void fmha_f16_prefix_kernel(F
 // or its V, and a unit's queries are shared out 64 at a time over as many workgroups.  What bounds either kernel is that
 // wait; with one workgroup per CU nothing covered it.  All of Q, K and V come by direct-to-LDS loads, whose number in
 // flight the waits below count; a wavefront requests 16 rows of every block.  12 heads, sequences of a third of the length
-// to the length, before and after: 32 x 128 keys 12.9 -> 5.8 us, 128 x 256 42.8 -> 35.7 us, 32 x 384 20.7 -> 20.1 us,
-// 128 x 384 71.5 -> 64.8 us.
+// to the length, that kernel / this one, us per plugin call: 32 x 128 keys 12.5 / 5.8, 128 x 256 41.7 / 37.5, 32 x 384
+// 19.8 / 19.6, 128 x 384 71.7 / 64.6, 16 x 512 22.8 / 19.5.  What is left is the L2: K and V of a unit are read once for every
+// 64 queries, 133 MB for the 35.8 MB of 32 x 384.
 // ------------------------------------------------------------------------------------------
 constexpr int kQueriesF16 = kWavesF16T * kQPerWave;
 __device__ u32x4 const kZeroRow[8] = {}; // 64 binary16 zeros, in memory

@@ -288,7 +288,7 @@ def config_rows(api, torch, steps: int = 100, seed: int = 1, cpu: bool = True, l
                     q, k, v = (cq[lo:hi, :, i].transpose(0, 1) for i in range(3))
                     torch.softmax(q @ k.transpose(1, 2) * 0.125, -1) @ v
             cpu_s = _cpu_time(attn_cpu)
-        report("C3", "QKV-to-context v5 (fmha_f16_prefix_kernel)", "fp16", f"B=32 N=12 S={S}, {T} tokens", t, ops=ops,
+        report("C3", "QKV-to-context v5 (fmha_f16_turns_kernel)", "fp16", f"B=32 N=12 S={S}, {T} tokens", t, ops=ops,
                peak_ops=PEAK_F16, cpu_s=cpu_s)
 
     # ---- C3, the fixed [S,B,N,3,d] layout with the packed key mask (v4 plugin with a mask input) ----------
