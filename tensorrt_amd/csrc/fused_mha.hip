@@ -57,7 +57,8 @@ __device__ inline float mul_rounded(float a, float b)
     return a * b;
 }
 
-// The MFMAs of the cu_seqlens kernels (fmha_i8_prefix_kernel, fmha_f16_prefix_kernel) go through these wrappers.  A
+// The MFMAs of the cu_seqlens kernels (fmha_i8_prefix_kernel, fmha_f16_turns_kernel, fmha_f16_prefix_kernel) go through
+// these wrappers.  A
 // library built with -DTRTAMD_ABLATE_ATTENTION_MFMA (`python -m tensorrt_amd.build --ablation` writes it to
 // lib/libtrtamd_ablation.so; `python -m tensorrt_amd.kernel_bench --ablation` times it; nothing else loads it) leaves
 // the instruction out: the result registers keep what they held and every other instruction of the kernel stays, so

@@ -1,6 +1,6 @@
-"""GPU parity of the unfused attention path (head sizes <= 128: one launch that keeps a query's scores in registers
-for S <= 512 and walks the keys twice beyond; larger head sizes: the strided batched GEMMs around the scaled/masked
-softmax) and of zeroPadding2d, through the C ABI."""
+"""GPU parity of the unfused attention path (head sizes <= 128: one launch; FP32 up to 1024 keys splits them between
+wavefronts, otherwise a query's scores stay in registers for S <= 512 and the keys are walked twice beyond; larger head
+sizes: the strided batched GEMMs around the scaled/masked softmax) and of zeroPadding2d, through the C ABI."""
 import ctypes as C
 
 import numpy as np
