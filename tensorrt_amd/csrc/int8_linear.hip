@@ -1965,7 +1965,7 @@ bool is_piece(int plan)
 // there is nothing left to share them between.
 int parts_of(int plan, LinearArgs const& a)
 {
-    if (plan != kPiece32x32 || a.T <= 0)
+    if (plan != kPiece32x32 || a.T <= 0 || a.T > kLinearPartialTokens || a.K < kLinearPartialK)
     {
         return 1;
     }

@@ -32,6 +32,8 @@ int linear_parts(trtamd_int8_linear_params const& p);
 int linear_parts(trtamd_fp16_linear_params const& p);
 // Bytes that the partial sums of any such layer fit in: they come from one workgroup per CU at most, 32 x 32 of them each.
 size_t linear_partial_bytes();
+// linear_parts is 1 for more tokens than these and for layers of fewer bytes of k.
+constexpr int kLinearPartialTokens = 255, kLinearPartialK = 2048;
 // `parts`: what linear_parts said.  The parameters are checked as the public calls check theirs.
 int int8_linear_partial(trtamd_stream_t stream, trtamd_int8_linear_params const& p, int parts, int32_t* partial,
     WeightPrefetch const& prefetch);

@@ -12,6 +12,7 @@
 #include "../host_utils.hpp"
 #include "../network_ops.hpp"
 
+#include <algorithm>
 #include <memory>
 #include <string>
 #include <vector>
@@ -274,13 +275,13 @@ public:
         return static_cast<int32_t>(mContexts.size());
     }
 
-    // emb fp16 | x | qkv | ctx | ao | h | m | f | dummy | emb's second output | partial sums of ffn2
+    // Enough for every number of tokens up to this one: those few that have the partial sums of ffn2 behind the tensors need
+    // more than somewhat more tokens without.
     size_t workspaceSize(int32_t tokens) const
     {
-        size_t const T = static_cast<size_t>(tokens > 0 ? tokens : 0);
-        size_t const E = static_cast<size_t>(mCfg.hidden), F = static_cast<size_t>(mCfg.ffn);
-        return align256(T * E * 2) + 5 * align256(T * E) + align256(3 * T * E) + align256(T * F)
-            + align256(sizeof(int32_t) * static_cast<size_t>(mCfg.max_seqlen)) + 256 + align256(linear_partial_bytes());
+        size_t const size = tensorBytes(tokens);
+        return sharesFfn2() ? std::max(size, tensorBytes(std::min(tokens, kLinearPartialTokens)) + align256(linear_partial_bytes()))
+                            : size;
     }
 
     int enqueue(int32_t const* ids, int32_t const* segs, int32_t const* cu, int32_t batch, int32_t tokens,
@@ -421,6 +422,21 @@ private:
         Side side;
     };
 
+    // Whether the second feed-forward layer of few tokens may be shared between workgroups, as partial sums.
+    bool sharesFfn2() const
+    {
+        return (mCfg.hidden == 768 || mCfg.hidden == 1024) && mCfg.ffn >= kLinearPartialK;
+    }
+
+    // emb fp16 | x | qkv | ctx | ao | h | m | f | dummy | emb's second output
+    size_t tensorBytes(int32_t tokens) const
+    {
+        size_t const T = static_cast<size_t>(tokens > 0 ? tokens : 0);
+        size_t const E = static_cast<size_t>(mCfg.hidden), F = static_cast<size_t>(mCfg.ffn);
+        return align256(T * E * 2) + 5 * align256(T * E) + align256(3 * T * E) + align256(T * F)
+            + align256(sizeof(int32_t) * static_cast<size_t>(mCfg.max_seqlen)) + 256;
+    }
+
     void requireComplete() const
     {
         TRTAMD_VALIDATE_MSG(mContexts[0].embedding != nullptr, "set_embedding has not been called");
@@ -477,7 +493,7 @@ private:
             f = reinterpret_cast<int8_t*>(carve(T * E));
             dummy = carve(sizeof(int32_t) * static_cast<size_t>(enc.mCfg.max_seqlen)); // only its extent is read
             emb2 = carve(256);
-            partial = reinterpret_cast<int32_t*>(carve(linear_partial_bytes()));
+            partial = reinterpret_cast<int32_t*>(base); // behind the tensors, where ffn2Parts says so
             if (enc.mLayers.empty())
             {
                 qkvAhead = projAhead = ffn1Ahead = ffn2Ahead = {nullptr, 0};
@@ -491,7 +507,7 @@ private:
             ffn1Ahead = prefetch_of(L.ffn1.params(h, m, tokens, TRTAMD_LINEAR_GELU, 1.f));
             auto const f2 = L.ffn2.params(m, f, tokens, TRTAMD_LINEAR_AFFINE, 1.f);
             ffn2Ahead = prefetch_of(f2);
-            ffn2Parts = enc.mCfg.hidden == 768 || enc.mCfg.hidden == 1024 ? linear_parts(f2) : 1;
+            ffn2Parts = enc.sharesFfn2() ? linear_parts(f2) : 1;
         }
 
         template <size_t NI, size_t NO>

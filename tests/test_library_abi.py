@@ -82,6 +82,15 @@ def test_encoder_runtime_rejects_bad_configurations(lib):
     assert h
     # emb fp16 + five hidden-wide INT8 tensors + QKV + FFN intermediate + the two small extras, each 256-byte aligned
     assert a.encoder_workspace_size(h, 100) == 25600 + 5 * 12800 + 38400 + 25600 + 512 + 256
+    large = capi.EncoderConfig(hidden=1024, heads=16, ffn=4096, layers=1, vocab=10, max_pos=8, type_vocab=2, max_seqlen=128)
+    big = a.encoder_create(ctypes.byref(large))
+    tensors = lambda t: t * 14 * 1024 + 512 + 256
+    # the sums of the second feed-forward layer stand behind the tensors of up to 255 tokens: 32 x 32 of them per CU
+    few = tensors(255) + 256 * 4096
+    assert a.encoder_workspace_size(big, 32) == tensors(32) + 256 * 4096
+    assert a.encoder_workspace_size(big, 255) == a.encoder_workspace_size(big, 256) == few
+    assert a.encoder_workspace_size(big, 33289) == tensors(33289)
+    a.encoder_destroy(big)
     assert a.encoder_enqueue(h, None, None, None, 1, 100, None, None, None) != 0
     assert "set_embedding" in a.last_error_str()
     assert a.encoder_set_layer(h, 3, ctypes.byref(capi.EncoderLayer())) != 0
