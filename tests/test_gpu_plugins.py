@@ -157,10 +157,13 @@ def emb_fields(w, fp16, extra=()):
             i32("output_fp16", fp16)] + list(extra)
 
 
-@pytest.mark.parametrize("S,mha_type,fp16", [(128, 1, 1), (384, 2, 1), (64, 1, 1), (100, 1, 1), (128, 0, 0)])
-def test_embln_v6_plugin(reg, S, mha_type, fp16):
+@pytest.mark.parametrize("S,mha_type,fp16,B,ld", [
+    (128, 1, 1, 4, 256), (384, 2, 1, 4, 256), (64, 1, 1, 4, 256), (100, 1, 1, 4, 256), (128, 0, 0, 4, 256),
+    # four tokens per wavefront (from 65536 on) behind either kind of mask workgroups, and rows that are no whole vectors
+    (384, 1, 1, 171, 64), (100, 1, 1, 657, 64), (128, 0, 0, 513, 32), (96, 1, 1, 5, 30), (70, 0, 0, 9, 31)])
+def test_embln_v6_plugin(reg, S, mha_type, fp16, B, ld):
     r = rng(110 + S)
-    ld, B, vocab = 256, 4, 500
+    vocab = 500
     w = emb_weights(r, ld, vocab, S)
     c = reg.get_creator(EMBLN, "6")
     p = through_runtime(c, c.create_plugin("emb", emb_fields(w, fp16, [i32("mha_type_id", mha_type)])))
