@@ -10,7 +10,8 @@
 
 #include "trtamd_plugin_c.h"
 
-#include <vector>
+#include <memory>
+#include <new>
 
 namespace
 {
@@ -115,7 +116,13 @@ public:
         mCount = PySequence_Fast_GET_SIZE(seq);
         if (mCount > kInline)
         {
-            mHeap.resize(static_cast<size_t>(mCount));
+            mHeap.reset(new (std::nothrow) T[static_cast<size_t>(mCount)]{}); // no exception may leave for the interpreter
+            if (!mHeap)
+            {
+                Py_DECREF(seq);
+                PyErr_NoMemory();
+                return false;
+            }
         }
         bool ok = true;
         for (Py_ssize_t i = 0; ok && i < mCount; ++i)
@@ -127,7 +134,7 @@ public:
     }
     T* data()
     {
-        return mCount > kInline ? mHeap.data() : mInline;
+        return mCount > kInline ? mHeap.get() : mInline;
     }
     int32_t count() const
     {
@@ -136,7 +143,7 @@ public:
 
 private:
     T mInline[kInline]{};
-    std::vector<T> mHeap;
+    std::unique_ptr<T[]> mHeap;
     Py_ssize_t mCount{0};
 };
 

@@ -143,3 +143,25 @@ def test_missing_library_is_loud(monkeypatch, tmp_path):
     monkeypatch.setattr(tensorrt_amd, "_LIB", str(tmp_path / "nope.so"))
     with pytest.raises(tensorrt_amd.LibraryNotBuilt):
         tensorrt_amd.load_library()
+
+
+def test_plugin_call_reports_lack_of_memory():
+    """Descriptions beyond those kept in place go to the heap: no memory for them is a MemoryError, not an abort."""
+    import subprocess
+    import sys
+    path = os.path.join(os.path.dirname(tensorrt_amd._LIB), "_plugin_call.so")
+    code = f"""
+import importlib.machinery, importlib.util, resource
+loader = importlib.machinery.ExtensionFileLoader("_plugin_call", {path!r})
+module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_plugin_call", loader))
+loader.exec_module(module)
+many = [None] * (8 << 20)  # at 56 bytes a description and more: 448 MiB
+used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (used + (256 << 20),) * 2)
+try:
+    module.on_shape_change(0, 0, many, [])
+except MemoryError:
+    print("MemoryError")
+"""
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert (out.returncode, out.stdout) == (0, "MemoryError\n"), out.stderr
