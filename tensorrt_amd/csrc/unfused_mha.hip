@@ -480,9 +480,9 @@ int can_vectorise(T const* base, GemmOperand const& o)
 
 // ------------------------------------------------------------------------------------------
 // The same attention in one launch, for sequences whose scores fit in registers (S <= 512, head size <= 128) and that
-// attention_split_keys (binary32) does not take or where it is the slower one: no score matrix goes to memory.  A workgroup
-// of four wavefronts owns 64 queries of one (batch, head), a wavefront 16 of them with ALL their keys, so the row maximum and sum need no exchange between wavefronts.  The matrix products
-// are computed transposed, S^T = K Q^T and O^T = V^T P^T, with the 16 x 16 MFMA tiles: a lane then holds, for its
+// attention_split_keys (binary32) does not take or where it is the slower one: no score matrix goes to memory.  A
+// workgroup of four wavefronts owns 64 queries of one (batch, head), a wavefront 16 of them with ALL their keys, so the
+// row maximum and sum need no exchange between wavefronts.  The matrix products are computed transposed, S^T = K Q^T and O^T = V^T P^T, with the 16 x 16 MFMA tiles: a lane then holds, for its
 // one query, four consecutive keys per tile — the softmax reductions run inside the lane (plus two lane exchanges),
 // and the probabilities are, as they stand in the accumulator registers, the B operand of the second product.  The
 // order in which a lane's eight (binary16) or four (binary32) k positions of a step map to dimensions / keys is
