@@ -1737,10 +1737,10 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
 // 1024-channel INT8 encoder with weights from memory, and the ones that decide from 2500 tokens on (large tiles, 128 x 256,
 // 128 x 128, 64 x 128, 128 x 128 deep) to whole passes of that encoder with the plans of one or two of its layers changed at a
 // time: what a launch takes by itself does not say what it costs the ones around it.  At 9084 tokens 128 x 128 tiles are the
-// faster ones for either feed-forward layer by itself, and the pass is 2.5 % faster with large tiles for both.  Over 28
-// sizes of 3300 to 21000 tokens the pass takes 1.1 % less than with constants for launches by themselves, none takes more,
-// and the best of the measured combinations would take another 1.1 % less (4 % at most).  32 sequences of up to 256 tokens:
-// 2945 -> 2798 us.
+// faster ones for either feed-forward layer by itself, and the pass is 2.5 % faster with large tiles for both.  Over 142
+// sizes of 2465 to 23000 tokens the pass takes 0.8 % less than with constants for launches by themselves, one of them more
+// than 0.8 % more (7399 tokens, 1.9 %), and the best of the measured combinations would take another 0.9 % less (4 % at
+// most).  32 sequences of up to 256 tokens: 2979 -> 2877 us.
 // Against 128 x 128 tiles staged through registers for every launch short of half a round of large tiles (single launches,
 // weights in the last-level cache): 40 tokens x (1024 -> 3072 / 4096 -> 1024) INT8 7.2 / 19.1 -> 3.7 / 4.7 us, 600 tokens
 // 7.4 / 19.0 -> 5.2 / 7.9 us, 5300 tokens 20.5 / 43.0 -> 20.9 / 27.1 us; FP16 40 tokens x (768 -> 2304 / 3072 -> 768) 9.7 /
@@ -1776,9 +1776,9 @@ constexpr TileCost kTileCosts[2][kLinearPlans] = {
         {128, 128, 2, 1.93f, 1.06f, 0.292f, 0.41f, 1.30f, 1.10f, 0.53f}, {64, 128, 3, 2.49f, 0.32f, 0.188f, 0.21f, 1.27f, 1.14f, 0.52f},
         {64, 64, 4, 2.29f, 0.30f, 0.138f, 0.13f, 0.94f, 0.89f, 0.47f}, {}, {}, {},
         {32, 64, 1, 2.88f, 0.30f, 0.071f, 0.05f, 0.57f, 1.91f, 0.80f}, {32, 32, 1, 2.38f, 0.34f, 0.053f, 0.13f, 1.48f, 1.49f, 0.68f}},
-    {{256, 256, 1, 0.00f, 3.72f, 0.513f, 4.84f, 0.f, 0.f, 0.f}, {128, 256, 2, 2.72f, 0.81f, 0.391f, 1.43f, 1.05f, 1.57f, 0.62f},
-        {128, 128, 3, 3.06f, 0.80f, 0.242f, 0.39f, 0.84f, 1.06f, 0.43f}, {64, 128, 3, 2.96f, 0.26f, 0.169f, 0.32f, 1.34f, 1.44f, 0.04f},
-        {64, 64, 4, 3.19f, 0.04f, 0.141f, 0.24f, 0.60f, 0.66f, 0.00f}, {128, 128, 2, 3.04f, 0.62f, 0.221f, 0.66f, 1.56f, 1.31f, 0.39f},
+    {{256, 256, 1, 0.00f, 3.34f, 0.542f, 4.36f, 0.f, 0.f, 0.f}, {128, 256, 2, 2.72f, 0.81f, 0.391f, 1.69f, 1.03f, 1.39f, 0.63f},
+        {128, 128, 3, 3.06f, 0.79f, 0.233f, 0.53f, 0.87f, 1.01f, 0.47f}, {64, 128, 3, 2.96f, 0.26f, 0.169f, 0.32f, 1.59f, 0.94f, 0.00f},
+        {64, 64, 4, 3.19f, 0.04f, 0.141f, 0.24f, 0.60f, 0.66f, 0.00f}, {128, 128, 2, 3.04f, 0.62f, 0.221f, 0.66f, 1.62f, 1.38f, 0.61f},
         {64, 128, 2, 2.54f, 0.60f, 0.150f, 0.32f, 1.22f, 0.93f, 0.35f}, {64, 64, 2, 2.46f, 0.54f, 0.100f, 0.35f, 0.93f, 0.91f, 0.46f},
         {32, 64, 2, 3.19f, 0.17f, 0.068f, 0.04f, 0.90f, 1.19f, 0.67f}, {32, 32, 4, 2.69f, 1.21f, 0.042f, 0.16f, 0.67f, 1.19f, 0.64f}}};
 
@@ -1806,11 +1806,11 @@ inline float large_tiles_time(TileCost const& c, bool il, LinearArgs const& a, i
     float rest = 0.f;
     if (a.pieces)
     {
-        rest = (float) (a.N / 64) * (float) ceil_div(a.T - a.tokMain * kBig, 64) / cus * (6.48f + 0.206f * stages);
+        rest = (float) (a.N / 64) * (float) ceil_div(a.T - a.tokMain * kBig, 64) / cus * (6.63f + 0.175f * stages);
     }
     else if (smallTiles)
     {
-        rest = std::ceil((float) smallTiles / cus) * (0.83f + (gelu ? 0.25f * c.gelu : 0.f) + 0.464f * stages);
+        rest = std::ceil((float) smallTiles / cus) * (0.83f + (gelu ? 0.25f * c.gelu : 0.f) + 0.51f * stages);
     }
     return c.launch + rounds * (c.tile + (gelu ? c.gelu : 0.f) + c.stage * stages) + rest;
 }
