@@ -116,7 +116,7 @@ def clock_ramp(torch, step, seconds=0.25):
 
 
 def run_encoder(args, api, torch):
-    """the full 24-layer encoder.  Returns the JSON record."""
+    """The full 24-layer encoder.  Returns the JSON record."""
     from tensorrt_amd import capi
     from tensorrt_amd.encoder import EncoderConfig, Int8BertEncoder
     cfg = EncoderConfig(layers=args.layers, seed=args.seed, max_seqlen=args.seqlen)
@@ -268,7 +268,7 @@ def run_encoder(args, api, torch):
         "dtype": "int8",
         "data": "synthetic",
         "config": {
-            "workload": f"full {cfg.layers}-layer BERT-large INT8 encoder (configs[4]): EmbLayerNorm v4, quantise, per "
+            "workload": f"full {cfg.layers}-layer BERT-large INT8 encoder: EmbLayerNorm v4, quantise, per "
                         "layer QKV GEMM / QKV-to-context v6 / projection GEMM / SkipLayerNorm v7 / FFN GEMM+GELU / FFN "
                         "GEMM / SkipLayerNorm v7, dequantise; random-init weights, scales calibrated on the batch",
             "batch": args.batch, "max_seq_len": args.seqlen, "heads": N, "head_size": 64, "hidden": E, "ffn": F,
@@ -649,7 +649,7 @@ def main():
         "dtype": "int8",
         "data": "synthetic",
         "config": {
-            "workload": "BERT-large INT8 layer plugin path (configs[3]): QKV-to-context INT8 v6 kernel "
+            "workload": "BERT-large INT8 layer plugin path: QKV-to-context INT8 v6 kernel "
                         "(32-interleaved, cu_seqlens) + SkipLayerNorm INT8 v7 kernel; the GEMMs between plugins are "
                         "not part of the step",
             "batch": wl.B, "max_seq_len": wl.S, "heads": N, "head_size": 64, "hidden": E, "tokens": T,

@@ -139,7 +139,7 @@ def _cpu_time(fn, budget_s=0.4):
 
 
 def config_rows(api, torch, steps: int = 100, seed: int = 1, cpu: bool = True, launch_floor_us: float | None = None) -> list:
-    """The kernels of configs[0..3] (and of the unfused attention path) at their stated sizes.  launch_floor_us: what
+    """The kernels one at a time (and the unfused attention path) at their stated sizes.  launch_floor_us: what
     an empty kernel costs back to back on this box (microbench()["empty_launch_us"]); bandwidth-bound rows then also
     carry the rate over the time above that floor, which is what the kernel itself decides at these small sizes."""
     from tensorrt_amd import capi, workloads
