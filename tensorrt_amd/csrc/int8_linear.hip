@@ -81,7 +81,7 @@ struct LinearArgs
     int tokMain;   // rows of 256 tokens they cover
     int panel;     // channel tiles per panel of the tile numbering (divides the number of channel tiles)
     int persist;   // persistent kernel: workgroups that loop over the 256 x 256 tiles
-    int pieces;    // direct-to-LDS kernel: the tokens behind the large tiles go in 64 x 64 pieces (see linear_piece64)
+    int pieces;    // large tiles: the tokens behind them go in 64 x 64 pieces (see linear_piece64)
     int parts;     // pieces: workgroups that share the k range of a piece, each with an output of its own
     WeightPrefetch prefetch; // by the workgroups behind mainTiles of the interleaved tile and piece kernels
 };
@@ -166,6 +166,33 @@ __device__ __forceinline__ BlockScales load_block_scales(float const* sAlpha, fl
     return s;
 }
 
+// The FP16 results of a 32 x 32 block: 16 consecutive channels, 16 (l/32) .. +15, of token l%32 per lane.
+template <int EPI>
+__device__ __forceinline__ void pack_half_block(AccT<EPI> const& acc, BlockScales const& sc, u32x4& first, u32x4& second)
+{
+    u32x2 w[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+    {
+        f16x4 h;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+        {
+            float const y = fmaf((float) acc[4 * g + e], sc.al[g][e], sc.be[g][e]);
+            h[e] = (f16) (EPI == kF16_GELU ? gelu_erf(y) : y);
+        }
+        w[g] = __builtin_bit_cast(u32x2, h);
+    }
+    // lanes l < 32 hold channels 8g..8g+3 of each group g, lanes l+32 the other four: after the swaps lane l has
+    // groups 0 and 1 whole, lane l+32 groups 2 and 3
+    auto const a0 = __builtin_amdgcn_permlane32_swap(w[0][0], w[2][0], false, false);
+    auto const a1 = __builtin_amdgcn_permlane32_swap(w[0][1], w[2][1], false, false);
+    auto const b0 = __builtin_amdgcn_permlane32_swap(w[1][0], w[3][0], false, false);
+    auto const b1 = __builtin_amdgcn_permlane32_swap(w[1][1], w[3][1], false, false);
+    first = u32x4{a0[0], a1[0], a0[1], a1[1]};
+    second = u32x4{b0[0], b1[0], b0[1], b1[1]};
+}
+
 template <bool IL_OUT, int EPI, bool FULL = false, bool THROUGH = false>
 __device__ __forceinline__ void store_block_scaled(
     LinearArgs const& p, AccT<EPI> const& acc, int const c0, int const tb, BlockScales const& sc)
@@ -190,27 +217,8 @@ __device__ __forceinline__ void store_block_scaled(
     }
     else if constexpr (EPI >= kF16_AFFINE || EPI == kHALF)
     {
-        u32x2 w[4];
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-        {
-            f16x4 h;
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-            {
-                float const y = fmaf((float) acc[4 * g + e], al[g][e], be[g][e]);
-                h[e] = (f16) (EPI == kF16_GELU ? gelu_erf(y) : y);
-            }
-            w[g] = __builtin_bit_cast(u32x2, h);
-        }
-        // lanes l < 32 hold channels 8g..8g+3 of each group g, lanes l+32 the other four: after the swaps lane l has
-        // groups 0 and 1 whole, lane l+32 groups 2 and 3: 16 consecutive channels, two 16-byte stores
-        auto const a0 = __builtin_amdgcn_permlane32_swap(w[0][0], w[2][0], false, false);
-        auto const a1 = __builtin_amdgcn_permlane32_swap(w[0][1], w[2][1], false, false);
-        auto const b0 = __builtin_amdgcn_permlane32_swap(w[1][0], w[3][0], false, false);
-        auto const b1 = __builtin_amdgcn_permlane32_swap(w[1][1], w[3][1], false, false);
-        u32x4 const first = {a0[0], a1[0], a0[1], a1[1]};
-        u32x4 const second = {b0[0], b1[0], b0[1], b1[1]};
+        u32x4 first, second;
+        pack_half_block<EPI>(acc, sc, first, second);
         if (live)
         {
             f16* dst = static_cast<f16*>(p.out) + (size_t) t * p.N + c0 + 16 * hi;
@@ -674,12 +682,8 @@ __device__ __forceinline__ void linear_tile_run(
 // and K of 256 bytes (the ring index is then the stage index modulo 4 in every tile).  One instruction fills 1 KB of
 // LDS with lane i's 16 bytes at offset 16 i, so the LDS swizzle is applied on the source side: lane i fetches the
 // 16 bytes that belong there.
-//   IL (both operands 32-interleaved): a load unit is one fragment, 32 rows x 32 bytes, contiguous in memory.
-//   otherwise (both operands linear [R][K], also the FP16 layers): a load unit is 16 rows x 64 bytes (four lanes
-//   per row, 64 contiguous bytes of it); in LDS the 16-byte chunk c of row r sits at chunk c ^ (r / 4), which makes
-//   the fragment reads (16 rows x one chunk per 16 lanes) conflict-free; fragment (block, ks) takes chunks 2 ks and
-//   2 ks + 1 of the block's two units.
-template <bool IL, bool IL_OUT, int EPI, typename Origin>
+// Both operands are 32-interleaved: a load unit is one fragment, 32 rows x 32 bytes, contiguous in memory.
+template <bool IL_OUT, int EPI, typename Origin>
 __device__ __forceinline__ void linear_tile_run_dma(
     LinearArgs const& p, int const count, Origin origin, uint8_t* __restrict__ lds, float* sScale)
 {
@@ -691,9 +695,9 @@ __device__ __forceinline__ void linear_tile_run_dma(
     constexpr int LB = BF / NWAVES;
     constexpr int STAGE = (AF + BF) * 1024;
     constexpr int kLoads = LA + LB;           // direct loads per wavefront and stage
-    // global stores per wavefront in a tile's epilogue: one 16-byte store per accumulator block (INT8), two (FP16)
-    constexpr int kStores = MT * NT * (EPI >= kF16_AFFINE ? 2 : 1);
-    static_assert(EPI == kAFFINE || EPI == kGELU || EPI == kF16_AFFINE || EPI == kF16_GELU, "store count per block");
+    // global stores per wavefront in a tile's epilogue: one 16-byte store per accumulator block
+    constexpr int kStores = MT * NT;
+    static_assert(EPI == kAFFINE || EPI == kGELU, "store count per block");
 
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -705,23 +709,11 @@ __device__ __forceinline__ void linear_tile_run_dma(
     // Lane i of a unit's load supplies LDS offset 16 i of the unit.  Its address is a wave-uniform part (the unit's
     // first row, kept in scalar registers and advanced by scalar arithmetic) plus a lane part that is the same for
     // every unit, tile and stage: the loop spends no vector-ALU instruction on addresses.
-    uint32_t laneOff;
-    if constexpr (IL)
-    {
-        int const r = lane >> 1; // row of the fragment; the half that the swizzle puts at this offset
-        uint32_t const half = (uint32_t) ((lane & 1) ^ ((r >> 3) & 1));
-        laneOff = (uint32_t) r * 32u + half * 16u;
-    }
-    else
-    {
-        int const rr = lane >> 2; // row of the 16-row unit; the chunk that the swizzle puts at this offset
-        uint32_t const chunk = (uint32_t) ((lane & 3) ^ (rr >> 2));
-        laneOff = (uint32_t) rr * (uint32_t) p.K + chunk * 16u;
-    }
+    int const loadRow = lane >> 1; // row of the fragment; the half that the swizzle puts at this offset
+    uint32_t const laneOff = (uint32_t) loadRow * 32u + (uint32_t) ((lane & 1) ^ ((loadRow >> 3) & 1)) * 16u;
     auto unit_base = [&](int u, int row0, int R) -> uint32_t {
         int const rb = u >> 1, sel = u & 1;
-        uint32_t const b = IL ? ((uint32_t) sel * (uint32_t) R + (uint32_t) (row0 + rb * 32)) * 32u
-                              : (uint32_t) (row0 + rb * 32 + sel * 16) * (uint32_t) p.K;
+        uint32_t const b = ((uint32_t) sel * (uint32_t) R + (uint32_t) (row0 + rb * 32)) * 32u;
         return (uint32_t) __builtin_amdgcn_readfirstlane((int) b);
     };
     auto address = [&](int n0, int t0, uint32_t(&oa)[LA], uint32_t(&ob)[LB]) {
@@ -736,8 +728,8 @@ __device__ __forceinline__ void linear_tile_run_dma(
             ob[q] = unit_base(q * NWAVES + wave, t0, p.T);
         }
     };
-    uint32_t const stepA = IL ? (uint32_t) KS * (uint32_t) p.N * 32u : 64u;
-    uint32_t const stepB = IL ? (uint32_t) KS * (uint32_t) p.T * 32u : 64u;
+    uint32_t const stepA = (uint32_t) KS * (uint32_t) p.N * 32u;
+    uint32_t const stepB = (uint32_t) KS * (uint32_t) p.T * 32u;
     int const nk = p.K / (32 * KS); // a multiple of 4
 
     uint32_t oaC[LA], obC[LB], oaN[LA], obN[LB];
@@ -766,15 +758,7 @@ __device__ __forceinline__ void linear_tile_run_dma(
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
     {
-        if constexpr (IL)
-        {
-            readOff[ks] = ks * 1024 + frag_offset(lane & 31, lane >> 5);
-        }
-        else
-        {
-            int const fr = lane & 31, rr = fr & 15;
-            readOff[ks] = (fr >> 4) * 1024 + rr * 64 + (((ks * 2 + (lane >> 5)) ^ (rr >> 2)) << 4);
-        }
+        readOff[ks] = ks * 1024 + frag_offset(lane & 31, lane >> 5);
     }
     auto multiply = [&](int slot) {
         uint8_t const* base = lds + slot * STAGE;
@@ -1179,36 +1163,59 @@ __device__ __forceinline__ void for_each_behind(int const rest, F&& f)
     }
 }
 
-// One tile of BM = WM*MT*32 channels x BN = WN*NT*32 tokens with the stages brought in by direct-to-LDS loads, for
-// launches that do not fill the chip with 256 x 256 tiles.  The LDS layout of a stage, its swizzles and its load units
-// are those of linear_tile_run_dma; a ring of RING stages, stage k + RING - 1 requested while stage k is multiplied and
-// one barrier per stage.  Rows behind the last one are read as the last one (their results are not stored), so any
-// T and N are taken; K a multiple of 64 bytes.  Operands both interleaved (IL) or both linear.
-template <bool IL, bool IL_OUT, int EPI, int WM, int WN, int MT, int NT, int RING>
+// Whether a tile's scale vectors come at its end, into a slot of the ring, since a place of their own would cost the CU its
+// second workgroup.
+constexpr bool scales_late(int ringBytes)
+{
+    constexpr int kHalfOfLds = 80 * 1024;
+    return ringBytes <= kHalfOfLds && ringBytes + 2 * kBigTile * 4 > kHalfOfLds;
+}
+
+// One tile of BM = WM*MT*32 channels x BN = WN*NT*32 tokens with the stages brought in by direct-to-LDS loads.  Rows behind
+// the last one are read as the last one (their results are not stored), so any T and N are taken.  Operands both
+// interleaved (IL) or both linear.
+//
+// Stages.  KS k-halves of 32 bytes.  Interleaved operands arrive in whole lines whatever the stage is.  Of a linear operand
+// a row's share of a stage is 32 KS bytes: with 64 of them every line crosses from the L2 to the CU twice, half of it for
+// nothing, so linear rows come in stages of 128 bytes (KS = 4; K a multiple of that, otherwise KS = 2).  A load unit is
+// 8 rows x 128 bytes, and in LDS the 16-byte chunk c of row r sits at chunk c ^ (r / 2) % 8 (KS = 2: 16 rows x 64 bytes,
+// chunk c ^ r / 4): 16 rows x one chunk, a quarter of a fragment read, then touch every bank once.
+//
+// Schedule.  All RING slots are requested ahead; a stage's slot is requested again as soon as everybody has read it.  What
+// a wavefront does between two matrix instructions is written out: the fragments of the next k-half are read while
+// this one's are multiplied, across the barrier too, and the loads of a stage are spread over the k-halves of the one
+// before, for a burst of them stalls the wavefront that issues it while the CU's one path to the L2 takes them in.
+//
+// What it is bound by: with every CU busy, by the power the chip may draw (768 channels, 7765 tokens x 3072 -> 768: 43 us on
+// normal operands, 35 us on zeros; 31 us with either the loads or the matrix instructions left out).
+// 7765 tokens, FP16, QKV / projection / feed-forward 1 / 2 of 768 channels, graph replays, the best plan of each, us:
+//   stages of 64 bytes, fragments read behind the barrier     39.8 / 16.9 / 52.4 / 50.4
+//   the same in tiles of 192 channels or tokens too           37.3 / 16.6 / 49.1 / 49.2
+//   stages of 128 bytes                                       39.8 / 16.0 / 47.8 / 44.5
+//   fragments read ahead                                      38.7 / 15.8 / 46.5 / 43.0
+//   loads spread out, order kept                              36.0 / 14.8 / 45.1 / 39.3
+//   rows stored whole, through the L2 (see the end)           32.6 / 12.5 / 41.2 / 35.5
+template <bool IL, bool IL_OUT, int EPI, int WM, int WN, int MT, int NT, int RING, int KS = 2>
 __device__ __forceinline__ void linear_tile_dma(
-    LinearArgs const& p, int const n0, int const t0, uint8_t* __restrict__ lds, float* sScale)
+    LinearArgs const& p, int const n0, int const t0, uint8_t* __restrict__ lds)
 {
     constexpr int NWAVES = WM * WN;
     constexpr int BM = WM * MT * 32;
     constexpr int BN = WN * NT * 32;
-    constexpr int AF = (BM / 32) * 2;
-    constexpr int BF = (BN / 32) * 2;
-    static_assert(AF % NWAVES == 0 && BF % NWAVES == 0, "load units divide evenly among the waves");
-    static_assert(BM <= kBigTile, "scale vectors");
-    constexpr int LA = AF / NWAVES;
-    constexpr int LB = BF / NWAVES;
-    constexpr int kLoads = LA + LB;
+    constexpr int AF = (BM / 32) * KS;
+    constexpr int BF = (BN / 32) * KS;
+    constexpr int kLoads = (AF + BF + NWAVES - 1) / NWAVES;
     constexpr int STAGE = (AF + BF) * 1024;
+    static_assert(BM <= kBigTile && STAGE >= 2 * kBigTile * 4, "scale vectors");
 
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int const wm = wave / WN;
     int const wn = wave % WN;
     uint32_t const ldsBase = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) lds;
-    uint32_t const scaleBase = (uint32_t) (size_t) (__attribute__((address_space(3))) float*) sScale;
 
     auto unit_offset = [&](int u, int row0, int R) -> uint32_t {
-        int const rb = u >> 1, sel = u & 1;
+        int const rb = u / KS, sel = u % KS;
         if constexpr (IL)
         {
             int const r = lane >> 1;
@@ -1217,36 +1224,34 @@ __device__ __forceinline__ void linear_tile_dma(
         }
         else
         {
-            int const rr = lane >> 2;
-            uint32_t const chunk = (uint32_t) ((lane & 3) ^ (rr >> 2));
-            return (uint32_t) min(row0 + rb * 32 + sel * 16 + rr, R - 1) * (uint32_t) p.K + chunk * 16u;
+            int const rr = lane / (2 * KS), r = sel * (32 / KS) + rr;
+            uint32_t const chunk = (uint32_t) ((lane & (2 * KS - 1)) ^ (KS == 2 ? rr >> 2 : (r >> 1) & 7));
+            return (uint32_t) min(row0 + rb * 32 + r, R - 1) * (uint32_t) p.K + chunk * 16u;
         }
     };
-    uint32_t offA[LA], offB[LB];
+    // Units 0 .. AF-1 are the weights', the ones behind them the tokens', dealt to the wavefronts in turn.  Where they do
+    // not come out even, the wavefronts without a last unit fetch the one before it again, to the same place: every
+    // wavefront then has the same number of loads in flight, which is what the waits below count.
+    uint32_t off[kLoads], step[kLoads], dstOff[kLoads];
+    int8_t const* src[kLoads];
 #pragma unroll
-    for (int q = 0; q < LA; ++q)
+    for (int q = 0; q < kLoads; ++q)
     {
-        offA[q] = unit_offset(q * NWAVES + wave, n0, p.N);
+        int const own = q * NWAVES + wave;
+        int const u = (q + 1) * NWAVES <= AF + BF || own < AF + BF ? own : own - NWAVES;
+        bool const weights = (q + 1) * NWAVES <= AF || (q * NWAVES < AF && u < AF);
+        off[q] = weights ? unit_offset(u, n0, p.N) : unit_offset(u - AF, t0, p.T);
+        src[q] = weights ? p.w : p.a;
+        step[q] = KS * 32u * (IL ? (uint32_t) (weights ? p.N : p.T) : 1u);
+        dstOff[q] = (uint32_t) u * 1024u;
     }
-#pragma unroll
-    for (int q = 0; q < LB; ++q)
-    {
-        offB[q] = unit_offset(q * NWAVES + wave, t0, p.T);
-    }
-    uint32_t const stepA = IL ? 2u * (uint32_t) p.N * 32u : 64u;
-    uint32_t const stepB = IL ? 2u * (uint32_t) p.T * 32u : 64u;
-    int const nk = p.K / 64;
+    int const nk = p.K / (32 * KS);
     auto fetch = [&](int kt, int slot) {
         uint32_t const dst = ldsBase + (uint32_t) slot * STAGE;
 #pragma unroll
-        for (int q = 0; q < LA; ++q)
+        for (int q = 0; q < kLoads; ++q)
         {
-            load_to_lds16_sbase(p.w + (uint64_t) kt * stepA, offA[q], dst + (uint32_t) (q * NWAVES + wave) * 1024u);
-        }
-#pragma unroll
-        for (int q = 0; q < LB; ++q)
-        {
-            load_to_lds16_sbase(p.a + (uint64_t) kt * stepB, offB[q], dst + (uint32_t) (AF + q * NWAVES + wave) * 1024u);
+            load_to_lds16_sbase(src[q] + (uint64_t) kt * step[q], off[q], dst + dstOff[q]);
         }
     };
     AccT<EPI> acc[MT][NT];
@@ -1263,9 +1268,9 @@ __device__ __forceinline__ void linear_tile_dma(
             }
         }
     }
-    int readOff[2];
+    int readOff[KS];
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
+    for (int ks = 0; ks < KS; ++ks)
     {
         if constexpr (IL)
         {
@@ -1273,68 +1278,186 @@ __device__ __forceinline__ void linear_tile_dma(
         }
         else
         {
-            int const fr = lane & 31, rr = fr & 15;
-            readOff[ks] = (fr >> 4) * 1024 + rr * 64 + (((ks * 2 + (lane >> 5)) ^ (rr >> 2)) << 4);
+            int const fr = lane & 31, rr = fr & 15, chunk = ks * 2 + (lane >> 5);
+            readOff[ks] = KS == 2 ? (fr >> 4) * 1024 + rr * 64 + ((chunk ^ (rr >> 2)) << 4)
+                                  : fr * 128 + ((chunk ^ ((fr >> 1) & 7)) << 4);
         }
     }
-    auto multiply = [&](int slot) {
-        uint8_t const* base = lds + slot * STAGE;
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
+    i32x4 fa[2][MT], fb[2][NT];
+    // fragment r of k-half ks of the stage in `slot`, in the order in which the matrix instructions ask for them
+    auto read_fragment = [&](auto setTag, int slot, int ks, int r) {
+        constexpr int S = decltype(setTag)::value;
+        uint8_t const* base = lds + slot * STAGE + readOff[ks];
+        if (r == 0 || r > NT)
         {
-            i32x4 fa[MT], fb[NT];
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-            {
-                fa[i] = *reinterpret_cast<i32x4 const*>(base + (wm * MT + i) * 2048 + readOff[ks]);
-            }
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-            {
-                fb[j] = *reinterpret_cast<i32x4 const*>(base + AF * 1024 + (wn * NT + j) * 2048 + readOff[ks]);
-            }
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-            {
-#pragma unroll
-                for (int j = 0; j < NT; ++j)
-                {
-                    acc[i][j] = mma<EPI>(fa[i], fb[j], acc[i][j]);
-                }
-            }
+            int const i = r == 0 ? 0 : r - NT;
+            fa[S][i] = *reinterpret_cast<i32x4 const*>(base + (wm * MT + i) * (KS * 1024));
+        }
+        else
+        {
+            fb[S][r - 1] = *reinterpret_cast<i32x4 const*>(base + AF * 1024 + (wn * NT + r - 1) * (KS * 1024));
         }
     };
-    // requested first, so the wait for stage 0 covers them
-    if (wave < 2 && lane < BM / 4)
+    // One k-half: the matrix instructions on fragment set S, and between them the reads of the next k-half's fragments
+    // (ks of `slot`, into the other set) and this k-half's share of the loads of stage kt.  The order is kept as it stands.
+    auto phase = [&](auto setTag, auto readTag, int slot, int ks, auto loadTag, int kt, int ktSlot) {
+        constexpr int S = decltype(setTag)::value;
+        constexpr bool READ = decltype(readTag)::value;
+        constexpr int PART = decltype(loadTag)::value; // -1: no loads
+        constexpr int M = MT * NT, R = MT + NT, kReadsAtOnce = (2 * R + M - 1) / M;
+        // two stages in the ring: the loads of a stage have to be on their way early in the one before it
+        constexpr int P = RING == 2 ? 2 : KS;
+        constexpr int L0 = PART < 0 || PART >= P ? 0 : PART * kLoads / P, L1 = PART < 0 || PART >= P ? 0 : (PART + 1) * kLoads / P;
+        uint32_t const dst = ldsBase + (uint32_t) ktSlot * STAGE;
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+        {
+            acc[m / NT][m % NT] = mma<EPI>(fa[S][m / NT], fb[S][m % NT], acc[m / NT][m % NT]);
+            if constexpr (READ)
+            {
+#pragma unroll
+                for (int r = m * kReadsAtOnce; r < (m + 1) * kReadsAtOnce && r < R; ++r)
+                {
+                    read_fragment(std::integral_constant<int, 1 - S>{}, slot, ks, r);
+                }
+            }
+#pragma unroll
+            for (int q = L0 + m * (L1 - L0) / M; q < L0 + (m + 1) * (L1 - L0) / M; ++q)
+            {
+                load_to_lds16_sbase(src[q] + (uint64_t) kt * step[q], off[q], dst + dstOff[q]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    using Even = std::integral_constant<int, 0>;
+    using Odd = std::integral_constant<int, 1>;
+    using Yes = std::true_type;
+    using No = std::false_type;
+    using NoLoads = std::integral_constant<int, -1>;
+    constexpr bool kLate = scales_late(RING * STAGE);
+    auto fetch_scales = [&](int at) {
+        if (wave < 2 && lane < BM / 4)
+        {
+            float const* from = (wave == 0 ? p.alpha : p.beta) + min(n0 + lane * 4, p.N - 4);
+            load_to_lds16(from, ldsBase + (uint32_t) (at + wave * kBigTile * 4));
+        }
+    };
+    if constexpr (!kLate)
     {
-        float const* src = (wave == 0 ? p.alpha : p.beta) + min(n0 + lane * 4, p.N - 4);
-        load_to_lds16(src, scaleBase + (uint32_t) (wave * kBigTile) * 4u);
+        fetch_scales(RING * STAGE); // requested first, so the wait for stage 0 covers them
     }
 #pragma unroll
-    for (int s = 0; s < RING - 1; ++s)
+    for (int s = 0; s < RING; ++s)
     {
         if (s < nk)
         {
             fetch(s, s);
         }
     }
-    int slot = 0, k = 0;
-    for (; k + RING - 1 < nk; ++k)
+    if (nk >= RING)
     {
-        wait_vmcnt<(RING - 2) * kLoads>(); // this wavefront's part of stage k has landed
-        __syncthreads();                   // everybody's has, and nobody reads stage k - 1 any more
-        fetch(k + RING - 1, slot == 0 ? RING - 1 : slot - 1);
-        multiply(slot);
-        slot = slot == RING - 1 ? 0 : slot + 1;
+        wait_vmcnt<(RING - 1) * kLoads>();
     }
-    // at most RING - 1 stages, all requested
-    for_each_behind<RING - 2>(nk - k, [&](auto behind) {
-        wait_vmcnt<decltype(behind)::value * kLoads>();
-        __syncthreads();
-        multiply(slot);
+    else
+    {
+        wait_vmcnt<0>();
+    }
+    __syncthreads();
+    int slot = 0, k = 0;
+#pragma unroll
+    for (int r = 0; r < MT + NT; ++r)
+    {
+        read_fragment(Even{}, 0, 0, r);
+    }
+    // the k-halves of stage k but its last; `loads`: with the rest of the loads of stage k + RING - 1, which go where
+    // stage k - 1 was
+    auto first_halves = [&](auto loads) {
+        constexpr bool LOADS = decltype(loads)::value;
+        int const before = slot == 0 ? RING - 1 : slot - 1;
+        phase(Even{}, Yes{}, slot, 1, std::integral_constant<int, LOADS ? 1 : -1>{}, k + RING - 1, before);
+        if constexpr (KS == 4)
+        {
+            phase(Odd{}, Yes{}, slot, 2, std::integral_constant<int, LOADS ? 2 : -1>{}, k + RING - 1, before);
+            phase(Even{}, Yes{}, slot, 3, std::integral_constant<int, LOADS ? 3 : -1>{}, k + RING - 1, before);
+        }
+    };
+    // stage k, with stage k + 1 landed before its last k-half; BEHIND: stages that may still be on their way then
+    auto stage = [&](auto restTag, auto behindTag, auto nextTag) {
+        first_halves(restTag);
+        wait_vmcnt<decltype(behindTag)::value * kLoads>(); // this wavefront's part of stage k + 1 has landed
+        __syncthreads();                                   // everybody's has, and everybody has read stage k
+        int const own = slot;
         slot = slot == RING - 1 ? 0 : slot + 1;
-    });
+        phase(Odd{}, Yes{}, slot, 0, std::integral_constant<int, decltype(nextTag)::value ? 0 : -1>{}, k + RING, own);
+        ++k;
+    };
+    using Behind = std::integral_constant<int, RING - 2>;
+    if (k + RING < nk)
+    {
+        stage(No{}, Behind{}, Yes{});
+        while (k + RING < nk)
+        {
+            stage(Yes{}, Behind{}, Yes{});
+        }
+        stage(Yes{}, Behind{}, No{});
+    }
+    for_each_behind<RING - 2>(nk - 1 - k, [&](auto behind) { stage(No{}, behind, No{}); });
+    int const scalesAt = kLate ? (slot == 0 ? RING - 1 : slot - 1) * STAGE : RING * STAGE;
+    if constexpr (kLate)
+    {
+        fetch_scales(scalesAt); // a slot that no further stage needs
+    }
+    first_halves(No{});
+    phase(Odd{}, No{}, 0, 0, NoLoads{}, 0, 0);
+    constexpr int kRow = MT * 64 + 16; // bytes; 16 of padding spread the rows over the banks
+    constexpr bool kStaged = EPI >= kF16_AFFINE && NWAVES * 32 * kRow <= STAGE;
+    if constexpr (kLate || kStaged)
+    {
+        wait_vmcnt<0>();
+        __syncthreads(); // the scales have come, and nobody reads the last stage any more
+    }
+    float const* const sScale = reinterpret_cast<float const*>(lds + scalesAt);
 
+    // FP16 rows leave through LDS, 32 tokens of the wavefront's channels at a time, so that a store writes whole lines, and can
+    // write through the L2: what is left in it at the kernel's end is written back while nothing else runs (up to 32 MB;
+    // stores of 16-byte pieces need the L2 to put them together, and cost 5 to 9 of the 44 us of feed-forward 1).
+    if constexpr (kStaged)
+    {
+        uint8_t* const own = lds + slot * STAGE + wave * (32 * kRow);
+        int const nw = n0 + wm * MT * 32;
+        BlockScales sc[MT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+        {
+            sc[i] = load_block_scales<EPI>(sScale + (wm * MT + i) * 32, sScale + kBigTile + (wm * MT + i) * 32);
+        }
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+        {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+            {
+                u32x4 first, second;
+                pack_half_block<EPI>(acc[i][j], sc[i], first, second);
+                u32x4* dst = reinterpret_cast<u32x4*>(own + (lane & 31) * kRow + i * 64 + (lane >> 5) * 32);
+                dst[0] = first;
+                dst[1] = second;
+            }
+            constexpr int kChunks = MT * 4; // 16-byte pieces of a row
+            int const tb = t0 + (wn * NT + j) * 32;
+#pragma unroll
+            for (int q = 0; q < kChunks / 2; ++q)
+            {
+                int const c = q * 64 + lane, r = c / kChunks, ch = c % kChunks;
+                u32x4 const v = *reinterpret_cast<u32x4 const*>(own + r * kRow + ch * 16);
+                if (tb + r < p.T && nw + ch * 8 < p.N)
+                {
+                    store_out<true>(static_cast<f16*>(p.out) + (size_t) (tb + r) * p.N + nw + ch * 8, v);
+                }
+            }
+        }
+        return;
+    }
     bool const full = t0 + BN <= p.T; // uniform
 #pragma unroll
     for (int i = 0; i < MT; ++i)
@@ -1363,7 +1486,7 @@ __device__ __forceinline__ void linear_tile_dma(
 }
 
 // The persistent tile plan with direct-to-LDS loads for the 256 x 256 tiles.
-template <bool IL, bool IL_OUT, int EPI>
+template <bool IL_OUT, int EPI>
 __global__ __launch_bounds__(512) void int8_linear_dma_kernel(LinearArgs const p)
 {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * 2 * (kBig / 32) * 2 * 1024];
@@ -1379,24 +1502,20 @@ __global__ __launch_bounds__(512) void int8_linear_dma_kernel(LinearArgs const p
             n0 = (int) (pan * pw + rem % pw) * kBig;
             t0 = (int) (rem / pw) * kBig;
         };
-        linear_tile_run_dma<IL, IL_OUT, EPI>(p, count, origin, lds, sScale);
+        linear_tile_run_dma<IL_OUT, EPI>(p, count, origin, lds, sScale);
     }
     else
     {
         uint32_t const tile = blockIdx.x - (uint32_t) p.persist;
-        if constexpr (IL && (EPI == kAFFINE || EPI == kGELU))
+        if (p.pieces)
         {
-            if (p.pieces)
-            {
-                uint32_t const nbm = (uint32_t) p.N / 64u;
-                linear_piece64<IL_OUT, EPI>(p, (int) (tile % nbm) * 64, p.tokMain * kBig + (int) (tile / nbm) * 64, lds,
-                    sScale);
-                return;
-            }
+            uint32_t const nbm = (uint32_t) p.N / 64u;
+            linear_piece64<IL_OUT, EPI>(p, (int) (tile % nbm) * 64, p.tokMain * kBig + (int) (tile / nbm) * 64, lds, sScale);
+            return;
         }
         uint32_t const nbm = (uint32_t) ((p.N + kSmall - 1) / kSmall);
-        linear_tile_dma<IL, IL_OUT, EPI, 2, 4, 2, 1, 4>(p, (int) (tile % nbm) * kSmall,
-            p.tokMain * kBig + (int) (tile / nbm) * kSmall, lds, sScale);
+        linear_tile_dma<true, IL_OUT, EPI, 2, 4, 2, 1, 4>(p, (int) (tile % nbm) * kSmall,
+            p.tokMain * kBig + (int) (tile / nbm) * kSmall, lds);
     }
 }
 
@@ -1426,11 +1545,11 @@ __device__ __forceinline__ void prefetch_weights(LinearArgs const& p)
     }
 }
 
-template <bool IL, bool IL_OUT, int EPI, int WM, int WN, int MT, int NT, int RING, int PER_SIMD>
+template <bool IL, bool IL_OUT, int EPI, int WM, int WN, int MT, int NT, int RING, int PER_SIMD, int KS = 2>
 __global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(LinearArgs const p)
 {
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[RING * (WM * MT + WN * NT) * 2 * 1024];
-    __shared__ __attribute__((aligned(16))) float sScale[2 * kBigTile];
+    constexpr int kRing = RING * (WM * MT + WN * NT) * KS * 1024;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[kRing + (scales_late(kRing) ? 0 : 2 * kBigTile * 4)];
     if constexpr (IL)
     {
         if ((int) blockIdx.x >= p.mainTiles)
@@ -1444,8 +1563,8 @@ __global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(Line
     uint32_t const perPanel = (uint32_t) p.tokMain * pw;
     uint32_t const tile = xcd_remap(blockIdx.x, (uint32_t) p.mainTiles);
     uint32_t const pan = tile / perPanel, rem = tile % perPanel;
-    linear_tile_dma<IL, IL_OUT, EPI, WM, WN, MT, NT, RING>(
-        p, (int) (pan * pw + rem % pw) * (WM * MT * 32), (int) (rem / pw) * (WN * NT * 32), lds, sScale);
+    linear_tile_dma<IL, IL_OUT, EPI, WM, WN, MT, NT, RING, KS>(
+        p, (int) (pan * pw + rem % pw) * (WM * MT * 32), (int) (rem / pw) * (WN * NT * 32), lds);
 }
 
 // A piece of CB x TB blocks of 32 channels x 32 tokens by one workgroup whose eight wavefronts split k, for launches
@@ -1724,16 +1843,22 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
 
 // Which kernel a launch with operands of one layout takes: the one with the lowest estimate of
 //
-//   launch + units(x) * (tile + gelu + stage * K / 64)                    [us]
+//   launch + units(x) * (tile + gelu + stage * (1 + busy * min(x, 1)) * K / 64)                    [us]
 //
 // where x is the number of tiles per CU.  Up to `resident` tiles run on a CU at once and share it, each behind the first
 // costing `share` of a tile's time on its own; the ones beyond that wait their turn at `turn` each.  The CUs with the
-// most tiles decide how long the launch takes as far as `whole` says (1: entirely, 0: an even spread).  Small tiles fill the
+// most tiles decide how long the launch takes as far as `whole` says (1: entirely, 0: an even spread).  `busy`: what a stage
+// takes longer when every CU works than when few do.  `spill`: GPUs differ in how many CUs each shader engine has left, and
+// workgroups are dealt to the engines evenly, so on some GPUs a launch of one workgroup per CU runs a second round from
+// 3/4 of the CUs on (7765 tokens x 768 -> 768, 246 workgroups: 12.3 us on one GPU, 16.8 us on another).  Small tiles fill the
 // chip where the problem has few of them, large ones move fewer bytes per multiplication where it has many, and the pieces
 // cut the chain of stages by eight where neither fills it.
 //
-// The constants are fits.  Linear operands: to launches by themselves on the four layers of a 768-channel FP16 encoder
-// (graph replays, weights in the last-level cache).  Interleaved operands: to launches by themselves on those of a
+// The constants are fits.  Linear operands: to launches by themselves on the four layers of 768- and 1024-channel FP16
+// encoders (graph replays, weights in the last-level cache), 16 to 33289 tokens, on two GPUs, one of them with the uneven
+// engines.  The plan they choose takes 0.8 % more than the best of all in the mean (24 % at most, a launch at the edge
+// of a second round); the kernels and the choice before took 13 % more (50 % at most).
+// Interleaved operands: to launches by themselves on those of a
 // 1024-channel INT8 encoder with weights from memory, and the ones that decide from 2500 tokens on (large tiles, 128 x 256,
 // 128 x 128, 64 x 128, 128 x 128 deep) to whole passes of that encoder with the plans of one or two of its layers changed at a
 // time: what a launch takes by itself does not say what it costs the ones around it.  At 9084 tokens 128 x 128 tiles are the
@@ -1741,24 +1866,20 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
 // sizes of 2465 to 23000 tokens the pass takes 0.8 % less than with constants for launches by themselves, one of them more
 // than 0.8 % more (7399 tokens, 1.9 %), and the best of the measured combinations would take another 0.9 % less (4 % at
 // most).  32 sequences of up to 256 tokens: 2979 -> 2877 us.
-// Against 128 x 128 tiles staged through registers for every launch short of half a round of large tiles (single launches,
-// weights in the last-level cache): 40 tokens x (1024 -> 3072 / 4096 -> 1024) INT8 7.2 / 19.1 -> 3.7 / 4.7 us, 600 tokens
-// 7.4 / 19.0 -> 5.2 / 7.9 us, 5300 tokens 20.5 / 43.0 -> 20.9 / 27.1 us; FP16 40 tokens x (768 -> 2304 / 3072 -> 768) 9.7 /
-// 29.9 -> 4.0 / 7.2 us, 9100 tokens x 3072 -> 768 80.0 -> 54.4 us.
 // Deep rings: where one workgroup per CU is all there is, a tile is bound by the trips to memory of its own stages, and
 // the LDS of the workgroups that do not come is better used for more of them (interleaved, weights from memory, 600 tokens
 // x 4096 -> 1024 in 64 x 64 tiles: 12.9 us with three stages ahead, 9.5 us with seven; 128 x 128 tiles, 1900 tokens 20.8
 // us with two, 17.4 us with three); with two and more per CU they are slower.  Sharing the k range of such a tile between
 // groups of wavefronts instead (two or four groups, rings of their own) measured 9.9-10.4 us on the first of these and
-// lost elsewhere.  Linear operands gain 1-5 % from them and go without.
+// lost elsewhere.
 struct TileCost
 {
     int channels, tokens, resident;
-    float launch, tile, stage, gelu, share, turn, whole;
+    float launch, tile, stage, gelu, share, turn, whole, busy, spill;
 };
 enum LinearPlan
 {
-    kLargeTiles = 0, // whole rounds of 256 x 256 tiles by persistent workgroups and smaller ones for the rest
+    kLargeTiles = 0, // interleaved: whole rounds of 256 x 256 tiles by persistent workgroups and smaller ones for the rest
     kTile128x256,
     kTile128x128,
     kTile64x128,
@@ -1768,41 +1889,50 @@ enum LinearPlan
     kTile64x64Deep,
     kPiece32x64,
     kPiece32x32,
+    kTile256x256,
+    kTile256x192,
+    kTile128x192,
+    kTile128x192Deep,
+    kTile128x64,
     kLinearPlans
 };
 // [0]: linear operands, [1]: interleaved ones.  No channels: the layout has no such kernel.
 constexpr TileCost kTileCosts[2][kLinearPlans] = {
-    {{256, 256, 1, 0.00f, 8.31f, 0.750f, 0.33f, 0.f, 0.f, 0.f}, {128, 256, 2, 2.06f, 2.05f, 0.430f, 0.64f, 1.50f, 1.22f, 0.62f},
-        {128, 128, 2, 1.93f, 1.06f, 0.292f, 0.41f, 1.30f, 1.10f, 0.53f}, {64, 128, 3, 2.49f, 0.32f, 0.188f, 0.21f, 1.27f, 1.14f, 0.52f},
-        {64, 64, 4, 2.29f, 0.30f, 0.138f, 0.13f, 0.94f, 0.89f, 0.47f}, {}, {}, {},
-        {32, 64, 1, 2.88f, 0.30f, 0.071f, 0.05f, 0.57f, 1.91f, 0.80f}, {32, 32, 1, 2.38f, 0.34f, 0.053f, 0.13f, 1.48f, 1.49f, 0.68f}},
+    {{}, {}, {128, 128, 2, 4.64f, 0.00f, 0.231f, 0.60f, 0.61f, 1.02f, 0.40f, 0.25f}, {},
+        {64, 64, 2, 3.82f, 0.29f, 0.082f, 0.23f, 0.70f, 0.89f, 0.63f, 0.34f},
+        {128, 128, 1, 4.02f, 0.77f, 0.142f, 0.99f, 0.f, 1.30f, 0.77f, 0.51f, 0.10f}, {}, {},
+        {32, 64, 1, 2.77f, 0.86f, 0.064f, 0.27f, 0.f, 1.03f, 0.71f, 0.62f, 0.00f},
+        {32, 32, 1, 2.90f, 0.65f, 0.046f, 0.20f, 0.f, 1.12f, 0.71f, 0.32f, 0.08f},
+        {256, 256, 1, 0.00f, 4.48f, 0.440f, 1.88f, 0.f, 1.02f, 0.54f, 0.97f, 0.11f},
+        {256, 192, 1, 5.13f, 0.01f, 0.388f, 1.26f, 0.f, 1.35f, 0.67f, 0.56f, 0.15f},
+        {128, 192, 2, 4.47f, 0.10f, 0.289f, 0.70f, 0.78f, 0.99f, 0.47f, 0.38f},
+        {128, 192, 1, 4.87f, 0.02f, 0.194f, 1.21f, 0.f, 1.45f, 0.62f, 0.55f, 0.11f},
+        {128, 64, 2, 3.91f, 0.15f, 0.116f, 0.37f, 0.90f, 1.02f, 0.61f, 0.38f}},
     {{256, 256, 1, 0.00f, 3.34f, 0.542f, 4.36f, 0.f, 0.f, 0.f}, {128, 256, 2, 2.72f, 0.81f, 0.391f, 1.69f, 1.03f, 1.39f, 0.63f},
         {128, 128, 3, 3.06f, 0.79f, 0.233f, 0.53f, 0.87f, 1.01f, 0.47f}, {64, 128, 3, 2.96f, 0.26f, 0.169f, 0.32f, 1.59f, 0.94f, 0.00f},
         {64, 64, 4, 3.19f, 0.04f, 0.141f, 0.24f, 0.60f, 0.66f, 0.00f}, {128, 128, 2, 3.04f, 0.62f, 0.221f, 0.66f, 1.62f, 1.38f, 0.61f},
         {64, 128, 2, 2.54f, 0.60f, 0.150f, 0.32f, 1.22f, 0.93f, 0.35f}, {64, 64, 2, 2.46f, 0.54f, 0.100f, 0.35f, 0.93f, 0.91f, 0.46f},
-        {32, 64, 2, 3.19f, 0.17f, 0.068f, 0.04f, 0.90f, 1.19f, 0.67f}, {32, 32, 4, 2.69f, 1.21f, 0.042f, 0.16f, 0.67f, 1.19f, 0.64f}}};
+        {32, 64, 2, 3.19f, 0.17f, 0.068f, 0.04f, 0.90f, 1.19f, 0.67f}, {32, 32, 4, 2.69f, 1.21f, 0.042f, 0.16f, 0.67f, 1.19f, 0.64f},
+        {}, {}, {}, {}, {}}};
 
 inline float tile_time(TileCost const& c, LinearArgs const& a, bool gelu)
 {
     float const x = (float) ceil_div(a.N, c.channels) * (float) ceil_div(a.T, c.tokens) / (float) num_cus();
-    float units = 1.f;
+    float units = 1.f + c.spill * std::max(0.f, 4.f * x - 3.f);
     if (x > 1.f)
     {
         float const y = c.whole * std::ceil(x) + (1.f - c.whole) * x, r = (float) c.resident;
-        units += c.share * (std::min(y, r) - 1.f) + c.turn * std::max(0.f, y - r);
+        units = 1.f + c.share * (std::min(y, r) - 1.f) + c.turn * std::max(0.f, y - r);
     }
-    return c.launch + units * (c.tile + (gelu ? c.gelu : 0.f) + c.stage * (float) (a.K / 64));
+    float const stage = c.stage * (1.f + c.busy * std::min(x, 1.f));
+    return c.launch + units * (c.tile + (gelu ? c.gelu : 0.f) + stage * (float) (a.K / 64));
 }
 
 // The same for the large tiles: whole rounds, and what is left behind them, as 64 x 64 pieces or as 128 x 128 tiles.
-inline float large_tiles_time(TileCost const& c, bool il, LinearArgs const& a, int64_t smallTiles, bool gelu)
+inline float large_tiles_time(TileCost const& c, LinearArgs const& a, int64_t smallTiles, bool gelu)
 {
     float const stages = (float) (a.K / 64), cus = (float) num_cus();
     float const rounds = (float) ceil_div(a.mainTiles, num_cus());
-    if (!il)
-    {
-        return c.launch + rounds * (c.tile + (gelu ? c.gelu : 0.f) + c.stage * stages) + (float) smallTiles / cus * 0.66f * stages;
-    }
     float rest = 0.f;
     if (a.pieces)
     {
@@ -1850,32 +1980,40 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
     a.parts = 1;
     a.mainTiles = (int) grid;
     auto run = [&](auto kernel, int threads) { return launch_tiles(stream, a, kernel, threads); };
-    switch (plan)
-    {
-    case kTile128x256: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 4, 2, 2, 3, 4>, 512);
-    case kTile128x128:
-        // four wavefronts and three workgroups per CU; linear operands gain from eight and a deeper ring
-        if constexpr (IL)
-        {
-            return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 2, 3, 3>, 256);
-        }
-        else
-        {
-            return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 4, 2, 1, 4, 4>, 512);
-        }
-    case kTile64x128: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 2, 4, 3>, 256);
-    case kTile64x64: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 1, 4, 4>, 256);
-    default: break;
-    }
     if constexpr (IL)
     {
         switch (plan)
         {
+        case kTile128x256: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 4, 2, 2, 3, 4>, 512);
+        case kTile128x128: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 2, 3, 3>, 256);
+        case kTile64x128: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 2, 4, 3>, 256);
+        case kTile64x64: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 1, 4, 4>, 256);
         case kTile128x128Deep: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 2, 4, 2>, 256);
         case kTile64x128Deep: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 2, 6, 2>, 256);
-        case kTile64x64Deep: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 1, 8, 2>, 256);
+        case kTile64x64Deep:
+            // 128 bytes of k per stage where k comes in those: half the barriers
+            return a.K % 128 == 0 ? run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 1, 4, 2, 4>, 256)
+                                  : run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 1, 8, 2>, 256);
         case kPiece32x64: return run(linear_piece_kernel<IL_OUT, EPI, 1, 2, 4, 4>, 512);
         case kPiece32x32: return run(linear_piece_kernel<IL_OUT, EPI, 1, 1, 8, 4>, 512);
+        default: break;
+        }
+    }
+    else if (plan == kPiece32x64)
+    {
+        return run(linear_piece_dma_kernel<IL_OUT, EPI, 1, 2, 3, 2>, 512);
+    }
+    else if (plan == kPiece32x32)
+    {
+        return run(linear_piece_dma_kernel<IL_OUT, EPI, 1, 1, 4, 2>, 512);
+    }
+    else if (a.K % 128 != 0)
+    {
+        // rows that end within a line: stages of 64 bytes
+        switch (plan)
+        {
+        case kTile128x128: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 2, 3, 2>, 256);
+        case kTile64x64: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 1, 4, 4>, 256);
         default: break;
         }
     }
@@ -1883,8 +2021,14 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
     {
         switch (plan)
         {
-        case kPiece32x64: return run(linear_piece_dma_kernel<IL_OUT, EPI, 1, 2, 3, 2>, 512);
-        case kPiece32x32: return run(linear_piece_dma_kernel<IL_OUT, EPI, 1, 1, 4, 2>, 512);
+        case kTile256x256: return run(linear_tile_kernel<IL, IL_OUT, EPI, 4, 2, 2, 4, 2, 2, 4>, 512);
+        case kTile256x192: return run(linear_tile_kernel<IL, IL_OUT, EPI, 4, 2, 2, 3, 2, 2, 4>, 512);
+        case kTile128x192: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 3, 2, 2, 4>, 256);
+        case kTile128x192Deep: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 3, 3, 1, 4>, 256);
+        case kTile128x128: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 2, 2, 2, 4>, 256);
+        case kTile128x128Deep: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 2, 4, 1, 4>, 256);
+        case kTile128x64: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 1, 3, 2, 4>, 256);
+        case kTile64x64: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 1, 5, 2, 4>, 256);
         default: break;
         }
     }
@@ -1912,28 +2056,31 @@ int launch_partial(hipStream_t stream, LinearArgs a, int parts, void* partial, W
 
 // The plan of a launch with operands of one layout and tokMain / mainTiles / pieces set up for the large tiles.
 template <bool IL>
-int choose_plan(LinearArgs const& a, int64_t smallTiles, bool gelu)
+int cheapest_plan(LinearArgs const& a, int64_t smallTiles, bool gelu, int plan)
 {
-    bool const large = a.N % kBig == 0 && a.K % 256 == 0 && a.mainTiles > 0;
-    int plan = tuning(Tuning::kLinearPlan);
-    if (plan >= 0 && plan < kLinearPlans && kTileCosts[IL][plan].channels != 0 && (plan != kLargeTiles || large))
+    bool const large = IL && a.N % kBig == 0 && a.K % 256 == 0 && a.mainTiles > 0;
+    auto const exists = [&](int q) {
+        if (q == kLargeTiles)
+        {
+            return large;
+        }
+        bool const halfLines = !IL && a.K % 128 != 0; // the tiles that have a kernel for those
+        return kTileCosts[IL][q].channels != 0
+            && (!halfLines || q == kTile128x128 || q == kTile64x64 || q == kPiece32x64 || q == kPiece32x32);
+    };
+    if (plan >= 0 && plan < kLinearPlans && exists(plan))
     {
         return plan;
     }
-    // Linear operands: the smaller tiles have to win by more than 8 %.  They read more bytes per multiplication, which a pass
-    // pays for in the launches around them too, and these constants are for launches by themselves (FP16 passes of 1000 to
-    // 25000 tokens without it: another choice at 5 of 17 sizes, 0.0 to 1.9 % slower; nowhere faster).
-    constexpr float kMargin = IL ? 1.f : 1.f / 1.08f;
-    float best = large ? kMargin * large_tiles_time(kTileCosts[IL][kLargeTiles], IL, a, smallTiles, gelu)
-                       : std::numeric_limits<float>::max();
-    plan = kLargeTiles;
-    for (int q = kTile128x256; q < kLinearPlans; ++q)
+    float best = std::numeric_limits<float>::max();
+    for (int q = kLargeTiles; q < kLinearPlans; ++q)
     {
-        if (kTileCosts[IL][q].channels == 0)
+        if (!exists(q))
         {
             continue;
         }
-        float const t = tile_time(kTileCosts[IL][q], a, gelu);
+        float const t = q == kLargeTiles ? large_tiles_time(kTileCosts[IL][q], a, smallTiles, gelu)
+                                         : tile_time(kTileCosts[IL][q], a, gelu);
         if (t < best)
         {
             best = t;
@@ -1943,11 +2090,34 @@ int choose_plan(LinearArgs const& a, int64_t smallTiles, bool gelu)
     return plan;
 }
 
+// The same, remembered by each thread for the sizes it asked for last: the layers of a pass ask for the same few plans over
+// and over, and the estimates take 0.3 us where a short launch costs the host 3.
+template <bool IL>
+int choose_plan(LinearArgs const& a, int64_t smallTiles, bool gelu)
+{
+    struct Choice
+    {
+        int T, K, N, mainTiles, pieces, gelu, setting, plan;
+        int64_t smallTiles;
+    };
+    constexpr int kChoices = 16;
+    thread_local Choice choices[kChoices] = {};
+    int const setting = tuning(Tuning::kLinearPlan);
+    Choice& c = choices[((uint32_t) a.T * 5u + (uint32_t) (a.K >> 6) * 3u + (uint32_t) (a.N >> 5) * 7u + (uint32_t) gelu) % kChoices];
+    if (c.T != a.T || c.K != a.K || c.N != a.N || c.mainTiles != a.mainTiles || c.pieces != a.pieces || c.gelu != (int) gelu
+        || c.setting != setting || c.smallTiles != smallTiles)
+    {
+        c = {a.T, a.K, a.N, a.mainTiles, a.pieces, (int) gelu, setting, cheapest_plan<IL>(a, smallTiles, gelu, setting), smallTiles};
+    }
+    return c.plan;
+}
+
 // The plan of a launch too short for large tiles, for callers that want to know ahead (-1: one that may have them).
 template <bool IL>
 int small_plan(LinearArgs a, bool gelu)
 {
-    if ((int64_t) ceil_div(a.N, kBig) * (a.T / kBig) > 0 || !tuning(Tuning::kLinearPersistent) || !tuning(Tuning::kLinearDirect))
+    bool const large = IL && (int64_t) ceil_div(a.N, kBig) * (a.T / kBig) > 0;
+    if (large || !tuning(Tuning::kLinearPersistent) || !tuning(Tuning::kLinearDirect))
     {
         return -1;
     }
@@ -2024,11 +2194,14 @@ int launch_shape(hipStream_t stream, LinearArgs a)
             {
                 return launch_plan<IL_W, IL_OUT, EPI>(stream, a, plan);
             }
-            a.persist = a.mainTiles < cus ? a.mainTiles : cus;
-            int64_t const behind = a.pieces ? (int64_t) (a.N / 64) * ceil_div(restTokens, 64) : smallTiles;
-            hipLaunchKernelGGL((int8_linear_dma_kernel<IL_W, IL_OUT, EPI>), dim3((uint32_t) (a.persist + behind)), dim3(512), 0,
-                stream, a);
-            return check_launch("int8_linear_dma_kernel");
+            if constexpr (IL_W && (EPI == kAFFINE || EPI == kGELU))
+            {
+                a.persist = a.mainTiles < cus ? a.mainTiles : cus;
+                int64_t const behind = a.pieces ? (int64_t) (a.N / 64) * ceil_div(restTokens, 64) : smallTiles;
+                hipLaunchKernelGGL((int8_linear_dma_kernel<IL_OUT, EPI>), dim3((uint32_t) (a.persist + behind)), dim3(512), 0,
+                    stream, a);
+                return check_launch("int8_linear_dma_kernel");
+            }
         }
     }
     if (persistent && a.K % 128 == 0)

@@ -129,6 +129,54 @@ def test_linear_plans(plan, T, K, N):
         assert_fp_close(got, ref, what=f"plan {plan} FP16")
 
 
+# tiles of linear operands: stages of 128 bytes of k (64 FP16 values), rings of two to five of them.  One stage, as many as
+# the ring has and one more; a last line that is half there; token and channel counts on both sides of a tile's edge.
+@pytest.mark.parametrize("plan", [2, 4, 5, 10, 11, 12, 13, 14])
+@pytest.mark.parametrize("T,K,N", [(1, 64, 32), (63, 128, 96), (191, 192, 128), (193, 256, 160), (257, 384, 288), (65, 160, 64),
+                                   (130, 608, 224)])
+def test_linear_tiles_of_whole_lines(plan, T, K, N):
+    """FP16 against binary64 and against the pieces' results; INT8 with linear operands byte for byte against the
+    register-staged kernel; nothing written behind the last row."""
+    r = rng(97 + T)
+    x = r.standard_normal((T, K)).astype(np.float16)
+    w = (0.05 * r.standard_normal((N, K))).astype(np.float16)
+    alpha, beta = r.uniform(0.5, 1.5, N).astype(np.float32), (0.1 * r.standard_normal(N)).astype(np.float32)
+    exact = (x.astype(np.float64) @ w.astype(np.float64).T) * alpha + beta
+    for gelu in (False, True):
+        with tuning("TRTAMD_LINEAR_PLAN", plan):
+            got = run_fp16(x, w, alpha, beta, gelu)
+        with tuning("TRTAMD_LINEAR_PLAN", 9):
+            pieces = run_fp16(x, w, alpha, beta, gelu)
+        assert_fp_close(got, oracle.fp16_linear(x, w, alpha, beta, gelu=gelu), what=f"plan {plan}")
+        # either kernel rounds a binary32 sum once: they differ by a unit in the last place where the sums straddle a tie
+        assert_fp_close(got, pieces, atol=2.0 ** -14, rtol=2.0 ** -10, what=f"plan {plan} against the pieces")
+        if not gelu:
+            assert_fp_close(got, exact, what=f"plan {plan} against binary64")
+    a, w8, al, be = problem(98 + T, T, 2 * K, N)
+    for out_il in (False, True):
+        with tuning("TRTAMD_LINEAR_DIRECT", 0):
+            want = run_gpu(a, w8, al, be, capi.LINEAR_AFFINE, out_il=out_il)
+        with tuning("TRTAMD_LINEAR_PLAN", plan):
+            got = run_gpu(a, w8, al, be, capi.LINEAR_AFFINE, out_il=out_il)
+        assert np.array_equal(got, want)
+
+
+def test_fp16_tiles_write_nothing_behind_the_last_row():
+    import torch
+    api = capi.api()
+    T, K, N = 130, 128, 96
+    r = rng(99)
+    x, w = dev(r.standard_normal((T, K)).astype(np.float16)), dev(r.standard_normal((N, K)).astype(np.float16))
+    one, zero = dev(np.ones(N, np.float32)), dev(np.zeros(N, np.float32))
+    for plan in (2, 4, 5, 10, 11, 12, 13, 14):
+        out = dev_empty((T + 200, N), np.float16, fill=-7)
+        p = capi.Fp16LinearParams(ptr(x), ptr(w), ptr(one), ptr(zero), ptr(out), T, K, N, capi.LINEAR_AFFINE)
+        with tuning("TRTAMD_LINEAR_PLAN", plan):
+            api.check(api.fp16_linear(stream(), C.byref(p)))
+        torch.cuda.synchronize()
+        assert (host(out)[T:] == -7).all() and (host(out)[:T] != -7).any()
+
+
 FMHA_SETTINGS = [("TRTAMD_FMHA_GENERIC", 1), ("TRTAMD_FMHA_QSPLIT", 1), ("TRTAMD_FMHA_QSPLIT", 2),
                  ("TRTAMD_FMHA_QSPLIT", 3), ("TRTAMD_FMHA_QSPLIT", 4), ("TRTAMD_FMHA_RANKED", 0),
                  ("TRTAMD_FMHA_RANKED", 1)]
