@@ -1866,6 +1866,12 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
 // sizes of 2465 to 23000 tokens the pass takes 0.8 % less than with constants for launches by themselves, one of them more
 // than 0.8 % more (7399 tokens, 1.9 %), and the best of the measured combinations would take another 0.9 % less (4 % at
 // most).  32 sequences of up to 256 tokens: 2979 -> 2877 us.
+// Interleaved tiles of 256 x 256, 256 x 192 and 128 x 192 fill the chip once where the ones above need a round and a bit
+// of it (128 x 128 tiles for 5012 tokens x 4096 -> 1024: 1.25 rounds; 128 x 192: 0.84): fitted to whole passes as well, 70
+// sizes on two GPUs with one layer's plan changed at a time, and only to launches of one round, where they were 1 to 5 % of
+// the pass faster or slower by the size alone; what they take beyond that follows no such line, and they are not taken
+// there.  0.4 us in `launch` is the margin by which they have to win (without it some passes are 2 % slower).  At these sizes
+// the pass takes 1.3 % less in the mean, 8.8 % at most (8200 tokens), and more than 0.5 % more at two of 140.
 // Deep rings: where one workgroup per CU is all there is, a tile is bound by the trips to memory of its own stages, and
 // the LDS of the workgroups that do not come is better used for more of them (interleaved, weights from memory, 600 tokens
 // x 4096 -> 1024 in 64 x 64 tiles: 12.9 us with three stages ahead, 9.5 us with seven; 128 x 128 tiles, 1900 tokens 20.8
@@ -1896,6 +1902,7 @@ enum LinearPlan
     kTile128x64,
     kLinearPlans
 };
+constexpr float kOneRound = 1e3f; // of tiles that are taken only where a launch has no more of them than CUs
 // [0]: linear operands, [1]: interleaved ones.  No channels: the layout has no such kernel.
 constexpr TileCost kTileCosts[2][kLinearPlans] = {
     {{}, {}, {128, 128, 2, 4.64f, 0.00f, 0.231f, 0.60f, 0.61f, 1.02f, 0.40f, 0.25f}, {},
@@ -1913,7 +1920,8 @@ constexpr TileCost kTileCosts[2][kLinearPlans] = {
         {64, 64, 4, 3.19f, 0.04f, 0.141f, 0.24f, 0.60f, 0.66f, 0.00f}, {128, 128, 2, 3.04f, 0.62f, 0.221f, 0.66f, 1.62f, 1.38f, 0.61f},
         {64, 128, 2, 2.54f, 0.60f, 0.150f, 0.32f, 1.22f, 0.93f, 0.35f}, {64, 64, 2, 2.46f, 0.54f, 0.100f, 0.35f, 0.93f, 0.91f, 0.46f},
         {32, 64, 2, 3.19f, 0.17f, 0.068f, 0.04f, 0.90f, 1.19f, 0.67f}, {32, 32, 4, 2.69f, 1.21f, 0.042f, 0.16f, 0.67f, 1.19f, 0.64f},
-        {}, {}, {}, {}, {}}};
+        {256, 256, 1, 5.39f, 0.f, 0.406f, 4.88f, 0.f, kOneRound, 1.f, 0.41f}, {256, 192, 1, 5.31f, 0.f, 0.217f, 2.67f, 0.f, kOneRound, 1.f, 1.50f},
+        {128, 192, 1, 4.55f, 0.f, 0.142f, 1.01f, 0.f, kOneRound, 1.f, 1.47f}, {}, {}}};
 
 inline float tile_time(TileCost const& c, LinearArgs const& a, bool gelu)
 {
@@ -1994,6 +2002,9 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
             // 128 bytes of k per stage where k comes in those: half the barriers
             return a.K % 128 == 0 ? run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 1, 4, 2, 4>, 256)
                                   : run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 1, 8, 2>, 256);
+        case kTile256x256: return run(linear_tile_kernel<IL, IL_OUT, EPI, 4, 2, 2, 4, 4, 2>, 512);
+        case kTile256x192: return run(linear_tile_kernel<IL, IL_OUT, EPI, 4, 2, 2, 3, 5, 2>, 512);
+        case kTile128x192: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 3, 4, 2>, 256);
         case kPiece32x64: return run(linear_piece_kernel<IL_OUT, EPI, 1, 2, 4, 4>, 512);
         case kPiece32x32: return run(linear_piece_kernel<IL_OUT, EPI, 1, 1, 8, 4>, 512);
         default: break;

@@ -161,6 +161,22 @@ def test_linear_tiles_of_whole_lines(plan, T, K, N):
         assert np.array_equal(got, want)
 
 
+# the same tiles of interleaved operands: stages of 64 bytes, rings of four and five
+@pytest.mark.parametrize("plan", [7, 10, 11, 12])
+@pytest.mark.parametrize("T,K,N", [(1, 64, 32), (191, 256, 128), (193, 320, 160), (257, 384, 288), (130, 1088, 224)])
+def test_linear_tiles_of_interleaved_operands(plan, T, K, N):
+    """Byte for byte against the register-staged kernel, affine and GELU, either output layout."""
+    a, w, alpha, beta = problem(94 + T, T, K, N)
+    for epi, scale, f in ((capi.LINEAR_AFFINE, 1.0, 1.0), (capi.LINEAR_GELU, float(np.float32(127.0 / 4.0)), 0.06)):
+        al, be = (alpha * f).astype(np.float32), (beta * f / 3).astype(np.float32)
+        for out_il in (False, True):
+            with tuning("TRTAMD_LINEAR_DIRECT", 0):
+                want = run_gpu(a, w, al, be, epi, out_scale=scale, a_il=True, w_il=True, out_il=out_il)
+            with tuning("TRTAMD_LINEAR_PLAN", plan):
+                got = run_gpu(a, w, al, be, epi, out_scale=scale, a_il=True, w_il=True, out_il=out_il)
+            assert np.array_equal(got, want)
+
+
 def test_fp16_tiles_write_nothing_behind_the_last_row():
     import torch
     api = capi.api()
