@@ -250,3 +250,33 @@ def test_fp16_attention_variants(name, value, S, lens):
         assert_fp_close(got, default, atol=1e-3, rtol=2e-3, what="general kernel vs prefix kernel")
     else:
         assert np.array_equal(got.view(np.uint16), default.view(np.uint16)), f"{name}={value}: bits differ from the default"
+
+
+@pytest.mark.parametrize("B", [1, 63, 64, 65, 127, 128, 129])
+def test_longest_first_order_reaches_every_sequence(B):
+    """The longest-first order on either side of what a wavefront keeps in its registers, with empty sequences, many of one
+    length and one longer than the kernel serves whole: the bytes of the natural order."""
+    r = rng(1500 + B)
+    lens = r.integers(0, 40, B)
+    lens[:: 3] = 17
+    lens[B // 2] = 70
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T, N, S = int(cu[-1]), 2, 64
+    qkv, s_q = quantize_amax(r.standard_normal((T, 3 * N * 64)).astype(np.float32))
+    d_qkv, d_cu = dev(interleave(qkv)), dev(cu)
+    api = capi.api()
+    outs = []
+    for ranked in (0, 1):
+        out = dev_empty((N * 2, T, 32), np.int8, fill=55)
+        p = capi.FmhaParams()
+        p.qkv_ptr, p.o_ptr, p.cu_seqlens = ptr(d_qkv), ptr(out), ptr(d_cu)
+        p.qkv_stride_in_bytes = p.o_stride_in_bytes = T
+        p.b, p.h, p.s, p.d, p.interleaved = B, N, S, 64, 1
+        bits = lambda x: int(np.float32(x).view(np.uint32))
+        p.scale_bmm1, p.scale_softmax, p.scale_bmm2 = bits(s_q * s_q * 0.125), bits(127.0), bits(s_q / 127.0 / 0.02)
+        with tuning("TRTAMD_FMHA_RANKED", ranked):
+            api.check(api.fused_mha_run(stream(), 2, C.byref(p)))
+            sync()
+        outs.append(host(out))
+    assert np.array_equal(outs[0], outs[1])
+    assert all((outs[0][:, cu[b]:cu[b + 1]] != 55).any() for b in range(B) if lens[b])
