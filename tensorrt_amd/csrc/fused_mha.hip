@@ -57,7 +57,7 @@ __device__ inline float mul_rounded(float a, float b)
     return a * b;
 }
 
-// The MFMAs of the cu_seqlens kernels (fmha_i8_prefix_kernel, fmha_f16_turns_kernel, fmha_f16_prefix_kernel) go through
+// The MFMAs of the cu_seqlens kernels (fmha_i8_prefix_kernel, fmha_f16_turns_kernel, fmha_f16_stream_kernel) go through
 // these wrappers.  A
 // library built with -DTRTAMD_ABLATE_ATTENTION_MFMA (`python -m tensorrt_amd.build --ablation` writes it to
 // lib/libtrtamd_ablation.so; `python -m tensorrt_amd.kernel_bench --ablation` times it; nothing else loads it) leaves
@@ -82,6 +82,17 @@ __device__ __forceinline__ f32x4 attention_mfma_f16(f16x8 const a, f16x8 const b
     return d;
 #else
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+#endif
+}
+
+__device__ __forceinline__ f32x16 attention_mfma_f16_32(f16x8 const a, f16x8 const b, f32x16 c)
+{
+#ifdef TRTAMD_ABLATE_ATTENTION_MFMA
+    f32x16 d;
+    asm volatile("; v_mfma_f32_32x32x16_f16 left out" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+    return d;
+#else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 #endif
 }
 
@@ -1406,310 +1417,7 @@ __global__ __launch_bounds__(kWavesF16* kWaveSize) void fmha_f16_kernel(FmhaArgs
 }
 
 // ------------------------------------------------------------------------------------------
-// FP16, prefix-valid keys, many units of more than 384: same specialisation on the number of 64-key blocks as the INT8
-// kernel.  K and V of a unit are staged once for all of its queries, at one workgroup of eight wavefronts per CU.
-// ------------------------------------------------------------------------------------------
-
-template <int KT>
-__device__ inline void stage_kv_prefix_f16(FmhaArgs const& a, int64_t seqBase, int64_t firstTok, int n, int nk,
-    int nkb, uint8_t* sK, uint8_t* sV)
-{
-    constexpr int kRowsPerPass = kWavesF16 * kWaveSize / 8;   // 8 chunks of 16 bytes per 128-byte row
-    constexpr int kPasses = 64 / kRowsPerPass;
-    constexpr int kRow = Lds<2>::kRow;
-    uint8_t const* src = static_cast<uint8_t const*>(a.qkv);
-    int const chunk = threadIdx.x & 7;
-    int const rowInPass = threadIdx.x >> 3;
-    u32x4 kv[KT][kPasses], vv[KT][kPasses];
-#pragma unroll
-    for (int kb = 0; kb < KT; ++kb)
-    {
-#pragma unroll
-        for (int p = 0; p < kPasses; ++p)
-        {
-            int const key = kb * 64 + p * kRowsPerPass + rowInPass;
-            kv[kb][p] = u32x4{0, 0, 0, 0};
-            vv[kb][p] = u32x4{0, 0, 0, 0};
-            if (key < nk)
-            {
-                kv[kb][p] = *reinterpret_cast<u32x4 const*>(
-                    src + qkv_chunk_offset<2, false>(a, seqBase, firstTok, key, n, 1, chunk));
-                vv[kb][p] = *reinterpret_cast<u32x4 const*>(
-                    src + qkv_chunk_offset<2, false>(a, seqBase, firstTok, key, n, 2, chunk));
-            }
-        }
-    }
-#pragma unroll
-    for (int kb = 0; kb < KT; ++kb)
-    {
-        if (kb < nkb)
-        {
-#pragma unroll
-            for (int p = 0; p < kPasses; ++p)
-            {
-                int const kk = p * kRowsPerPass + rowInPass;
-                int const kr = kb * 64 + kk;
-                int const vr = kb * 64 + v_row<2>(kk);
-                *reinterpret_cast<u32x4*>(sK + kr * kRow + swz<2>(kr, chunk) * 16) = kv[kb][p];
-                *reinterpret_cast<u32x4*>(sV + vr * kRow + swz<2>(vr, chunk) * 16) = vv[kb][p];
-            }
-        }
-    }
-}
-
-template <int NKB, bool DEBUG>
-__device__ __forceinline__ void attend_f16(FmhaArgs const& a, SeqInfo const& sq, int const b, int const n,
-    int const qtBegin, int const qtEnd, uint8_t const* sK, uint8_t const* sV, f16x8 const qFirst0,
-    f16x8 const qFirst1)
-{
-    constexpr int kRow = Lds<2>::kRow;
-    constexpr int NT = NKB * 4;
-    int const lane = threadIdx.x & (kWaveSize - 1);
-    int const wave = threadIdx.x >> 6;
-    int const lq = lane & 15;
-    int const g = lane >> 4;
-    uint8_t const* src = static_cast<uint8_t const*>(a.qkv);
-    f16x8 ones;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-    {
-        ones[i] = (f16) 1.f;
-    }
-    int const lastKeys = sq.nk - (NKB - 1) * 64;
-    int const lastHalves = (lastKeys + 31) >> 5;   // 32-key halves of the last block that hold keys
-    int const lastRel = lastKeys - 4 * g;          // key 16u + j of this lane group exists iff 16u + j < lastRel
-
-    auto load_q = [&](int qt, int h) -> f16x8 {
-        int const qq = qt * kQPerWave + lq;
-        u32x4 raw = {0, 0, 0, 0};
-        if (qq < sq.nq)
-        {
-            raw = *reinterpret_cast<u32x4 const*>(
-                src + qkv_chunk_offset<2, false>(a, sq.seqBaseIn, sq.firstTok, qq, n, 0, h * 4 + g));
-        }
-        return __builtin_bit_cast(f16x8, raw);
-    };
-    f16x8 qnext[2] = {qFirst0, qFirst1};
-    for (int qt = qtBegin + wave; qt < qtEnd; qt += kWavesF16)
-    {
-        int const q = qt * kQPerWave + lq;
-        bool const qValid = q < sq.nq;
-        f16x8 const qreg[2] = {qnext[0], qnext[1]};
-        qnext[0] = load_q(qt + kWavesF16, 0);
-        qnext[1] = load_q(qt + kWavesF16, 1);
-
-        // ---- S^T = K Q^T (binary32 accumulation); absent keys start from -infinity
-        f32x4 acc[NT];
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-        {
-            int const key = t * 16 + lq;
-            f32x4 sd = {0.f, 0.f, 0.f, 0.f};
-            if (t >= NT - 4)
-            {
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                {
-                    sd[j] = (16 * (t & 3) + j) < lastRel ? 0.f : -__builtin_inff();
-                }
-            }
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-            {
-                f16x8 const kreg = *reinterpret_cast<f16x8 const*>(sK + key * kRow + swz<2>(key, h * 4 + g) * 16);
-                sd = attention_mfma_f16(kreg, qreg[h], sd);
-            }
-            acc[t] = sd;
-        }
-        __builtin_amdgcn_sched_barrier(0);
-
-        if (DEBUG && a.dbgAcc1 && qValid)
-        {
-            for (int t = 0; t < NT; ++t)
-            {
-                for (int j = 0; j < 4; ++j)
-                {
-                    int const key = t * 16 + g * 4 + j;
-                    if (key < sq.nk)
-                    {
-                        a.dbgAcc1[(((int64_t) b * a.N + n) * a.S + q) * a.S + key] = __float_as_int(acc[t][j]);
-                    }
-                }
-            }
-        }
-
-        // ---- row max
-        float mxA = -__builtin_inff(), mxB = -__builtin_inff();
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-        {
-            mxA = fmaxf(fmaxf(mxA, acc[t][0]), acc[t][1]);
-            mxB = fmaxf(fmaxf(mxB, acc[t][2]), acc[t][3]);
-        }
-        float mx = fmaxf(mxA, mxB);
-        mx = reduce_step<16>(mx, [](float x, float y) { return fmaxf(x, y); });
-        mx = reduce_step<32>(mx, [](float x, float y) { return fmaxf(x, y); });
-        __builtin_amdgcn_sched_barrier(0);
-
-        // ---- p = 2^((s - max) * c) rounded to binary16; O^T = V^T P^T; row sum by a tile of ones
-        float const negK0 = -mx * a.c; // nk >= 1: the maximum is finite
-        f32x4 oacc[4];
-        f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-        {
-            oacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb)
-        {
-#pragma unroll
-            for (int hb = 0; hb < 2; ++hb)
-            {
-                if (kb == NKB - 1 && hb >= lastHalves)
-                {
-                    continue; // no key in this half
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                f16x8 preg;
-#pragma unroll
-                for (int w = 0; w < 2; ++w)
-                {
-                    int const t = kb * 4 + hb * 2 + w;
-                    float pr[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                    {
-                        pr[j] = __builtin_amdgcn_exp2f(fmaf(acc[t][j], a.c, negK0));
-                    }
-                    f16x2 const p01 = __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(pr[0], pr[1]));
-                    f16x2 const p23 = __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(pr[2], pr[3]));
-                    preg[w * 4 + 0] = p01[0];
-                    preg[w * 4 + 1] = p01[1];
-                    preg[w * 4 + 2] = p23[0];
-                    preg[w * 4 + 3] = p23[1];
-                }
-                int const vrow = kb * 64 + hb * 32 + 4 * g + (lq >> 2);
-                uint8_t const* vbase = sV + vrow * kRow + 8 * (lq & 1);
-#pragma unroll
-                for (int dt = 0; dt < 4; ++dt)
-                {
-                    int const sc = swz<2>(vrow, 2 * dt + ((lq >> 1) & 1)) * 16;
-                    i16x4 const v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*) (vbase + sc));
-                    i16x4 const v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*) (vbase + 16 * kRow + sc));
-                    typedef short i16x8 __attribute__((ext_vector_type(8)));
-                    i16x8 const both = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
-                    oacc[dt] = attention_mfma_f16(__builtin_bit_cast(f16x8, both), preg, oacc[dt]);
-                }
-                sacc = attention_mfma_f16(ones, preg, sacc);
-            }
-        }
-
-        // Lane (g, query) holds 8 bytes of each 32-byte quarter dt of the query's 128-byte row; a 4 x 4 transpose over
-        // the four rows of 16 lanes (v_permlane32_swap, v_permlane16_swap, once for each dword) leaves it with the
-        // whole quarter dt = g, which goes out as two 16-byte stores.
-        {
-            float const rinv = 1.f / sacc[0];
-            uint32_t lo[4], hi[4];
-#pragma unroll
-            for (int dt = 0; dt < 4; ++dt)
-            {
-                f16x4 y;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                {
-                    y[j] = (f16) (oacc[dt][j] * rinv);
-                }
-                u32x2 const w = __builtin_bit_cast(u32x2, y);
-                lo[dt] = w[0];
-                hi[dt] = w[1];
-            }
-            rows_transpose(lo);
-            rows_transpose(hi);
-            if (qValid)
-            {
-                uint8_t* dst = static_cast<uint8_t*>(a.out);
-                int64_t const off
-                    = sq.seqBaseOut + (int64_t) q * a.tokStrideOut + ((int64_t) n * kHeadSize + g * 16) * 2;
-                u32x4 const first = {lo[0], hi[0], lo[1], hi[1]};
-                u32x4 const second = {lo[2], hi[2], lo[3], hi[3]};
-                *reinterpret_cast<u32x4*>(dst + off) = first;
-                *reinterpret_cast<u32x4*>(dst + off + 16) = second;
-            }
-        }
-    }
-}
-
-template <int KT, bool DEBUG>
-__global__ __launch_bounds__(kWavesF16* kWaveSize) void fmha_f16_prefix_kernel(FmhaArgs const a)
-{
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    uint8_t* sK = smem;
-    uint8_t* sV = smem + Lds<2>::matBytes(KT);
-    __shared__ PickLds sPick;
-    UnitPart const up = unit_of_workgroup(blockIdx.x, gridDim.x, a.qSplit);
-    int const part = up.part;
-    int const n = up.unit % a.N;
-    int b;
-    SeqInfo const sq = pick_sequence_info<kWavesF16 * kWaveSize>(a, up.unit / a.N, KT * 64, sPick, b);
-    int const nqt = (sq.nq + kQPerWave - 1) / kQPerWave;
-    int const per = kWavesF16 * ((nqt + kWavesF16 * a.qSplit - 1) / (kWavesF16 * a.qSplit));
-    int const qtBegin = min(part * per, nqt);
-    int const qtEnd = min(qtBegin + per, nqt);
-    if (qtBegin >= qtEnd)
-    {
-        return;
-    }
-    int const nkb = (sq.nk + 63) >> 6;
-    f16x8 qFirst[2];
-    {
-        int const qt = qtBegin + (int) (threadIdx.x >> 6);
-        int const qq = qt * kQPerWave + (int) (threadIdx.x & 15);
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-        {
-            u32x4 raw = {0, 0, 0, 0};
-            if (qq < sq.nq && qt < qtEnd)
-            {
-                raw = *reinterpret_cast<u32x4 const*>(static_cast<uint8_t const*>(a.qkv)
-                    + qkv_chunk_offset<2, false>(a, sq.seqBaseIn, sq.firstTok, qq, n, 0,
-                        h * 4 + (int) ((threadIdx.x & 63) >> 4)));
-            }
-            qFirst[h] = __builtin_bit_cast(f16x8, raw);
-        }
-    }
-    stage_kv_prefix_f16<KT>(a, sq.seqBaseIn, sq.firstTok, n, sq.nk, nkb, sK, sV);
-    __syncthreads();
-    switch (nkb)
-    {
-    case 1: attend_f16<1, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst[0], qFirst[1]); break;
-    case 2:
-        if (KT >= 2) attend_f16<(KT >= 2 ? 2 : 1), DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst[0], qFirst[1]);
-        break;
-    case 3:
-        if (KT >= 3) attend_f16<(KT >= 3 ? 3 : 1), DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst[0], qFirst[1]);
-        break;
-    case 4:
-        if (KT >= 4) attend_f16<(KT >= 4 ? 4 : 1), DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst[0], qFirst[1]);
-        break;
-    case 5:
-        if (KT >= 5) attend_f16<(KT >= 5 ? 5 : 1), DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst[0], qFirst[1]);
-        break;
-    case 6:
-        if (KT >= 6) attend_f16<(KT >= 6 ? 6 : 1), DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst[0], qFirst[1]);
-        break;
-    case 7:
-        if (KT >= 7) attend_f16<(KT >= 7 ? 7 : 1), DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst[0], qFirst[1]);
-        break;
-    case 8:
-        if (KT >= 8) attend_f16<(KT >= 8 ? 8 : 1), DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst[0], qFirst[1]);
-        break;
-    default: break;
-    }
-}
-
-// ------------------------------------------------------------------------------------------
-// FP16, prefix-valid keys, up to 384 of them (or few units): the same specialisation, but K and V take turns in LDS, one
+// FP16, prefix-valid keys, launches that leave CUs idle: the same specialisation, but K and V take turns in LDS, one
 // block of V in the place of each block of K as soon as every wavefront has multiplied it.  48 KB for 384 keys instead of
 // 96 KB: three workgroups of four wavefronts share a CU, so that one computes while another waits for its sequence, its K
 // or its V, and a unit's queries are shared out 64 at a time over as many workgroups.  What bounds either kernel is that
@@ -2022,6 +1730,295 @@ __global__ __launch_bounds__(kWavesF16T* kWaveSize)
 }
 
 // ------------------------------------------------------------------------------------------
+// FP16, prefix-valid keys, launches that fill the chip: 32 queries per wavefront, K and V in blocks of 64 keys through two
+// slots of LDS, the softmax kept up from block to block.  A workgroup takes 128 queries, so K and V come from the L2 half
+// as often as above, every fragment read from LDS serves twice the queries, and 36 KB let four workgroups share a CU.
+// The weights are relative to a running maximum that is only moved when it would be passed by more than a factor of 2^8,
+// which they and their binary32 sums hold without loss: a branch that is rarely taken after the first block.  What bounds it
+// is issue: per wavefront and block 512 cycles of matrix instructions, as many of exponentials and 400 of other vector work,
+// which overlap in part (~2000 cycles measured).  12 heads, sequences of a third of the length to the length, the
+// kernels it took the place of / this one, us: 32 x 256 keys 13.9 / 13.1, 32 x 384 21.6 / 19.0, 128 x 256 36.5 / 33.2,
+// 64 x 384 35.8 / 32.8, 16 x 512 22.7 / 18.0, 16 heads x 128 x 384 98.5 / 82.4, 128 x 512 145 / 134.
+// ------------------------------------------------------------------------------------------
+constexpr int kWavesStream = 4;
+constexpr int kStreamQueries = 32; // per wavefront
+constexpr int kStreamBlock = 64 * Lds<2>::kRow;     // bytes of 64 rows of K or V
+constexpr int kStreamStage = 2 * kStreamBlock;
+constexpr int kStreamLds = 2 * kStreamStage;
+
+template <bool DEBUG>
+__global__ __launch_bounds__(kWavesStream* kWaveSize) __attribute__((amdgpu_waves_per_eu(4))) void fmha_f16_stream_kernel(
+    FmhaArgs const a, int const capacity)
+{
+    constexpr int kRow = Lds<2>::kRow;
+    constexpr int kLoads = 2 * 8 / kWavesStream; // direct loads per wavefront and block: 8 rows each, of K and of V
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    __shared__ PickLds sPick;
+    UnitPart const up = unit_of_workgroup(blockIdx.x, gridDim.x, a.qSplit);
+    int const n = __builtin_amdgcn_readfirstlane(up.unit % a.N);
+    int b;
+    SeqInfo sq = pick_sequence_info<kWavesStream * kWaveSize>(a, up.unit / a.N, capacity, sPick, b);
+    // the same in every lane, which the compiler cannot see where they come from LDS: scalars keep the addresses scalar
+    b = __builtin_amdgcn_readfirstlane(b);
+    int const nq = __builtin_amdgcn_readfirstlane(sq.nq), nk = __builtin_amdgcn_readfirstlane(sq.nk);
+    int const firstTok = __builtin_amdgcn_readfirstlane((int) sq.firstTok);
+    int64_t const baseIn = a.cuSeqlens ? firstTok * a.tokStrideIn : b * a.seqStrideIn;
+    int64_t const baseOut = a.cuSeqlens ? firstTok * a.tokStrideOut : b * a.seqStrideOut;
+    int const lane = threadIdx.x & (kWaveSize - 1);
+    int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int const q0 = __builtin_amdgcn_readfirstlane(up.part) * (kWavesStream * kStreamQueries);
+    if (q0 >= nq)
+    {
+        return;
+    }
+    int const qw = q0 + wave * kStreamQueries; // this wavefront's first query
+    bool const active = qw < nq;               // if not, it only brings in its rows
+    int const lq = lane & 31, h = lane >> 5;
+    uint32_t const ldsBase = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) lds;
+    uint8_t const* const unit = static_cast<uint8_t const*>(a.qkv) + baseIn + (int64_t) n * 3 * kRow;
+    uint32_t const stride = (uint32_t) a.tokStrideIn;
+
+    // 8 rows of matrix `mat` from `row` on to LDS byte `to`; unless complete, those at or behind `limit` as the last one, or
+    // for V as zeros: 0, the weight of such a key, times an infinite V would not be 0
+    int const r8 = lane >> 3;
+    uint32_t const chunk = (uint32_t) (((lane & 7) ^ r8) * 16); // the swizzle of swz<2>, on the source side
+    uint32_t const whole = (uint32_t) r8 * stride + chunk;
+    auto request = [&](int mat, int row, int limit, int to, bool complete) {
+        int const first = complete ? row : min(row, limit - 1);
+        uint8_t const* const src = unit + (int64_t) first * a.tokStrideIn + mat * kRow;
+        uint32_t const dst = ldsBase + (uint32_t) to;
+        uint32_t off = whole;
+        if (!complete && row + 8 > limit)
+        {
+            if (mat == 2)
+            {
+                load_to_lds16(row + r8 < limit ? src + whole : reinterpret_cast<uint8_t const*>(kZeroRow) + chunk, dst);
+                return;
+            }
+            off = (uint32_t) min(r8, limit - 1 - first) * stride + chunk;
+        }
+        load_to_lds16_sbase(src, off, dst);
+    };
+    int const nb = (nk + 63) >> 6;
+    // A block that is all there: one address, advanced from block to block (a wavefront that waits for its own scalar
+    // arithmetic here is late with the next block and everything behind it).
+    uint64_t const step8 = (uint64_t) (8 * kWavesStream) * stride;
+    uint64_t kNext = reinterpret_cast<uint64_t>(unit) + (uint64_t) (8 * wave) * stride + kRow;
+    auto request_block = [&](int kb, int slot) {
+        uint32_t const to = (uint32_t) (slot * kStreamStage + wave * 8 * kRow);
+        if (kb * 64 + 64 <= nk)
+        {
+#pragma unroll
+            for (int i = 0; i < kLoads / 2; ++i)
+            {
+                void const* const src = reinterpret_cast<void const*>(kNext + i * step8);
+                load_to_lds16_sbase(src, whole, ldsBase + to + (uint32_t) (i * kWavesStream * 8 * kRow));
+                load_to_lds16_sbase(src, whole + kRow, ldsBase + to + (uint32_t) (kStreamBlock + i * kWavesStream * 8 * kRow));
+            }
+            kNext += 64ull * stride;
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < kLoads / 2; ++i)
+        {
+            int const r = (i * kWavesStream + wave) * 8;
+            request(1, kb * 64 + r, nk, slot * kStreamStage + r * kRow, false);
+            request(2, kb * 64 + r, nk, slot * kStreamStage + kStreamBlock + r * kRow, false);
+        }
+    };
+
+    // Q passes through the second slot
+    static_assert(kWavesStream * kStreamQueries * kRow <= kStreamStage, "Q in a slot");
+    int const qAt = kStreamStage + wave * kStreamQueries * kRow;
+#pragma unroll
+    for (int i = 0; i < kStreamQueries / 8; ++i)
+    {
+        request(0, qw + 8 * i, nq, qAt + 8 * i * kRow, false);
+    }
+    request_block(0, 0);
+    wait_vmcnt<kLoads>();
+    asm volatile("" ::: "memory");
+    f16x8 qreg[4]; // B operand: query lq, elements 16 s + 8 h .. + 7
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+    {
+        qreg[s] = *reinterpret_cast<f16x8 const*>(lds + qAt + lq * kRow + swz<2>(lq, 2 * s + h) * 16);
+    }
+
+    f32x16 out[2]; // O^T: elements 32 d + 8 (v / 4) + 4 h + v % 4 of query lq
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+    {
+        out[0][v] = out[1][v] = 0.f;
+    }
+    float negMax = 0.f;  // -maximum * c of the scores that the weights are relative to
+    float sum[2] = {0.f, 0.f}; // of this lane's keys, in two chains
+    int const tr = (lane & 15) >> 2; // transposing reads: 16 lanes take 4 rows of 16 elements
+    int const trBase = (4 * h + tr) * kRow + (lane & 1) * 8;
+    int const trChunk = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);
+
+    for (int kb = 0; kb < nb; ++kb)
+    {
+        wait_vmcnt<0>();
+        __syncthreads(); // everybody's rows of block kb have landed, and everybody has read block kb - 1 (and Q)
+        uint8_t const* const sK = lds + (kb & 1) * kStreamStage;
+        uint8_t const* const sV = sK + kStreamBlock;
+        auto request_next = [&] {
+            if (kb + 1 < nb)
+            {
+                request_block(kb + 1, (kb + 1) & 1);
+            }
+        };
+        if (!active)
+        {
+            request_next();
+            continue;
+        }
+        int const keys = nk - kb * 64; // of this block, 64 and more: all
+        // ---- S^T = K Q^T: keys 32 t + 8 (v / 4) + 4 h + v % 4 of query lq
+        f32x16 acc[2];
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+        {
+            acc[0][v] = acc[1][v] = 0.f;
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+        {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+            {
+                int const key = 32 * t + lq;
+                f16x8 const kreg = *reinterpret_cast<f16x8 const*>(sK + key * kRow + swz<2>(key, 2 * s + h) * 16);
+                acc[t] = attention_mfma_f16_32(kreg, qreg[s], acc[t]);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        request_next(); // while the matrix instructions run
+        __builtin_amdgcn_sched_barrier(0);
+        if (DEBUG && a.dbgAcc1 && qw + lq < nq)
+        {
+            for (int v = 0; v < 32; ++v)
+            {
+                int const key = kb * 64 + 32 * (v >> 4) + 8 * ((v & 15) >> 2) + 4 * h + (v & 3);
+                if (key < nk)
+                {
+                    a.dbgAcc1[(((int64_t) b * a.N + n) * a.S + qw + lq) * a.S + key] = __float_as_int(acc[v >> 4][v & 15]);
+                }
+            }
+        }
+        if (keys < 64) // uniform: absent keys weigh nothing
+        {
+#pragma unroll
+            for (int v = 0; v < 32; ++v)
+            {
+                int const key = 32 * (v >> 4) + 8 * ((v & 15) >> 2) + (v & 3);
+                acc[v >> 4][v & 15] = key < keys - 4 * h ? acc[v >> 4][v & 15] : -__builtin_inff();
+            }
+        }
+        float mxA = fmaxf(acc[0][0], acc[0][1]), mxB = fmaxf(acc[1][0], acc[1][1]);
+#pragma unroll
+        for (int v = 2; v < 16; v += 2)
+        {
+            mxA = fmaxf(fmaxf(mxA, acc[0][v]), acc[0][v + 1]);
+            mxB = fmaxf(fmaxf(mxB, acc[1][v]), acc[1][v + 1]);
+        }
+        float const mx = reduce_step<32>(fmaxf(mxA, mxB), [](float x, float y) { return fmaxf(x, y); });
+        // finite, so that a block whose scores are all -infinity weighs nothing
+        float const negNew = -fmaxf(mx, -3.402823466e+38f) * a.c;
+        if (kb == 0)
+        {
+            negMax = negNew;
+        }
+        else if (__ballot(negNew < negMax - 8.f) != 0)
+        {
+            // Weights may grow to 2^8 before the sums so far are brought to the new maximum.
+            float const to = fminf(negNew, negMax);
+            float const f = __builtin_amdgcn_exp2f(to - negMax);
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+            {
+                out[0][v] *= f;
+                out[1][v] *= f;
+            }
+            sum[0] *= f;
+            sum[1] *= f;
+            negMax = to;
+        }
+        // ---- p = 2^(s * c - max * c) rounded to binary16; O^T = V^T P^T
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+        {
+            if (t == 1 && keys <= 32)
+            {
+                break; // no key in this half
+            }
+#pragma unroll
+            for (int w = 0; w < 2; ++w)
+            {
+                f16x8 preg;
+#pragma unroll
+                for (int j = 0; j < 8; j += 2)
+                {
+                    float const p0 = __builtin_amdgcn_exp2f(fmaf(acc[t][8 * w + j], a.c, negMax));
+                    float const p1 = __builtin_amdgcn_exp2f(fmaf(acc[t][8 * w + j + 1], a.c, negMax));
+                    f16x2 const pp = __builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_pkrtz(p0, p1));
+                    f16x2 const ones = {(f16) 1.f, (f16) 1.f};
+                    sum[(j >> 1) & 1] = __builtin_amdgcn_fdot2(pp, ones, sum[(j >> 1) & 1], false);
+                    preg[j] = pp[0];
+                    preg[j + 1] = pp[1];
+                }
+#pragma unroll
+                for (int d = 0; d < 2; ++d)
+                {
+                    int const row = 32 * t + 16 * w + 4 * h + tr;
+                    uint8_t const* const v0 = sV + (32 * t + 16 * w) * kRow + trBase + swz<2>(row, 4 * d + trChunk) * 16;
+                    i16x4 const lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*) v0);
+                    i16x4 const hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*) (v0 + 8 * kRow));
+                    typedef short i16x8 __attribute__((ext_vector_type(8)));
+                    i16x8 const both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                    out[d] = attention_mfma_f16_32(__builtin_bit_cast(f16x8, both), preg, out[d]);
+                }
+            }
+        }
+    }
+
+    // The two lanes of a query hold four consecutive elements in turn; after two swaps per 32 elements each has 16 of them.
+    if (active)
+    {
+        float const rinv = 1.f / reduce_step<32>(sum[0] + sum[1], [](float x, float y) { return x + y; });
+        uint8_t* const dst = static_cast<uint8_t*>(a.out) + baseOut + (int64_t) (qw + lq) * a.tokStrideOut + (int64_t) n * kRow;
+#pragma unroll
+        for (int d = 0; d < 2; ++d)
+        {
+            u32x2 w[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+            {
+                f16x4 y;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                {
+                    y[j] = (f16) (out[d][4 * g + j] * rinv);
+                }
+                w[g] = __builtin_bit_cast(u32x2, y);
+            }
+            auto const a0 = __builtin_amdgcn_permlane32_swap(w[0][0], w[2][0], false, false);
+            auto const a1 = __builtin_amdgcn_permlane32_swap(w[0][1], w[2][1], false, false);
+            auto const b0 = __builtin_amdgcn_permlane32_swap(w[1][0], w[3][0], false, false);
+            auto const b1 = __builtin_amdgcn_permlane32_swap(w[1][1], w[3][1], false, false);
+            u32x4 const first = {a0[0], a1[0], a0[1], a1[1]};
+            u32x4 const second = {b0[0], b1[0], b0[1], b1[1]};
+            if (qw + lq < nq)
+            {
+                *reinterpret_cast<u32x4*>(dst + d * 64 + h * 32) = first;
+                *reinterpret_cast<u32x4*>(dst + d * 64 + h * 32 + 16) = second;
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------------------------
 
@@ -2122,11 +2119,30 @@ int run_i8(hipStream_t stream, FmhaArgs const& a, bool interleaved)
     return set_error(TRTAMD_STATUS_NOT_SUPPORTED, "fused MHA: sequence length %d exceeds 512", a.S);
 }
 
+// Which of the FP16 kernels a launch takes.
+enum class F16Kernel
+{
+    kGENERAL, // packed masks, and strides beyond the 32-bit offsets of the direct-to-LDS loads
+    kTURNS,
+    kSTREAM
+};
+
 template <bool DEBUG>
-int run_f16(hipStream_t stream, FmhaArgs const& a, bool turns)
+int run_f16(hipStream_t stream, FmhaArgs const& a, F16Kernel which)
 {
     int const kt = pick_kt(a.S);
-    if (turns)
+    if (which == F16Kernel::kSTREAM)
+    {
+        int const st = ensure_lds(reinterpret_cast<void const*>(fmha_f16_stream_kernel<DEBUG>), "fmha_f16_stream", kStreamLds);
+        if (st)
+        {
+            return st;
+        }
+        hipLaunchKernelGGL((fmha_f16_stream_kernel<DEBUG>), dim3((uint32_t) a.B * (uint32_t) a.N * (uint32_t) a.qSplit),
+            dim3(kWavesStream * kWaveSize), kStreamLds, stream, a, kt * 64);
+        return check_launch("fmha_f16_stream");
+    }
+    if (which == F16Kernel::kTURNS)
     {
 #define TRTAMD_F16T(KT)                                                                                                \
     case KT:                                                                                                           \
@@ -2143,10 +2159,6 @@ int run_f16(hipStream_t stream, FmhaArgs const& a, bool turns)
         default: break;
         }
 #undef TRTAMD_F16T
-    }
-    if (a.packedMask == nullptr && kt == 8 && !tuning(Tuning::kFmhaGeneric))
-    {
-        return launch_fmha(fmha_f16_prefix_kernel<8, DEBUG>, "fmha_f16_prefix", stream, a, Lds<2>::total(8), kWavesF16);
     }
 #define TRTAMD_F16(KT)                                                                                                 \
     case KT: return launch_fmha(fmha_f16_kernel<KT, DEBUG>, "fmha_f16", stream, a, Lds<2>::total(KT), kWavesF16)
@@ -2178,11 +2190,6 @@ int prepare_kt()
     st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_i8_kernel<KT, false, false>), "fmha_i8", Lds<1>::total(KT));
     st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_f16_turns_kernel<KT, false>), "fmha_f16_turns",
                       Lds<2>::matBytes(KT));
-    if constexpr (KT == 8)
-    {
-        st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_f16_prefix_kernel<KT, false>), "fmha_f16_prefix",
-                          Lds<2>::total(KT));
-    }
     st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_f16_kernel<KT, false>), "fmha_f16", Lds<2>::total(KT));
     return st;
 }
@@ -2257,23 +2264,27 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
     a.N = p->h;
     a.S = p->s;
     int const kt = pick_kt(p->s);
-    // FP16, prefix-valid keys: K and V take turns in LDS, save where there are whole units of more than 384 keys for all of
-    // the 256 CUs.  The scores of 512 keys leave room for two wavefronts per SIMD in either kernel, and staging K and V for
-    // 64 queries at a time then costs more than the wait it hides (12 heads x 32 sequences of 171-512 keys: 33.8 us
-    // against 27.6; 12 x 16: 20.2 us against 23.5).
-    bool const turns = dataType == 1 && (p->cu_seqlens || !p->packed_mask_ptr) && !tuning(Tuning::kFmhaGeneric)
-        && (kt < 8 || (int64_t) p->b * p->h <= 256)
-        && p->qkv_stride_in_bytes < (1LL << 29); // eight tokens within a 32-bit offset
+    // FP16, prefix-valid keys: 128 queries per workgroup where that makes three workgroups and more for each of the 256 CUs,
+    // 64 of them and the scores of all their keys in registers where it does not (12 heads: 16 x 256 keys, 384 workgroups of
+    // 128, 7.9 against 8.8 us; 32 x 256, 768 of them, 13.9 against 13.1; 16 heads, 8 x 384, 384: 9.6 against 10.2).
+    constexpr int kStreamTile = kWavesStream * kStreamQueries;
+    int const streamParts = ceil_div(kt * 64, kStreamTile);
+    F16Kernel f16 = F16Kernel::kGENERAL;
+    if (dataType == 1 && (p->cu_seqlens || !p->packed_mask_ptr) && !tuning(Tuning::kFmhaGeneric)
+        && p->qkv_stride_in_bytes < (1LL << 29)) // eight tokens within a 32-bit offset
+    {
+        f16 = (int64_t) p->b * p->h * streamParts >= 768 ? F16Kernel::kSTREAM : F16Kernel::kTURNS;
+    }
     {
         // Workgroups per (sequence, head).  Every extra workgroup stages K and V again, so a unit is only shared
         // while the launch would otherwise leave the chip partly idle or badly balanced.  INT8 (three workgroups per
         // CU, 768 places): below 896 units two workgroups per unit, which also evens out a single round of units of
         // very different lengths (768 units of 128-384 keys: 24.9 against 27.8 us; 512 units: 18.7 against 23.1 us;
         // 896 units: 29.1 against 28.1 us), and more of them only to reach one round (256 units: three, 12.6 us
-        // against 13.1 with two and 17.4 with one; at most four).  FP16 (its K and V take most of a CU's LDS, one
-        // workgroup per CU, and staging them is 40 % of a workgroup's time): only below 160 units (192 units of 192-384
-        // keys: 15.3 us alone, 17.5 us shared by two; 144 units: 14.9 against 12.9 us).  Where K and V take turns, 64
-        // queries each, one for each block of 64 keys that the kernel has room for: a sequence longer than s that still fits
+        // against 13.1 with two and 17.4 with one; at most four).  FP16 with a packed mask (its K and V take most of a
+        // CU's LDS, one workgroup per CU, and staging them is 40 % of a workgroup's time): only below 160 units (192 units
+        // of 192-384 keys: 15.3 us alone, 17.5 us shared by two; 144 units: 14.9 against 12.9 us).  The other FP16 kernels
+        // take 64 or 128 queries each, of as many as the kernel has room for: a sequence longer than s that still fits
         // is served whole, as by the kernels that walk the queries.
         int const waves = dataType == 2 ? kWavesI8 : kWavesF16;
         int const maxSplit = std::max(1, ceil_div(ceil_div(p->s, kQPerWave), waves));
@@ -2283,9 +2294,9 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         {
             split = heads >= 896 ? 1 : (int) std::max<int64_t>(2, std::min<int64_t>(4, ceil_div<int64_t>(768, heads)));
         }
-        else if (turns)
+        else if (f16 != F16Kernel::kGENERAL)
         {
-            split = kt;
+            split = f16 == F16Kernel::kTURNS ? kt : streamParts;
         }
         else
         {
@@ -2294,10 +2305,10 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
                 split *= 2;
             }
         }
-        a.qSplit = turns ? split : std::min(split, maxSplit);
+        a.qSplit = f16 != F16Kernel::kGENERAL ? split : std::min(split, maxSplit);
         // tuning override: TRTAMD_FMHA_QSPLIT=<n> forces the number of workgroups per head
         int const forced = tuning(Tuning::kFmhaQsplit);
-        if (forced > 0 && !turns)
+        if (forced > 0 && f16 == F16Kernel::kGENERAL)
         {
             a.qSplit = std::min(forced, maxSplit);
         }
@@ -2309,10 +2320,21 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         // first, so that the short ones fill the tail).  When every workgroup of the launch is resident at once it
         // changes nothing, and the workgroups skip the ranking (a trip to LDS and two barriers before their loads).
         // Workgroups of 64 queries are short enough to even out by themselves (12 heads x 128 sequences of 67-200 keys:
-        // 29.1 us in natural order, 36.8 ranked).
-        int64_t const lds = dataType == 2 ? Lds<1>::total(kt) : Lds<2>::total(kt);
-        int64_t const perCu = std::max<int64_t>(1, std::min<int64_t>(dataType == 2 ? 3 : 2, (160 * 1024) / std::max<int64_t>(lds, 1)));
-        a.ranked = !turns && (int64_t) a.B * a.N * a.qSplit > perCu * 256 ? 1 : 0;
+        // 29.1 us in natural order, 36.8 ranked); those of 128 queries are all resident at once up to four per CU, and the
+        // order then spreads the long ones over the CUs (12 heads, ranked / not: 16 x 512 18.0 / 21.2 us, 32 x 384 19.0 / 20.4,
+        // 64 x 384 32.8 / 33.6), until there are several rounds of them (16 heads, 128 x 384: 85.6 / 82.4).
+        int64_t const workgroups = (int64_t) a.B * a.N * a.qSplit;
+        if (f16 == F16Kernel::kSTREAM)
+        {
+            a.ranked = workgroups < 3072 ? 1 : 0;
+        }
+        else
+        {
+            int64_t const lds = dataType == 2 ? Lds<1>::total(kt) : Lds<2>::total(kt);
+            int64_t const perCu
+                = std::max<int64_t>(1, std::min<int64_t>(dataType == 2 ? 3 : 2, (160 * 1024) / std::max<int64_t>(lds, 1)));
+            a.ranked = f16 == F16Kernel::kGENERAL && workgroups > perCu * 256 ? 1 : 0;
+        }
         // tuning override: TRTAMD_FMHA_RANKED=0 / 1 forces natural order / the longest-first order
         int const forcedRank = tuning(Tuning::kFmhaRanked);
         if (forcedRank >= 0)
@@ -2407,7 +2429,7 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
     a.c = s1 * kLog2e;
     a.scaleSoftmax = 1.f;
     a.scaleBmm2 = 1.f;
-    return dbgAcc1 ? run_f16<true>(stream, a, turns) : run_f16<false>(stream, a, turns);
+    return dbgAcc1 ? run_f16<true>(stream, a, f16) : run_f16<false>(stream, a, f16);
 }
 
 } // namespace
@@ -2436,6 +2458,7 @@ extern "C" int trtamd_fused_mha_prepare(void)
     st = st ? st : prepare_kt<4>();
     st = st ? st : prepare_kt<6>();
     st = st ? st : prepare_kt<8>();
+    st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_f16_stream_kernel<false>), "fmha_f16_stream", kStreamLds);
     return st;
 }
 

@@ -280,3 +280,75 @@ def test_longest_first_order_reaches_every_sequence(B):
         outs.append(host(out))
     assert np.array_equal(outs[0], outs[1])
     assert all((outs[0][:, cu[b]:cu[b + 1]] != 55).any() for b in range(B) if lens[b])
+
+
+# launches that fill the chip (768 workgroups of 128 queries): lengths on either side of a wavefront's 32 queries, a
+# workgroup's 128, half a block and a block of keys; scores whose maximum grows from block to block and scores of one size
+@pytest.mark.parametrize("S,B,N", [(64, 192, 4), (384, 64, 4), (512, 48, 4)])
+@pytest.mark.parametrize("growing", [False, True])
+@pytest.mark.parametrize("ranked", [0, 1])
+def test_fp16_attention_of_full_launches(S, B, N, growing, ranked):
+    api = capi.api()
+    r = rng(1600 + S)
+    edges = [n for n in (1, 31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129, 161, 255, 257, 383, 384, 449, 511, 512) if n <= S]
+    lens = np.array([edges[i % len(edges)] for i in range(B)])
+    lens[3] = 0
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T = int(cu[-1])
+    qkv = r.standard_normal((T, N, 3, 64))
+    if growing:
+        for b in range(B):
+            # scores up to about +-8 x 90 x 0.125: a block's largest is e^10 and more above the one before
+            qkv[cu[b]:cu[b + 1], :, 1] *= (1 + np.arange(lens[b]) * 0.25)[:, None, None]
+    qkv = qkv.astype(np.float16)
+    d_qkv, d_cu = dev(qkv), dev(cu)
+    out = dev_empty((T + 64, N * 64), np.float16, fill=-7)
+    p = capi.FmhaParams()
+    p.qkv_ptr, p.o_ptr, p.cu_seqlens = ptr(d_qkv), ptr(out), ptr(d_cu)
+    p.qkv_stride_in_bytes, p.o_stride_in_bytes = 2 * 3 * N * 64, 2 * N * 64
+    p.b, p.h, p.s, p.d = B, N, S, 64
+    p.scale_bmm1, p.scale_softmax, p.scale_bmm2 = half2_bits(0.125), half2_bits(1.0), half2_bits(1.0)
+    with tuning("TRTAMD_FMHA_RANKED", ranked):
+        api.check(api.fused_mha_run(stream(), 1, C.byref(p)))
+        sync()
+    got = host(out)
+    assert (got[T:] == -7).all()
+    for b in range(min(B, 2 * len(edges))):
+        lo, hi = int(cu[b]), int(cu[b + 1])
+        if lo == hi:
+            continue
+        n = b % N
+        want = attention_f64(qkv[lo:hi, n, 0], qkv[lo:hi, n, 1], qkv[lo:hi, n, 2], 0.125)
+        assert_fp_close(got[lo:hi, n * 64:(n + 1) * 64], want, what=f"sequence {b} of {hi - lo}, head {n}")
+
+
+def test_fp16_attention_of_full_launches_keeps_infinite_scores_apart():
+    """Keys with a score of -infinity weigh nothing, also where they are a whole block or the first one; an infinite V
+    behind the last key of a sequence does not reach it."""
+    api = capi.api()
+    r = rng(1700)
+    B, N, S = 200, 4, 128
+    lens = np.full(B, 100)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T = int(cu[-1])
+    qkv = r.standard_normal((T, N, 3, 64)).astype(np.float16)
+    qkv[:, :, 0, 0] = np.abs(qkv[:, :, 0, 0]) + np.float16(0.5)
+    qkv[cu[1]:cu[1] + 64, :, 1, 0] = -np.inf        # sequence 1: the first block
+    qkv[cu[2] + 64:cu[2] + 100, :, 1, 0] = -np.inf  # sequence 2: the last one
+    qkv[cu[4]:cu[5], :, 2, 5] = np.inf              # sequence 4: V, next to sequences 3 and 5
+    d_qkv, d_cu = dev(qkv), dev(cu)
+    out = dev_empty((T, N * 64), np.float16, fill=0)
+    p = capi.FmhaParams()
+    p.qkv_ptr, p.o_ptr, p.cu_seqlens = ptr(d_qkv), ptr(out), ptr(d_cu)
+    p.qkv_stride_in_bytes, p.o_stride_in_bytes = 2 * 3 * N * 64, 2 * N * 64
+    p.b, p.h, p.s, p.d = B, N, S, 64
+    p.scale_bmm1, p.scale_softmax, p.scale_bmm2 = half2_bits(0.125), half2_bits(1.0), half2_bits(1.0)
+    api.check(api.fused_mha_run(stream(), 1, C.byref(p)))
+    sync()
+    got = host(out)
+    for b, keys in ((0, slice(0, 100)), (1, slice(64, 100)), (2, slice(0, 64)), (3, slice(0, 100)), (5, slice(0, 100))):
+        lo = int(cu[b])
+        k, v = qkv[lo:lo + 100][keys], qkv[lo:lo + 100][keys]
+        want = attention_f64(qkv[lo:lo + 100, 1, 0], k[:, 1, 1], v[:, 1, 2], 0.125)
+        assert_fp_close(got[lo:lo + 100, 64:128], want, what=f"sequence {b}")
+    assert np.isinf(got[cu[4]:cu[5], 64 + 5]).all()
