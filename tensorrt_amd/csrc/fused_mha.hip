@@ -128,6 +128,7 @@ struct FmhaArgs
     int32_t qSplit;              // workgroups per (sequence, head)
     int32_t total;               // interleaved: total token count
     int32_t warpsM, warpsN;      // geometry of the packed mask
+    uint32_t spanInverse;        // 2^20 / (16 warpsN) rounded up: key * this >> 20 is key / (16 warpsN) for keys below 512
     float c;                     // scale_bmm1 * log2(e)
     float scaleSoftmax;
     float scaleBmm2;
@@ -833,6 +834,59 @@ __device__ inline SeqInfo pick_sequence_info(FmhaArgs const& a, int rank, int ca
 // number of 64-key blocks so that a query tile is one straight-line instruction stream.
 // ------------------------------------------------------------------------------------------
 
+// The keys that a packed mask leaves a sequence: 64 of them in each m, their number up to the last one in sq.nk; true where
+// keys before that one are masked.  By every wavefront for itself, one key per lane and block, in one trip to memory: no
+// LDS, no barrier (FP16, 16 x 12 x 128: 6.2 us with the mask built in LDS by the workgroup, 5.7 us).  Masks that are a
+// prefix, which is what the embedding layer packs, then cost no more than lengths do.  us per launch with the general
+// kernel / with this: FP16 16 x 12 x 128 6.3 / 5.7, 64 x 12 x 128 14.6 / 12.3, 32 x 12 x 384 40.6 / 25.0; INT8 64 x 12 x 128
+// 12.3 / 11.5, 8 x 12 x 384 14.8 / 12.2, 64 x 16 x 384 68.6 / 50.2.
+template <int KT>
+__device__ inline bool packed_mask_keys(FmhaArgs const& a, int b, SeqInfo& sq, uint64_t (&m)[KT])
+{
+    int const lane = threadIdx.x & (kWaveSize - 1);
+    uint32_t const* const pm = a.packedMask + (int64_t) b * a.maskStrideWords;
+    uint32_t word[KT], bit[KT];
+#pragma unroll
+    for (int i = 0; i < KT; ++i)
+    {
+        // the layout that build_key_mask reads
+        int const key = 64 * i + lane, ni = (int) (((uint32_t) key * a.spanInverse) >> 20), r = key - ni * 16 * a.warpsN;
+        int const r2 = r & 15;
+        bit[i] = (uint32_t) (8 * ni + (r2 & 1) + ((r2 & 8) ? 4 : 0));
+        word[i] = key < sq.nk ? pm[(r >> 4) * a.warpsM * 32 + ((r2 & 7) >> 1)] : 0u;
+    }
+    int used = 0;
+#pragma unroll
+    for (int i = 0; i < KT; ++i)
+    {
+        m[i] = __ballot(((word[i] >> (bit[i] & 31u)) & 1u) != 0);
+        used = m[i] ? 64 * i + 64 - __builtin_clzll(m[i]) : used;
+    }
+    sq.nk = used;
+    bool holes = false;
+#pragma unroll
+    for (int i = 0; i < KT; ++i)
+    {
+        int const here = used - 64 * i;
+        uint64_t const all = here >= 64 ? ~0ull : here > 0 ? (1ull << here) - 1ull : 0ull;
+        holes = holes || m[i] != all;
+    }
+    return holes;
+}
+
+// Rows q0 .. of a sequence that has no key at all are zeros: `queries` of them by the whole workgroup.
+template <int ESIZE>
+__device__ inline void store_zero_rows(FmhaArgs const& a, SeqInfo const& sq, int n, int q0, int queries)
+{
+    int const end = min(q0 + queries, sq.nq) - q0;
+    for (int i = threadIdx.x; i < end * 4 * ESIZE; i += blockDim.x)
+    {
+        *reinterpret_cast<u32x4*>(static_cast<uint8_t*>(a.out) + sq.seqBaseOut + (int64_t) (q0 + i / (4 * ESIZE)) * a.tokStrideOut
+            + (int64_t) n * Lds<ESIZE>::kRow + (i % (4 * ESIZE)) * 16)
+            = u32x4{0, 0, 0, 0};
+    }
+}
+
 // Stage K and V of one (sequence, head): rows < nk from memory, the rest of the last block zero.
 template <int KT, bool INTERLEAVED>
 __device__ inline void stage_kv_prefix_i8(FmhaArgs const& a, int64_t seqBase, int64_t firstTok, int n, int nk, int nkb,
@@ -890,7 +944,7 @@ __device__ inline void stage_kv_prefix_i8(FmhaArgs const& a, int64_t seqBase, in
 // sequence).  sK / sV: the head's keys and values in LDS as stage_kv_prefix_i8 lays them out.
 template <int NKB, bool INTERLEAVED, bool DEBUG>
 __device__ __forceinline__ void tile_i8(FmhaArgs const& a, SeqInfo const& sq, int const b, int const n, int const qt,
-    uint8_t const* sK, uint8_t const* sV, i32x4 const qreg)
+    uint8_t const* sK, uint8_t const* sV, i32x4 const qreg, uint64_t const* const masks, bool const holes)
 {
     constexpr int kRow = Lds<1>::kRow;
     constexpr int NT = NKB * 4;
@@ -924,6 +978,19 @@ __device__ __forceinline__ void tile_i8(FmhaArgs const& a, SeqInfo const& sq, in
             }
         }
         acc[t] = attention_mfma_i8(kreg, qreg, seed);
+    }
+    if (holes)
+    {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+        {
+            uint32_t const bits = (uint32_t) (masks[t >> 2] >> (32 * ((t >> 1) & 1))) >> (16 * (t & 1) + 4 * g);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            {
+                acc[t][j] = (bits >> j) & 1u ? acc[t][j] : kNegInfBits;
+            }
+        }
     }
     __builtin_amdgcn_sched_barrier(0);
 
@@ -1105,7 +1172,8 @@ __device__ __forceinline__ i32x4 load_q_i8(FmhaArgs const& a, SeqInfo const& sq,
 // All query tiles of this wavefront for a sequence of exactly NKB key blocks.
 template <int NKB, bool INTERLEAVED, bool DEBUG>
 __device__ __forceinline__ void attend_i8(FmhaArgs const& a, SeqInfo const& sq, int const b, int const n,
-    int const qtBegin, int const qtEnd, uint8_t const* sK, uint8_t const* sV, i32x4 const qFirst)
+    int const qtBegin, int const qtEnd, uint8_t const* sK, uint8_t const* sV, i32x4 const qFirst, uint64_t const* const masks,
+    bool const holes)
 {
     int const wave = threadIdx.x >> 6;
     constexpr int qtStep = kWavesI8;
@@ -1114,11 +1182,12 @@ __device__ __forceinline__ void attend_i8(FmhaArgs const& a, SeqInfo const& sq, 
     {
         i32x4 const qreg = qnext;
         qnext = load_q_i8<INTERLEAVED>(a, sq, n, qt + qtStep);
-        tile_i8<NKB, INTERLEAVED, DEBUG>(a, sq, b, n, qt, sK, sV, qreg);
+        tile_i8<NKB, INTERLEAVED, DEBUG>(a, sq, b, n, qt, sK, sV, qreg, masks, holes);
     }
 }
 
-template <int KT, bool INTERLEAVED, bool DEBUG>
+// MASKED: the keys come from a packed mask (a kernel of its own: the other one keeps its registers).
+template <int KT, bool INTERLEAVED, bool DEBUG, bool MASKED = false>
 __global__ __launch_bounds__(kWavesI8* kWaveSize) __attribute__((amdgpu_waves_per_eu(KT <= 6 ? 3 : 2))) void fmha_i8_prefix_kernel(FmhaArgs const a)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -1136,7 +1205,7 @@ __global__ __launch_bounds__(kWavesI8* kWaveSize) __attribute__((amdgpu_waves_pe
     int const part = up.part;
     int const n = up.unit % a.N;
     int b;
-    SeqInfo const sq = pick_sequence_info<kWavesI8 * kWaveSize>(a, up.unit / a.N, KT * 64, sPick, b);
+    SeqInfo sq = pick_sequence_info<kWavesI8 * kWaveSize>(a, up.unit / a.N, KT * 64, sPick, b);
     // contiguous tile ranges, each a multiple of one round of the workgroup's wavefronts
     int const nqt = (sq.nq + kQPerWave - 1) / kQPerWave;
     int const per = kWavesI8 * ((nqt + kWavesI8 * a.qSplit - 1) / (kWavesI8 * a.qSplit));
@@ -1145,6 +1214,17 @@ __global__ __launch_bounds__(kWavesI8* kWaveSize) __attribute__((amdgpu_waves_pe
     if (qtBegin >= qtEnd)
     {
         return; // no query tile for this workgroup (also: empty sequence)
+    }
+    uint64_t masks[KT] = {};
+    bool holes = false;
+    if constexpr (MASKED)
+    {
+        holes = packed_mask_keys<KT>(a, b, sq, masks);
+        if (sq.nk == 0)
+        {
+            store_zero_rows<1>(a, sq, n, qtBegin * kQPerWave, (qtEnd - qtBegin) * kQPerWave);
+            return;
+        }
     }
     int const nkb = (sq.nk + 63) >> 6;
     // the first query tile of this wavefront travels with K and V
@@ -1161,27 +1241,27 @@ __global__ __launch_bounds__(kWavesI8* kWaveSize) __attribute__((amdgpu_waves_pe
     __syncthreads();
     switch (nkb)
     {
-    case 1: attend_i8<1, INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst); break;
+    case 1: attend_i8<1, INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst, masks, holes); break;
     case 2:
-        if (KT >= 2) attend_i8<(KT >= 2 ? 2 : 1), INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst);
+        if (KT >= 2) attend_i8<(KT >= 2 ? 2 : 1), INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst, masks, holes);
         break;
     case 3:
-        if (KT >= 3) attend_i8<(KT >= 3 ? 3 : 1), INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst);
+        if (KT >= 3) attend_i8<(KT >= 3 ? 3 : 1), INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst, masks, holes);
         break;
     case 4:
-        if (KT >= 4) attend_i8<(KT >= 4 ? 4 : 1), INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst);
+        if (KT >= 4) attend_i8<(KT >= 4 ? 4 : 1), INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst, masks, holes);
         break;
     case 5:
-        if (KT >= 5) attend_i8<(KT >= 5 ? 5 : 1), INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst);
+        if (KT >= 5) attend_i8<(KT >= 5 ? 5 : 1), INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst, masks, holes);
         break;
     case 6:
-        if (KT >= 6) attend_i8<(KT >= 6 ? 6 : 1), INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst);
+        if (KT >= 6) attend_i8<(KT >= 6 ? 6 : 1), INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst, masks, holes);
         break;
     case 7:
-        if (KT >= 7) attend_i8<(KT >= 7 ? 7 : 1), INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst);
+        if (KT >= 7) attend_i8<(KT >= 7 ? 7 : 1), INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst, masks, holes);
         break;
     case 8:
-        if (KT >= 8) attend_i8<(KT >= 8 ? 8 : 1), INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst);
+        if (KT >= 8) attend_i8<(KT >= 8 ? 8 : 1), INTERLEAVED, DEBUG>(a, sq, b, n, qtBegin, qtEnd, sK, sV, qFirst, masks, holes);
         break;
     default: break;
     }
@@ -1442,7 +1522,8 @@ __device__ __forceinline__ void for_each_block(F&& f)
 
 template <int NKB, bool DEBUG>
 __device__ __forceinline__ void attend_f16_turns(
-    FmhaArgs const& a, SeqInfo const& sq, int const b, int const n, int const q0, uint8_t* const lds)
+    FmhaArgs const& a, SeqInfo const& sq, int const b, int const n, int const q0, uint8_t* const lds,
+    uint64_t const* const masks, bool const holes)
 {
     constexpr int kRow = Lds<2>::kRow;
     constexpr int NT = NKB * 4;
@@ -1539,6 +1620,19 @@ __device__ __forceinline__ void attend_f16_turns(
                 }
                 acc[t] = sd;
             }
+            if (holes)
+            {
+#pragma unroll
+                for (int t = kb * 4; t < kb * 4 + 4; ++t)
+                {
+                    uint32_t const bits = (uint32_t) (masks[kb] >> (32 * ((t >> 1) & 1))) >> (16 * (t & 1) + 4 * g);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                    {
+                        acc[t][j] = (bits >> j) & 1u ? acc[t][j] : -__builtin_inff();
+                    }
+                }
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -1578,7 +1672,7 @@ __device__ __forceinline__ void attend_f16_turns(
         float mx = fmaxf(mxA, mxB);
         mx = reduce_step<16>(mx, [](float x, float y) { return fmaxf(x, y); });
         mx = reduce_step<32>(mx, [](float x, float y) { return fmaxf(x, y); });
-        negK0 = -mx * a.c; // nk >= 1: the maximum is finite
+        negK0 = a.packedMask && mx == -__builtin_inff() ? 0.f : -mx * a.c; // a mask's row without a score is zeros
     }
 
     // ---- p = 2^((s - max) * c) rounded to binary16; O^T = V^T P^T; row sum by a tile of ones
@@ -1651,7 +1745,7 @@ __device__ __forceinline__ void attend_f16_turns(
     // whole quarter dt = g, which goes out as two 16-byte stores.
     if (active)
     {
-        float const rinv = 1.f / sacc[0];
+        float const rinv = a.packedMask && !(sacc[0] > 0.f) ? 0.f : 1.f / sacc[0];
         uint32_t lo[4], hi[4];
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt)
@@ -1710,11 +1804,22 @@ __global__ __launch_bounds__(kWavesF16T* kWaveSize)
     {
         return;
     }
+    uint64_t masks[KT] = {};
+    bool holes = false;
+    if (a.packedMask)
+    {
+        holes = packed_mask_keys<KT>(a, b, sq, masks);
+        if (sq.nk == 0)
+        {
+            store_zero_rows<2>(a, sq, n, q0, kQueriesF16);
+            return;
+        }
+    }
     switch ((sq.nk + 63) >> 6)
     {
 #define TRTAMD_BLOCKS(NKB)                                                                                             \
     case NKB:                                                                                                          \
-        if constexpr (KT >= NKB) attend_f16_turns<NKB, DEBUG>(a, sq, b, n, q0, smem);                                        \
+        if constexpr (KT >= NKB) attend_f16_turns<NKB, DEBUG>(a, sq, b, n, q0, smem, masks, holes);                                        \
         break
         TRTAMD_BLOCKS(1);
         TRTAMD_BLOCKS(2);
@@ -1754,13 +1859,14 @@ __global__ __launch_bounds__(kWavesStream* kWaveSize) __attribute__((amdgpu_wave
     constexpr int kLoads = 2 * 8 / kWavesStream; // direct loads per wavefront and block: 8 rows each, of K and of V
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ PickLds sPick;
+    __shared__ uint64_t sMask[8];
     UnitPart const up = unit_of_workgroup(blockIdx.x, gridDim.x, a.qSplit);
     int const n = __builtin_amdgcn_readfirstlane(up.unit % a.N);
     int b;
     SeqInfo sq = pick_sequence_info<kWavesStream * kWaveSize>(a, up.unit / a.N, capacity, sPick, b);
     // the same in every lane, which the compiler cannot see where they come from LDS: scalars keep the addresses scalar
     b = __builtin_amdgcn_readfirstlane(b);
-    int const nq = __builtin_amdgcn_readfirstlane(sq.nq), nk = __builtin_amdgcn_readfirstlane(sq.nk);
+    int const nq = __builtin_amdgcn_readfirstlane(sq.nq);
     int const firstTok = __builtin_amdgcn_readfirstlane((int) sq.firstTok);
     int64_t const baseIn = a.cuSeqlens ? firstTok * a.tokStrideIn : b * a.seqStrideIn;
     int64_t const baseOut = a.cuSeqlens ? firstTok * a.tokStrideOut : b * a.seqStrideOut;
@@ -1771,6 +1877,26 @@ __global__ __launch_bounds__(kWavesStream* kWaveSize) __attribute__((amdgpu_wave
     {
         return;
     }
+    bool holes = false;
+    if (a.packedMask)
+    {
+        uint64_t masks[8];
+        holes = packed_mask_keys<8>(a, b, sq, masks);
+        if (threadIdx.x == 0) // read behind the barrier before block 0
+        {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+            {
+                sMask[i] = masks[i];
+            }
+        }
+        if (sq.nk == 0)
+        {
+            store_zero_rows<2>(a, sq, n, q0, kWavesStream * kStreamQueries);
+            return;
+        }
+    }
+    int const nk = __builtin_amdgcn_readfirstlane(sq.nk);
     int const qw = q0 + wave * kStreamQueries; // this wavefront's first query
     bool const active = qw < nq;               // if not, it only brings in its rows
     int const lq = lane & 31, h = lane >> 5;
@@ -1916,6 +2042,19 @@ __global__ __launch_bounds__(kWavesStream* kWaveSize) __attribute__((amdgpu_wave
                 acc[v >> 4][v & 15] = key < keys - 4 * h ? acc[v >> 4][v & 15] : -__builtin_inff();
             }
         }
+        if (holes)
+        {
+#pragma unroll
+            for (int v = 0; v < 32; v += 4)
+            {
+                uint32_t const bits = (uint32_t) (sMask[kb] >> (2 * v)) >> (4 * h);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                {
+                    acc[v >> 4][(v & 15) + j] = (bits >> j) & 1u ? acc[v >> 4][(v & 15) + j] : -__builtin_inff();
+                }
+            }
+        }
         float mxA = fmaxf(acc[0][0], acc[0][1]), mxB = fmaxf(acc[1][0], acc[1][1]);
 #pragma unroll
         for (int v = 2; v < 16; v += 2)
@@ -1986,7 +2125,8 @@ __global__ __launch_bounds__(kWavesStream* kWaveSize) __attribute__((amdgpu_wave
     // The two lanes of a query hold four consecutive elements in turn; after two swaps per 32 elements each has 16 of them.
     if (active)
     {
-        float const rinv = 1.f / reduce_step<32>(sum[0] + sum[1], [](float x, float y) { return x + y; });
+        float const total = reduce_step<32>(sum[0] + sum[1], [](float x, float y) { return x + y; });
+        float const rinv = a.packedMask && !(total > 0.f) ? 0.f : 1.f / total; // a mask's row without a score is zeros
         uint8_t* const dst = static_cast<uint8_t*>(a.out) + baseOut + (int64_t) (qw + lq) * a.tokStrideOut + (int64_t) n * kRow;
 #pragma unroll
         for (int d = 0; d < 2; ++d)
@@ -2076,14 +2216,15 @@ template <bool DEBUG>
 int run_i8(hipStream_t stream, FmhaArgs const& a, bool interleaved)
 {
     int const kt = pick_kt(a.S);
-    // keys are a valid prefix (cu_seqlens, or no mask) and probabilities cannot leave the INT8 range:
-    // the kernel specialised on the number of key blocks serves the launch
+    // probabilities cannot leave the INT8 range: the kernel specialised on the number of key blocks serves the launch
     int const noFast = tuning(Tuning::kFmhaGeneric);
-    if (a.packedMask == nullptr && !a.clampP && !noFast)
+    if (!a.clampP && !noFast)
     {
 #define TRTAMD_I8P(KT)                                                                                                 \
     case KT:                                                                                                           \
-        return interleaved ? launch_fmha(fmha_i8_prefix_kernel<KT, true, DEBUG>, "fmha_i8_prefix_interleaved", stream, \
+        return a.packedMask ? launch_fmha(fmha_i8_prefix_kernel<KT, false, DEBUG, true>, "fmha_i8_masked", stream, a,  \
+                   Lds<1>::total(KT), kWavesI8)                                                                        \
+            : interleaved ? launch_fmha(fmha_i8_prefix_kernel<KT, true, DEBUG>, "fmha_i8_prefix_interleaved", stream, \
                    a, Lds<1>::total(KT), kWavesI8)                                                                     \
                            : launch_fmha(fmha_i8_prefix_kernel<KT, false, DEBUG>, "fmha_i8_prefix", stream, a,         \
                                Lds<1>::total(KT), kWavesI8)
@@ -2185,6 +2326,8 @@ int prepare_kt()
 
     st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_i8_prefix_kernel<KT, false, false>), "fmha_i8_prefix",
                       Lds<1>::total(KT));
+    st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_i8_prefix_kernel<KT, false, false, true>), "fmha_i8_masked",
+                      Lds<1>::total(KT));
     st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_i8_kernel<KT, true, false>), "fmha_i8_interleaved",
                       Lds<1>::total(KT));
     st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_i8_kernel<KT, false, false>), "fmha_i8", Lds<1>::total(KT));
@@ -2270,7 +2413,7 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
     constexpr int kStreamTile = kWavesStream * kStreamQueries;
     int const streamParts = ceil_div(kt * 64, kStreamTile);
     F16Kernel f16 = F16Kernel::kGENERAL;
-    if (dataType == 1 && (p->cu_seqlens || !p->packed_mask_ptr) && !tuning(Tuning::kFmhaGeneric)
+    if (dataType == 1 && !tuning(Tuning::kFmhaGeneric)
         && p->qkv_stride_in_bytes < (1LL << 29)) // eight tokens within a 32-bit offset
     {
         f16 = (int64_t) p->b * p->h * streamParts >= 768 ? F16Kernel::kSTREAM : F16Kernel::kTURNS;
@@ -2398,6 +2541,7 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         a.packedMask = static_cast<uint32_t const*>(p->packed_mask_ptr);
         a.warpsM = wm;
         a.warpsN = wn;
+        a.spanInverse = ((1u << 20) + 16u * (uint32_t) wn - 1u) / (16u * (uint32_t) wn);
         a.maskStrideWords = p->packed_mask_stride_in_bytes / 4;
         int const xn = ceil_div(p->s, 16 * wn);
         if (xn > 4 || a.maskStrideWords < (int64_t) wm * wn * 32)

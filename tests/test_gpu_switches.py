@@ -352,3 +352,59 @@ def test_fp16_attention_of_full_launches_keeps_infinite_scores_apart():
         want = attention_f64(qkv[lo:lo + 100, 1, 0], k[:, 1, 1], v[:, 1, 2], 0.125)
         assert_fp_close(got[lo:lo + 100, 64:128], want, what=f"sequence {b}")
     assert np.isinf(got[cu[4]:cu[5], 64 + 5]).all()
+
+
+# packed masks: launches of either FP16 kernel (768 workgroups of 128 queries and fewer) and INT8
+@pytest.mark.parametrize("dtype", [1, 2])
+@pytest.mark.parametrize("S,B,N", [(64, 9, 2), (96, 9, 2), (128, 9, 2), (384, 9, 2), (128, 200, 4), (384, 70, 4)])
+def test_attention_with_packed_masks(dtype, S, B, N):
+    """Masks that are a prefix of every kind of length, that have holes in the first, a middle and the last block, that
+    leave one key or none: the general kernel's results to the bar, zeros where no key is left."""
+    api = capi.api()
+    r = rng(1800 + S + B)
+    mask = np.zeros((S, B), np.int32)
+    for b in range(B):
+        n = [S, 1, 0, S - 1, min(64, S), min(65, S - 1), S // 2 + 3, S, S][b % 9]
+        mask[:n, b] = 1
+        if b % 9 >= 7:
+            mask[:, b] = r.integers(0, 2, S)
+    mask[:, 8] = 0
+    mask[S - 1, 8] = 1
+    packed, _ = oracle.convert_mask(mask, *((1, 8) if S == 384 else (2, 2)))
+    x = r.standard_normal((S, B, N, 3, 64))
+    if dtype == 2:
+        qkv, s_q = quantize_amax(x.astype(np.float32))
+        bits = lambda v: int(np.float32(v).view(np.uint32))
+        scales = bits(s_q * s_q * 0.125), bits(127.0), bits(s_q / 127.0 / 0.02)
+    else:
+        qkv, scales = x.astype(np.float16), (half2_bits(0.125), half2_bits(1.0), half2_bits(1.0))
+    size = qkv.itemsize
+    d_qkv, d_mask = dev(qkv), dev(packed)
+
+    def run():
+        out = dev_empty((S, B, N * 64), qkv.dtype.type, fill=55)
+        p = capi.FmhaParams()
+        p.qkv_ptr, p.o_ptr, p.packed_mask_ptr = ptr(d_qkv), ptr(out), ptr(d_mask)
+        p.qkv_stride_in_bytes, p.o_stride_in_bytes = size * 3 * B * N * 64, size * B * N * 64
+        p.packed_mask_stride_in_bytes = packed.shape[1] * 4
+        p.b, p.h, p.s, p.d = B, N, S, 64
+        p.scale_bmm1, p.scale_softmax, p.scale_bmm2 = scales
+        api.check(api.fused_mha_run(stream(), dtype, C.byref(p)))
+        sync()
+        return host(out)
+
+    got = run()
+    with tuning("TRTAMD_FMHA_GENERIC", 1):
+        want = run()
+    assert (got[:, 2] == 0).all()
+    if dtype == 2:
+        # the two kernels add a row's weights up in different orders: a unit in the last place of the sum turns one of
+        # 384 quantised weights in 10^5 over, and the output by one where it was next to a tie
+        assert_int8_close(got, want, what="general kernel", max_frac_off=1e-3)
+    else:
+        assert_fp_close(got, want, atol=1e-3, rtol=2e-3, what="general kernel")
+        for b in (0, 1, 3, 5, 7, 8, B - 1):
+            keep = mask[:, b] == 1
+            if keep.any():
+                ref = attention_f64(qkv[:, b, 1, 0], qkv[keep, b, 1, 1], qkv[keep, b, 1, 2], 0.125)
+                assert_fp_close(got[:, b, 64:128], ref, what=f"sequence {b}")
