@@ -1098,9 +1098,30 @@ __device__ __forceinline__ void linear_piece64(
     }
 }
 
+// The scales and offsets of the four channels that a lane of a piece stores: requested with the operands, since a trip to
+// memory behind the sums is as long as everything else behind the operands' (see linear_piece_kernel).
+struct QuadScales
+{
+    f32x4 al, be;
+};
+
+template <int EPI>
+__device__ __forceinline__ QuadScales load_quad_scales(LinearArgs const& p, int const c)
+{
+    QuadScales s{};
+    if constexpr (EPI != kRAW && EPI != kF16_RAW)
+    {
+        int const at = min(c, p.N - 4);
+        s.al = *reinterpret_cast<f32x4 const*>(p.alpha + at);
+        s.be = *reinterpret_cast<f32x4 const*>(p.beta + at);
+    }
+    return s;
+}
+
 // The results of one lane for four consecutive channels (c .. c+3) of one token, packed and stored.
 template <bool IL_OUT, int EPI, typename Acc4>
-__device__ __forceinline__ void store_quad(LinearArgs const& p, Acc4 const& acc, int const c, int const t, int const part)
+__device__ __forceinline__ void store_quad(
+    LinearArgs const& p, Acc4 const& acc, QuadScales const& sc, int const c, int const t, int const part)
 {
     if constexpr (EPI == kRAW || EPI == kF16_RAW)
     {
@@ -1110,8 +1131,8 @@ __device__ __forceinline__ void store_quad(LinearArgs const& p, Acc4 const& acc,
         }
         return;
     }
-    f32x4 const al = *reinterpret_cast<f32x4 const*>(p.alpha + c);
-    f32x4 const be = *reinterpret_cast<f32x4 const*>(p.beta + c);
+    f32x4 const& al = sc.al;
+    f32x4 const& be = sc.be;
     if (t >= p.T)
     {
         return;
@@ -1604,6 +1625,8 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(LinearArgs 
         offB[b] = r * 32u + (uint32_t) half * 16u;
     }
     uint32_t const slabA = (uint32_t) p.N * 32u, slabB = (uint32_t) p.T * 32u;
+    static_assert(CB * TB * 4 <= NW, "a quarter of a block for each wavefront at most");
+    QuadScales const scales = load_quad_scales<EPI>(p, n0 + (wave / (4 * TB)) * 32 + 8 * (wave & 3) + 4 * half);
     // this workgroup's k-slabs, and the consecutive ones of this wavefront
     int const perPart = ceil_div(p.K / 32, p.parts);
     int const slabs = min(p.K / 32, (kpart + 1) * perPart);
@@ -1683,7 +1706,7 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(LinearArgs 
         }
     }
     __syncthreads();
-    for (int u = wave; u < CB * TB * 4; u += NW)
+    if (int const u = wave; u < CB * TB * 4)
     {
         Acc4 t = part[u * 64 + lane];
 #pragma unroll
@@ -1694,7 +1717,7 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(LinearArgs 
         int const b = u >> 2, q = u & 3, cb = n0 + (b / TB) * 32, tb = t0 + (b % TB) * 32;
         if (cb < p.N)
         {
-            store_quad<IL_OUT, EPI>(p, t, cb + 8 * q + 4 * half, tb + row, kpart);
+            store_quad<IL_OUT, EPI>(p, t, scales, cb + 8 * q + 4 * half, tb + row, kpart);
         }
     }
 }
@@ -1729,6 +1752,8 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
         int const g = u < 2 * CB ? min(n0 + r, p.N - 1) : min(t0 + r - 32 * CB, p.T - 1);
         off[u] = (uint32_t) g * (uint32_t) p.K + chunk;
     }
+    static_assert(CB * TB * 4 <= NW, "a quarter of a block for each wavefront at most");
+    QuadScales const scales = load_quad_scales<EPI>(p, n0 + (wave / (4 * TB)) * 32 + 8 * (wave & 3) + 4 * half);
     int const perPart = ceil_div(p.K / 64, p.parts); // stages of this workgroup
     int const nk = min(p.K / 64, (kpart + 1) * perPart);
     int const per = ceil_div(perPart, NW), first = kpart * perPart + wave * per;
@@ -1825,7 +1850,7 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
         }
     }
     __syncthreads();
-    for (int u = wave; u < CB * TB * 4; u += NW)
+    if (int const u = wave; u < CB * TB * 4)
     {
         Acc4 t = reinterpret_cast<Acc4 const*>(lds)[u * 64 + lane];
 #pragma unroll
@@ -1836,7 +1861,7 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
         int const b = u >> 2, q = u & 3, cb = n0 + (b / TB) * 32, tb = t0 + (b % TB) * 32;
         if (cb < p.N)
         {
-            store_quad<IL_OUT, EPI>(p, t, cb + 8 * q + 4 * half, tb + row, kpart);
+            store_quad<IL_OUT, EPI>(p, t, scales, cb + 8 * q + 4 * half, tb + row, kpart);
         }
     }
 }
