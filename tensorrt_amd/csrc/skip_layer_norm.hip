@@ -39,12 +39,18 @@ struct Vec16
 // The residual sum is formed in T like the reference (skipLayerNormKernel.cu:121-134);
 // statistics are a Welford/Chan merge in binary32; epsilon is the caller's.
 // ------------------------------------------------------------------------------------------
-template <typename T, int NV, int R, bool HAS_BIAS>
+// FEW: a launch bound by the trips to memory in a row, not by the bytes.  All arguments come in one trip and all of a
+// wavefront's loads in a second (the conditions of the other form made up to five and three of them).
+template <typename T, int NV, int R, bool HAS_BIAS, bool FEW>
 __global__ __launch_bounds__(kBlock) void skipln_rows_kernel(int const ld, int64_t const rows, T const* __restrict__ in,
     T const* __restrict__ skip, T const* __restrict__ beta, T const* __restrict__ gamma, T const* __restrict__ bias,
     T* __restrict__ out, float const eps)
 {
     constexpr int VPT = Vec16<T>::kN;
+    if constexpr (FEW)
+    {
+        asm volatile("" ::"s"(ld), "s"(rows), "s"(in), "s"(skip), "s"(beta), "s"(gamma), "s"(bias), "s"(out), "s"(eps));
+    }
     int const lane = threadIdx.x & (kWaveSize - 1);
     int64_t const wave = (int64_t) blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
     int64_t const row0 = wave * R;
@@ -54,31 +60,52 @@ __global__ __launch_bounds__(kBlock) void skipln_rows_kernel(int const ld, int64
     }
     int const nvec = ld / VPT;
 
-    Vec16<T> xin[R][NV], xsk[R][NV];
-#pragma unroll
-    for (int r = 0; r < R; ++r)
+    Vec16<T> xin[R][NV], xsk[R][NV], g[NV], b[NV], bs[NV];
+    if constexpr (FEW)
     {
+        static_assert(R == 1, "one row per wavefront");
 #pragma unroll
         for (int j = 0; j < NV; ++j)
         {
             int const vi = lane + kWaveSize * j;
-            bool const ok = vi < nvec && row0 + r < rows;
-            int64_t const off = (row0 + r) * ld + (int64_t) vi * VPT;
-            xin[r][j].u = ok ? *reinterpret_cast<u32x4 const*>(in + off) : u32x4{0, 0, 0, 0};
-            xsk[r][j].u = ok ? *reinterpret_cast<u32x4 const*>(skip + off) : u32x4{0, 0, 0, 0};
+            int const c = vi < nvec ? vi * VPT : 0; // lanes behind the end of the row re-read its start
+            xin[0][j].u = *reinterpret_cast<u32x4 const*>(in + row0 * ld + c);
+            xsk[0][j].u = *reinterpret_cast<u32x4 const*>(skip + row0 * ld + c);
+            g[j].u = *reinterpret_cast<u32x4 const*>(gamma + c);
+            b[j].u = *reinterpret_cast<u32x4 const*>(beta + c);
+            if (HAS_BIAS)
+            {
+                bs[j].u = *reinterpret_cast<u32x4 const*>(bias + c);
+            }
         }
+        __builtin_amdgcn_sched_barrier(0);
     }
-    Vec16<T> g[NV], b[NV], bs[NV];
-#pragma unroll
-    for (int j = 0; j < NV; ++j)
+    else
     {
-        int const vi = lane + kWaveSize * j;
-        bool const ok = vi < nvec;
-        g[j].u = ok ? *reinterpret_cast<u32x4 const*>(gamma + vi * VPT) : u32x4{0, 0, 0, 0};
-        b[j].u = ok ? *reinterpret_cast<u32x4 const*>(beta + vi * VPT) : u32x4{0, 0, 0, 0};
-        if (HAS_BIAS)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
         {
-            bs[j].u = ok ? *reinterpret_cast<u32x4 const*>(bias + vi * VPT) : u32x4{0, 0, 0, 0};
+#pragma unroll
+            for (int j = 0; j < NV; ++j)
+            {
+                int const vi = lane + kWaveSize * j;
+                bool const ok = vi < nvec && row0 + r < rows;
+                int64_t const off = (row0 + r) * ld + (int64_t) vi * VPT;
+                xin[r][j].u = ok ? *reinterpret_cast<u32x4 const*>(in + off) : u32x4{0, 0, 0, 0};
+                xsk[r][j].u = ok ? *reinterpret_cast<u32x4 const*>(skip + off) : u32x4{0, 0, 0, 0};
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+        {
+            int const vi = lane + kWaveSize * j;
+            bool const ok = vi < nvec;
+            g[j].u = ok ? *reinterpret_cast<u32x4 const*>(gamma + vi * VPT) : u32x4{0, 0, 0, 0};
+            b[j].u = ok ? *reinterpret_cast<u32x4 const*>(beta + vi * VPT) : u32x4{0, 0, 0, 0};
+            if (HAS_BIAS)
+            {
+                bs[j].u = ok ? *reinterpret_cast<u32x4 const*>(bias + vi * VPT) : u32x4{0, 0, 0, 0};
+            }
         }
     }
 
@@ -126,6 +153,14 @@ __global__ __launch_bounds__(kBlock) void skipln_rows_kernel(int const ld, int64
             }
         }
         w = group_welford<kWaveSize>(w);
+        if constexpr (FEW)
+        {
+#pragma unroll
+            for (int j = 0; j < NV; ++j)
+            {
+                asm volatile("" : "+v"(g[j].u), "+v"(b[j].u)); // not sunk to where the lanes are masked
+            }
+        }
         float const mu = w.mean;
         float const rsigma = rsqrtf(w.m2 * rld + eps);
 #pragma unroll
@@ -187,23 +222,36 @@ __global__ __launch_bounds__(kBlock) void skipln_generic_kernel(int const ld, in
     }
 }
 
-template <typename T, int NV, int R>
-int launch_rows(hipStream_t stream, int ld, int64_t rows, T const* in, T const* skip, T const* beta, T const* gamma,
+template <typename T, int NV, int R, bool FEW>
+int launch_rows_as(hipStream_t stream, int ld, int64_t rows, T const* in, T const* skip, T const* beta, T const* gamma,
     T const* bias, T* out, float eps)
 {
     int64_t const waves = ceil_div<int64_t>(rows, R);
     dim3 const grid((unsigned) ceil_div<int64_t>(waves, kWavesPerBlock));
-    if (bias)
+    auto const launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, stream, ld, rows, in, skip, beta, gamma, bias, out, eps);
+        return check_launch("skipln_rows_kernel");
+    };
+    return bias ? launch(skipln_rows_kernel<T, NV, R, true, FEW>) : launch(skipln_rows_kernel<T, NV, R, false, FEW>);
+}
+
+// Up to here one form is the faster throughout, beyond it the bytes set the time of either (us, masked loads / FEW: FP32 x 768,
+// 128 rows 2.89 / 2.77, 1024 rows 4.09 / 3.73, 2048 rows 5.00 / 4.60, 8192 rows 12.6 / 12.4, 32000 rows 45.1 / 47.3; FP16 x
+// 384, 128 rows 2.40 / 2.25, 8192 rows 6.14 / 6.16, 32000 rows 18.1 / 18.7).
+constexpr int64_t kFewRows = 8192;
+
+template <typename T, int NV, int R>
+int launch_rows(hipStream_t stream, int ld, int64_t rows, T const* in, T const* skip, T const* beta, T const* gamma,
+    T const* bias, T* out, float eps)
+{
+    if constexpr (R == 1)
     {
-        hipLaunchKernelGGL((skipln_rows_kernel<T, NV, R, true>), grid, dim3(kBlock), 0, stream, ld, rows, in, skip, beta,
-            gamma, bias, out, eps);
+        if (rows <= kFewRows)
+        {
+            return launch_rows_as<T, NV, 1, true>(stream, ld, rows, in, skip, beta, gamma, bias, out, eps);
+        }
     }
-    else
-    {
-        hipLaunchKernelGGL((skipln_rows_kernel<T, NV, R, false>), grid, dim3(kBlock), 0, stream, ld, rows, in, skip,
-            beta, gamma, bias, out, eps);
-    }
-    return check_launch("skipln_rows_kernel");
+    return launch_rows_as<T, NV, R, false>(stream, ld, rows, in, skip, beta, gamma, bias, out, eps);
 }
 
 template <typename T>
@@ -243,7 +291,7 @@ int skip_layer_norm(hipStream_t stream, int32_t ld, int64_t n, T const* in, T co
     {
         if constexpr (sizeof(T) == 2)
         {
-            if (rows > 8192)
+            if (rows > kFewRows)
             {
                 return launch_rows<T, 2, 2>(stream, ld, rows, in, skip, beta, gamma, bias, out, eps);
             }
@@ -289,6 +337,8 @@ __global__ __launch_bounds__(kBlock) void skipln_rows_partial_kernel(int const l
     PartialSums<float> const sums, f16 const* __restrict__ skip, f16 const* __restrict__ beta, f16 const* __restrict__ gamma,
     f16 const* __restrict__ bias, f16* __restrict__ out, float const eps)
 {
+    asm volatile("" ::"s"(ld), "s"(rows), "s"(sums.sums), "s"(sums.parts), "s"(sums.alpha), "s"(sums.beta), "s"(skip), "s"(beta),
+                 "s"(gamma), "s"(bias), "s"(out), "s"(eps));
     int const lane = threadIdx.x & (kWaveSize - 1);
     int const row = (int) blockIdx.x * kWavesPerBlock + (int) (threadIdx.x >> 6);
     if (row >= rows)
@@ -296,41 +346,48 @@ __global__ __launch_bounds__(kBlock) void skipln_rows_partial_kernel(int const l
         return;
     }
     int const nvec = ld / 8;
-    f32x4 x[NV][2];
+    f32x4 x[NV][2], sum4[NV][kMaxLinearParts][2], al[NV][2], be[NV][2];
     Vec16<f16> xs[NV], g[NV], b[NV], bs[NV];
 #pragma unroll
     for (int j = 0; j < NV; ++j)
     {
         int const vi = lane + kWaveSize * j;
-        bool const ok = vi < nvec;
-        int const c = ok ? vi * 8 : 0;
-        f32x4 v[kMaxLinearParts][2];
-#pragma unroll
-        for (int s = 0; s < kMaxLinearParts; ++s)
-        {
-            float const* src = sums.sums + ((int64_t) min(s, sums.parts - 1) * rows + row) * ld + c;
-            v[s][0] = *reinterpret_cast<f32x4 const*>(src);
-            v[s][1] = *reinterpret_cast<f32x4 const*>(src + 4);
-        }
-        xs[j].u = ok ? *reinterpret_cast<u32x4 const*>(skip + (int64_t) row * ld + c) : u32x4{0, 0, 0, 0};
-        g[j].u = ok ? *reinterpret_cast<u32x4 const*>(gamma + c) : u32x4{0, 0, 0, 0};
-        b[j].u = ok ? *reinterpret_cast<u32x4 const*>(beta + c) : u32x4{0, 0, 0, 0};
-        bs[j].u = ok ? *reinterpret_cast<u32x4 const*>(bias + c) : u32x4{0, 0, 0, 0};
+        int const c = vi < nvec ? vi * 8 : 0; // lanes behind the end re-read the start, and count and store nothing
 #pragma unroll
         for (int h = 0; h < 2; ++h)
         {
-            x[j][h] = v[0][h];
+#pragma unroll
+            for (int s = 0; s < kMaxLinearParts; ++s)
+            {
+                sum4[j][s][h] = *reinterpret_cast<f32x4 const*>(
+                    sums.sums + ((int64_t) min(s, sums.parts - 1) * rows + row) * ld + c + 4 * h);
+            }
+            al[j][h] = *reinterpret_cast<f32x4 const*>(sums.alpha + c + 4 * h);
+            be[j][h] = *reinterpret_cast<f32x4 const*>(sums.beta + c + 4 * h);
+        }
+        xs[j].u = *reinterpret_cast<u32x4 const*>(skip + (int64_t) row * ld + c);
+        bs[j].u = *reinterpret_cast<u32x4 const*>(bias + c);
+        g[j].u = *reinterpret_cast<u32x4 const*>(gamma + c);
+        b[j].u = *reinterpret_cast<u32x4 const*>(beta + c);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+    {
+        bool const ok = lane + kWaveSize * j < nvec;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+        {
+            x[j][h] = sum4[j][0][h];
 #pragma unroll
             for (int s = 1; s < kMaxLinearParts; ++s)
             {
-                x[j][h] += s < sums.parts ? v[s][h] : f32x4{0.f, 0.f, 0.f, 0.f};
+                x[j][h] += s < sums.parts ? sum4[j][s][h] : f32x4{0.f, 0.f, 0.f, 0.f};
             }
-            f32x4 const al = *reinterpret_cast<f32x4 const*>(sums.alpha + c + 4 * h);
-            f32x4 const be = *reinterpret_cast<f32x4 const*>(sums.beta + c + 4 * h);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
             {
-                x[j][h][e] = ok ? fmaf(x[j][h][e], al[e], be[e]) : 0.f;
+                x[j][h][e] = ok ? fmaf(x[j][h][e], al[j][h][e], be[j][h][e]) : 0.f;
             }
         }
     }
@@ -365,6 +422,11 @@ __global__ __launch_bounds__(kBlock) void skipln_rows_partial_kernel(int const l
         }
     }
     w = group_welford<kWaveSize>(w);
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+    {
+        asm volatile("" : "+v"(g[j].u), "+v"(b[j].u)); // not sunk to where the lanes are masked
+    }
     float const rsigma = rsqrtf(w.m2 * (1.f / (float) ld) + eps);
 #pragma unroll
     for (int j = 0; j < NV; ++j)
@@ -570,6 +632,8 @@ __global__ __launch_bounds__(W * kWaveSize) void skipln_interleaved_kernel(int c
     constexpr int SUBS = kWaveSize / LPG;      // channel groups per load instruction
     constexpr int NI = G / (SUBS * W);
     static_assert(G % (SUBS * W) == 0 && NI <= 8, "every lane keeps its part of the row in registers");
+    asm volatile("" ::"s"(total), "s"(gridDim.x), "s"(in), "s"(skip), "s"(beta), "s"(gamma), "s"(out), "s"(preln), "s"(dqIn),
+                 "s"(dqSkip), "s"(qScale), "s"(eps));
     __shared__ float sGamma[LD];
     __shared__ float sBeta[LD];
     __shared__ int sStat[W][TOK][5];
@@ -841,6 +905,8 @@ __global__ __launch_bounds__(kBlock) void skipln_interleaved_token_kernel(int co
 {
     constexpr int LD = G * 32;
     constexpr int NE = (G + 31) / 32; // loads per tensor and lane: 32 channel groups x 2 halves each
+    asm volatile("" ::"s"(total), "s"(in), "s"(skip), "s"(beta), "s"(gamma), "s"(out), "s"(preln), "s"(dqIn), "s"(dqSkip),
+                 "s"(qScale), "s"(eps));
     int const lane = threadIdx.x & (kWaveSize - 1);
     int const hf = lane & 1;
     int const token = (int) blockIdx.x * kWavesPerBlock + (int) (threadIdx.x >> 6);
@@ -854,11 +920,10 @@ __global__ __launch_bounds__(kBlock) void skipln_interleaved_token_kernel(int co
 #pragma unroll
     for (int e = 0; e < NE; ++e)
     {
-        int const grp = e * 32 + (lane >> 1);
-        bool const live = grp < G;
+        int const grp = min(e * 32 + (lane >> 1), G - 1); // lanes behind the last group re-read it
         int64_t const off = (int64_t) grp * groupStride + (int64_t) token * 32 + hf * 16;
-        xi[e] = live ? *reinterpret_cast<u32x4 const*>(in + off) : u32x4{0, 0, 0, 0};
-        xs[e] = live ? *reinterpret_cast<u32x4 const*>(skip + off) : u32x4{0, 0, 0, 0};
+        xi[e] = *reinterpret_cast<u32x4 const*>(in + off);
+        xs[e] = *reinterpret_cast<u32x4 const*>(skip + off);
     }
 #pragma unroll
     for (int e = 0; e < NE; ++e)
@@ -872,10 +937,14 @@ __global__ __launch_bounds__(kBlock) void skipln_interleaved_token_kernel(int co
             b[e][q] = *reinterpret_cast<f16x8 const*>(beta + ch + 8 * q);
         }
     }
+    __builtin_amdgcn_sched_barrier(0);
     int sIn = 0, sSk = 0, sII = 0, sIS = 0, sSS = 0;
 #pragma unroll
     for (int e = 0; e < NE; ++e)
     {
+        bool const live = e * 32 + (lane >> 1) < G;
+        xi[e] = live ? xi[e] : u32x4{0, 0, 0, 0};
+        xs[e] = live ? xs[e] : u32x4{0, 0, 0, 0};
 #pragma unroll
         for (int q = 0; q < 4; ++q)
         {
@@ -891,6 +960,11 @@ __global__ __launch_bounds__(kBlock) void skipln_interleaved_token_kernel(int co
     sII = wave_sum_i32(sII);
     sIS = wave_sum_i32(sIS);
     sSS = wave_sum_i32(sSS);
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+    {
+        asm volatile("" : "+v"(g[e][0]), "+v"(g[e][1]), "+v"(b[e][0]), "+v"(b[e][1])); // not sunk to where lanes are masked
+    }
     double const dIn = (double) dqIn, dSk = (double) dqSkip;
     double const mean = (dIn * sIn + dSk * sSk) * (1.0 / LD);
     double const ex2 = (dIn * dIn * sII + 2.0 * dIn * dSk * sIS + dSk * dSk * sSS) * (1.0 / LD);
@@ -950,6 +1024,8 @@ __global__ __launch_bounds__(G * 8) void skipln_interleaved_sums_kernel(int cons
 {
     constexpr int LD = G * 32, WAVES = G / 8;
     __shared__ int sStat[WAVES][5];
+    asm volatile("" ::"s"(total), "s"(sums.sums), "s"(sums.parts), "s"(sums.alpha), "s"(sums.beta), "s"(skip), "s"(beta),
+                 "s"(gamma), "s"(out), "s"(dqIn), "s"(dqSkip), "s"(qScale), "s"(eps));
     int const token = (int) blockIdx.x;
     int const wave = (int) (threadIdx.x >> 6);
     int const ch = (int) threadIdx.x * 4;

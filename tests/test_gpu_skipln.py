@@ -62,6 +62,17 @@ def test_skipln_fp(api, dt, rows, ld, has_bias):
     assert_fp_close(got, ref, what="vs oracle")
 
 
+# the launches whose loads are unconditional: lanes and whole columns behind the end of a row (one to eight vectors per lane),
+# a last workgroup of one wavefront, and either side of the 8192 rows up to which they are chosen
+@pytest.mark.parametrize("dt,ld", [(np.float32, 36), (np.float32, 768), (np.float32, 1996), (np.float16, 40), (np.float16, 520),
+                                   (np.float16, 1032), (np.float16, 4088)])
+@pytest.mark.parametrize("rows", [1, 6, 8192, 8193])
+def test_skipln_fp_few_rows(api, dt, rows, ld):
+    if rows > 6 and ld > 1032:
+        rows = 9
+    test_skipln_fp(api, dt, rows, ld, rows % 2 == 0)
+
+
 def test_skipln_fp_errors(api):
     assert api.skip_layer_norm_fp32(None, 768, 100, 0, 0, 0, 0, 0, 0) != 0   # n % ld != 0
     assert "multiple" in api.last_error_str()
