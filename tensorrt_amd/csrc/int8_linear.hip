@@ -83,6 +83,7 @@ struct LinearArgs
     int persist;   // persistent kernel: workgroups that loop over the 256 x 256 tiles
     int pieces;    // large tiles: the tokens behind them go in 64 x 64 pieces (see linear_piece64)
     int parts;     // pieces: workgroups that share the k range of a piece, each with an output of its own
+    int perPart;   // pieces: 32-byte k-slabs (interleaved operands) or 64-byte stages of each
     WeightPrefetch prefetch; // by the workgroups behind mainTiles of the interleaved tile and piece kernels
 };
 
@@ -1544,13 +1545,16 @@ __global__ __launch_bounds__(512) void int8_linear_dma_kernel(LinearArgs const p
 // whose L2 the launch that uses them will look in (ids are dealt to the 8 XCDs in turn), waits for them and drops them.
 constexpr int kPrefetchLoads = 4; // per wavefront, 1 KB each
 
-__device__ __forceinline__ void prefetch_weights(LinearArgs const& p)
+__device__ __forceinline__ void prefetch_weights(LinearArgs const& p, uint32_t id, uint32_t waves)
 {
     int const lane = threadIdx.x & 63;
-    uint32_t const waves = blockDim.x >> 6;
-    uint32_t const xcd = blockIdx.x & 7u, rank = (blockIdx.x - (uint32_t) p.mainTiles) >> 3;
+    uint32_t const xcd = id & 7u, rank = (id - (uint32_t) p.mainTiles) >> 3;
     uint32_t const perXcd = p.prefetch.units / 8u;
     uint32_t const first = (rank * waves + (threadIdx.x >> 6)) * kPrefetchLoads;
+    if (first >= perXcd)
+    {
+        return;
+    }
     i32x4 v[kPrefetchLoads];
 #pragma unroll
     for (int i = 0; i < kPrefetchLoads; ++i)
@@ -1575,7 +1579,7 @@ __global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(Line
     {
         if ((int) blockIdx.x >= p.mainTiles)
         {
-            prefetch_weights(p);
+            prefetch_weights(p, blockIdx.x, WM * WN);
             return;
         }
     }
@@ -1588,13 +1592,24 @@ __global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(Line
         p, (int) (pan * pw + rem % pw) * (WM * MT * 32), (int) (rem / pw) * (WN * NT * 32), lds);
 }
 
+// Asks for what the piece kernels read of their arguments at once: left to its first use, each trip of the scalar loads
+// delays a launch of few tokens by 0.1 to 0.2 us, and there were up to five one after the other.  With the divisions that
+// the numbering of the pieces took (they have a grid of three extents now), a pass of one request: INT8, 24 layers of 1024
+// channels, 632 -> 590 us; FP16, 12 layers of 768, 386 -> 379 us.
+__device__ __forceinline__ void pin_piece_args(LinearArgs const& p)
+{
+    asm volatile("" ::"s"(p.a), "s"(p.w), "s"(p.alpha), "s"(p.beta), "s"(p.out), "s"(p.T), "s"(p.K), "s"(p.N), "s"(p.qOut),
+                 "s"(p.tokMain), "s"(p.parts), "s"(p.perPart), "s"(p.mainTiles), "s"(p.prefetch.data), "s"(p.prefetch.units));
+}
+
 // A piece of CB x TB blocks of 32 channels x 32 tokens by one workgroup whose eight wavefronts split k, for launches
 // with too few tokens to fill the chip with tiles that walk k one stage after the other: bound by the latency of one trip
 // to memory and by what one CU can read (64 bytes a clock), not by the matrix cores.  Interleaved operands, as in
 // linear_piece64: a fragment is 1 KB of consecutive memory and goes straight into the operand registers, DEPTH k-slabs
 // in flight per wavefront, no LDS stage and no barrier before the eight partial accumulators meet in LDS; every wavefront
 // then adds up and stores quarters of blocks.  40 tokens x 4096 -> 1024: 19.1 us in 128 x 128 tiles, 4.7 us in 32 x 32
-// pieces; K any multiple of 32 bytes, N and T any.
+// pieces; K any multiple of 32 bytes, N and T any.  The grid is (channel pieces, token pieces, parts and what prefetches):
+// no division stands between a wavefront's start and its first request, and all arguments come in one trip.
 template <bool IL_OUT, int EPI, int CB, int TB, int DEPTH, int PER_SIMD>
 __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(LinearArgs const p)
 {
@@ -1603,14 +1618,14 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(LinearArgs 
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int const row = lane & 31, half = lane >> 5;
-    if ((int) blockIdx.x >= p.mainTiles)
+    pin_piece_args(p);
+    if ((int) blockIdx.z >= p.parts)
     {
-        prefetch_weights(p);
+        uint32_t const nbm = (uint32_t) ceil_div(p.N, 32 * CB);
+        prefetch_weights(p, (blockIdx.z * (uint32_t) p.tokMain + blockIdx.y) * nbm + blockIdx.x, NW);
         return;
     }
-    uint32_t const nbm = (uint32_t) ceil_div(p.N, 32 * CB);
-    int const n0 = (int) (blockIdx.x % nbm) * (32 * CB);
-    int const kpart = (int) (blockIdx.x / nbm) / p.tokMain, t0 = (int) (blockIdx.x / nbm) % p.tokMain * (32 * TB);
+    int const n0 = (int) blockIdx.x * (32 * CB), t0 = (int) blockIdx.y * (32 * TB), kpart = (int) blockIdx.z;
     uint32_t offA[CB], offB[TB];
 #pragma unroll
     for (int b = 0; b < CB; ++b)
@@ -1628,9 +1643,8 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(LinearArgs 
     static_assert(CB * TB * 4 <= NW, "a quarter of a block for each wavefront at most");
     QuadScales const scales = load_quad_scales<EPI>(p, n0 + (wave / (4 * TB)) * 32 + 8 * (wave & 3) + 4 * half);
     // this workgroup's k-slabs, and the consecutive ones of this wavefront
-    int const perPart = ceil_div(p.K / 32, p.parts);
-    int const slabs = min(p.K / 32, (kpart + 1) * perPart);
-    int const per = ceil_div(perPart, NW), first = kpart * perPart + wave * per;
+    int const slabs = min(p.K / 32, (kpart + 1) * p.perPart);
+    int const per = ceil_div(p.perPart, NW), first = kpart * p.perPart + wave * per;
     int const steps = max(0, min(per, slabs - first));
     i32x4 fa[DEPTH][CB], fb[DEPTH][TB];
     auto fetch = [&](int slot, int step) {
@@ -1737,9 +1751,8 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int const row = lane & 31, half = lane >> 5;
-    uint32_t const nbm = (uint32_t) ceil_div(p.N, 32 * CB);
-    int const n0 = (int) (blockIdx.x % nbm) * (32 * CB);
-    int const kpart = (int) (blockIdx.x / nbm) / p.tokMain, t0 = (int) (blockIdx.x / nbm) % p.tokMain * (32 * TB);
+    pin_piece_args(p);
+    int const n0 = (int) blockIdx.x * (32 * CB), t0 = (int) blockIdx.y * (32 * TB), kpart = (int) blockIdx.z;
     uint8_t* const own = lds + wave * (RING * STAGE);
     uint32_t const ownBase = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) own;
     int const rr = lane >> 2;
@@ -1754,9 +1767,8 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
     }
     static_assert(CB * TB * 4 <= NW, "a quarter of a block for each wavefront at most");
     QuadScales const scales = load_quad_scales<EPI>(p, n0 + (wave / (4 * TB)) * 32 + 8 * (wave & 3) + 4 * half);
-    int const perPart = ceil_div(p.K / 64, p.parts); // stages of this workgroup
-    int const nk = min(p.K / 64, (kpart + 1) * perPart);
-    int const per = ceil_div(perPart, NW), first = kpart * perPart + wave * per;
+    int const nk = min(p.K / 64, (kpart + 1) * p.perPart); // stages up to the end of this workgroup's
+    int const per = ceil_div(p.perPart, NW), first = kpart * p.perPart + wave * per;
     int const steps = max(0, min(per, nk - first));
     auto fetch = [&](int step, int slot) {
         uint64_t const k = (uint64_t) (first + step) * 64u;
@@ -1978,16 +1990,38 @@ inline float large_tiles_time(TileCost const& c, LinearArgs const& a, int64_t sm
     return c.launch + rounds * (c.tile + (gelu ? c.gelu : 0.f) + c.stage * stages) + rest;
 }
 
-// The workgroups of a.mainTiles tiles, with those that fetch a.prefetch behind them where the launch leaves CUs idle.
+bool is_piece(int plan)
+{
+    return plan == kPiece32x64 || plan == kPiece32x32;
+}
+
+// What fetches a.prefetch behind the tiles, where the launch leaves CUs idle.
+uint32_t prefetch_workgroups(LinearArgs const& a, int threads)
+{
+    return a.prefetch.data && a.mainTiles <= num_cus()
+        ? 8u * ceil_div(a.prefetch.units / 8u, (uint32_t) (threads / 64 * kPrefetchLoads))
+        : 0u;
+}
+
+// The workgroups of a.mainTiles tiles, with those behind them.
 template <typename Kernel>
 int launch_tiles(hipStream_t stream, LinearArgs const& a, Kernel kernel, int threads)
 {
-    uint32_t behind = 0;
-    if (a.prefetch.data && a.mainTiles <= num_cus())
-    {
-        behind = 8u * ceil_div(a.prefetch.units / 8u, (uint32_t) (threads / 64 * kPrefetchLoads));
-    }
-    hipLaunchKernelGGL(kernel, dim3((uint32_t) a.mainTiles + behind), dim3(threads), 0, stream, a);
+    hipLaunchKernelGGL(kernel, dim3((uint32_t) a.mainTiles + prefetch_workgroups(a, threads)), dim3(threads), 0, stream, a);
+    return check_launch("int8_linear");
+}
+
+// The same for pieces of `channels` x `tokens`, in as many parts as a.parts says.
+template <bool IL, typename Kernel>
+int launch_pieces(hipStream_t stream, LinearArgs a, Kernel kernel, int channels, int tokens)
+{
+    uint32_t const nbm = (uint32_t) ceil_div(a.N, channels);
+    a.tokMain = ceil_div(a.T, tokens);
+    a.mainTiles = (int) nbm * a.tokMain * a.parts;
+    a.perPart = ceil_div(a.K / (IL ? 32 : 64), a.parts);
+    uint32_t const behind = IL ? prefetch_workgroups(a, 512) : 0u;
+    hipLaunchKernelGGL(kernel, dim3(nbm, (uint32_t) a.tokMain, (uint32_t) a.parts + ceil_div(behind, nbm * (uint32_t) a.tokMain)),
+        dim3(512), 0, stream, a);
     return check_launch("int8_linear");
 }
 
@@ -2030,18 +2064,18 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
         case kTile256x256: return run(linear_tile_kernel<IL, IL_OUT, EPI, 4, 2, 2, 4, 4, 2>, 512);
         case kTile256x192: return run(linear_tile_kernel<IL, IL_OUT, EPI, 4, 2, 2, 3, 5, 2>, 512);
         case kTile128x192: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 3, 4, 2>, 256);
-        case kPiece32x64: return run(linear_piece_kernel<IL_OUT, EPI, 1, 2, 4, 4>, 512);
-        case kPiece32x32: return run(linear_piece_kernel<IL_OUT, EPI, 1, 1, 8, 4>, 512);
+        case kPiece32x64: return launch_pieces<IL>(stream, a, linear_piece_kernel<IL_OUT, EPI, 1, 2, 4, 4>, 32, 64);
+        case kPiece32x32: return launch_pieces<IL>(stream, a, linear_piece_kernel<IL_OUT, EPI, 1, 1, 8, 4>, 32, 32);
         default: break;
         }
     }
     else if (plan == kPiece32x64)
     {
-        return run(linear_piece_dma_kernel<IL_OUT, EPI, 1, 2, 3, 2>, 512);
+        return launch_pieces<IL>(stream, a, linear_piece_dma_kernel<IL_OUT, EPI, 1, 2, 3, 2>, 32, 64);
     }
     else if (plan == kPiece32x32)
     {
-        return run(linear_piece_dma_kernel<IL_OUT, EPI, 1, 1, 4, 2>, 512);
+        return launch_pieces<IL>(stream, a, linear_piece_dma_kernel<IL_OUT, EPI, 1, 1, 4, 2>, 32, 32);
     }
     else if (a.K % 128 != 0)
     {
@@ -2078,15 +2112,13 @@ int launch_partial(hipStream_t stream, LinearArgs a, int parts, void* partial, W
     a.out = partial;
     a.parts = parts;
     a.prefetch = prefetch;
-    a.tokMain = ceil_div(a.T, 32);
-    a.mainTiles = ceil_div(a.N, 32) * a.tokMain * parts;
     if constexpr (IL)
     {
-        return launch_tiles(stream, a, linear_piece_kernel<false, EPI, 1, 1, 8, 4>, 512);
+        return launch_pieces<IL>(stream, a, linear_piece_kernel<false, EPI, 1, 1, 8, 4>, 32, 32);
     }
     else
     {
-        return launch_tiles(stream, a, linear_piece_dma_kernel<false, EPI, 1, 1, 4, 2>, 512);
+        return launch_pieces<IL>(stream, a, linear_piece_dma_kernel<false, EPI, 1, 1, 4, 2>, 32, 32);
     }
 }
 
@@ -2099,6 +2131,10 @@ int cheapest_plan(LinearArgs const& a, int64_t smallTiles, bool gelu, int plan)
         if (q == kLargeTiles)
         {
             return large;
+        }
+        if (is_piece(q) && ceil_div(a.T, kTileCosts[IL][q].tokens) > 65535)
+        {
+            return false; // the second extent of their grid
         }
         bool const halfLines = !IL && a.K % 128 != 0; // the tiles that have a kernel for those
         return kTileCosts[IL][q].channels != 0
@@ -2159,11 +2195,6 @@ int small_plan(LinearArgs a, bool gelu)
     }
     a.mainTiles = 0;
     return choose_plan<IL>(a, 0, gelu);
-}
-
-bool is_piece(int plan)
-{
-    return plan == kPiece32x64 || plan == kPiece32x32;
 }
 
 // Parts of a layer whose launch is `plan`: as many as bring its workgroups to one per CU, and no less than 1 KB of k for

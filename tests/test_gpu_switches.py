@@ -129,6 +129,16 @@ def test_linear_plans(plan, T, K, N):
         assert_fp_close(got, ref, what=f"plan {plan} FP16")
 
 
+@pytest.mark.parametrize("plan,T", [(9, 65535 * 32), (9, 65535 * 32 + 1), (8, 65535 * 32 + 1)])
+def test_pieces_up_to_the_extent_of_their_grid(plan, T):
+    """More pieces of tokens than the second extent of a grid holds are left to another plan."""
+    a, w, alpha, beta = problem(99, T, 64, 32)
+    want = run_gpu(a, w, alpha, beta, capi.LINEAR_AFFINE, a_il=True, out_il=True, w_il=True)
+    with tuning("TRTAMD_LINEAR_PLAN", plan):
+        got = run_gpu(a, w, alpha, beta, capi.LINEAR_AFFINE, a_il=True, out_il=True, w_il=True)
+    assert np.array_equal(got, want)
+
+
 # tiles of linear operands: stages of 128 bytes of k (64 FP16 values), rings of two to five of them.  One stage, as many as
 # the ring has and one more; a last line that is half there; token and channel counts on both sides of a tile's edge.
 @pytest.mark.parametrize("plan", [2, 4, 5, 10, 11, 12, 13, 14])
