@@ -254,6 +254,30 @@ __device__ inline uint32_t xcd_remap(uint32_t bid, uint32_t nblocks)
     return (bid % kXcds) * per + bid / kXcds;
 }
 
+// Division by a number that the host knows, as part of a launch's arguments: a division by any other value is some forty
+// dependent instructions, which a workgroup would spend on finding its place before its first request.  Exact for all
+// 32-bit values (Granlund and Montgomery, "Division by Invariant Integers using Multiplication", figure 4.1).
+struct FastDiv
+{
+    uint32_t d, mul, shift1, shift2;
+};
+
+inline FastDiv fast_div(uint32_t d)
+{
+    uint32_t l = 0;
+    while ((uint64_t) 1 << l < d)
+    {
+        ++l;
+    }
+    return {d, (uint32_t) (((((uint64_t) 1 << l) - d) << 32) / d + 1u), l ? 1u : 0u, l ? l - 1u : 0u};
+}
+
+__host__ __device__ inline uint32_t operator/(uint32_t n, FastDiv const& v)
+{
+    uint32_t const t = (uint32_t) ((uint64_t) n * v.mul >> 32);
+    return (t + ((n - t) >> v.shift1)) >> v.shift2;
+}
+
 // Which unit of work and which of its `parts` a workgroup takes when several workgroups share a unit's data (the
 // attention kernels: a (sequence, head) unit's K and V, read by every workgroup that takes some of its queries).
 // Workgroup ids are dealt round-robin to the 8 XCDs, so ids 8 q m + 8 p + x take unit 8 m + x, part p: the parts of a
@@ -279,6 +303,22 @@ __device__ inline UnitPart unit_of_workgroup(uint32_t bid, uint32_t nblocks, int
         return {m * 8u + x % 8u, (int) (x / 8u)};
     }
     return {bid / q, (int) (bid % q)};
+}
+
+// The same with the divisors at hand: `span` is 8 * parts.
+__device__ inline UnitPart unit_of_workgroup(uint32_t bid, uint32_t nblocks, FastDiv const& parts, FastDiv const& span)
+{
+    if (parts.d <= 1)
+    {
+        return {bid, 0};
+    }
+    uint32_t const m = bid / span, x = bid - m * span.d;
+    if ((m + 1) * span.d <= nblocks)
+    {
+        return {m * 8u + x % 8u, (int) (x / 8u)};
+    }
+    uint32_t const unit = bid / parts;
+    return {unit, (int) (bid - unit * parts.d)};
 }
 
 // 16 bytes per lane from global memory straight into LDS (global_load_lds_dwordx4): lane i's bytes land at LDS byte

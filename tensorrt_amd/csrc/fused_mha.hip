@@ -136,7 +136,20 @@ struct FmhaArgs
     int32_t* dbgAcc1;            // optional [B][N][S][S] int32 (INT8) / float bits (FP16)
     int8_t* dbgP8;               // optional [B][N][S][S]
     int32_t ranked;              // serve the longest sequences first (pointless when one round holds every workgroup)
+    FastDiv partDiv, spanDiv;    // by qSplit and 8 qSplit (unit_of_workgroup)
+    FastDiv headDiv, turnDiv;    // by N and kWavesI8 qSplit
 };
+
+// Asks for what the cu_seqlens kernels read of their arguments at once: left to the first uses, the trips of the scalar
+// loads stand one behind the other ahead of a workgroup's first request.
+__device__ __forceinline__ void pin_args(FmhaArgs const& a)
+{
+    asm volatile("" ::"s"(a.qkv), "s"(a.out), "s"(a.cuSeqlens), "s"(a.packedMask), "s"(a.tokStrideIn), "s"(a.tokStrideOut),
+                 "s"(a.seqStrideIn), "s"(a.seqStrideOut), "s"(a.B), "s"(a.S), "s"(a.total), "s"(a.c), "s"(a.scaleBmm2),
+                 "s"(a.ranked), "s"(gridDim.x), "s"(a.partDiv.d), "s"(a.partDiv.mul), "s"(a.partDiv.shift1),
+                 "s"(a.partDiv.shift2), "s"(a.spanDiv.d), "s"(a.spanDiv.mul), "s"(a.spanDiv.shift1), "s"(a.spanDiv.shift2),
+                 "s"(a.headDiv.d), "s"(a.headDiv.mul), "s"(a.headDiv.shift1), "s"(a.headDiv.shift2));
+}
 
 template <int ESIZE>
 struct Lds
@@ -1194,7 +1207,9 @@ __global__ __launch_bounds__(kWavesI8* kWaveSize) __attribute__((amdgpu_waves_pe
     uint8_t* sK = smem;
     uint8_t* sV = smem + Lds<1>::matBytes(KT);
     __shared__ PickLds sPick;
-    UnitPart up = unit_of_workgroup(blockIdx.x, gridDim.x, a.qSplit);
+    pin_args(a);
+    asm volatile("" ::"s"(a.turnDiv.d), "s"(a.turnDiv.mul), "s"(a.turnDiv.shift1), "s"(a.turnDiv.shift2));
+    UnitPart up = unit_of_workgroup(blockIdx.x, gridDim.x, a.partDiv, a.spanDiv);
     if (!INTERLEAVED && a.qSplit == 1 && (a.N & 1) == 0)
     {
         // Linear layout ([token][head][Q K V][64 bytes]): V of head n and Q of head n + 1 lie in one 128-byte line, so
@@ -1203,12 +1218,13 @@ __global__ __launch_bounds__(kWavesI8* kWaveSize) __attribute__((amdgpu_waves_pe
         up.unit = pair.unit * 2u + (uint32_t) pair.part;
     }
     int const part = up.part;
-    int const n = up.unit % a.N;
+    uint32_t const rank = up.unit / a.headDiv;
+    int const n = (int) (up.unit - rank * a.headDiv.d);
     int b;
-    SeqInfo sq = pick_sequence_info<kWavesI8 * kWaveSize>(a, up.unit / a.N, KT * 64, sPick, b);
+    SeqInfo sq = pick_sequence_info<kWavesI8 * kWaveSize>(a, (int) rank, KT * 64, sPick, b);
     // contiguous tile ranges, each a multiple of one round of the workgroup's wavefronts
     int const nqt = (sq.nq + kQPerWave - 1) / kQPerWave;
-    int const per = kWavesI8 * ((nqt + kWavesI8 * a.qSplit - 1) / (kWavesI8 * a.qSplit));
+    int const per = kWavesI8 * (int) ((uint32_t) (nqt + (int) a.turnDiv.d - 1) / a.turnDiv);
     int const qtBegin = min(part * per, nqt);
     int const qtEnd = min(qtBegin + per, nqt);
     if (qtBegin >= qtEnd)
@@ -1780,11 +1796,13 @@ __global__ __launch_bounds__(kWavesF16T* kWaveSize)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     __shared__ PickLds sPick;
-    UnitPart const up = unit_of_workgroup(blockIdx.x, gridDim.x, a.qSplit);
-    int const n = __builtin_amdgcn_readfirstlane(up.unit % a.N);
+    pin_args(a);
+    UnitPart const up = unit_of_workgroup(blockIdx.x, gridDim.x, a.partDiv, a.spanDiv);
+    uint32_t const rank = up.unit / a.headDiv;
+    int const n = __builtin_amdgcn_readfirstlane((int) (up.unit - rank * a.headDiv.d));
     int const q0 = __builtin_amdgcn_readfirstlane(up.part) * kQueriesF16;
     int b;
-    SeqInfo sq = pick_sequence_info<kWavesF16T * kWaveSize>(a, up.unit / a.N, KT * 64, sPick, b);
+    SeqInfo sq = pick_sequence_info<kWavesF16T * kWaveSize>(a, (int) rank, KT * 64, sPick, b);
     // the same in every lane, which the compiler cannot see where they come from LDS: scalars keep the addresses scalar
     b = __builtin_amdgcn_readfirstlane(b);
     sq.nq = __builtin_amdgcn_readfirstlane(sq.nq);
@@ -1860,10 +1878,12 @@ __global__ __launch_bounds__(kWavesStream* kWaveSize) __attribute__((amdgpu_wave
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ PickLds sPick;
     __shared__ uint64_t sMask[8];
-    UnitPart const up = unit_of_workgroup(blockIdx.x, gridDim.x, a.qSplit);
-    int const n = __builtin_amdgcn_readfirstlane(up.unit % a.N);
+    pin_args(a);
+    UnitPart const up = unit_of_workgroup(blockIdx.x, gridDim.x, a.partDiv, a.spanDiv);
+    uint32_t const rank = up.unit / a.headDiv;
+    int const n = __builtin_amdgcn_readfirstlane((int) (up.unit - rank * a.headDiv.d));
     int b;
-    SeqInfo sq = pick_sequence_info<kWavesStream * kWaveSize>(a, up.unit / a.N, capacity, sPick, b);
+    SeqInfo sq = pick_sequence_info<kWavesStream * kWaveSize>(a, (int) rank, capacity, sPick, b);
     // the same in every lane, which the compiler cannot see where they come from LDS: scalars keep the addresses scalar
     b = __builtin_amdgcn_readfirstlane(b);
     int const nq = __builtin_amdgcn_readfirstlane(sq.nq);
@@ -2456,6 +2476,10 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
             a.qSplit = std::min(forced, maxSplit);
         }
     }
+    a.partDiv = fast_div((uint32_t) a.qSplit);
+    a.spanDiv = fast_div(8u * (uint32_t) a.qSplit);
+    a.headDiv = fast_div((uint32_t) a.N);
+    a.turnDiv = fast_div((uint32_t) (kWavesI8 * a.qSplit));
     a.dbgAcc1 = dbgAcc1;
     a.dbgP8 = dbgP8;
     {

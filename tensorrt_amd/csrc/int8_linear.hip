@@ -84,6 +84,7 @@ struct LinearArgs
     int pieces;    // large tiles: the tokens behind them go in 64 x 64 pieces (see linear_piece64)
     int parts;     // pieces: workgroups that share the k range of a piece, each with an output of its own
     int perPart;   // pieces: 32-byte k-slabs (interleaved operands) or 64-byte stages of each
+    FastDiv panelDiv, perPanelDiv; // tiles: by panel and tokMain * panel
     WeightPrefetch prefetch; // by the workgroups behind mainTiles of the interleaved tile and piece kernels
 };
 
@@ -1575,6 +1576,10 @@ __global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(Line
 {
     constexpr int kRing = RING * (WM * MT + WN * NT) * KS * 1024;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[kRing + (scales_late(kRing) ? 0 : 2 * kBigTile * 4)];
+    // all arguments in one trip of the scalar loads, as in the piece kernels
+    asm volatile("" ::"s"(p.a), "s"(p.w), "s"(p.alpha), "s"(p.beta), "s"(p.out), "s"(p.T), "s"(p.K), "s"(p.N), "s"(p.mainTiles),
+                 "s"(p.panelDiv.d), "s"(p.panelDiv.mul), "s"(p.panelDiv.shift1), "s"(p.panelDiv.shift2), "s"(p.perPanelDiv.d),
+                 "s"(p.perPanelDiv.mul), "s"(p.perPanelDiv.shift1), "s"(p.perPanelDiv.shift2));
     if constexpr (IL)
     {
         if ((int) blockIdx.x >= p.mainTiles)
@@ -1584,12 +1589,11 @@ __global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(Line
         }
     }
     // panel numbering as for the large tiles (see int8_linear_kernel)
-    uint32_t const pw = (uint32_t) p.panel;
-    uint32_t const perPanel = (uint32_t) p.tokMain * pw;
     uint32_t const tile = xcd_remap(blockIdx.x, (uint32_t) p.mainTiles);
-    uint32_t const pan = tile / perPanel, rem = tile % perPanel;
+    uint32_t const pan = tile / p.perPanelDiv, rem = tile - pan * p.perPanelDiv.d;
+    uint32_t const tokenTile = rem / p.panelDiv, inPanel = rem - tokenTile * p.panelDiv.d;
     linear_tile_dma<IL, IL_OUT, EPI, WM, WN, MT, NT, RING, KS>(
-        p, (int) (pan * pw + rem % pw) * (WM * MT * 32), (int) (rem / pw) * (WN * NT * 32), lds);
+        p, (int) (pan * p.panelDiv.d + inPanel) * (WM * MT * 32), (int) tokenTile * (WN * NT * 32), lds);
 }
 
 // Asks for what the piece kernels read of their arguments at once: left to its first use, each trip of the scalar loads
@@ -2046,6 +2050,8 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
     }
     a.parts = 1;
     a.mainTiles = (int) grid;
+    a.panelDiv = fast_div((uint32_t) a.panel);
+    a.perPanelDiv = fast_div((uint32_t) a.panel * (uint32_t) a.tokMain);
     auto run = [&](auto kernel, int threads) { return launch_tiles(stream, a, kernel, threads); };
     if constexpr (IL)
     {
