@@ -38,23 +38,25 @@ struct Vec16
     };
 };
 
-// Token of this wave: fills tokenIdx (row of ids and of the output) and pos (row of the
-// position table).  Returns false when the wave has nothing to do.
+// Token of a slot (of S * B < 2^31): fills tokenIdx (row of ids and of the output) and pos (row of the
+// position table).  Returns false when the slot is empty.  `inner` divides by B (kFIXED) or S.
 template <int MODE>
-__device__ inline bool locate_token(int64_t wave, int B, int S, int32_t const* cu, int64_t& tokenIdx, int& pos)
+__device__ inline bool locate_token(
+    uint32_t slot, int B, int S, FastDiv const& inner, int32_t const* cu, int64_t& tokenIdx, int& pos)
 {
-    if (wave >= (int64_t) S * B)
+    if (slot >= (uint32_t) S * (uint32_t) B)
     {
         return false;
     }
+    uint32_t const outer = slot / inner;
     if (MODE == kFIXED)
     {
-        tokenIdx = wave;
-        pos = (int) (wave / B);
+        tokenIdx = slot;
+        pos = (int) outer;
         return true;
     }
-    int const b = (int) (wave / S);
-    int const s = (int) (wave % S);
+    int const b = (int) outer;
+    int const s = (int) (slot - outer * inner.d);
     int const first = cu[b];
     int const len = cu[b + 1] - first;
     if (s >= len)
@@ -76,11 +78,19 @@ __device__ __forceinline__ void mask_idx(
         return;
     }
     int first = S;
-    for (int s = lane; s < S; s += kWaveSize)
+    constexpr int kAtOnce = 4; // values of a lane, requested together; behind the end the last one again
+    for (int s0 = lane; s0 < S; s0 += kAtOnce * kWaveSize)
     {
-        if (mask[(int64_t) s * B + b] == 0)
+        int32_t m[kAtOnce];
+#pragma unroll
+        for (int i = 0; i < kAtOnce; ++i)
         {
-            first = min(first, s);
+            m[i] = mask[(int64_t) min(s0 + i * kWaveSize, S - 1) * B + b];
+        }
+#pragma unroll
+        for (int i = 0; i < kAtOnce; ++i)
+        {
+            first = m[i] == 0 ? min(first, min(s0 + i * kWaveSize, S - 1)) : first;
         }
     }
     first = wave_min_i32(first);
@@ -99,7 +109,8 @@ __global__ __launch_bounds__(kBlock) void mask_idx_kernel(
 // Packed mask (embLayerNormKernel.cu:41-96): word (b, mi, tidx) holds, for each ni, the mask at
 // columns off, off+1, off, off+1, off+8, off+9, off+8, off+9 with
 // off = ni*16*warps_n + (tidx/32/warps_m)*16 + (tidx%4)*2; identical for every mi.
-// Columns at or beyond S count as masked.
+// Columns at or beyond S count as masked; xmmas_n is at most 4, and all values of a word are requested together (under the
+// condition k < S each, they were up to sixteen trips to memory, the longest chain of an embedding launch).
 __device__ __forceinline__ void convert_mask(uint32_t const bi, uint32_t const threads, uint32_t const warps_m,
     uint32_t const warps_n, uint32_t const S, uint32_t const B, uint32_t const xmmas_m, uint32_t const xmmas_n,
     int32_t const* __restrict__ maskSB, uint32_t* __restrict__ maskX)
@@ -107,12 +118,24 @@ __device__ __forceinline__ void convert_mask(uint32_t const bi, uint32_t const t
     uint32_t const tidx = threadIdx.x;
     uint32_t const warp_n = (tidx / 32) / warps_m;
     uint32_t const col = warp_n * 16 + (tidx % 4) * 2;
-    auto at = [&](uint32_t k) -> uint32_t { return (k < S && maskSB[(int64_t) k * B + bi] == 1) ? 1u : 0u; };
+    int32_t m[4][4];
+#pragma unroll
+    for (uint32_t ni = 0; ni < 4; ++ni)
+    {
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i)
+        {
+            uint32_t const k = ni * 16 * warps_n + col + (i >> 1) * 8 + (i & 1);
+            m[ni][i] = maskSB[(int64_t) min(k, S - 1) * B + bi];
+        }
+    }
     uint32_t word = 0;
-    for (uint32_t ni = 0; ni < xmmas_n; ++ni)
+#pragma unroll
+    for (uint32_t ni = 0; ni < 4; ++ni)
     {
         uint32_t const off = ni * 16 * warps_n + col;
-        uint32_t const m0 = at(off), m1 = at(off + 1), m8 = at(off + 8), m9 = at(off + 9);
+        auto at = [&](uint32_t i) -> uint32_t { return ni < xmmas_n && off + (i >> 1) * 8 + (i & 1) < S && m[ni][i] == 1 ? 1u : 0u; };
+        uint32_t const m0 = at(0), m1 = at(1), m8 = at(2), m9 = at(3);
         uint32_t const byte = m0 | (m1 << 1) | (m0 << 2) | (m1 << 3) | (m8 << 4) | (m9 << 5) | (m8 << 6) | (m9 << 7);
         word |= byte << (8 * ni);
     }
@@ -168,14 +191,19 @@ __device__ __forceinline__ void mask_workgroup(MaskJob const& job, uint32_t cons
 // bytes a token pulls through the vector cache.
 // With the plugin's mask output, whose workgroups come first (MaskJob): B = 32, S = 128, 768 channels FP16 takes 6.0 us
 // where the embedding and the mask as two launches took 9.5.
+// With one token slot per wavefront the trips to memory in a row set the time: the arguments are one, the ids the second,
+// and every row and vector the third; the position takes no division.
 template <typename T, int NV, int MODE, int TPW>
 __global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B, int const S,
     int32_t const* __restrict__ inputIds, int32_t const* __restrict__ tokenIds, int32_t const* __restrict__ cuSeqlens,
     float const* __restrict__ beta, float const* __restrict__ gamma, T const* __restrict__ wordEmb,
     T const* __restrict__ posEmb, T const* __restrict__ tokEmb, int32_t const wordSize, int32_t const tokSize,
-    T* __restrict__ output, T* __restrict__ skipOut, MaskJob const job)
+    T* __restrict__ output, T* __restrict__ skipOut, FastDiv const inner, MaskJob const job)
 {
     constexpr int VPT = Vec16<T>::kN;
+    asm volatile("" ::"s"(ld), "s"(B), "s"(S), "s"(inputIds), "s"(tokenIds), "s"(cuSeqlens), "s"(beta), "s"(gamma), "s"(wordEmb),
+                 "s"(posEmb), "s"(tokEmb), "s"(wordSize), "s"(tokSize), "s"(output), "s"(skipOut), "s"(inner.d), "s"(inner.mul),
+                 "s"(inner.shift1), "s"(inner.shift2), "s"(job.blocks));
     if constexpr (MODE == kFIXED)
     {
         if (blockIdx.x < job.blocks)
@@ -185,29 +213,42 @@ __global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B
         }
     }
     int const lane = threadIdx.x & (kWaveSize - 1);
-    int64_t const wave = __builtin_amdgcn_readfirstlane(
-        (int) ((int64_t) (blockIdx.x - (MODE == kFIXED ? job.blocks : 0u)) * kWavesPerBlock + (threadIdx.x >> 6)));
+    uint32_t const wave = (uint32_t) __builtin_amdgcn_readfirstlane(
+        (int) ((blockIdx.x - (MODE == kFIXED ? job.blocks : 0u)) * kWavesPerBlock + (threadIdx.x >> 6)));
     int const nvec = ld / VPT;
 
     // gamma/beta take the output type first: `const R g(gamma[i])`, common.cuh:275-276
+    f32x4 g4[NV][VPT / 4], b4[NV][VPT / 4];
     float gk[NV][VPT], bk[NV][VPT];
+    auto load_scales = [&] {
 #pragma unroll
-    for (int j = 0; j < NV; ++j)
-    {
-        int const vi = lane + kWaveSize * j;
-        bool const ok = vi < nvec;
-#pragma unroll
-        for (int q = 0; q < VPT / 4; ++q)
+        for (int j = 0; j < NV; ++j)
         {
-            f32x4 const g4 = ok ? *reinterpret_cast<f32x4 const*>(gamma + vi * VPT + q * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
-            f32x4 const b4 = ok ? *reinterpret_cast<f32x4 const*>(beta + vi * VPT + q * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+            int const c = lane + kWaveSize * j < nvec ? (lane + kWaveSize * j) * VPT : 0;
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
+            for (int q = 0; q < VPT / 4; ++q)
             {
-                gk[j][q * 4 + e] = (float) (T) g4[e];
-                bk[j][q * 4 + e] = (float) (T) b4[e];
+                g4[j][q] = *reinterpret_cast<f32x4 const*>(gamma + c + q * 4);
+                b4[j][q] = *reinterpret_cast<f32x4 const*>(beta + c + q * 4);
             }
         }
+    };
+    auto convert_scales = [&] {
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+        {
+#pragma unroll
+            for (int k = 0; k < VPT; ++k)
+            {
+                gk[j][k] = (float) (T) g4[j][k / 4][k % 4];
+                bk[j][k] = (float) (T) b4[j][k / 4][k % 4];
+            }
+        }
+    };
+    if constexpr (TPW > 1)
+    {
+        load_scales();
+        convert_scales();
     }
 
 #pragma unroll 1
@@ -215,7 +256,7 @@ __global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B
     {
         int64_t tokenIdx;
         int pos;
-        if (!locate_token<MODE>(wave * TPW + it, B, S, cuSeqlens, tokenIdx, pos))
+        if (!locate_token<MODE>(wave * TPW + (uint32_t) it, B, S, inner, cuSeqlens, tokenIdx, pos))
         {
             continue;
         }
@@ -224,14 +265,24 @@ __global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B
         bool const inRange = wordId >= 0 && wordId < wordSize && tokId >= 0 && tokId < tokSize;
 
         Vec16<T> w[NV], t[NV], p[NV];
+        if constexpr (TPW == 1)
+        {
+            load_scales();
+        }
 #pragma unroll
         for (int j = 0; j < NV; ++j)
         {
             int const vi = lane + kWaveSize * j;
-            bool const ok = vi < nvec && inRange;
-            w[j].u = ok ? *reinterpret_cast<u32x4 const*>(wordEmb + (int64_t) wordId * ld + vi * VPT) : u32x4{0, 0, 0, 0};
-            t[j].u = ok ? *reinterpret_cast<u32x4 const*>(tokEmb + (int64_t) tokId * ld + vi * VPT) : u32x4{0, 0, 0, 0};
-            p[j].u = ok ? *reinterpret_cast<u32x4 const*>(posEmb + (int64_t) pos * ld + vi * VPT) : u32x4{0, 0, 0, 0};
+            if (vi < nvec && inRange)
+            {
+                w[j].u = *reinterpret_cast<u32x4 const*>(wordEmb + (int64_t) wordId * ld + vi * VPT);
+                t[j].u = *reinterpret_cast<u32x4 const*>(tokEmb + (int64_t) tokId * ld + vi * VPT);
+                p[j].u = *reinterpret_cast<u32x4 const*>(posEmb + (int64_t) pos * ld + vi * VPT);
+            }
+            else
+            {
+                w[j].u = t[j].u = p[j].u = u32x4{0, 0, 0, 0};
+            }
         }
 
         float v[NV][VPT];
@@ -275,6 +326,10 @@ __global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B
         // No epsilon (plugin/common/common.cuh:269).  Ids out of range leave the reference's row
         // undefined; here such a row is the LayerNorm of zeros with rsigma forced to 0, i.e. beta.
         float const rsigma = inRange ? rsqrtf(st.m2 / (float) ld) : 0.f;
+        if constexpr (TPW == 1)
+        {
+            convert_scales();
+        }
 #pragma unroll
         for (int j = 0; j < NV; ++j)
         {
@@ -299,7 +354,7 @@ __global__ __launch_bounds__(kBlock) void embln_generic_kernel(int const ld, int
     int32_t const* __restrict__ inputIds, int32_t const* __restrict__ tokenIds, int32_t const* __restrict__ cuSeqlens,
     float const* __restrict__ beta, float const* __restrict__ gamma, T const* __restrict__ wordEmb,
     T const* __restrict__ posEmb, T const* __restrict__ tokEmb, int32_t const wordSize, int32_t const tokSize,
-    T* __restrict__ output, T* __restrict__ skipOut, MaskJob const job)
+    T* __restrict__ output, T* __restrict__ skipOut, FastDiv const inner, MaskJob const job)
 {
     if (blockIdx.x < job.blocks)
     {
@@ -307,11 +362,11 @@ __global__ __launch_bounds__(kBlock) void embln_generic_kernel(int const ld, int
         return;
     }
     int const lane = threadIdx.x & (kWaveSize - 1);
-    int64_t const wave = __builtin_amdgcn_readfirstlane(
-        (int) ((int64_t) (blockIdx.x - job.blocks) * kWavesPerBlock + (threadIdx.x >> 6)));
+    uint32_t const wave = (uint32_t) __builtin_amdgcn_readfirstlane(
+        (int) ((blockIdx.x - job.blocks) * kWavesPerBlock + (threadIdx.x >> 6)));
     int64_t tokenIdx;
     int pos;
-    if (!locate_token<MODE>(wave, B, S, cuSeqlens, tokenIdx, pos))
+    if (!locate_token<MODE>(wave, B, S, inner, cuSeqlens, tokenIdx, pos))
     {
         return;
     }
@@ -380,18 +435,19 @@ int emb_layer_norm(hipStream_t stream, int32_t ld, int32_t B, int32_t S, int32_t
     dim3 const grid((unsigned) ceil_div<int64_t>((int64_t) S * B, kWavesPerBlock) + job.blocks);
     // several tokens per wavefront once there are enough token slots to keep every SIMD busy anyway
     int64_t const slots = (int64_t) S * B;
+    FastDiv const inner = fast_div((uint32_t) (MODE == kFIXED ? B : S));
     bool const multi = slots >= 65536;
     dim3 const grid4((unsigned) ceil_div<int64_t>(ceil_div<int64_t>(slots, 4), kWavesPerBlock) + job.blocks);
 #define TRTAMD_EMB_LAUNCH(NVV)                                                                                         \
     if (multi)                                                                                                         \
     {                                                                                                                  \
         hipLaunchKernelGGL((embln_kernel<T, NVV, MODE, 4>), grid4, dim3(kBlock), 0, stream, ld, B, S, inputIds,          \
-            tokenIds, cuSeqlens, beta, gamma, wordEmb, posEmb, tokEmb, wordSize, tokSize, output, skipOut, job);            \
+            tokenIds, cuSeqlens, beta, gamma, wordEmb, posEmb, tokEmb, wordSize, tokSize, output, skipOut, inner, job);     \
     }                                                                                                                  \
     else                                                                                                               \
     {                                                                                                                  \
         hipLaunchKernelGGL((embln_kernel<T, NVV, MODE, 1>), grid, dim3(kBlock), 0, stream, ld, B, S, inputIds,           \
-            tokenIds, cuSeqlens, beta, gamma, wordEmb, posEmb, tokEmb, wordSize, tokSize, output, skipOut, job);            \
+            tokenIds, cuSeqlens, beta, gamma, wordEmb, posEmb, tokEmb, wordSize, tokSize, output, skipOut, inner, job);     \
     }
     if (vec_ok && nv == 1)
     {
@@ -408,7 +464,7 @@ int emb_layer_norm(hipStream_t stream, int32_t ld, int32_t B, int32_t S, int32_t
     else
     {
         hipLaunchKernelGGL((embln_generic_kernel<T, MODE>), grid, dim3(kBlock), 0, stream, ld, B, S, inputIds, tokenIds,
-            cuSeqlens, beta, gamma, wordEmb, posEmb, tokEmb, wordSize, tokSize, output, skipOut, job);
+            cuSeqlens, beta, gamma, wordEmb, posEmb, tokEmb, wordSize, tokSize, output, skipOut, inner, job);
     }
 #undef TRTAMD_EMB_LAUNCH
     return check_launch("embln_kernel");
