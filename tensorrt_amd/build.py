@@ -24,10 +24,12 @@ PLUGIN_CALL_NAME = "_plugin_call.so"              # CPython module: the plugins'
 OBJ_DIR = os.path.join(CSRC, "_obj")
 
 ARCH = "gfx950"
-# packed-fp32 code generation is switched off: hipcc -O3 otherwise forms v_pk_*_f32 by itself
+# packed-fp32 code generation is switched off: hipcc -O3 otherwise forms v_pk_*_f32 by itself.
+# The first 14 dwords of a kernel's arguments (all that fits beside the pointer to them) come in scalar registers with each
+# workgroup, up to the first that is a struct: without that every workgroup begins with a trip to memory for them.
 COMMON_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall", "-Wno-unused-function",
-    "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=14",
     f"-I{INCLUDE}", f"-I{CSRC}", f"-I{os.path.join(CSRC, 'plugin')}",
 ]
 

@@ -259,7 +259,7 @@ __device__ inline uint32_t xcd_remap(uint32_t bid, uint32_t nblocks)
 // 32-bit values (Granlund and Montgomery, "Division by Invariant Integers using Multiplication", figure 4.1).
 struct FastDiv
 {
-    uint32_t d, mul, shift1, shift2;
+    uint32_t d, mul, shifts; // the first shift (0 or 1) in bit 0, the second above it
 };
 
 inline FastDiv fast_div(uint32_t d)
@@ -269,13 +269,13 @@ inline FastDiv fast_div(uint32_t d)
     {
         ++l;
     }
-    return {d, (uint32_t) (((((uint64_t) 1 << l) - d) << 32) / d + 1u), l ? 1u : 0u, l ? l - 1u : 0u};
+    return {d, (uint32_t) (((((uint64_t) 1 << l) - d) << 32) / d + 1u), l ? 1u | (l - 1u) << 1 : 0u};
 }
 
 __host__ __device__ inline uint32_t operator/(uint32_t n, FastDiv const& v)
 {
     uint32_t const t = (uint32_t) ((uint64_t) n * v.mul >> 32);
-    return (t + ((n - t) >> v.shift1)) >> v.shift2;
+    return (t + ((n - t) >> (v.shifts & 1u))) >> (v.shifts >> 1);
 }
 
 // Which unit of work and which of its `parts` a workgroup takes when several workgroups share a unit's data (the

@@ -191,22 +191,20 @@ __device__ __forceinline__ void mask_workgroup(MaskJob const& job, uint32_t cons
 // bytes a token pulls through the vector cache.
 // With the plugin's mask output, whose workgroups come first (MaskJob): B = 32, S = 128, 768 channels FP16 takes 6.0 us
 // where the embedding and the mask as two launches took 9.5.
-// With one token slot per wavefront the trips to memory in a row set the time: the arguments are one, the ids the second,
-// and every row and vector the third; the position takes no division.
+// With one token slot per wavefront the trips to memory in a row set the time: the ids are one and every row and vector the
+// second, the arguments come preloaded or meanwhile, and the position takes no division.
 template <typename T, int NV, int MODE, int TPW>
-__global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B, int const S,
-    int32_t const* __restrict__ inputIds, int32_t const* __restrict__ tokenIds, int32_t const* __restrict__ cuSeqlens,
-    float const* __restrict__ beta, float const* __restrict__ gamma, T const* __restrict__ wordEmb,
-    T const* __restrict__ posEmb, T const* __restrict__ tokEmb, int32_t const wordSize, int32_t const tokSize,
-    T* __restrict__ output, T* __restrict__ skipOut, FastDiv const inner, MaskJob const job)
+__global__ __launch_bounds__(kBlock) void embln_kernel(uint32_t const maskBlocks, int const ld, int const B, int const S,
+    uint32_t const innerMul, uint32_t const innerShifts, int32_t const* __restrict__ inputIds,
+    int32_t const* __restrict__ tokenIds, int32_t const* __restrict__ cuSeqlens, float const* __restrict__ beta,
+    float const* __restrict__ gamma, T const* __restrict__ wordEmb, T const* __restrict__ posEmb, T const* __restrict__ tokEmb,
+    int32_t const wordSize, int32_t const tokSize, T* __restrict__ output, T* __restrict__ skipOut, MaskJob const job)
 {
     constexpr int VPT = Vec16<T>::kN;
-    asm volatile("" ::"s"(ld), "s"(B), "s"(S), "s"(inputIds), "s"(tokenIds), "s"(cuSeqlens), "s"(beta), "s"(gamma), "s"(wordEmb),
-                 "s"(posEmb), "s"(tokEmb), "s"(wordSize), "s"(tokSize), "s"(output), "s"(skipOut), "s"(inner.d), "s"(inner.mul),
-                 "s"(inner.shift1), "s"(inner.shift2), "s"(job.blocks));
+    FastDiv const inner{(uint32_t) (MODE == kFIXED ? B : S), innerMul, innerShifts};
     if constexpr (MODE == kFIXED)
     {
-        if (blockIdx.x < job.blocks)
+        if (blockIdx.x < maskBlocks)
         {
             mask_workgroup(job, (uint32_t) S, (uint32_t) B);
             return;
@@ -214,7 +212,7 @@ __global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B
     }
     int const lane = threadIdx.x & (kWaveSize - 1);
     uint32_t const wave = (uint32_t) __builtin_amdgcn_readfirstlane(
-        (int) ((blockIdx.x - (MODE == kFIXED ? job.blocks : 0u)) * kWavesPerBlock + (threadIdx.x >> 6)));
+        (int) ((blockIdx.x - (MODE == kFIXED ? maskBlocks : 0u)) * kWavesPerBlock + (threadIdx.x >> 6)));
     int const nvec = ld / VPT;
 
     // gamma/beta take the output type first: `const R g(gamma[i])`, common.cuh:275-276
@@ -260,8 +258,13 @@ __global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B
         {
             continue;
         }
-        int const wordId = __builtin_amdgcn_readfirstlane(inputIds[tokenIdx]);
-        int const tokId = __builtin_amdgcn_readfirstlane(tokenIds[tokenIdx]);
+        int const wordAt = inputIds[tokenIdx], tokAt = tokenIds[tokenIdx];
+        __builtin_amdgcn_sched_barrier(0);
+        // the arguments that do not come preloaded, while the ids are on their way
+        asm volatile("" ::"s"(beta), "s"(gamma), "s"(wordEmb), "s"(posEmb), "s"(tokEmb), "s"(wordSize), "s"(tokSize), "s"(output),
+                     "s"(skipOut));
+        int const wordId = __builtin_amdgcn_readfirstlane(wordAt);
+        int const tokId = __builtin_amdgcn_readfirstlane(tokAt);
         bool const inRange = wordId >= 0 && wordId < wordSize && tokId >= 0 && tokId < tokSize;
 
         Vec16<T> w[NV], t[NV], p[NV];
@@ -285,6 +288,10 @@ __global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B
             }
         }
 
+        if constexpr (TPW == 1)
+        {
+            convert_scales();
+        }
         float v[NV][VPT];
         float sum = 0.f, cnt = 0.f;
 #pragma unroll
@@ -326,10 +333,6 @@ __global__ __launch_bounds__(kBlock) void embln_kernel(int const ld, int const B
         // No epsilon (plugin/common/common.cuh:269).  Ids out of range leave the reference's row
         // undefined; here such a row is the LayerNorm of zeros with rsigma forced to 0, i.e. beta.
         float const rsigma = inRange ? rsqrtf(st.m2 / (float) ld) : 0.f;
-        if constexpr (TPW == 1)
-        {
-            convert_scales();
-        }
 #pragma unroll
         for (int j = 0; j < NV; ++j)
         {
@@ -441,13 +444,15 @@ int emb_layer_norm(hipStream_t stream, int32_t ld, int32_t B, int32_t S, int32_t
 #define TRTAMD_EMB_LAUNCH(NVV)                                                                                         \
     if (multi)                                                                                                         \
     {                                                                                                                  \
-        hipLaunchKernelGGL((embln_kernel<T, NVV, MODE, 4>), grid4, dim3(kBlock), 0, stream, ld, B, S, inputIds,          \
-            tokenIds, cuSeqlens, beta, gamma, wordEmb, posEmb, tokEmb, wordSize, tokSize, output, skipOut, inner, job);     \
+        hipLaunchKernelGGL((embln_kernel<T, NVV, MODE, 4>), grid4, dim3(kBlock), 0, stream, job.blocks, ld, B, S, \
+            inner.mul, inner.shifts, inputIds, tokenIds, cuSeqlens, beta, gamma, wordEmb, posEmb, tokEmb, wordSize, tokSize, \
+            output, skipOut, job);                                                                                     \
     }                                                                                                                  \
     else                                                                                                               \
     {                                                                                                                  \
-        hipLaunchKernelGGL((embln_kernel<T, NVV, MODE, 1>), grid, dim3(kBlock), 0, stream, ld, B, S, inputIds,           \
-            tokenIds, cuSeqlens, beta, gamma, wordEmb, posEmb, tokEmb, wordSize, tokSize, output, skipOut, inner, job);     \
+        hipLaunchKernelGGL((embln_kernel<T, NVV, MODE, 1>), grid, dim3(kBlock), 0, stream, job.blocks, ld, B, S, \
+            inner.mul, inner.shifts, inputIds, tokenIds, cuSeqlens, beta, gamma, wordEmb, posEmb, tokEmb, wordSize, tokSize, \
+            output, skipOut, job);                                                                                     \
     }
     if (vec_ok && nv == 1)
     {

@@ -146,9 +146,8 @@ __device__ __forceinline__ void pin_args(FmhaArgs const& a)
 {
     asm volatile("" ::"s"(a.qkv), "s"(a.out), "s"(a.cuSeqlens), "s"(a.packedMask), "s"(a.tokStrideIn), "s"(a.tokStrideOut),
                  "s"(a.seqStrideIn), "s"(a.seqStrideOut), "s"(a.B), "s"(a.S), "s"(a.total), "s"(a.c), "s"(a.scaleBmm2),
-                 "s"(a.ranked), "s"(gridDim.x), "s"(a.partDiv.d), "s"(a.partDiv.mul), "s"(a.partDiv.shift1),
-                 "s"(a.partDiv.shift2), "s"(a.spanDiv.d), "s"(a.spanDiv.mul), "s"(a.spanDiv.shift1), "s"(a.spanDiv.shift2),
-                 "s"(a.headDiv.d), "s"(a.headDiv.mul), "s"(a.headDiv.shift1), "s"(a.headDiv.shift2));
+                 "s"(a.ranked), "s"(gridDim.x), "s"(a.partDiv.d), "s"(a.partDiv.mul), "s"(a.partDiv.shifts), "s"(a.spanDiv.d), "s"(a.spanDiv.mul), "s"(a.spanDiv.shifts),
+                 "s"(a.headDiv.d), "s"(a.headDiv.mul), "s"(a.headDiv.shifts));
 }
 
 template <int ESIZE>
@@ -1208,7 +1207,7 @@ __global__ __launch_bounds__(kWavesI8* kWaveSize) __attribute__((amdgpu_waves_pe
     uint8_t* sV = smem + Lds<1>::matBytes(KT);
     __shared__ PickLds sPick;
     pin_args(a);
-    asm volatile("" ::"s"(a.turnDiv.d), "s"(a.turnDiv.mul), "s"(a.turnDiv.shift1), "s"(a.turnDiv.shift2));
+    asm volatile("" ::"s"(a.turnDiv.d), "s"(a.turnDiv.mul), "s"(a.turnDiv.shifts));
     UnitPart up = unit_of_workgroup(blockIdx.x, gridDim.x, a.partDiv, a.spanDiv);
     if (!INTERLEAVED && a.qSplit == 1 && (a.N & 1) == 0)
     {

@@ -1578,8 +1578,8 @@ __global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(Line
     __shared__ __attribute__((aligned(1024))) uint8_t lds[kRing + (scales_late(kRing) ? 0 : 2 * kBigTile * 4)];
     // all arguments in one trip of the scalar loads, as in the piece kernels
     asm volatile("" ::"s"(p.a), "s"(p.w), "s"(p.alpha), "s"(p.beta), "s"(p.out), "s"(p.T), "s"(p.K), "s"(p.N), "s"(p.mainTiles),
-                 "s"(p.panelDiv.d), "s"(p.panelDiv.mul), "s"(p.panelDiv.shift1), "s"(p.panelDiv.shift2), "s"(p.perPanelDiv.d),
-                 "s"(p.perPanelDiv.mul), "s"(p.perPanelDiv.shift1), "s"(p.perPanelDiv.shift2));
+                 "s"(p.panelDiv.d), "s"(p.panelDiv.mul), "s"(p.panelDiv.shifts), "s"(p.perPanelDiv.d),
+                 "s"(p.perPanelDiv.mul), "s"(p.perPanelDiv.shifts));
     if constexpr (IL)
     {
         if ((int) blockIdx.x >= p.mainTiles)

@@ -39,18 +39,14 @@ struct Vec16
 // The residual sum is formed in T like the reference (skipLayerNormKernel.cu:121-134);
 // statistics are a Welford/Chan merge in binary32; epsilon is the caller's.
 // ------------------------------------------------------------------------------------------
-// FEW: a launch bound by the trips to memory in a row, not by the bytes.  All arguments come in one trip and all of a
-// wavefront's loads in a second (the conditions of the other form made up to five and three of them).
+// FEW: a launch bound by the trips to memory in a row, not by the bytes.  All of a wavefront's loads are one trip (the
+// conditions of the other form made three of them), and what they need of the arguments comes preloaded.
 template <typename T, int NV, int R, bool HAS_BIAS, bool FEW>
 __global__ __launch_bounds__(kBlock) void skipln_rows_kernel(int const ld, int64_t const rows, T const* __restrict__ in,
     T const* __restrict__ skip, T const* __restrict__ beta, T const* __restrict__ gamma, T const* __restrict__ bias,
     T* __restrict__ out, float const eps)
 {
     constexpr int VPT = Vec16<T>::kN;
-    if constexpr (FEW)
-    {
-        asm volatile("" ::"s"(ld), "s"(rows), "s"(in), "s"(skip), "s"(beta), "s"(gamma), "s"(bias), "s"(out), "s"(eps));
-    }
     int const lane = threadIdx.x & (kWaveSize - 1);
     int64_t const wave = (int64_t) blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
     int64_t const row0 = wave * R;
@@ -79,6 +75,7 @@ __global__ __launch_bounds__(kBlock) void skipln_rows_kernel(int const ld, int64
             }
         }
         __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::"s"(out), "s"(eps)); // behind the arguments that come preloaded: requested together, below the loads
     }
     else
     {
@@ -320,25 +317,15 @@ int skip_layer_norm(hipStream_t stream, int32_t ld, int64_t n, T const* in, T co
     return check_launch("skipln_generic_kernel");
 }
 
-// The output of an affine linear layer as the partial sums of its accumulators (network_ops.hpp).
-template <typename Acc>
-struct PartialSums
-{
-    Acc const* sums; // [parts][rows][ld]
-    int parts;
-    float const* alpha;
-    float const* beta;
-};
-
-// The same rows (binary16, one per wavefront) behind a linear layer that left partial sums: its output is formed here as
-// that layer's epilogue forms it, f16(fmaf(sum, alpha, beta)), and never stored.  ld a multiple of 8, at most 1024.
+// The same rows (binary16, one per wavefront) behind a linear layer that left partial sums [parts][rows][ld]
+// (network_ops.hpp): its output is formed here as that layer's epilogue forms it, f16(fmaf(sum, alpha, beta)), and never
+// stored.  ld a multiple of 8, at most 1024.
 template <int NV>
-__global__ __launch_bounds__(kBlock) void skipln_rows_partial_kernel(int const ld, int const rows,
-    PartialSums<float> const sums, f16 const* __restrict__ skip, f16 const* __restrict__ beta, f16 const* __restrict__ gamma,
-    f16 const* __restrict__ bias, f16* __restrict__ out, float const eps)
+__global__ __launch_bounds__(kBlock) void skipln_rows_partial_kernel(int const ld, int const rows, float const* __restrict__ sums,
+    float const* __restrict__ alpha, float const* __restrict__ linearBeta, f16 const* __restrict__ skip,
+    f16 const* __restrict__ bias, int const parts, f16 const* __restrict__ beta, f16 const* __restrict__ gamma,
+    f16* __restrict__ out, float const eps)
 {
-    asm volatile("" ::"s"(ld), "s"(rows), "s"(sums.sums), "s"(sums.parts), "s"(sums.alpha), "s"(sums.beta), "s"(skip), "s"(beta),
-                 "s"(gamma), "s"(bias), "s"(out), "s"(eps));
     int const lane = threadIdx.x & (kWaveSize - 1);
     int const row = (int) blockIdx.x * kWavesPerBlock + (int) (threadIdx.x >> 6);
     if (row >= rows)
@@ -360,13 +347,20 @@ __global__ __launch_bounds__(kBlock) void skipln_rows_partial_kernel(int const l
             for (int s = 0; s < kMaxLinearParts; ++s)
             {
                 sum4[j][s][h] = *reinterpret_cast<f32x4 const*>(
-                    sums.sums + ((int64_t) min(s, sums.parts - 1) * rows + row) * ld + c + 4 * h);
+                    sums + ((int64_t) min(s, parts - 1) * rows + row) * ld + c + 4 * h);
             }
-            al[j][h] = *reinterpret_cast<f32x4 const*>(sums.alpha + c + 4 * h);
-            be[j][h] = *reinterpret_cast<f32x4 const*>(sums.beta + c + 4 * h);
+            al[j][h] = *reinterpret_cast<f32x4 const*>(alpha + c + 4 * h);
+            be[j][h] = *reinterpret_cast<f32x4 const*>(linearBeta + c + 4 * h);
         }
         xs[j].u = *reinterpret_cast<u32x4 const*>(skip + (int64_t) row * ld + c);
         bs[j].u = *reinterpret_cast<u32x4 const*>(bias + c);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::"s"(beta), "s"(gamma), "s"(out), "s"(eps)); // the arguments that do not come preloaded
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+    {
+        int const c = lane + kWaveSize * j < nvec ? (lane + kWaveSize * j) * 8 : 0;
         g[j].u = *reinterpret_cast<u32x4 const*>(gamma + c);
         b[j].u = *reinterpret_cast<u32x4 const*>(beta + c);
     }
@@ -382,7 +376,7 @@ __global__ __launch_bounds__(kBlock) void skipln_rows_partial_kernel(int const l
 #pragma unroll
             for (int s = 1; s < kMaxLinearParts; ++s)
             {
-                x[j][h] += s < sums.parts ? sum4[j][s][h] : f32x4{0.f, 0.f, 0.f, 0.f};
+                x[j][h] += s < parts ? sum4[j][s][h] : f32x4{0.f, 0.f, 0.f, 0.f};
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e)
@@ -632,8 +626,6 @@ __global__ __launch_bounds__(W * kWaveSize) void skipln_interleaved_kernel(int c
     constexpr int SUBS = kWaveSize / LPG;      // channel groups per load instruction
     constexpr int NI = G / (SUBS * W);
     static_assert(G % (SUBS * W) == 0 && NI <= 8, "every lane keeps its part of the row in registers");
-    asm volatile("" ::"s"(total), "s"(gridDim.x), "s"(in), "s"(skip), "s"(beta), "s"(gamma), "s"(out), "s"(preln), "s"(dqIn),
-                 "s"(dqSkip), "s"(qScale), "s"(eps));
     __shared__ float sGamma[LD];
     __shared__ float sBeta[LD];
     __shared__ int sStat[W][TOK][5];
@@ -643,7 +635,8 @@ __global__ __launch_bounds__(W * kWaveSize) void skipln_interleaved_kernel(int c
     int const sub = lane / LPG;
     int const tok = (lane % LPG) >> 1;
     int const hf = lane & 1;
-    uint32_t const block = token_block_of_workgroup(blockIdx.x, gridDim.x);
+    uint32_t const blocks = TAIL ? gridDim.x : ((uint32_t) total + TOK - 1) / TOK; // not an argument that comes preloaded
+    uint32_t const block = token_block_of_workgroup(blockIdx.x, blocks);
     int64_t const tRaw = (int64_t) block * TOK + tok;
     bool const valid = tRaw < total;
     // lanes past the last token re-read the last token (and store nothing): no divergent loads
@@ -666,7 +659,7 @@ __global__ __launch_bounds__(W * kWaveSize) void skipln_interleaved_kernel(int c
     // vector registers held), and normalises it after the block.
     constexpr int kExtraLoads = (G + 31) / 32; // load instructions per tensor: 32 channel groups x 2 halves each
     __shared__ __attribute__((aligned(16))) uint8_t sExtra[2][TAIL ? kExtraLoads * 1024 : 16];
-    int64_t const extraTok = (int64_t) gridDim.x * TOK + block;
+    int64_t const extraTok = (int64_t) blocks * TOK + block;
     bool const hasExtra = TAIL && extraTok < total; // the same for every lane of the workgroup
     if (TAIL && hasExtra && wave == 0)
     {
@@ -905,8 +898,6 @@ __global__ __launch_bounds__(kBlock) void skipln_interleaved_token_kernel(int co
 {
     constexpr int LD = G * 32;
     constexpr int NE = (G + 31) / 32; // loads per tensor and lane: 32 channel groups x 2 halves each
-    asm volatile("" ::"s"(total), "s"(in), "s"(skip), "s"(beta), "s"(gamma), "s"(out), "s"(preln), "s"(dqIn), "s"(dqSkip),
-                 "s"(qScale), "s"(eps));
     int const lane = threadIdx.x & (kWaveSize - 1);
     int const hf = lane & 1;
     int const token = (int) blockIdx.x * kWavesPerBlock + (int) (threadIdx.x >> 6);
@@ -938,6 +929,7 @@ __global__ __launch_bounds__(kBlock) void skipln_interleaved_token_kernel(int co
         }
     }
     __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::"s"(dqIn), "s"(dqSkip), "s"(qScale), "s"(eps)); // the arguments that do not come preloaded
     int sIn = 0, sSk = 0, sII = 0, sIS = 0, sSS = 0;
 #pragma unroll
     for (int e = 0; e < NE; ++e)
@@ -1018,14 +1010,13 @@ __global__ __launch_bounds__(kBlock) void skipln_interleaved_token_kernel(int co
 // all parts, 16 bytes per thread each, are one trip to memory; with a wavefront per token and 16 channels per lane as above
 // the launch took 4.7 us at 32 tokens and four parts.
 template <int G>
-__global__ __launch_bounds__(G * 8) void skipln_interleaved_sums_kernel(int const total, PartialSums<int32_t> const sums,
+__global__ __launch_bounds__(G * 8) void skipln_interleaved_sums_kernel(int const total, int const parts,
+    int32_t const* __restrict__ sums, float const* __restrict__ alpha, float const* __restrict__ linearBeta,
     int8_t const* __restrict__ skip, f16 const* __restrict__ beta, f16 const* __restrict__ gamma, int8_t* __restrict__ out,
     float const dqIn, float const dqSkip, float const qScale, float const eps)
 {
     constexpr int LD = G * 32, WAVES = G / 8;
     __shared__ int sStat[WAVES][5];
-    asm volatile("" ::"s"(total), "s"(sums.sums), "s"(sums.parts), "s"(sums.alpha), "s"(sums.beta), "s"(skip), "s"(beta),
-                 "s"(gamma), "s"(out), "s"(dqIn), "s"(dqSkip), "s"(qScale), "s"(eps));
     int const token = (int) blockIdx.x;
     int const wave = (int) (threadIdx.x >> 6);
     int const ch = (int) threadIdx.x * 4;
@@ -1035,18 +1026,20 @@ __global__ __launch_bounds__(G * 8) void skipln_interleaved_sums_kernel(int cons
     for (int s = 0; s < kMaxLinearParts; ++s)
     {
         // a part that does not exist re-reads the last one
-        v[s] = *reinterpret_cast<i32x4 const*>(sums.sums + ((int64_t) min(s, sums.parts - 1) * total + token) * LD + ch);
+        v[s] = *reinterpret_cast<i32x4 const*>(sums + ((int64_t) min(s, parts - 1) * total + token) * LD + ch);
     }
     uint32_t const xs = *reinterpret_cast<uint32_t const*>(skip + off);
-    f32x4 const al = *reinterpret_cast<f32x4 const*>(sums.alpha + ch);
-    f32x4 const be = *reinterpret_cast<f32x4 const*>(sums.beta + ch);
+    f32x4 const al = *reinterpret_cast<f32x4 const*>(alpha + ch);
+    f32x4 const be = *reinterpret_cast<f32x4 const*>(linearBeta + ch);
     f16x4 const g = *reinterpret_cast<f16x4 const*>(gamma + ch);
     f16x4 const b = *reinterpret_cast<f16x4 const*>(beta + ch);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::"s"(out), "s"(dqIn), "s"(dqSkip), "s"(qScale), "s"(eps)); // the arguments that do not come preloaded
     i32x4 acc = v[0];
 #pragma unroll
     for (int s = 1; s < kMaxLinearParts; ++s)
     {
-        acc += s < sums.parts ? v[s] : i32x4{0, 0, 0, 0};
+        acc += s < parts ? v[s] : i32x4{0, 0, 0, 0};
     }
     uint32_t xi = 0;
 #pragma unroll
@@ -1227,11 +1220,10 @@ int skipln_interleaved_from_partial(trtamd_stream_t stream, bool large, int32_t 
     {
         return set_error(TRTAMD_STATUS_NOT_SUPPORTED, "SkipLayerNorm from partial sums: unsupported problem");
     }
-    PartialSums<int32_t> const sums{partial, parts, alpha, beta};
     float const eps = large ? 1.1920928955078125e-07f : 0.0009765625f;
     auto const launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned) total), dim3((unsigned) ld / 4), 0, as_stream(stream), total, sums, skip,
-            reinterpret_cast<f16 const*>(lnBeta), reinterpret_cast<f16 const*>(lnGamma), output, dqScaleIn, dqScaleSkip, qScale,
+        hipLaunchKernelGGL(kernel, dim3((unsigned) total), dim3((unsigned) ld / 4), 0, as_stream(stream), total, parts, partial,
+            alpha, beta, skip, reinterpret_cast<f16 const*>(lnBeta), reinterpret_cast<f16 const*>(lnGamma), output, dqScaleIn, dqScaleSkip, qScale,
             eps);
         return check_launch("skipln_interleaved_sums_kernel");
     };
@@ -1246,12 +1238,11 @@ int skip_layer_norm_fp16_from_partial(trtamd_stream_t stream, int32_t ld, int32_
     {
         return set_error(TRTAMD_STATUS_NOT_SUPPORTED, "SkipLayerNorm from partial sums: unsupported problem");
     }
-    PartialSums<float> const sums{partial, parts, alpha, beta};
     float const eps = (ld == 768 || ld == 1024) ? 0.0009765625f : 0.f; // as skip_layer_norm
     auto const half = [](trtamd_half_t const* x) { return reinterpret_cast<f16 const*>(x); };
     auto const launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned) ceil_div(rows, kWavesPerBlock)), dim3(kBlock), 0, as_stream(stream), ld, rows,
-            sums, half(skip), half(lnBeta), half(lnGamma), half(bias), reinterpret_cast<f16*>(output), eps);
+            partial, alpha, beta, half(skip), half(bias), parts, half(lnBeta), half(lnGamma), reinterpret_cast<f16*>(output), eps);
         return check_launch("skipln_rows_partial_kernel");
     };
     return ld <= 512 ? launch(skipln_rows_partial_kernel<1>) : launch(skipln_rows_partial_kernel<2>);
