@@ -305,15 +305,15 @@ __device__ inline UnitPart unit_of_workgroup(uint32_t bid, uint32_t nblocks, int
     return {bid / q, (int) (bid % q)};
 }
 
-// The same with the divisors at hand: `span` is 8 * parts.
-__device__ inline UnitPart unit_of_workgroup(uint32_t bid, uint32_t nblocks, FastDiv const& parts, FastDiv const& span)
+// The same with the divisor at hand.
+__device__ inline UnitPart unit_of_workgroup(uint32_t bid, uint32_t nblocks, FastDiv const& parts)
 {
     if (parts.d <= 1)
     {
         return {bid, 0};
     }
-    uint32_t const m = bid / span, x = bid - m * span.d;
-    if ((m + 1) * span.d <= nblocks)
+    uint32_t const span = 8u * parts.d, m = (bid >> 3) / parts, x = bid - m * span;
+    if ((m + 1) * span <= nblocks)
     {
         return {m * 8u + x % 8u, (int) (x / 8u)};
     }

@@ -28,8 +28,8 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
-#include <type_traits>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace trtamd
@@ -136,18 +136,42 @@ struct FmhaArgs
     int32_t* dbgAcc1;            // optional [B][N][S][S] int32 (INT8) / float bits (FP16)
     int8_t* dbgP8;               // optional [B][N][S][S]
     int32_t ranked;              // serve the longest sequences first (pointless when one round holds every workgroup)
-    FastDiv partDiv, spanDiv;    // by qSplit and 8 qSplit (unit_of_workgroup)
-    FastDiv headDiv, turnDiv;    // by N and kWavesI8 qSplit
+    FastDiv partDiv, headDiv;    // by qSplit and N
 };
 
-// Asks for what the cu_seqlens kernels read of their arguments at once: left to the first uses, the trips of the scalar
-// loads stand one behind the other ahead of a workgroup's first request.
+// The arguments of the cu_seqlens kernels: what a workgroup needs to find its sequence comes preloaded, as the leading scalars
+// of the argument list, ...
+#define TRTAMD_FMHA_LEADING_PARAMS                                                                                     \
+    void const *qkv, int32_t const *cuSeqlens, uint32_t const qSplit, uint32_t const qSplitMul,                        \
+        uint32_t const qSplitShifts, uint32_t const N, uint32_t const headMul, uint32_t const headShifts, int const B, \
+        int const S, int const ranked, int const total
+#define TRTAMD_FMHA_LEADING_ARGS(a)                                                                                    \
+    (a).qkv, (a).cuSeqlens, (a).partDiv.d, (a).partDiv.mul, (a).partDiv.shifts, (a).headDiv.d, (a).headDiv.mul,        \
+        (a).headDiv.shifts, (a).B, (a).S, (a).ranked, (a).total
+#define TRTAMD_FMHA_ARGS_OF(rest)                                                                                      \
+    fmha_args(qkv, cuSeqlens, {qSplit, qSplitMul, qSplitShifts}, {N, headMul, headShifts}, B, S, ranked, total, rest)
+__device__ __forceinline__ FmhaArgs fmha_args(void const* qkv, int32_t const* cuSeqlens, FastDiv const& partDiv,
+    FastDiv const& headDiv, int B, int S, int ranked, int total, FmhaArgs const& rest)
+{
+    FmhaArgs a = rest;
+    a.qkv = qkv;
+    a.cuSeqlens = cuSeqlens;
+    a.partDiv = partDiv;
+    a.headDiv = headDiv;
+    a.qSplit = (int) partDiv.d;
+    a.N = (int) headDiv.d;
+    a.B = B;
+    a.S = S;
+    a.ranked = ranked;
+    a.total = total;
+    return a;
+}
+
+// ... and the others are requested together while the bounds of the sequence are on their way.
 __device__ __forceinline__ void pin_args(FmhaArgs const& a)
 {
-    asm volatile("" ::"s"(a.qkv), "s"(a.out), "s"(a.cuSeqlens), "s"(a.packedMask), "s"(a.tokStrideIn), "s"(a.tokStrideOut),
-                 "s"(a.seqStrideIn), "s"(a.seqStrideOut), "s"(a.B), "s"(a.S), "s"(a.total), "s"(a.c), "s"(a.scaleBmm2),
-                 "s"(a.ranked), "s"(gridDim.x), "s"(a.partDiv.d), "s"(a.partDiv.mul), "s"(a.partDiv.shifts), "s"(a.spanDiv.d), "s"(a.spanDiv.mul), "s"(a.spanDiv.shifts),
-                 "s"(a.headDiv.d), "s"(a.headDiv.mul), "s"(a.headDiv.shifts));
+    asm volatile("" ::"s"(a.out), "s"(a.packedMask), "s"(a.tokStrideIn), "s"(a.tokStrideOut), "s"(a.seqStrideIn),
+                 "s"(a.seqStrideOut), "s"(a.c), "s"(a.scaleBmm2));
 }
 
 template <int ESIZE>
@@ -334,8 +358,9 @@ __device__ inline SeqInfo seq_info(FmhaArgs const& a, int b, int capacity)
     SeqInfo s;
     if (a.cuSeqlens)
     {
-        int const first = a.cuSeqlens[b];
-        int const len = min(max(a.cuSeqlens[b + 1] - first, 0), capacity);
+        int const first = a.cuSeqlens[b], end = a.cuSeqlens[b + 1];
+        pin_args(a);
+        int const len = min(max(end - first, 0), capacity);
         s.firstTok = first;
         s.seqBaseIn = (int64_t) first * a.tokStrideIn;
         s.seqBaseOut = (int64_t) first * a.tokStrideOut;
@@ -719,6 +744,7 @@ __device__ inline SeqInfo pick_sequence_in_registers(FmhaArgs const& a, int rank
         first[i] = a.cuSeqlens[t];
         end[i] = a.cuSeqlens[t + 1];
     }
+    pin_args(a);
 #pragma unroll
     for (int i = 0; i < kPicksPerLane; ++i)
     {
@@ -1200,20 +1226,20 @@ __device__ __forceinline__ void attend_i8(FmhaArgs const& a, SeqInfo const& sq, 
 
 // MASKED: the keys come from a packed mask (a kernel of its own: the other one keeps its registers).
 template <int KT, bool INTERLEAVED, bool DEBUG, bool MASKED = false>
-__global__ __launch_bounds__(kWavesI8* kWaveSize) __attribute__((amdgpu_waves_per_eu(KT <= 6 ? 3 : 2))) void fmha_i8_prefix_kernel(FmhaArgs const a)
+__global__ __launch_bounds__(kWavesI8* kWaveSize) __attribute__((amdgpu_waves_per_eu(KT <= 6 ? 3 : 2))) void fmha_i8_prefix_kernel(
+    TRTAMD_FMHA_LEADING_PARAMS, FmhaArgs const rest)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     uint8_t* sK = smem;
     uint8_t* sV = smem + Lds<1>::matBytes(KT);
     __shared__ PickLds sPick;
-    pin_args(a);
-    asm volatile("" ::"s"(a.turnDiv.d), "s"(a.turnDiv.mul), "s"(a.turnDiv.shifts));
-    UnitPart up = unit_of_workgroup(blockIdx.x, gridDim.x, a.partDiv, a.spanDiv);
+    FmhaArgs const a = TRTAMD_FMHA_ARGS_OF(rest);
+    UnitPart up = unit_of_workgroup(blockIdx.x, B * N * qSplit, a.partDiv);
     if (!INTERLEAVED && a.qSplit == 1 && (a.N & 1) == 0)
     {
         // Linear layout ([token][head][Q K V][64 bytes]): V of head n and Q of head n + 1 lie in one 128-byte line, so
         // the two heads of a pair go to one XCD (18239 tokens x 16 heads: 36.2 -> 35.2 us)
-        UnitPart const pair = unit_of_workgroup(blockIdx.x, gridDim.x, 2);
+        UnitPart const pair = unit_of_workgroup(blockIdx.x, B * N * qSplit, 2);
         up.unit = pair.unit * 2u + (uint32_t) pair.part;
     }
     int const part = up.part;
@@ -1223,7 +1249,7 @@ __global__ __launch_bounds__(kWavesI8* kWaveSize) __attribute__((amdgpu_waves_pe
     SeqInfo sq = pick_sequence_info<kWavesI8 * kWaveSize>(a, (int) rank, KT * 64, sPick, b);
     // contiguous tile ranges, each a multiple of one round of the workgroup's wavefronts
     int const nqt = (sq.nq + kQPerWave - 1) / kQPerWave;
-    int const per = kWavesI8 * (int) ((uint32_t) (nqt + (int) a.turnDiv.d - 1) / a.turnDiv);
+    int const per = kWavesI8 * (int) ((uint32_t) ((nqt + kWavesI8 * a.qSplit - 1) / kWavesI8) / a.partDiv);
     int const qtBegin = min(part * per, nqt);
     int const qtEnd = min(qtBegin + per, nqt);
     if (qtBegin >= qtEnd)
@@ -1791,12 +1817,13 @@ __device__ __forceinline__ void attend_f16_turns(
 
 template <int KT, bool DEBUG>
 __global__ __launch_bounds__(kWavesF16T* kWaveSize)
-    __attribute__((amdgpu_waves_per_eu(KT <= 4 ? 4 : KT <= 6 ? 3 : 2))) void fmha_f16_turns_kernel(FmhaArgs const a)
+    __attribute__((amdgpu_waves_per_eu(KT <= 4 ? 4 : KT <= 6 ? 3 : 2))) void fmha_f16_turns_kernel(
+    TRTAMD_FMHA_LEADING_PARAMS, FmhaArgs const rest)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     __shared__ PickLds sPick;
-    pin_args(a);
-    UnitPart const up = unit_of_workgroup(blockIdx.x, gridDim.x, a.partDiv, a.spanDiv);
+    FmhaArgs const a = TRTAMD_FMHA_ARGS_OF(rest);
+    UnitPart const up = unit_of_workgroup(blockIdx.x, B * N * qSplit, a.partDiv);
     uint32_t const rank = up.unit / a.headDiv;
     int const n = __builtin_amdgcn_readfirstlane((int) (up.unit - rank * a.headDiv.d));
     int const q0 = __builtin_amdgcn_readfirstlane(up.part) * kQueriesF16;
@@ -1870,15 +1897,15 @@ constexpr int kStreamLds = 2 * kStreamStage;
 
 template <bool DEBUG>
 __global__ __launch_bounds__(kWavesStream* kWaveSize) __attribute__((amdgpu_waves_per_eu(4))) void fmha_f16_stream_kernel(
-    FmhaArgs const a, int const capacity)
+    TRTAMD_FMHA_LEADING_PARAMS, FmhaArgs const rest, int const capacity)
 {
     constexpr int kRow = Lds<2>::kRow;
     constexpr int kLoads = 2 * 8 / kWavesStream; // direct loads per wavefront and block: 8 rows each, of K and of V
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ PickLds sPick;
     __shared__ uint64_t sMask[8];
-    pin_args(a);
-    UnitPart const up = unit_of_workgroup(blockIdx.x, gridDim.x, a.partDiv, a.spanDiv);
+    FmhaArgs const a = TRTAMD_FMHA_ARGS_OF(rest);
+    UnitPart const up = unit_of_workgroup(blockIdx.x, B * N * qSplit, a.partDiv);
     uint32_t const rank = up.unit / a.headDiv;
     int const n = __builtin_amdgcn_readfirstlane((int) (up.unit - rank * a.headDiv.d));
     int b;
@@ -2215,7 +2242,14 @@ int launch_fmha(K kernel, char const* name, hipStream_t stream, FmhaArgs const& 
         return st;
     }
     unsigned const blocks = (unsigned) args.B * args.N * args.qSplit;
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(waves * kWaveSize), ldsBytes, stream, args);
+    if constexpr (std::is_invocable_v<K, FmhaArgs>)
+    {
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(waves * kWaveSize), ldsBytes, stream, args);
+    }
+    else
+    {
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(waves * kWaveSize), ldsBytes, stream, TRTAMD_FMHA_LEADING_ARGS(args), args);
+    }
     return check_launch(name);
 }
 
@@ -2299,7 +2333,7 @@ int run_f16(hipStream_t stream, FmhaArgs const& a, F16Kernel which)
             return st;
         }
         hipLaunchKernelGGL((fmha_f16_stream_kernel<DEBUG>), dim3((uint32_t) a.B * (uint32_t) a.N * (uint32_t) a.qSplit),
-            dim3(kWavesStream * kWaveSize), kStreamLds, stream, a, kt * 64);
+            dim3(kWavesStream * kWaveSize), kStreamLds, stream, TRTAMD_FMHA_LEADING_ARGS(a), a, kt * 64);
         return check_launch("fmha_f16_stream");
     }
     if (which == F16Kernel::kTURNS)
@@ -2476,9 +2510,7 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         }
     }
     a.partDiv = fast_div((uint32_t) a.qSplit);
-    a.spanDiv = fast_div(8u * (uint32_t) a.qSplit);
     a.headDiv = fast_div((uint32_t) a.N);
-    a.turnDiv = fast_div((uint32_t) (kWavesI8 * a.qSplit));
     a.dbgAcc1 = dbgAcc1;
     a.dbgP8 = dbgP8;
     {

@@ -1572,14 +1572,21 @@ __device__ __forceinline__ void prefetch_weights(LinearArgs const& p, uint32_t i
 }
 
 template <bool IL, bool IL_OUT, int EPI, int WM, int WN, int MT, int NT, int RING, int PER_SIMD, int KS = 2>
-__global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(LinearArgs const p)
+__global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(int8_t const* w, int8_t const* a, int const K, int const T,
+    int const N, int const mainTiles, uint32_t const panel, uint32_t const panelMul, uint32_t const panelShifts,
+    uint32_t const perPanel, uint32_t const perPanelMul, uint32_t const perPanelShifts, LinearArgs const rest)
 {
+    LinearArgs p = rest; // what a workgroup needs before its first request comes preloaded instead
+    p.w = w;
+    p.a = a;
+    p.K = K;
+    p.T = T;
+    p.N = N;
+    p.mainTiles = mainTiles;
+    p.panelDiv = {panel, panelMul, panelShifts};
+    p.perPanelDiv = {perPanel, perPanelMul, perPanelShifts};
     constexpr int kRing = RING * (WM * MT + WN * NT) * KS * 1024;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[kRing + (scales_late(kRing) ? 0 : 2 * kBigTile * 4)];
-    // all arguments in one trip of the scalar loads, as in the piece kernels
-    asm volatile("" ::"s"(p.a), "s"(p.w), "s"(p.alpha), "s"(p.beta), "s"(p.out), "s"(p.T), "s"(p.K), "s"(p.N), "s"(p.mainTiles),
-                 "s"(p.panelDiv.d), "s"(p.panelDiv.mul), "s"(p.panelDiv.shifts), "s"(p.perPanelDiv.d),
-                 "s"(p.perPanelDiv.mul), "s"(p.perPanelDiv.shifts));
     if constexpr (IL)
     {
         if ((int) blockIdx.x >= p.mainTiles)
@@ -1596,14 +1603,24 @@ __global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(Line
         p, (int) (pan * p.panelDiv.d + inPanel) * (WM * MT * 32), (int) tokenTile * (WN * NT * 32), lds);
 }
 
-// Asks for what the piece kernels read of their arguments at once: left to its first use, each trip of the scalar loads
-// delays a launch of few tokens by 0.1 to 0.2 us, and there were up to five one after the other.  With the divisions that
-// the numbering of the pieces took (they have a grid of three extents now), a pass of one request: INT8, 24 layers of 1024
-// channels, 632 -> 590 us; FP16, 12 layers of 768, 386 -> 379 us.
-__device__ __forceinline__ void pin_piece_args(LinearArgs const& p)
+// The arguments of the piece kernels: what a wavefront needs for its requests comes preloaded, as the leading scalars of the
+// argument list.  Left to their first uses in the struct, they were up to five trips of scalar loads of 0.1 to 0.2 us, one
+// behind the other, and the divisions that took a piece's number apart (it is a grid of three extents now) as much again: a
+// pass of one request, INT8, 24 layers of 1024 channels, 632 -> 590 us; FP16, 12 layers of 768, 386 -> 379 us.
+__device__ __forceinline__ LinearArgs piece_args(int8_t const* w, int8_t const* a, float const* alpha, float const* beta, int K,
+    int T, int N, int parts, int perPart, LinearArgs const& rest)
 {
-    asm volatile("" ::"s"(p.a), "s"(p.w), "s"(p.alpha), "s"(p.beta), "s"(p.out), "s"(p.T), "s"(p.K), "s"(p.N), "s"(p.qOut),
-                 "s"(p.tokMain), "s"(p.parts), "s"(p.perPart), "s"(p.mainTiles), "s"(p.prefetch.data), "s"(p.prefetch.units));
+    LinearArgs p = rest;
+    p.w = w;
+    p.a = a;
+    p.alpha = alpha;
+    p.beta = beta;
+    p.K = K;
+    p.T = T;
+    p.N = N;
+    p.parts = parts;
+    p.perPart = perPart;
+    return p;
 }
 
 // A piece of CB x TB blocks of 32 channels x 32 tokens by one workgroup whose eight wavefronts split k, for launches
@@ -1613,16 +1630,17 @@ __device__ __forceinline__ void pin_piece_args(LinearArgs const& p)
 // in flight per wavefront, no LDS stage and no barrier before the eight partial accumulators meet in LDS; every wavefront
 // then adds up and stores quarters of blocks.  40 tokens x 4096 -> 1024: 19.1 us in 128 x 128 tiles, 4.7 us in 32 x 32
 // pieces; K any multiple of 32 bytes, N and T any.  The grid is (channel pieces, token pieces, parts and what prefetches):
-// no division stands between a wavefront's start and its first request, and all arguments come in one trip.
+// neither a division nor a trip for an argument stands between a wavefront's start and its first request.
 template <bool IL_OUT, int EPI, int CB, int TB, int DEPTH, int PER_SIMD>
-__global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(LinearArgs const p)
+__global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(int8_t const* w, int8_t const* a, float const* alpha,
+    float const* beta, int const K, int const T, int const N, int const parts, int const perPart, LinearArgs const rest)
 {
     constexpr int NW = 8;
+    LinearArgs const p = piece_args(w, a, alpha, beta, K, T, N, parts, perPart, rest);
     __shared__ __attribute__((aligned(16))) uint8_t lds[NW * CB * TB * 4096];
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int const row = lane & 31, half = lane >> 5;
-    pin_piece_args(p);
     if ((int) blockIdx.z >= p.parts)
     {
         uint32_t const nbm = (uint32_t) ceil_div(p.N, 32 * CB);
@@ -1745,9 +1763,11 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(LinearArgs 
 // direct-to-LDS loads of its own (units, swizzle and fragment reads of the linear tiles; 7.2 us), so there is still no
 // barrier before the partial accumulators meet.  K a multiple of 64 bytes.
 template <bool IL_OUT, int EPI, int CB, int TB, int RING, int PER_SIMD>
-__global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearArgs const p)
+__global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(int8_t const* w, int8_t const* a, float const* alpha,
+    float const* beta, int const K, int const T, int const N, int const parts, int const perPart, LinearArgs const rest)
 {
     constexpr int NW = 8;
+    LinearArgs const p = piece_args(w, a, alpha, beta, K, T, N, parts, perPart, rest);
     constexpr int kLoads = (CB + TB) * 2;
     constexpr int STAGE = kLoads * 1024;
     static_assert(CB * TB * 4096 <= RING * STAGE, "the partial accumulators go where the wavefront's stages were");
@@ -1755,7 +1775,6 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(LinearA
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int const row = lane & 31, half = lane >> 5;
-    pin_piece_args(p);
     int const n0 = (int) blockIdx.x * (32 * CB), t0 = (int) blockIdx.y * (32 * TB), kpart = (int) blockIdx.z;
     uint8_t* const own = lds + wave * (RING * STAGE);
     uint32_t const ownBase = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) own;
@@ -2011,7 +2030,9 @@ uint32_t prefetch_workgroups(LinearArgs const& a, int threads)
 template <typename Kernel>
 int launch_tiles(hipStream_t stream, LinearArgs const& a, Kernel kernel, int threads)
 {
-    hipLaunchKernelGGL(kernel, dim3((uint32_t) a.mainTiles + prefetch_workgroups(a, threads)), dim3(threads), 0, stream, a);
+    hipLaunchKernelGGL(kernel, dim3((uint32_t) a.mainTiles + prefetch_workgroups(a, threads)), dim3(threads), 0, stream, a.w, a.a,
+        a.K, a.T, a.N, a.mainTiles, a.panelDiv.d, a.panelDiv.mul, a.panelDiv.shifts, a.perPanelDiv.d, a.perPanelDiv.mul,
+        a.perPanelDiv.shifts, a);
     return check_launch("int8_linear");
 }
 
@@ -2025,7 +2046,7 @@ int launch_pieces(hipStream_t stream, LinearArgs a, Kernel kernel, int channels,
     a.perPart = ceil_div(a.K / (IL ? 32 : 64), a.parts);
     uint32_t const behind = IL ? prefetch_workgroups(a, 512) : 0u;
     hipLaunchKernelGGL(kernel, dim3(nbm, (uint32_t) a.tokMain, (uint32_t) a.parts + ceil_div(behind, nbm * (uint32_t) a.tokMain)),
-        dim3(512), 0, stream, a);
+        dim3(512), 0, stream, a.w, a.a, a.alpha, a.beta, a.K, a.T, a.N, a.parts, a.perPart, a);
     return check_launch("int8_linear");
 }
 
