@@ -2018,6 +2018,17 @@ bool is_piece(int plan)
     return plan == kPiece32x64 || plan == kPiece32x32;
 }
 
+// The widest panel of at most `limit` channel tiles that divides their number.
+int widest_panel(int tiles, int limit)
+{
+    int w = std::max(limit, 1);
+    while (tiles % w != 0)
+    {
+        --w;
+    }
+    return w;
+}
+
 // What fetches a.prefetch behind the tiles, where the launch leaves CUs idle.
 uint32_t prefetch_workgroups(LinearArgs const& a, int threads)
 {
@@ -2059,20 +2070,16 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
     {
         return set_error(TRTAMD_STATUS_NOT_SUPPORTED, "int8_linear: too many tiles");
     }
-    // panels of at most 2 MB of weights: half of an XCD's L2
-    a.tokMain = ceil_div(a.T, c.tokens);
-    a.panel = 1;
-    for (int w = 1; w <= nbm && (int64_t) w * c.channels * a.K <= 2 << 20; ++w)
-    {
-        if (nbm % w == 0)
-        {
-            a.panel = w;
-        }
-    }
     a.parts = 1;
-    a.mainTiles = (int) grid;
-    a.panelDiv = fast_div((uint32_t) a.panel);
-    a.perPanelDiv = fast_div((uint32_t) a.panel * (uint32_t) a.tokMain);
+    if (!is_piece(plan))
+    {
+        // panels of at most 2 MB of weights: half of an XCD's L2
+        a.tokMain = ceil_div(a.T, c.tokens);
+        a.mainTiles = (int) grid;
+        a.panel = widest_panel((int) nbm, (int) std::min<int64_t>(nbm, (2 << 20) / ((int64_t) c.channels * a.K)));
+        a.panelDiv = fast_div((uint32_t) a.panel);
+        a.perPanelDiv = fast_div((uint32_t) a.panel * (uint32_t) a.tokMain);
+    }
     auto run = [&](auto kernel, int threads) { return launch_tiles(stream, a, kernel, threads); };
     if constexpr (IL)
     {
@@ -2254,15 +2261,6 @@ int launch_shape(hipStream_t stream, LinearArgs a)
     }
     a.tokMain = (int) (roundedTiles / nbmBig);
     a.mainTiles = a.tokMain * nbmBig;
-    constexpr int kMaxPanel = 8; // 8 x 256 channels x K = 1024 of weights is half of an XCD's 4 MB L2
-    a.panel = 1;
-    for (int w = 1; w <= kMaxPanel && w <= nbmBig; ++w)
-    {
-        if (nbmBig % w == 0)
-        {
-            a.panel = w;
-        }
-    }
     int const restTokens = a.T - a.tokMain * kBig;
     int64_t const grid = (int64_t) a.mainTiles + (int64_t) ceil_div(a.N, kSmall) * ceil_div(restTokens, kSmall);
     if (grid >= (int64_t) 1 << 31)
@@ -2271,6 +2269,7 @@ int launch_shape(hipStream_t stream, LinearArgs a)
     }
     int const persistent = tuning(Tuning::kLinearPersistent);
     int const direct = tuning(Tuning::kLinearDirect);
+    constexpr int kMaxPanel = 8; // 8 x 256 channels x K = 1024 of weights is half of an XCD's 4 MB L2
     if constexpr (IL_W == IL_IN && (EPI == kAFFINE || EPI == kGELU || EPI == kF16_AFFINE || EPI == kF16_GELU))
     {
         if (persistent && direct)
@@ -2284,12 +2283,13 @@ int launch_shape(hipStream_t stream, LinearArgs a)
                 a.pieces = restTokens > 0 && smallTiles * 100 <= (int64_t) tuning(Tuning::kLinearPieces) * cus;
             }
             int const plan = choose_plan<IL_W>(a, smallTiles, gelu);
-            if (plan != kLargeTiles)
+            if (plan != kLargeTiles) // numbers its tiles itself
             {
                 return launch_plan<IL_W, IL_OUT, EPI>(stream, a, plan);
             }
             if constexpr (IL_W && (EPI == kAFFINE || EPI == kGELU))
             {
+                a.panel = widest_panel(nbmBig, std::min(nbmBig, kMaxPanel));
                 a.persist = a.mainTiles < cus ? a.mainTiles : cus;
                 int64_t const behind = a.pieces ? (int64_t) (a.N / 64) * ceil_div(restTokens, 64) : smallTiles;
                 hipLaunchKernelGGL((int8_linear_dma_kernel<IL_OUT, EPI>), dim3((uint32_t) (a.persist + behind)), dim3(512), 0,
@@ -2298,6 +2298,7 @@ int launch_shape(hipStream_t stream, LinearArgs a)
             }
         }
     }
+    a.panel = widest_panel(nbmBig, std::min(nbmBig, kMaxPanel));
     if (persistent && a.K % 128 == 0)
     {
         a.persist = a.mainTiles < cus ? a.mainTiles : cus;
