@@ -170,7 +170,12 @@ __global__ __launch_bounds__(kBlock) void skipln_rows_kernel(int const ld, int64
 #pragma unroll
                 for (int k = 0; k < VPT; ++k)
                 {
-                    y.e[k] = (T) ((float) g[j].e[k] * (v[j][k] - mu) * rsigma + (float) b[j].e[k]);
+                    float value = (float) g[j].e[k] * (v[j][k] - mu) * rsigma + (float) b[j].e[k];
+                    if constexpr (FEW)
+                    {
+                        asm("" : "+v"(value)); // rounded to binary32 and then to T, as the compiler does in the other form
+                    }
+                    y.e[k] = (T) value;
                 }
                 store_through_l2(out + (row0 + r) * ld + (int64_t) vi * VPT, y.u);
             }

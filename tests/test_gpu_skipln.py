@@ -73,6 +73,22 @@ def test_skipln_fp_few_rows(api, dt, rows, ld):
     test_skipln_fp(api, dt, rows, ld, rows % 2 == 0)
 
 
+@pytest.mark.parametrize("dt,ld", [(np.float32, 768), (np.float16, 384), (np.float16, 1032), (np.float16, 2048)])
+def test_skipln_fp_rows_do_not_depend_on_their_number(api, dt, ld):
+    """A row gives the same bytes in a launch of few rows and in one of many, whose loads are other ones."""
+    r, rows = rng(2), 8200
+    x, skip = r.standard_normal((rows, ld)).astype(dt), r.standard_normal((rows, ld)).astype(dt)
+    d = [dev(a) for a in (x, skip, *_ln_params(r, ld, dt))]
+    fn = api.skip_layer_norm_fp32 if dt == np.float32 else api.skip_layer_norm_fp16
+    got = []
+    for n in (rows, 77):
+        o = dev_empty((rows, ld), dt, fill=0)
+        api.check(fn(stream(), ld, n * ld, ptr(d[0]), ptr(d[1]), ptr(d[3]), ptr(d[2]), ptr(o), ptr(d[4])))
+        sync()
+        got.append(host(o)[:77])
+    assert np.array_equal(got[0], got[1])
+
+
 def test_skipln_fp_errors(api):
     assert api.skip_layer_norm_fp32(None, 768, 100, 0, 0, 0, 0, 0, 0) != 0   # n % ld != 0
     assert "multiple" in api.last_error_str()
