@@ -254,6 +254,20 @@ __device__ inline uint32_t xcd_remap(uint32_t bid, uint32_t nblocks)
     return (bid % kXcds) * per + bid / kXcds;
 }
 
+// Addresses as launch arguments.  The runtime looks every pointer among a launch's arguments up in its table of allocations
+// (six of them: 2.41 us a launch, as integers or in a struct 2.28), which a pass of short launches waits for; as integers they
+// still come preloaded, which members of a struct do not.  Only for kernels whose loads do not rely on __restrict__.
+inline uint64_t address(void const* p)
+{
+    return reinterpret_cast<uint64_t>(p);
+}
+
+template <typename T>
+__device__ __forceinline__ T* global_ptr(uint64_t a)
+{
+    return (T*) reinterpret_cast<T __attribute__((address_space(1)))*>(a);
+}
+
 // Division by a number that the host knows, as part of a launch's arguments: a division by any other value is some forty
 // dependent instructions, which a workgroup would spend on finding its place before its first request.  Exact for all
 // 32-bit values (Granlund and Montgomery, "Division by Invariant Integers using Multiplication", figure 4.1).

@@ -142,20 +142,20 @@ struct FmhaArgs
 // The arguments of the cu_seqlens kernels: what a workgroup needs to find its sequence comes preloaded, as the leading scalars
 // of the argument list, ...
 #define TRTAMD_FMHA_LEADING_PARAMS                                                                                     \
-    void const *qkv, int32_t const *cuSeqlens, uint32_t const qSplit, uint32_t const qSplitMul,                        \
+    uint64_t const qkv, uint64_t const cuSeqlens, uint32_t const qSplit, uint32_t const qSplitMul,                      \
         uint32_t const qSplitShifts, uint32_t const N, uint32_t const headMul, uint32_t const headShifts, int const B, \
         int const S, int const ranked, int const total
 #define TRTAMD_FMHA_LEADING_ARGS(a)                                                                                    \
-    (a).qkv, (a).cuSeqlens, (a).partDiv.d, (a).partDiv.mul, (a).partDiv.shifts, (a).headDiv.d, (a).headDiv.mul,        \
-        (a).headDiv.shifts, (a).B, (a).S, (a).ranked, (a).total
+    address((a).qkv), address((a).cuSeqlens), (a).partDiv.d, (a).partDiv.mul, (a).partDiv.shifts, (a).headDiv.d,       \
+        (a).headDiv.mul, (a).headDiv.shifts, (a).B, (a).S, (a).ranked, (a).total
 #define TRTAMD_FMHA_ARGS_OF(rest)                                                                                      \
     fmha_args(qkv, cuSeqlens, {qSplit, qSplitMul, qSplitShifts}, {N, headMul, headShifts}, B, S, ranked, total, rest)
-__device__ __forceinline__ FmhaArgs fmha_args(void const* qkv, int32_t const* cuSeqlens, FastDiv const& partDiv,
+__device__ __forceinline__ FmhaArgs fmha_args(uint64_t qkv, uint64_t cuSeqlens, FastDiv const& partDiv,
     FastDiv const& headDiv, int B, int S, int ranked, int total, FmhaArgs const& rest)
 {
     FmhaArgs a = rest;
-    a.qkv = qkv;
-    a.cuSeqlens = cuSeqlens;
+    a.qkv = global_ptr<void const>(qkv);
+    a.cuSeqlens = global_ptr<int32_t const>(cuSeqlens);
     a.partDiv = partDiv;
     a.headDiv = headDiv;
     a.qSplit = (int) partDiv.d;

@@ -1572,13 +1572,13 @@ __device__ __forceinline__ void prefetch_weights(LinearArgs const& p, uint32_t i
 }
 
 template <bool IL, bool IL_OUT, int EPI, int WM, int WN, int MT, int NT, int RING, int PER_SIMD, int KS = 2>
-__global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(int8_t const* w, int8_t const* a, int const K, int const T,
+__global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(uint64_t const w, uint64_t const a, int const K, int const T,
     int const N, int const mainTiles, uint32_t const panel, uint32_t const panelMul, uint32_t const panelShifts,
     uint32_t const perPanel, uint32_t const perPanelMul, uint32_t const perPanelShifts, LinearArgs const rest)
 {
     LinearArgs p = rest; // what a workgroup needs before its first request comes preloaded instead
-    p.w = w;
-    p.a = a;
+    p.w = global_ptr<int8_t const>(w);
+    p.a = global_ptr<int8_t const>(a);
     p.K = K;
     p.T = T;
     p.N = N;
@@ -1607,14 +1607,14 @@ __global__ __launch_bounds__(WM* WN * 64, PER_SIMD) void linear_tile_kernel(int8
 // argument list.  Left to their first uses in the struct, they were up to five trips of scalar loads of 0.1 to 0.2 us, one
 // behind the other, and the divisions that took a piece's number apart (it is a grid of three extents now) as much again: a
 // pass of one request, INT8, 24 layers of 1024 channels, 632 -> 590 us; FP16, 12 layers of 768, 386 -> 379 us.
-__device__ __forceinline__ LinearArgs piece_args(int8_t const* w, int8_t const* a, float const* alpha, float const* beta, int K,
+__device__ __forceinline__ LinearArgs piece_args(uint64_t w, uint64_t a, uint64_t alpha, uint64_t beta, int K,
     int T, int N, int parts, int perPart, LinearArgs const& rest)
 {
     LinearArgs p = rest;
-    p.w = w;
-    p.a = a;
-    p.alpha = alpha;
-    p.beta = beta;
+    p.w = global_ptr<int8_t const>(w);
+    p.a = global_ptr<int8_t const>(a);
+    p.alpha = global_ptr<float const>(alpha);
+    p.beta = global_ptr<float const>(beta);
     p.K = K;
     p.T = T;
     p.N = N;
@@ -1632,8 +1632,8 @@ __device__ __forceinline__ LinearArgs piece_args(int8_t const* w, int8_t const* 
 // pieces; K any multiple of 32 bytes, N and T any.  The grid is (channel pieces, token pieces, parts and what prefetches):
 // neither a division nor a trip for an argument stands between a wavefront's start and its first request.
 template <bool IL_OUT, int EPI, int CB, int TB, int DEPTH, int PER_SIMD>
-__global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(int8_t const* w, int8_t const* a, float const* alpha,
-    float const* beta, int const K, int const T, int const N, int const parts, int const perPart, LinearArgs const rest)
+__global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(uint64_t const w, uint64_t const a, uint64_t const alpha,
+    uint64_t const beta, int const K, int const T, int const N, int const parts, int const perPart, LinearArgs const rest)
 {
     constexpr int NW = 8;
     LinearArgs const p = piece_args(w, a, alpha, beta, K, T, N, parts, perPart, rest);
@@ -1763,8 +1763,8 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(int8_t cons
 // direct-to-LDS loads of its own (units, swizzle and fragment reads of the linear tiles; 7.2 us), so there is still no
 // barrier before the partial accumulators meet.  K a multiple of 64 bytes.
 template <bool IL_OUT, int EPI, int CB, int TB, int RING, int PER_SIMD>
-__global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(int8_t const* w, int8_t const* a, float const* alpha,
-    float const* beta, int const K, int const T, int const N, int const parts, int const perPart, LinearArgs const rest)
+__global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(uint64_t const w, uint64_t const a, uint64_t const alpha,
+    uint64_t const beta, int const K, int const T, int const N, int const parts, int const perPart, LinearArgs const rest)
 {
     constexpr int NW = 8;
     LinearArgs const p = piece_args(w, a, alpha, beta, K, T, N, parts, perPart, rest);
@@ -2041,8 +2041,8 @@ uint32_t prefetch_workgroups(LinearArgs const& a, int threads)
 template <typename Kernel>
 int launch_tiles(hipStream_t stream, LinearArgs const& a, Kernel kernel, int threads)
 {
-    hipLaunchKernelGGL(kernel, dim3((uint32_t) a.mainTiles + prefetch_workgroups(a, threads)), dim3(threads), 0, stream, a.w, a.a,
-        a.K, a.T, a.N, a.mainTiles, a.panelDiv.d, a.panelDiv.mul, a.panelDiv.shifts, a.perPanelDiv.d, a.perPanelDiv.mul,
+    hipLaunchKernelGGL(kernel, dim3((uint32_t) a.mainTiles + prefetch_workgroups(a, threads)), dim3(threads), 0, stream, address(a.w),
+        address(a.a), a.K, a.T, a.N, a.mainTiles, a.panelDiv.d, a.panelDiv.mul, a.panelDiv.shifts, a.perPanelDiv.d, a.perPanelDiv.mul,
         a.perPanelDiv.shifts, a);
     return check_launch("int8_linear");
 }
@@ -2057,7 +2057,8 @@ int launch_pieces(hipStream_t stream, LinearArgs a, Kernel kernel, int channels,
     a.perPart = ceil_div(a.K / (IL ? 32 : 64), a.parts);
     uint32_t const behind = IL ? prefetch_workgroups(a, 512) : 0u;
     hipLaunchKernelGGL(kernel, dim3(nbm, (uint32_t) a.tokMain, (uint32_t) a.parts + ceil_div(behind, nbm * (uint32_t) a.tokMain)),
-        dim3(512), 0, stream, a.w, a.a, a.alpha, a.beta, a.K, a.T, a.N, a.parts, a.perPart, a);
+        dim3(512), 0, stream, address(a.w), address(a.a), address(a.alpha), address(a.beta), a.K, a.T, a.N, a.parts,
+        a.perPart, a);
     return check_launch("int8_linear");
 }
 

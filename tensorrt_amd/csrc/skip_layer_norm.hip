@@ -42,10 +42,16 @@ struct Vec16
 // FEW: a launch bound by the trips to memory in a row, not by the bytes.  All of a wavefront's loads are one trip (the
 // conditions of the other form made three of them), and what they need of the arguments comes preloaded.
 template <typename T, int NV, int R, bool HAS_BIAS, bool FEW>
-__global__ __launch_bounds__(kBlock) void skipln_rows_kernel(int const ld, int64_t const rows, T const* __restrict__ in,
-    T const* __restrict__ skip, T const* __restrict__ beta, T const* __restrict__ gamma, T const* __restrict__ bias,
-    T* __restrict__ out, float const eps)
+__global__ __launch_bounds__(kBlock) void skipln_rows_kernel(int const ld, int64_t const rows, uint64_t const inAt,
+    uint64_t const skipAt, uint64_t const betaAt, uint64_t const gammaAt, uint64_t const biasAt,
+    uint64_t const outAt, float const eps)
 {
+    T const* const in = global_ptr<T const>(inAt);
+    T const* const skip = global_ptr<T const>(skipAt);
+    T const* const beta = global_ptr<T const>(betaAt);
+    T const* const gamma = global_ptr<T const>(gammaAt);
+    T const* const bias = global_ptr<T const>(biasAt);
+    T* const out = global_ptr<T>(outAt);
     constexpr int VPT = Vec16<T>::kN;
     int const lane = threadIdx.x & (kWaveSize - 1);
     int64_t const wave = (int64_t) blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
@@ -231,7 +237,8 @@ int launch_rows_as(hipStream_t stream, int ld, int64_t rows, T const* in, T cons
     int64_t const waves = ceil_div<int64_t>(rows, R);
     dim3 const grid((unsigned) ceil_div<int64_t>(waves, kWavesPerBlock));
     auto const launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, stream, ld, rows, in, skip, beta, gamma, bias, out, eps);
+        hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, stream, ld, rows, address(in), address(skip), address(beta),
+            address(gamma), address(bias), address(out), eps);
         return check_launch("skipln_rows_kernel");
     };
     return bias ? launch(skipln_rows_kernel<T, NV, R, true, FEW>) : launch(skipln_rows_kernel<T, NV, R, false, FEW>);
@@ -326,11 +333,19 @@ int skip_layer_norm(hipStream_t stream, int32_t ld, int64_t n, T const* in, T co
 // (network_ops.hpp): its output is formed here as that layer's epilogue forms it, f16(fmaf(sum, alpha, beta)), and never
 // stored.  ld a multiple of 8, at most 1024.
 template <int NV>
-__global__ __launch_bounds__(kBlock) void skipln_rows_partial_kernel(int const ld, int const rows, float const* __restrict__ sums,
-    float const* __restrict__ alpha, float const* __restrict__ linearBeta, f16 const* __restrict__ skip,
-    f16 const* __restrict__ bias, int const parts, f16 const* __restrict__ beta, f16 const* __restrict__ gamma,
-    f16* __restrict__ out, float const eps)
+__global__ __launch_bounds__(kBlock) void skipln_rows_partial_kernel(int const ld, int const rows, uint64_t const sumsAt,
+    uint64_t const alphaAt, uint64_t const linearBetaAt, uint64_t const skipAt,
+    uint64_t const biasAt, int const parts, uint64_t const betaAt, uint64_t const gammaAt,
+    uint64_t const outAt, float const eps)
 {
+    float const* const sums = global_ptr<float const>(sumsAt);
+    float const* const alpha = global_ptr<float const>(alphaAt);
+    float const* const linearBeta = global_ptr<float const>(linearBetaAt);
+    f16 const* const skip = global_ptr<f16 const>(skipAt);
+    f16 const* const bias = global_ptr<f16 const>(biasAt);
+    f16 const* const beta = global_ptr<f16 const>(betaAt);
+    f16 const* const gamma = global_ptr<f16 const>(gammaAt);
+    f16* const out = global_ptr<f16>(outAt);
     int const lane = threadIdx.x & (kWaveSize - 1);
     int const row = (int) blockIdx.x * kWavesPerBlock + (int) (threadIdx.x >> 6);
     if (row >= rows)
@@ -618,10 +633,16 @@ __device__ inline uint32_t token_block_of_workgroup(uint32_t bid, uint32_t nbloc
 
 template <int G, int W, int TOK, bool PRELN, bool TAIL>
 __global__ __launch_bounds__(W * kWaveSize) void skipln_interleaved_kernel(int const total,
-    int8_t const* __restrict__ in, int8_t const* __restrict__ skip, f16 const* __restrict__ beta,
-    f16 const* __restrict__ gamma, int8_t* __restrict__ out, int8_t* __restrict__ preln, float const dqIn,
+    uint64_t const inAt, uint64_t const skipAt, uint64_t const betaAt,
+    uint64_t const gammaAt, uint64_t const outAt, uint64_t const prelnAt, float const dqIn,
     float const dqSkip, float const qScale, float const qSkipScale, float const eps, float const prelnMin)
 {
+    int8_t const* const in = global_ptr<int8_t const>(inAt);
+    int8_t const* const skip = global_ptr<int8_t const>(skipAt);
+    f16 const* const beta = global_ptr<f16 const>(betaAt);
+    f16 const* const gamma = global_ptr<f16 const>(gammaAt);
+    int8_t* const out = global_ptr<int8_t>(outAt);
+    int8_t* const preln = global_ptr<int8_t>(prelnAt);
     // A workgroup of W wavefronts owns TOK consecutive tokens.  Lane = (sub, token, half): one load
     // instruction of a wavefront reads SUBS channel groups x TOK tokens x 32 bytes, TOK*32 contiguous
     // bytes per group; the W wavefronts take interleaved sets of SUBS groups, NI sets each.
@@ -896,11 +917,17 @@ __global__ __launch_bounds__(W * kWaveSize) void skipln_interleaved_kernel(int c
 // of tokens spreads over as many CUs and nothing is exchanged between wavefronts.  (The 32-token blocks put 48 tokens on
 // two CUs, which then take longer over the arithmetic than over the loads.)
 template <int G, bool PRELN>
-__global__ __launch_bounds__(kBlock) void skipln_interleaved_token_kernel(int const total, int8_t const* __restrict__ in,
-    int8_t const* __restrict__ skip, f16 const* __restrict__ beta, f16 const* __restrict__ gamma, int8_t* __restrict__ out,
-    int8_t* __restrict__ preln, float const dqIn, float const dqSkip, float const qScale, float const qSkipScale,
+__global__ __launch_bounds__(kBlock) void skipln_interleaved_token_kernel(int const total, uint64_t const inAt,
+    uint64_t const skipAt, uint64_t const betaAt, uint64_t const gammaAt, uint64_t const outAt,
+    uint64_t const prelnAt, float const dqIn, float const dqSkip, float const qScale, float const qSkipScale,
     float const eps, float const prelnMin)
 {
+    int8_t const* const in = global_ptr<int8_t const>(inAt);
+    int8_t const* const skip = global_ptr<int8_t const>(skipAt);
+    f16 const* const beta = global_ptr<f16 const>(betaAt);
+    f16 const* const gamma = global_ptr<f16 const>(gammaAt);
+    int8_t* const out = global_ptr<int8_t>(outAt);
+    int8_t* const preln = global_ptr<int8_t>(prelnAt);
     constexpr int LD = G * 32;
     constexpr int NE = (G + 31) / 32; // loads per tensor and lane: 32 channel groups x 2 halves each
     int const lane = threadIdx.x & (kWaveSize - 1);
@@ -1016,10 +1043,17 @@ __global__ __launch_bounds__(kBlock) void skipln_interleaved_token_kernel(int co
 // the launch took 4.7 us at 32 tokens and four parts.
 template <int G>
 __global__ __launch_bounds__(G * 8) void skipln_interleaved_sums_kernel(int const total, int const parts,
-    int32_t const* __restrict__ sums, float const* __restrict__ alpha, float const* __restrict__ linearBeta,
-    int8_t const* __restrict__ skip, f16 const* __restrict__ beta, f16 const* __restrict__ gamma, int8_t* __restrict__ out,
+    uint64_t const sumsAt, uint64_t const alphaAt, uint64_t const linearBetaAt,
+    uint64_t const skipAt, uint64_t const betaAt, uint64_t const gammaAt, uint64_t const outAt,
     float const dqIn, float const dqSkip, float const qScale, float const eps)
 {
+    int32_t const* const sums = global_ptr<int32_t const>(sumsAt);
+    float const* const alpha = global_ptr<float const>(alphaAt);
+    float const* const linearBeta = global_ptr<float const>(linearBetaAt);
+    int8_t const* const skip = global_ptr<int8_t const>(skipAt);
+    f16 const* const beta = global_ptr<f16 const>(betaAt);
+    f16 const* const gamma = global_ptr<f16 const>(gammaAt);
+    int8_t* const out = global_ptr<int8_t>(outAt);
     constexpr int LD = G * 32, WAVES = G / 8;
     __shared__ int sStat[WAVES][5];
     int const token = (int) blockIdx.x;
@@ -1128,8 +1162,8 @@ int launch_interleaved_as(hipStream_t stream, int32_t total, int8_t const* in, i
     if ((int64_t) total * (G * 32) <= kFewBytes && aligned16(gamma) && aligned16(beta))
     {
         hipLaunchKernelGGL((skipln_interleaved_token_kernel<G, PRELN>),
-            dim3((unsigned) ceil_div(total, kWavesPerBlock)), dim3(kBlock), 0, stream, total, in, skip, beta, gamma, out, preln,
-            dqIn, dqSkip, qScale, qSkipScale, eps, prelnMin);
+            dim3((unsigned) ceil_div(total, kWavesPerBlock)), dim3(kBlock), 0, stream, total, address(in), address(skip),
+            address(beta), address(gamma), address(out), address(preln), dqIn, dqSkip, qScale, qSkipScale, eps, prelnMin);
         return check_launch("skipln_interleaved_token_kernel");
     }
     // One workgroup per block of TOK tokens.  When that is a few workgroups more than the chip holds at once, the
@@ -1144,12 +1178,12 @@ int launch_interleaved_as(hipStream_t stream, int32_t total, int8_t const* in, i
         && (int64_t) residentTail * (TOK + 1) >= total)
     {
         hipLaunchKernelGGL((skipln_interleaved_kernel<G, W, TOK, PRELN, true>), dim3((unsigned) residentTail), block, 0,
-            stream, total, in, skip, beta, gamma, out, preln, dqIn, dqSkip, qScale, qSkipScale, eps, prelnMin);
+            stream, total, address(in), address(skip), address(beta), address(gamma), address(out), address(preln), dqIn, dqSkip, qScale, qSkipScale, eps, prelnMin);
     }
     else
     {
         hipLaunchKernelGGL((skipln_interleaved_kernel<G, W, TOK, PRELN, false>), dim3((unsigned) blocks), block, 0, stream,
-            total, in, skip, beta, gamma, out, preln, dqIn, dqSkip, qScale, qSkipScale, eps, prelnMin);
+            total, address(in), address(skip), address(beta), address(gamma), address(out), address(preln), dqIn, dqSkip, qScale, qSkipScale, eps, prelnMin);
     }
     return check_launch("skipln_interleaved_kernel");
 }
@@ -1227,8 +1261,8 @@ int skipln_interleaved_from_partial(trtamd_stream_t stream, bool large, int32_t 
     }
     float const eps = large ? 1.1920928955078125e-07f : 0.0009765625f;
     auto const launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned) total), dim3((unsigned) ld / 4), 0, as_stream(stream), total, parts, partial,
-            alpha, beta, skip, reinterpret_cast<f16 const*>(lnBeta), reinterpret_cast<f16 const*>(lnGamma), output, dqScaleIn, dqScaleSkip, qScale,
+        hipLaunchKernelGGL(kernel, dim3((unsigned) total), dim3((unsigned) ld / 4), 0, as_stream(stream), total, parts,
+            address(partial), address(alpha), address(beta), address(skip), address(lnBeta), address(lnGamma), address(output), dqScaleIn, dqScaleSkip, qScale,
             eps);
         return check_launch("skipln_interleaved_sums_kernel");
     };
@@ -1244,10 +1278,10 @@ int skip_layer_norm_fp16_from_partial(trtamd_stream_t stream, int32_t ld, int32_
         return set_error(TRTAMD_STATUS_NOT_SUPPORTED, "SkipLayerNorm from partial sums: unsupported problem");
     }
     float const eps = (ld == 768 || ld == 1024) ? 0.0009765625f : 0.f; // as skip_layer_norm
-    auto const half = [](trtamd_half_t const* x) { return reinterpret_cast<f16 const*>(x); };
     auto const launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned) ceil_div(rows, kWavesPerBlock)), dim3(kBlock), 0, as_stream(stream), ld, rows,
-            partial, alpha, beta, half(skip), half(bias), parts, half(lnBeta), half(lnGamma), reinterpret_cast<f16*>(output), eps);
+            address(partial), address(alpha), address(beta), address(skip), address(bias), parts, address(lnBeta), address(lnGamma),
+            address(output), eps);
         return check_launch("skipln_rows_partial_kernel");
     };
     return ld <= 512 ? launch(skipln_rows_partial_kernel<1>) : launch(skipln_rows_partial_kernel<2>);
