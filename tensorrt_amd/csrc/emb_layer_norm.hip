@@ -195,11 +195,21 @@ __device__ __forceinline__ void mask_workgroup(MaskJob const& job, uint32_t cons
 // second, the arguments come preloaded or meanwhile, and the position takes no division.
 template <typename T, int NV, int MODE, int TPW>
 __global__ __launch_bounds__(kBlock) void embln_kernel(uint32_t const maskBlocks, int const ld, int const B, int const S,
-    uint32_t const innerMul, uint32_t const innerShifts, int32_t const* __restrict__ inputIds,
-    int32_t const* __restrict__ tokenIds, int32_t const* __restrict__ cuSeqlens, float const* __restrict__ beta,
-    float const* __restrict__ gamma, T const* __restrict__ wordEmb, T const* __restrict__ posEmb, T const* __restrict__ tokEmb,
-    int32_t const wordSize, int32_t const tokSize, T* __restrict__ output, T* __restrict__ skipOut, MaskJob const job)
+    uint32_t const innerMul, uint32_t const innerShifts, uint64_t const inputIdsAt,
+    uint64_t const tokenIdsAt, uint64_t const cuSeqlensAt, uint64_t const betaAt,
+    uint64_t const gammaAt, uint64_t const wordEmbAt, uint64_t const posEmbAt, uint64_t const tokEmbAt,
+    int32_t const wordSize, int32_t const tokSize, uint64_t const outputAt, uint64_t const skipOutAt, MaskJob const job)
 {
+    int32_t const* const inputIds = global_ptr<int32_t const>(inputIdsAt);
+    int32_t const* const tokenIds = global_ptr<int32_t const>(tokenIdsAt);
+    int32_t const* const cuSeqlens = global_ptr<int32_t const>(cuSeqlensAt);
+    float const* const beta = global_ptr<float const>(betaAt);
+    float const* const gamma = global_ptr<float const>(gammaAt);
+    T const* const wordEmb = global_ptr<T const>(wordEmbAt);
+    T const* const posEmb = global_ptr<T const>(posEmbAt);
+    T const* const tokEmb = global_ptr<T const>(tokEmbAt);
+    T* const output = global_ptr<T>(outputAt);
+    T* const skipOut = global_ptr<T>(skipOutAt);
     constexpr int VPT = Vec16<T>::kN;
     FastDiv const inner{(uint32_t) (MODE == kFIXED ? B : S), innerMul, innerShifts};
     if constexpr (MODE == kFIXED)
@@ -445,14 +455,16 @@ int emb_layer_norm(hipStream_t stream, int32_t ld, int32_t B, int32_t S, int32_t
     if (multi)                                                                                                         \
     {                                                                                                                  \
         hipLaunchKernelGGL((embln_kernel<T, NVV, MODE, 4>), grid4, dim3(kBlock), 0, stream, job.blocks, ld, B, S, \
-            inner.mul, inner.shifts, inputIds, tokenIds, cuSeqlens, beta, gamma, wordEmb, posEmb, tokEmb, wordSize, tokSize, \
-            output, skipOut, job);                                                                                     \
+            inner.mul, inner.shifts, address(inputIds), address(tokenIds), address(cuSeqlens), address(beta),           \
+            address(gamma), address(wordEmb), address(posEmb), address(tokEmb), wordSize, tokSize, address(output),     \
+            address(skipOut), job);                                                                                    \
     }                                                                                                                  \
     else                                                                                                               \
     {                                                                                                                  \
         hipLaunchKernelGGL((embln_kernel<T, NVV, MODE, 1>), grid, dim3(kBlock), 0, stream, job.blocks, ld, B, S, \
-            inner.mul, inner.shifts, inputIds, tokenIds, cuSeqlens, beta, gamma, wordEmb, posEmb, tokEmb, wordSize, tokSize, \
-            output, skipOut, job);                                                                                     \
+            inner.mul, inner.shifts, address(inputIds), address(tokenIds), address(cuSeqlens), address(beta),           \
+            address(gamma), address(wordEmb), address(posEmb), address(tokEmb), wordSize, tokSize, address(output),     \
+            address(skipOut), job);                                                                                    \
     }
     if (vec_ok && nv == 1)
     {
