@@ -2109,8 +2109,8 @@ __global__ __launch_bounds__(kWavesStream* kWaveSize) __attribute__((amdgpu_wave
             mxB = fmaxf(fmaxf(mxB, acc[1][v]), acc[1][v + 1]);
         }
         float const mx = reduce_step<32>(fmaxf(mxA, mxB), [](float x, float y) { return fmaxf(x, y); });
-        // finite, so that a block whose scores are all -infinity weighs nothing
-        float const negNew = -fmaxf(mx, -3.402823466e+38f) * a.c;
+        // finite, whatever the scale is, so that a block whose scores are all -infinity weighs nothing
+        float const negNew = fminf(-mx * a.c, 3.402823466e+38f);
         if (kb == 0)
         {
             negMax = negNew;
