@@ -34,6 +34,17 @@ struct Vec16
     };
 };
 
+// A result as binary32 and then as T.  Kernels whose loads are unconditional need it: the compiler otherwise folds the
+// multiply-add in front of a conversion to binary16 into it, which rounds once instead of twice, and a row would differ in one
+// value of 10^4 from what the form with masked loads gives.  (That form it converts in pairs, which cannot be folded; with this
+// it no longer adds in pairs either, and 8193 rows of 768 or 1024 values take 1 to 1.5 % more.  Tests compare all three.)
+template <typename T>
+__device__ __forceinline__ T through_binary32(float value)
+{
+    asm("" : "+v"(value));
+    return (T) value;
+}
+
 // ------------------------------------------------------------------------------------------
 // FP32 / FP16 rows, ld a multiple of the 16-byte vector width: register-resident rows.
 // The residual sum is formed in T like the reference (skipLayerNormKernel.cu:121-134);
@@ -176,12 +187,8 @@ __global__ __launch_bounds__(kBlock) void skipln_rows_kernel(int const ld, int64
 #pragma unroll
                 for (int k = 0; k < VPT; ++k)
                 {
-                    float value = (float) g[j].e[k] * (v[j][k] - mu) * rsigma + (float) b[j].e[k];
-                    if constexpr (FEW)
-                    {
-                        asm("" : "+v"(value)); // rounded to binary32 and then to T, as the compiler does in the other form
-                    }
-                    y.e[k] = (T) value;
+                    float const value = (float) g[j].e[k] * (v[j][k] - mu) * rsigma + (float) b[j].e[k];
+                    y.e[k] = FEW ? through_binary32<T>(value) : (T) value;
                 }
                 store_through_l2(out + (row0 + r) * ld + (int64_t) vi * VPT, y.u);
             }
@@ -452,7 +459,7 @@ __global__ __launch_bounds__(kBlock) void skipln_rows_partial_kernel(int const l
 #pragma unroll
             for (int k = 0; k < 8; ++k)
             {
-                y.e[k] = (f16) ((float) g[j].e[k] * (v[j][k] - w.mean) * rsigma + (float) b[j].e[k]);
+                y.e[k] = through_binary32<f16>((float) g[j].e[k] * (v[j][k] - w.mean) * rsigma + (float) b[j].e[k]);
             }
             store_through_l2(out + (int64_t) row * ld + vi * 8, y.u);
         }

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import oracle
-from helpers import assert_fp_close, rng
+from helpers import assert_fp_close, dev, dev_empty, host, ptr, rng, stream, sync
 from tensorrt_amd.encoder import EncoderConfig
 from tensorrt_amd.encoder_fp16 import Fp16BertEncoder
 
@@ -129,6 +129,50 @@ def test_normalisation_of_partial_sums(one_layer, hidden, ffn, lens):
     half = lambda a: a.astype(np.float16)
     want = oracle.skipln(f, h, half(L["ln2_beta"]), half(L["ln2_gamma"]), half(L["ln2_bias"]))
     assert_fp_close(out.cpu().numpy(), want, what="SkipLayerNorm of partial sums")
+
+
+@pytest.mark.parametrize("hidden,ffn", [(768, 3072), (1024, 4096), (512, 2048), (320, 2048)])
+@pytest.mark.parametrize("scaled", [False, True])
+def test_normalisation_of_partial_sums_rounds_as_the_layer_and_the_normalisation_do(one_layer, hidden, ffn, scaled):
+    """The bytes of the normalisation that reads partial sums are those of the normalisation by itself behind a layer with
+    the same sums: the layer's multiply-add rounded to binary16 once (`scaled`: by an alpha and a beta that leave something
+    to round), the normalisation's rounded to binary32 first."""
+    import torch
+    enc = one_layer(hidden, ffn)
+    api, L = enc.api, enc.layers[0]
+    r = rng(48 + hidden)
+    c = np.array([0, 20, 64], np.int32)
+    t = int(c[-1])
+    ids, segs = r.integers(0, 500, t).astype(np.int32), r.integers(0, 2, t).astype(np.int32)
+    alpha, beta = np.ones(hidden, np.float32), np.zeros(hidden, np.float32)
+    if scaled:
+        alpha, beta = r.uniform(0.5, 1.5, hidden).astype(np.float32), (0.1 * r.standard_normal(hidden)).astype(np.float32)
+    lin = L["ffn2"]
+    d = [dev(L[k].astype(np.float16)) for k in ("ln2_beta", "ln2_gamma", "ln2_bias")]
+    got, want = [], []
+    lin.alpha.copy_(torch.from_numpy(alpha))
+    lin.beta.copy_(torch.from_numpy(beta))
+    try:
+        for _ in range(8):   # one result in some 10^4 depends on how often it was rounded
+            enc._partial.zero_()
+            ids = np.roll(ids, 1)
+            out = enc.enqueue(ids, segs, c)
+            sync()
+            got.append(host(out))
+            sums = enc._partial.view(torch.float32)[:4 * t * hidden].cpu().numpy().reshape(4, t, hidden)
+            assert np.abs(sums[1]).max() > 0, "more than one part"
+            total = ((sums[0] + sums[1]) + sums[2]) + sums[3]   # binary32, in the kernel's order
+            f = (total.astype(np.float64) * alpha + beta).astype(np.float16)
+            o, d_f = dev_empty((t, hidden), np.float16), dev(f)
+            api.check(api.skip_layer_norm_fp16(stream(), hidden, t * hidden, ptr(d_f), ptr(enc.buf["h"]), ptr(d[0]), ptr(d[1]),
+                                               ptr(o), ptr(d[2])))
+            sync()
+            want.append(host(o))
+    finally:
+        lin.alpha.fill_(1.0)
+        lin.beta.zero_()
+    got, want = np.array(got).view(np.uint16), np.array(want).view(np.uint16)
+    assert np.array_equal(got, want), f"{int((got != want).sum())} of {got.size} values differ"
 
 
 def test_passes_asked_for_on_another_stream(setup):
