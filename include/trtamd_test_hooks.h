@@ -32,6 +32,10 @@ TRTAMD_API int trtamd_fused_mha_run_debug(trtamd_stream_t stream, int32_t data_t
 TRTAMD_API int trtamd_test_set_tuning(char const* name, int32_t value);
 TRTAMD_API int trtamd_test_reset_tuning(char const* name);
 
+/* The number (TRTAMD_LINEAR_PLAN) of the kernel that a linear layer with both operands interleaved, or both linear, takes at
+ * these sizes under the switches as they are; row_bytes: K in INT8, 2 K in FP16.  -1: sizes that no layer has. */
+TRTAMD_API int trtamd_test_linear_plan(int32_t interleaved, int32_t T, int32_t row_bytes, int32_t N, int32_t gelu);
+
 #ifdef __cplusplus
 }
 #endif

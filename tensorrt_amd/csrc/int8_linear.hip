@@ -24,6 +24,7 @@
 #include "host_utils.hpp"
 #include "network_ops.hpp"
 #include "trtamd_encoder_ops.h"
+#include "trtamd_test_hooks.h"
 
 #include <algorithm>
 #include <cmath>
@@ -1918,6 +1919,12 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(uint64_
 // encoders (graph replays, weights in the last-level cache), 16 to 33289 tokens, on two GPUs, one of them with the uneven
 // engines.  The plan they choose takes 0.8 % more than the best of all in the mean (24 % at most, a launch at the edge
 // of a second round); the kernels and the choice before took 13 % more (50 % at most).
+// Linear operands whose rows end within a line have kernels and constants of their own: stages of 64 bytes, tiles of up to 128 x
+// 256, and constants fitted to launches by themselves before the other linear operands had stages of whole lines.  10 layers of
+// 96 to 3104 channels, 40 to 33289 tokens, FP16 and INT8, 240 launches: 6.5 % less in the mean than when all linear operands
+// had those kernels (launches of 3 us up to 8 % more, others up to 4 %), 0.4 % more than the best of the six plans.  With only 128 x 128 and
+// 64 x 64 tiles and the constants of the whole lines it was 2.5 % more, 29 % at most (7765 tokens x 3104 -> 768, FP16: 50.2 us
+// then, 64.4 so, 50.3 now).
 // Interleaved operands: to launches by themselves on those of a
 // 1024-channel INT8 encoder with weights from memory, and the ones that decide from 2500 tokens on (large tiles, 128 x 256,
 // 128 x 128, 64 x 128, 128 x 128 deep) to whole passes of that encoder with the plans of one or two of its layers changed at a
@@ -1963,8 +1970,9 @@ enum LinearPlan
     kLinearPlans
 };
 constexpr float kOneRound = 1e3f; // of tiles that are taken only where a launch has no more of them than CUs
-// [0]: linear operands, [1]: interleaved ones.  No channels: the layout has no such kernel.
-constexpr TileCost kTileCosts[2][kLinearPlans] = {
+// [0]: linear operands, [1]: interleaved ones, [2]: linear ones whose rows end within a line of 128 bytes.  No channels: the
+// layout has no such kernel.
+constexpr TileCost kTileCosts[3][kLinearPlans] = {
     {{}, {}, {128, 128, 2, 4.64f, 0.00f, 0.231f, 0.60f, 0.61f, 1.02f, 0.40f, 0.25f}, {},
         {64, 64, 2, 3.82f, 0.29f, 0.082f, 0.23f, 0.70f, 0.89f, 0.63f, 0.34f},
         {128, 128, 1, 4.02f, 0.77f, 0.142f, 0.99f, 0.f, 1.30f, 0.77f, 0.51f, 0.10f}, {}, {},
@@ -1981,7 +1989,17 @@ constexpr TileCost kTileCosts[2][kLinearPlans] = {
         {64, 128, 2, 2.54f, 0.60f, 0.150f, 0.32f, 1.22f, 0.93f, 0.35f}, {64, 64, 2, 2.46f, 0.54f, 0.100f, 0.35f, 0.93f, 0.91f, 0.46f},
         {32, 64, 2, 3.19f, 0.17f, 0.068f, 0.04f, 0.90f, 1.19f, 0.67f}, {32, 32, 4, 2.69f, 1.21f, 0.042f, 0.16f, 0.67f, 1.19f, 0.64f},
         {256, 256, 1, 5.39f, 0.f, 0.406f, 4.88f, 0.f, kOneRound, 1.f, 0.41f}, {256, 192, 1, 5.31f, 0.f, 0.217f, 2.67f, 0.f, kOneRound, 1.f, 1.50f},
-        {128, 192, 1, 4.55f, 0.f, 0.142f, 1.01f, 0.f, kOneRound, 1.f, 1.47f}, {}, {}}};
+        {128, 192, 1, 4.55f, 0.f, 0.142f, 1.01f, 0.f, kOneRound, 1.f, 1.47f}, {}, {}},
+    {{}, {128, 256, 2, 2.06f, 2.05f, 0.430f, 0.64f, 1.50f, 1.22f, 0.62f}, {128, 128, 2, 1.93f, 1.06f, 0.292f, 0.41f, 1.30f, 1.10f, 0.53f},
+        {64, 128, 3, 2.49f, 0.32f, 0.188f, 0.21f, 1.27f, 1.14f, 0.52f}, {64, 64, 4, 2.29f, 0.30f, 0.138f, 0.13f, 0.94f, 0.89f, 0.47f},
+        {}, {}, {}, {32, 64, 1, 2.88f, 0.30f, 0.071f, 0.05f, 0.57f, 1.91f, 0.80f}, {32, 32, 1, 2.38f, 0.34f, 0.053f, 0.13f, 1.48f, 1.49f, 0.68f}}};
+
+// The costs of a launch's plans.
+template <bool IL>
+TileCost const* tile_costs(LinearArgs const& a)
+{
+    return kTileCosts[IL ? 1 : a.K % 128 == 0 ? 0 : 2];
+}
 
 inline float tile_time(TileCost const& c, LinearArgs const& a, bool gelu)
 {
@@ -2065,7 +2083,7 @@ int launch_pieces(hipStream_t stream, LinearArgs a, Kernel kernel, int channels,
 template <bool IL, bool IL_OUT, int EPI>
 int launch_plan(hipStream_t stream, LinearArgs a, int plan)
 {
-    TileCost const& c = kTileCosts[IL][plan];
+    TileCost const& c = tile_costs<IL>(a)[plan];
     int64_t const nbm = ceil_div(a.N, c.channels), grid = nbm * ceil_div(a.T, c.tokens);
     if (grid >= (int64_t) 1 << 31)
     {
@@ -2117,7 +2135,9 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
         // rows that end within a line: stages of 64 bytes
         switch (plan)
         {
-        case kTile128x128: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 2, 3, 2>, 256);
+        case kTile128x256: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 4, 2, 2, 3, 4>, 512);
+        case kTile128x128: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 4, 2, 1, 4, 4>, 512);
+        case kTile64x128: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 2, 4, 3>, 256);
         case kTile64x64: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 1, 4, 4>, 256);
         default: break;
         }
@@ -2162,18 +2182,17 @@ template <bool IL>
 int cheapest_plan(LinearArgs const& a, int64_t smallTiles, bool gelu, int plan)
 {
     bool const large = IL && a.N % kBig == 0 && a.K % 256 == 0 && a.mainTiles > 0;
+    TileCost const* const costs = tile_costs<IL>(a);
     auto const exists = [&](int q) {
         if (q == kLargeTiles)
         {
             return large;
         }
-        if (is_piece(q) && ceil_div(a.T, kTileCosts[IL][q].tokens) > 65535)
+        if (is_piece(q) && ceil_div(a.T, costs[q].tokens) > 65535)
         {
             return false; // the second extent of their grid
         }
-        bool const halfLines = !IL && a.K % 128 != 0; // the tiles that have a kernel for those
-        return kTileCosts[IL][q].channels != 0
-            && (!halfLines || q == kTile128x128 || q == kTile64x64 || q == kPiece32x64 || q == kPiece32x32);
+        return costs[q].channels != 0;
     };
     if (plan >= 0 && plan < kLinearPlans && exists(plan))
     {
@@ -2186,8 +2205,7 @@ int cheapest_plan(LinearArgs const& a, int64_t smallTiles, bool gelu, int plan)
         {
             continue;
         }
-        float const t = q == kLargeTiles ? large_tiles_time(kTileCosts[IL][q], a, smallTiles, gelu)
-                                         : tile_time(kTileCosts[IL][q], a, gelu);
+        float const t = q == kLargeTiles ? large_tiles_time(costs[q], a, smallTiles, gelu) : tile_time(costs[q], a, gelu);
         if (t < best)
         {
             best = t;
@@ -2245,15 +2263,14 @@ int parts_of(int plan, LinearArgs const& a)
     return std::max(1, std::min({kMaxLinearParts, num_cus() / grid, a.K / 1024}));
 }
 
-template <bool IL_W, bool IL_IN, bool IL_OUT, int EPI>
-int launch_shape(hipStream_t stream, LinearArgs a)
+// Large tiles for as many whole rows of 256 tokens as fit in full rounds of one workgroup per CU, plus a last partial round when
+// it would occupy more than `partial` per cent of the CUs: in 128 x 128 tiles that remainder needs three rounds or more, which
+// take longer than one round of large tiles.  Returns the 128 x 128 tiles behind them.
+int64_t place_large_tiles(LinearArgs& a)
 {
-    // big tiles for as many whole token-tile rows as fit in full rounds of one workgroup per CU
     int const nbmBig = ceil_div(a.N, kBig);
     int64_t const bigTiles = (int64_t) nbmBig * (a.T / kBig);
     int const cus = num_cus();
-    // ... plus a last partial round when it would occupy more than `partial` per cent of the CUs: in 128 x 128
-    // tiles that remainder needs three rounds or more, which take longer than one round of large tiles
     int const partial = tuning(Tuning::kLinearPartialRound);
     int64_t roundedTiles = (bigTiles / cus) * cus;
     if ((bigTiles - roundedTiles) * 100 > (int64_t) partial * cus)
@@ -2262,8 +2279,23 @@ int launch_shape(hipStream_t stream, LinearArgs a)
     }
     a.tokMain = (int) (roundedTiles / nbmBig);
     a.mainTiles = a.tokMain * nbmBig;
-    int const restTokens = a.T - a.tokMain * kBig;
-    int64_t const grid = (int64_t) a.mainTiles + (int64_t) ceil_div(a.N, kSmall) * ceil_div(restTokens, kSmall);
+    return (int64_t) ceil_div(a.N, kSmall) * ceil_div(a.T - a.tokMain * kBig, kSmall);
+}
+
+// The plan of a launch whose large tiles are placed.  Few 128 x 128 tiles behind them (no more than TRTAMD_LINEAR_PIECES per cent
+// of the CUs busy with a long k loop each): the same tokens as 64 x 64 pieces whose wavefronts split k (linear_piece64).
+template <bool IL>
+int plan_behind_large_tiles(LinearArgs& a, int64_t smallTiles, bool gelu)
+{
+    a.pieces = IL && a.T > a.tokMain * kBig && smallTiles * 100 <= (int64_t) tuning(Tuning::kLinearPieces) * num_cus();
+    return choose_plan<IL>(a, smallTiles, gelu);
+}
+
+template <bool IL_W, bool IL_IN, bool IL_OUT, int EPI>
+int launch_shape(hipStream_t stream, LinearArgs a)
+{
+    int const nbmBig = ceil_div(a.N, kBig), cus = num_cus();
+    int64_t const smallTiles = place_large_tiles(a), grid = a.mainTiles + smallTiles;
     if (grid >= (int64_t) 1 << 31)
     {
         return set_error(TRTAMD_STATUS_NOT_SUPPORTED, "int8_linear: too many tiles");
@@ -2275,15 +2307,7 @@ int launch_shape(hipStream_t stream, LinearArgs a)
     {
         if (persistent && direct)
         {
-            constexpr bool gelu = EPI == kGELU || EPI == kF16_GELU;
-            // few 128 x 128 tiles behind the large ones (no more than TRTAMD_LINEAR_PIECES per cent of the CUs busy with
-            // a long k loop each): the same tokens as 64 x 64 pieces whose wavefronts split k (linear_piece64)
-            int64_t const smallTiles = grid - a.mainTiles;
-            if constexpr (IL_W && (EPI == kAFFINE || EPI == kGELU))
-            {
-                a.pieces = restTokens > 0 && smallTiles * 100 <= (int64_t) tuning(Tuning::kLinearPieces) * cus;
-            }
-            int const plan = choose_plan<IL_W>(a, smallTiles, gelu);
+            int const plan = plan_behind_large_tiles<IL_W>(a, smallTiles, EPI == kGELU || EPI == kF16_GELU);
             if (plan != kLargeTiles) // numbers its tiles itself
             {
                 return launch_plan<IL_W, IL_OUT, EPI>(stream, a, plan);
@@ -2292,7 +2316,7 @@ int launch_shape(hipStream_t stream, LinearArgs a)
             {
                 a.panel = widest_panel(nbmBig, std::min(nbmBig, kMaxPanel));
                 a.persist = a.mainTiles < cus ? a.mainTiles : cus;
-                int64_t const behind = a.pieces ? (int64_t) (a.N / 64) * ceil_div(restTokens, 64) : smallTiles;
+                int64_t const behind = a.pieces ? (int64_t) (a.N / 64) * ceil_div(a.T - a.tokMain * kBig, 64) : smallTiles;
                 hipLaunchKernelGGL((int8_linear_dma_kernel<IL_OUT, EPI>), dim3((uint32_t) (a.persist + behind)), dim3(512), 0,
                     stream, a);
                 return check_launch("int8_linear_dma_kernel");
@@ -2542,6 +2566,21 @@ int fp16_linear_check(trtamd_fp16_linear_params const& p)
 }
 
 } // namespace trtamd
+
+extern "C" int trtamd_test_linear_plan(int32_t interleaved, int32_t T, int32_t row_bytes, int32_t N, int32_t gelu)
+{
+    using namespace trtamd;
+    if (T <= 0 || row_bytes <= 0 || N <= 0 || row_bytes % 64 != 0 || N % 32 != 0)
+    {
+        return -1;
+    }
+    LinearArgs a{};
+    a.T = T;
+    a.K = row_bytes;
+    a.N = N;
+    int64_t const smallTiles = place_large_tiles(a);
+    return interleaved ? plan_behind_large_tiles<true>(a, smallTiles, gelu != 0) : plan_behind_large_tiles<false>(a, smallTiles, gelu != 0);
+}
 
 extern "C" int trtamd_int8_linear(trtamd_stream_t stream, trtamd_int8_linear_params const* p)
 {

@@ -140,13 +140,21 @@ def test_pieces_up_to_the_extent_of_their_grid(plan, T):
 
 
 # tiles of linear operands: stages of 128 bytes of k (64 FP16 values), rings of two to five of them.  One stage, as many as
-# the ring has and one more; a last line that is half there; token and channel counts on both sides of a tile's edge.
-@pytest.mark.parametrize("plan", [2, 4, 5, 10, 11, 12, 13, 14])
-@pytest.mark.parametrize("T,K,N", [(1, 64, 32), (63, 128, 96), (191, 192, 128), (193, 256, 160), (257, 384, 288), (65, 160, 64),
-                                   (130, 608, 224)])
-def test_linear_tiles_of_whole_lines(plan, T, K, N):
+# the ring has and one more; token and channel counts on both sides of a tile's edge.
+WHOLE_LINES = [(plan, *shape) for plan in (2, 4, 5, 10, 11, 12, 13, 14) for shape in
+               [(1, 64, 32), (63, 128, 96), (191, 192, 128), (193, 256, 160), (257, 384, 288)]]
+# rows that end within a line: stages of 64 bytes and tiles of their own, k longer than their rings (three and four stages) and
+# as long as one stage
+HALF_LINES = [(plan, *shape) for plan in (1, 2, 3, 4) for shape in
+              [(1, 32, 32), (65, 160, 64), (130, 608, 224), (257, 96, 160), (255, 288, 128)]]
+
+
+@pytest.mark.parametrize("plan,T,K,N", WHOLE_LINES + HALF_LINES)
+def test_linear_tiles_of_linear_operands(plan, T, K, N):
     """FP16 against binary64 and against the pieces' results; INT8 with linear operands byte for byte against the
-    register-staged kernel; nothing written behind the last row."""
+    register-staged kernel; every shape through the kernel that it is listed for."""
+    with tuning("TRTAMD_LINEAR_PLAN", plan):
+        assert capi.api().test_linear_plan(0, T, 2 * K, N, 0) == plan == capi.api().test_linear_plan(0, T, 2 * K, N, 1)
     r = rng(97 + T)
     x = r.standard_normal((T, K)).astype(np.float16)
     w = (0.05 * r.standard_normal((N, K))).astype(np.float16)

@@ -1,0 +1,42 @@
+"""Which kernel a linear layer's sizes lead to, asked of the launcher itself (include/trtamd_test_hooks.h); no launch is made."""
+import pytest
+
+from tensorrt_amd import capi
+
+INTERLEAVED, LINEAR = 1, 0
+# the plans (TRTAMD_LINEAR_PLAN) that have a kernel: interleaved operands, linear ones whose rows are whole lines of 128
+# bytes, linear ones whose rows end within a line
+KERNELS = {(INTERLEAVED, 1024): {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12}, (LINEAR, 1536): {2, 4, 5, 8, 9, 10, 11, 12, 13, 14},
+           (LINEAR, 1472): {1, 2, 3, 4, 8, 9}}
+
+
+def plan(layout, T, row_bytes, N, gelu=0):
+    return capi.api().test_linear_plan(layout, T, row_bytes, N, gelu)
+
+
+@pytest.fixture
+def forced():
+    api = capi.api()
+    yield lambda n: api.check(api.test_set_tuning(b"TRTAMD_LINEAR_PLAN", n))
+    api.check(api.test_reset_tuning(b"TRTAMD_LINEAR_PLAN"))
+
+
+def test_sizes_that_no_layer_has():
+    for sizes in ((0, 64, 32), (1, 0, 32), (1, 96, 32), (1, 64, 0), (1, 64, 48), (-1, 64, 32)):
+        assert plan(LINEAR, *sizes) == -1
+
+
+@pytest.mark.parametrize("layout,row_bytes", KERNELS)
+def test_a_plan_is_taken_where_it_has_a_kernel_and_passed_over_where_not(forced, layout, row_bytes):
+    chosen = plan(layout, 130, row_bytes, 96)
+    for n in range(0, 16):
+        forced(n)
+        assert plan(layout, 130, row_bytes, 96) == (n if n in KERNELS[layout, row_bytes] else chosen), n
+
+
+@pytest.mark.parametrize("T,row_bytes,N", [(16384, 2112, 3168), (33289, 1472, 2208), (7765, 6208, 768), (2048, 4160, 1024)])
+@pytest.mark.parametrize("gelu", [0, 1])
+def test_many_tokens_with_rows_that_end_within_a_line(T, row_bytes, N, gelu):
+    """The layers whose launches tiles of 128 x 256 shorten most against the 128 x 128 and 64 x 64 ones take them, or at 2048
+    tokens something else than those two."""
+    assert plan(LINEAR, T, row_bytes, N, gelu) in ({1} if T > 2048 else {1, 3})
