@@ -35,6 +35,8 @@ TRTAMD_API int trtamd_test_reset_tuning(char const* name);
 /* The number (TRTAMD_LINEAR_PLAN) of the kernel that a linear layer with both operands interleaved, or both linear, takes at
  * these sizes under the switches as they are; row_bytes: K in INT8, 2 K in FP16.  -1: sizes that no layer has. */
 TRTAMD_API int trtamd_test_linear_plan(int32_t interleaved, int32_t T, int32_t row_bytes, int32_t N, int32_t gelu);
+/* How often the calling thread has worked such a number out, rather than remembered it. */
+TRTAMD_API int64_t trtamd_test_linear_estimates(void);
 
 #ifdef __cplusplus
 }

@@ -2215,8 +2215,11 @@ int cheapest_plan(LinearArgs const& a, int64_t smallTiles, bool gelu, int plan)
     return plan;
 }
 
+thread_local int64_t gLinearEstimates = 0; // plans worked out rather than remembered, for trtamd_test_linear_estimates
+
 // The same, remembered by each thread for the sizes it asked for last: the layers of a pass ask for the same few plans over
-// and over, and the estimates take 0.3 us where a short launch costs the host 3.
+// and over, and the estimates take 0.3 us where a short launch costs the host 3.  Four layers and two halves of a batch are
+// eight sizes; any sixteen of them have a place each, the oldest making room for the next.
 template <bool IL>
 int choose_plan(LinearArgs const& a, int64_t smallTiles, bool gelu)
 {
@@ -2227,13 +2230,23 @@ int choose_plan(LinearArgs const& a, int64_t smallTiles, bool gelu)
     };
     constexpr int kChoices = 16;
     thread_local Choice choices[kChoices] = {};
+    thread_local int oldest = 0;
     int const setting = tuning(Tuning::kLinearPlan);
-    Choice& c = choices[((uint32_t) a.T * 5u + (uint32_t) (a.K >> 6) * 3u + (uint32_t) (a.N >> 5) * 7u + (uint32_t) gelu) % kChoices];
-    if (c.T != a.T || c.K != a.K || c.N != a.N || c.mainTiles != a.mainTiles || c.pieces != a.pieces || c.gelu != (int) gelu
-        || c.setting != setting || c.smallTiles != smallTiles)
+    bool const large = IL && a.mainTiles > 0; // if not, there is nothing for the other tiles to stand behind
+    int const mainTiles = large ? a.mainTiles : 0, pieces = large ? a.pieces : 0;
+    int64_t const behind = large ? smallTiles : 0;
+    for (Choice const& c : choices)
     {
-        c = {a.T, a.K, a.N, a.mainTiles, a.pieces, (int) gelu, setting, cheapest_plan<IL>(a, smallTiles, gelu, setting), smallTiles};
+        if (c.T == a.T && c.K == a.K && c.N == a.N && c.gelu == (int) gelu && c.mainTiles == mainTiles && c.pieces == pieces
+            && c.smallTiles == behind && c.setting == setting)
+        {
+            return c.plan;
+        }
     }
+    ++gLinearEstimates;
+    Choice& c = choices[oldest];
+    oldest = (oldest + 1) % kChoices;
+    c = {a.T, a.K, a.N, mainTiles, pieces, (int) gelu, setting, cheapest_plan<IL>(a, smallTiles, gelu, setting), behind};
     return c.plan;
 }
 
@@ -2580,6 +2593,11 @@ extern "C" int trtamd_test_linear_plan(int32_t interleaved, int32_t T, int32_t r
     a.N = N;
     int64_t const smallTiles = place_large_tiles(a);
     return interleaved ? plan_behind_large_tiles<true>(a, smallTiles, gelu != 0) : plan_behind_large_tiles<false>(a, smallTiles, gelu != 0);
+}
+
+extern "C" int64_t trtamd_test_linear_estimates(void)
+{
+    return trtamd::gLinearEstimates;
 }
 
 extern "C" int trtamd_int8_linear(trtamd_stream_t stream, trtamd_int8_linear_params const* p)

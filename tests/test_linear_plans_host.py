@@ -40,3 +40,32 @@ def test_many_tokens_with_rows_that_end_within_a_line(T, row_bytes, N, gelu):
     """The layers whose launches tiles of 128 x 256 shorten most against the 128 x 128 and 64 x 64 ones take them, or at 2048
     tokens something else than those two."""
     assert plan(LINEAR, T, row_bytes, N, gelu) in ({1} if T > 2048 else {1, 3})
+
+
+def layers(layout, size, hidden, ffn):
+    """The four linear layers of an encoder layer: row bytes, channels, GELU."""
+    return [(layout, size * hidden, 3 * hidden, 0), (layout, size * hidden, hidden, 0), (layout, size * hidden, ffn, 1),
+            (layout, size * ffn, hidden, 0)]
+
+
+@pytest.mark.parametrize("T", [[1], [48], [255], [256], [600], [4096], [9084, 8231], [16384, 16640], [24000, 23999]])
+@pytest.mark.parametrize("model", [(INTERLEAVED, 1, 1024, 4096), (LINEAR, 2, 768, 3072), (LINEAR, 2, 1024, 4096),
+                                   (INTERLEAVED, 1, 768, 3072), (INTERLEAVED, 1, 512, 2048)])
+def test_the_layers_of_a_pass_are_estimated_once(model, T):
+    """One encoder layer after the other asks for the same few plans, as two halves of a batch do in turn: nothing is worked
+    out again."""
+    asked = [(layout, t, row_bytes, n, gelu) for t in T for layout, row_bytes, n, gelu in layers(*model)]
+    first = [plan(*a) for a in asked]
+    before = capi.api().test_linear_estimates()
+    for _ in range(24):
+        assert [plan(*a) for a in asked] == first
+    assert capi.api().test_linear_estimates() == before
+
+
+def test_plans_are_remembered_for_the_switches_that_they_were_made_under(forced):
+    want = plan(LINEAR, 7000, 1536, 768)
+    for n in (10, 14, 2):
+        forced(n)
+        assert plan(LINEAR, 7000, 1536, 768) == n
+    forced(-1)
+    assert plan(LINEAR, 7000, 1536, 768) == want
