@@ -68,8 +68,6 @@ def test_skipln_fp(api, dt, rows, ld, has_bias):
                                    (np.float16, 1032), (np.float16, 4088)])
 @pytest.mark.parametrize("rows", [1, 6, 8192, 8193])
 def test_skipln_fp_few_rows(api, dt, rows, ld):
-    if rows > 6 and ld > 1032:
-        rows = 9
     test_skipln_fp(api, dt, rows, ld, rows % 2 == 0)
 
 
