@@ -868,8 +868,8 @@ __device__ inline SeqInfo pick_sequence_info(FmhaArgs const& a, int rank, int ca
 }
 
 // ------------------------------------------------------------------------------------------
-// INT8, prefix-valid keys (cu_seqlens or no mask at all): the usual case, specialised on the exact
-// number of 64-key blocks so that a query tile is one straight-line instruction stream.
+// INT8, the usual case (cu_seqlens, a packed mask with holes or without, or no mask; scales that keep probabilities within
+// INT8): specialised on the exact number of 64-key blocks so that a query tile is one straight-line instruction stream.
 // ------------------------------------------------------------------------------------------
 
 // The keys that a packed mask leaves a sequence: 64 of them in each m, their number up to the last one in sq.nk; true where
@@ -1538,8 +1538,8 @@ __global__ __launch_bounds__(kWavesF16* kWaveSize) void fmha_f16_kernel(FmhaArgs
 }
 
 // ------------------------------------------------------------------------------------------
-// FP16, prefix-valid keys, launches that leave CUs idle: the same specialisation, but K and V take turns in LDS, one
-// block of V in the place of each block of K as soon as every wavefront has multiplied it.  48 KB for 384 keys instead of
+// FP16, launches that leave CUs idle, on cu_seqlens or a packed mask (with holes too): the same specialisation, but K and V
+// take turns in LDS, one block of V in the place of each block of K as soon as every wavefront has multiplied it.  48 KB for 384 keys instead of
 // 96 KB: three workgroups of four wavefronts share a CU, so that one computes while another waits for its sequence, its K
 // or its V, and a unit's queries are shared out 64 at a time over as many workgroups.  What bounds either kernel is that
 // wait; with one workgroup per CU nothing covered it.  All of Q, K and V come by direct-to-LDS loads, whose number in
@@ -1879,13 +1879,15 @@ __global__ __launch_bounds__(kWavesF16T* kWaveSize)
 }
 
 // ------------------------------------------------------------------------------------------
-// FP16, prefix-valid keys, launches that fill the chip: 32 queries per wavefront, K and V in blocks of 64 keys through two
-// slots of LDS, the softmax kept up from block to block.  A workgroup takes 128 queries, so K and V come from the L2 half
-// as often as above, every fragment read from LDS serves twice the queries, and 36 KB let four workgroups share a CU.
+// FP16, launches that fill the chip, on cu_seqlens or a packed mask (with holes too): 32 queries per wavefront, K and V in
+// blocks of 64 keys through two slots of LDS, the softmax kept up from block to block.  A workgroup takes 128 queries, so K and
+// V come from the L2 half as often as above (32 x 384: 78 MB read there with Q, where the kernel above reads 133), every
+// fragment read from LDS serves twice the queries, and 36 KB let four workgroups share a CU.
 // The weights are relative to a running maximum that is only moved when it would be passed by more than a factor of 2^8,
 // which they and their binary32 sums hold without loss: a branch that is rarely taken after the first block.  What bounds it
-// is issue: per wavefront and block 512 cycles of matrix instructions, as many of exponentials and 400 of other vector work,
-// which overlap in part (~2000 cycles measured).  12 heads, sequences of a third of the length to the length, the
+// is issue, and what does not overlap of it: per wavefront and block 512 cycles of matrix instructions, as many of exponentials
+// and 400 of other vector work, of 2240 that pass (32 x 384, counters: vector ALU 45 %, matrix pipe 23 % of the launch, its
+// start and tail among the rest); with the matrix instructions left out launches take 15 to 23 % less.  12 heads, sequences of a third of the length to the length, the
 // kernels it took the place of / this one, us: 32 x 256 keys 13.9 / 13.1, 32 x 384 21.6 / 19.0, 128 x 256 36.5 / 33.2,
 // 64 x 384 35.8 / 32.8, 16 x 512 22.7 / 18.0, 16 heads x 128 x 384 98.5 / 82.4, 128 x 512 145 / 134.
 // ------------------------------------------------------------------------------------------
@@ -2316,7 +2318,7 @@ int run_i8(hipStream_t stream, FmhaArgs const& a, bool interleaved)
 // Which of the FP16 kernels a launch takes.
 enum class F16Kernel
 {
-    kGENERAL, // packed masks, and strides beyond the 32-bit offsets of the direct-to-LDS loads
+    kGENERAL, // TRTAMD_FMHA_GENERIC, and strides beyond the 32-bit offsets of the direct-to-LDS loads
     kTURNS,
     kSTREAM
 };
@@ -2460,7 +2462,7 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
     a.N = p->h;
     a.S = p->s;
     int const kt = pick_kt(p->s);
-    // FP16, prefix-valid keys: 128 queries per workgroup where that makes three workgroups and more for each of the 256 CUs,
+    // FP16: 128 queries per workgroup where that makes three workgroups and more for each of the 256 CUs,
     // 64 of them and the scores of all their keys in registers where it does not (12 heads: 16 x 256 keys, 384 workgroups of
     // 128, 7.9 against 8.8 us; 32 x 256, 768 of them, 13.9 against 13.1; 16 heads, 8 x 384, 384: 9.6 against 10.2).
     constexpr int kStreamTile = kWavesStream * kStreamQueries;
@@ -2477,7 +2479,7 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         // CU, 768 places): below 896 units two workgroups per unit, which also evens out a single round of units of
         // very different lengths (768 units of 128-384 keys: 24.9 against 27.8 us; 512 units: 18.7 against 23.1 us;
         // 896 units: 29.1 against 28.1 us), and more of them only to reach one round (256 units: three, 12.6 us
-        // against 13.1 with two and 17.4 with one; at most four).  FP16 with a packed mask (its K and V take most of a
+        // against 13.1 with two and 17.4 with one; at most four).  The general FP16 kernel (its K and V take most of a
         // CU's LDS, one workgroup per CU, and staging them is 40 % of a workgroup's time): only below 160 units (192 units
         // of 192-384 keys: 15.3 us alone, 17.5 us shared by two; 144 units: 14.9 against 12.9 us).  The other FP16 kernels
         // take 64 or 128 queries each, of as many as the kernel has room for: a sequence longer than s that still fits

@@ -11,11 +11,17 @@
 // either layout.
 //
 // Tiling: a workgroup owns BM channels x BN tokens, its waves a WM x WN grid of (MT*32) x (NT*32)
-// sub-tiles kept in INT32 accumulators.  One stage is 64 bytes of k for the whole tile (two MFMA
-// steps).  Global loads are 16 bytes per lane with consecutive lanes on consecutive addresses; a
-// fragment sits in LDS row-major with a one-bit swizzle, so LDS writes and the 16-byte-per-lane
-// fragment reads are both conflict-free.  Stages are double-buffered in LDS and the loads run two
-// stages ahead of the multiplication through two register sets.
+// sub-tiles kept in INT32 (FP16 operands: binary32) accumulators.  Global loads are 16 bytes per lane,
+// and a swizzle keeps the 16-byte-per-lane fragment reads from LDS conflict-free.  Three ways to bring
+// a tile's operands in:
+//   operands of one layout, chip-filling or middling launches: rings of stages of 64 or, for linear rows
+//     of whole lines, 128 bytes of k by direct-to-LDS loads (linear_tile_dma; persistent 256 x 256 tiles of
+//     interleaved operands: linear_tile_run_dma);
+//   operands of one layout, few tokens: pieces whose eight wavefronts split k (linear_piece_kernel,
+//     linear_piece_dma_kernel, linear_piece64);
+//   operands of two layouts, INT32 and FP16 outputs of INT8 operands, or TRTAMD_LINEAR_DIRECT=0: stages of
+//     64 bytes, double-buffered in LDS, through two register sets that run two stages ahead (linear_tile,
+//     linear_tile_run).
 //
 // Activations, weights and outputs may be in the linear layout [R][C] or in the 32-interleaved
 // layout [C/32][R][32] that the interleaved encoder plugins use; the interleaved one makes every

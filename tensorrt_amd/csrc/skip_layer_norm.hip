@@ -251,7 +251,7 @@ int launch_rows_as(hipStream_t stream, int ld, int64_t rows, T const* in, T cons
     return bias ? launch(skipln_rows_kernel<T, NV, R, true, FEW>) : launch(skipln_rows_kernel<T, NV, R, false, FEW>);
 }
 
-// Up to here one form is the faster throughout, beyond it the bytes set the time of either (us, masked loads / FEW: FP32 x 768,
+// Up to here FEW is the faster or as fast within the noise, beyond it the bytes set the time of either (us, masked loads / FEW: FP32 x 768,
 // 128 rows 2.89 / 2.77, 1024 rows 4.09 / 3.73, 2048 rows 5.00 / 4.60, 8192 rows 12.6 / 12.4, 32000 rows 45.1 / 47.3; FP16 x
 // 384, 128 rows 2.40 / 2.25, 8192 rows 6.14 / 6.16, 32000 rows 18.1 / 18.7).
 constexpr int64_t kFewRows = 8192;

@@ -262,6 +262,8 @@ def config_rows(api, torch, steps: int = 100, seed: int = 1, cpu: bool = True, l
     del sets
 
     # ---- C3: fused attention FP16, BERT-base, B=32, var-seqlen (v5) ---------------------------------
+    # 384 (sequence, head) units are 384 workgroups of 128 queries at S=128 and 1152 at S=384; launches of 768 and more take those
+    f16_kernel = {128: "fmha_f16_turns_kernel", 384: "fmha_f16_stream_kernel"}.get
     for S in (128, 384):
         B, N, d = 32, 12, 64
         lens = r.integers(S // 2, S + 1, B)
@@ -288,7 +290,7 @@ def config_rows(api, torch, steps: int = 100, seed: int = 1, cpu: bool = True, l
                     q, k, v = (cq[lo:hi, :, i].transpose(0, 1) for i in range(3))
                     torch.softmax(q @ k.transpose(1, 2) * 0.125, -1) @ v
             cpu_s = _cpu_time(attn_cpu)
-        report("C3", "QKV-to-context v5 (fmha_f16_turns_kernel)", "fp16", f"B=32 N=12 S={S}, {T} tokens", t, ops=ops,
+        report("C3", f"QKV-to-context v5 ({f16_kernel(S)})", "fp16", f"B=32 N=12 S={S}, {T} tokens", t, ops=ops,
                peak_ops=PEAK_F16, cpu_s=cpu_s)
 
     # ---- C3, the fixed [S,B,N,3,d] layout with the packed key mask (v4 plugin with a mask input) ----------
@@ -310,7 +312,7 @@ def config_rows(api, torch, steps: int = 100, seed: int = 1, cpu: bool = True, l
         p.b, p.h, p.s, p.d = B, N, S, d
         p.scale_bmm1, p.scale_softmax, p.scale_bmm2 = half2_bits(0.125), half2_bits(1.0), half2_bits(1.0)
         t = timeit(lambda: api.check(api.fused_mha_run(stream, 1, C.byref(p))))
-        report("C3", "QKV-to-context v4, packed mask (fmha_f16_kernel)", "fp16", f"S={S} B=32 N=12, fixed layout", t,
+        report("C3", f"QKV-to-context v4, packed mask ({f16_kernel(S)})", "fp16", f"S={S} B=32 N=12, fixed layout", t,
                ops=4.0 * d * N * float(np.sum(lens.astype(np.float64) ** 2)), peak_ops=PEAK_F16,
                note="every query row of the S x B tensor is computed; ops count valid lengths only")
 
