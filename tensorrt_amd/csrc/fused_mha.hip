@@ -1886,7 +1886,7 @@ __global__ __launch_bounds__(kWavesF16T* kWaveSize)
 // The weights are relative to a running maximum that is only moved when it would be passed by more than a factor of 2^8,
 // which they and their binary32 sums hold without loss: a branch that is rarely taken after the first block.  What bounds it
 // is issue, and what does not overlap of it: per wavefront and block 512 cycles of matrix instructions, as many of exponentials
-// and 400 of other vector work, of 2240 that pass (32 x 384, counters: vector ALU 45 %, matrix pipe 23 % of the launch, its
+// and 400 of other vector work, of 2180 that pass (32 x 384, counters: vector ALU 45 %, matrix pipe 23 % of the launch, its
 // start and tail among the rest); with the matrix instructions left out launches take 15 to 23 % less.  12 heads, sequences of a third of the length to the length, the
 // kernels it took the place of / this one, us: 32 x 256 keys 13.9 / 13.1, 32 x 384 21.6 / 19.0, 128 x 256 36.5 / 33.2,
 // 64 x 384 35.8 / 32.8, 16 x 512 22.7 / 18.0, 16 heads x 128 x 384 98.5 / 82.4, 128 x 512 145 / 134.
