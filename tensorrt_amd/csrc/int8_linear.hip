@@ -1767,16 +1767,24 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_kernel(uint64_t co
 
 // The same pieces for linear operands, where the 32 rows of a fragment are 32 separate lines (read straight into
 // registers, 40 tokens x 3072 -> 768 in FP16 take 16 us): every wavefront brings its own k range in through a ring of
-// direct-to-LDS loads of its own (units, swizzle and fragment reads of the linear tiles; 7.2 us), so there is still no
-// barrier before the partial accumulators meet.  K a multiple of 64 bytes.
-template <bool IL_OUT, int EPI, int CB, int TB, int RING, int PER_SIMD>
-__global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(uint64_t const w, uint64_t const a, uint64_t const alpha,
+// direct-to-LDS loads of its own (units, swizzle and fragment reads of the linear tiles), so there is still no barrier before
+// the partial accumulators meet.  K a multiple of 32 KS bytes.
+//
+// KS = 4, rows in whole lines of 128 bytes, wherever K comes in those: what bounds a piece is what its CU can read from the L2,
+// and that is 65 bytes a clock in whole lines and 31 in halves of them (168 workgroups of 96 rows x 6144 bytes, loads alone:
+// 5.8 against 9.9 us).  The stages are twice as long for it, so four wavefronts share k instead of eight, with the LDS of the
+// other four for their rings: 448 tokens x 3072 -> 768, FP16, pieces of 32 x 64: 11.5 -> 9.2 us by itself.  Pieces of 32 x 32
+// leave room for two workgroups on a CU; rings of four stages, or eight wavefronts with rings of two, are slower.
+template <bool IL_OUT, int EPI, int CB, int TB, int RING, int NW, int KS, int PER_SIMD>
+__global__ __launch_bounds__(NW * 64, PER_SIMD) void linear_piece_dma_kernel(uint64_t const w, uint64_t const a, uint64_t const alpha,
     uint64_t const beta, int const K, int const T, int const N, int const parts, int const perPart, LinearArgs const rest)
 {
-    constexpr int NW = 8;
     LinearArgs const p = piece_args(w, a, alpha, beta, K, T, N, parts, perPart, rest);
-    constexpr int kLoads = (CB + TB) * 2;
+    constexpr int kLoads = (CB + TB) * KS;
     constexpr int STAGE = kLoads * 1024;
+    constexpr int kUnits = CB * TB * 4; // quarters of blocks: what a wavefront adds up and stores at a time
+    constexpr int kOwn = kUnits / NW > 1 ? kUnits / NW : 1;
+    static_assert(kUnits % NW == 0 || kUnits < NW, "the same number of them for each wavefront that has any");
     static_assert(CB * TB * 4096 <= RING * STAGE, "the partial accumulators go where the wavefront's stages were");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[NW * RING * STAGE];
     int const lane = threadIdx.x & 63;
@@ -1785,27 +1793,31 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(uint64_
     int const n0 = (int) blockIdx.x * (32 * CB), t0 = (int) blockIdx.y * (32 * TB), kpart = (int) blockIdx.z;
     uint8_t* const own = lds + wave * (RING * STAGE);
     uint32_t const ownBase = (uint32_t) (size_t) (__attribute__((address_space(3))) uint8_t*) own;
-    int const rr = lane >> 2;
-    uint32_t const chunk = (uint32_t) ((lane & 3) ^ (rr >> 2)) * 16u;
     uint32_t off[kLoads];
 #pragma unroll
     for (int u = 0; u < kLoads; ++u)
     {
-        int const r = (u >> 1) * 32 + (u & 1) * 16 + rr;
-        int const g = u < 2 * CB ? min(n0 + r, p.N - 1) : min(t0 + r - 32 * CB, p.T - 1);
-        off[u] = (uint32_t) g * (uint32_t) p.K + chunk;
+        int const r = u * (32 / KS) + lane / (2 * KS); // row of the stage: weights, then tokens
+        int const g = u < KS * CB ? min(n0 + r, p.N - 1) : min(t0 + r - 32 * CB, p.T - 1);
+        uint32_t const chunk = (uint32_t) ((lane & (2 * KS - 1)) ^ (KS == 2 ? (r >> 2) & 3 : (r >> 1) & 7));
+        off[u] = (uint32_t) g * (uint32_t) p.K + chunk * 16u;
     }
-    static_assert(CB * TB * 4 <= NW, "a quarter of a block for each wavefront at most");
-    QuadScales const scales = load_quad_scales<EPI>(p, n0 + (wave / (4 * TB)) * 32 + 8 * (wave & 3) + 4 * half);
-    int const nk = min(p.K / 64, (kpart + 1) * p.perPart); // stages up to the end of this workgroup's
+    QuadScales scales[kOwn];
+#pragma unroll
+    for (int v = 0; v < kOwn; ++v)
+    {
+        int const u = v * NW + wave;
+        scales[v] = load_quad_scales<EPI>(p, n0 + (u / (4 * TB)) * 32 + 8 * (u & 3) + 4 * half);
+    }
+    int const nk = min(p.K / (32 * KS), (kpart + 1) * p.perPart); // stages up to the end of this workgroup's
     int const per = ceil_div(p.perPart, NW), first = kpart * p.perPart + wave * per;
     int const steps = max(0, min(per, nk - first));
     auto fetch = [&](int step, int slot) {
-        uint64_t const k = (uint64_t) (first + step) * 64u;
+        uint64_t const k = (uint64_t) (first + step) * (32u * KS);
 #pragma unroll
         for (int u = 0; u < kLoads; ++u)
         {
-            load_to_lds16_sbase((u < 2 * CB ? p.w : p.a) + k, off[u], ownBase + (uint32_t) (slot * STAGE + u * 1024));
+            load_to_lds16_sbase((u < KS * CB ? p.w : p.a) + k, off[u], ownBase + (uint32_t) (slot * STAGE + u * 1024));
         }
     };
     AccT<EPI> acc[CB][TB];
@@ -1825,20 +1837,21 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(uint64_
     auto multiply = [&](int slot) {
         uint8_t const* base = own + slot * STAGE;
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
+        for (int ks = 0; ks < KS; ++ks)
         {
-            int const fr = row & 15;
-            int const o = (row >> 4) * 1024 + fr * 64 + (((ks * 2 + half) ^ (fr >> 2)) << 4);
+            int const chunk = ks * 2 + half, fr = row & 15;
+            int const o = KS == 2 ? (row >> 4) * 1024 + fr * 64 + ((chunk ^ (fr >> 2)) << 4)
+                                  : row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4);
             i32x4 fa[CB], fb[TB];
 #pragma unroll
             for (int i = 0; i < CB; ++i)
             {
-                fa[i] = *reinterpret_cast<i32x4 const*>(base + i * 2048 + o);
+                fa[i] = *reinterpret_cast<i32x4 const*>(base + i * (KS * 1024) + o);
             }
 #pragma unroll
             for (int j = 0; j < TB; ++j)
             {
-                fb[j] = *reinterpret_cast<i32x4 const*>(base + (CB + j) * 2048 + o);
+                fb[j] = *reinterpret_cast<i32x4 const*>(base + (CB + j) * (KS * 1024) + o);
             }
 #pragma unroll
             for (int i = 0; i < CB; ++i)
@@ -1892,8 +1905,14 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(uint64_
         }
     }
     __syncthreads();
-    if (int const u = wave; u < CB * TB * 4)
+#pragma unroll
+    for (int v = 0; v < kOwn; ++v)
     {
+        int const u = v * NW + wave;
+        if (u >= kUnits)
+        {
+            break;
+        }
         Acc4 t = reinterpret_cast<Acc4 const*>(lds)[u * 64 + lane];
 #pragma unroll
         for (int w = 1; w < NW; ++w)
@@ -1903,7 +1922,7 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(uint64_
         int const b = u >> 2, q = u & 3, cb = n0 + (b / TB) * 32, tb = t0 + (b % TB) * 32;
         if (cb < p.N)
         {
-            store_quad<IL_OUT, EPI>(p, t, scales, cb + 8 * q + 4 * half, tb + row, kpart);
+            store_quad<IL_OUT, EPI>(p, t, scales[v], cb + 8 * q + 4 * half, tb + row, kpart);
         }
     }
 }
@@ -1924,7 +1943,9 @@ __global__ __launch_bounds__(512, PER_SIMD) void linear_piece_dma_kernel(uint64_
 // The constants are fits.  Linear operands: to launches by themselves on the four layers of 768- and 1024-channel FP16
 // encoders (graph replays, weights in the last-level cache), 16 to 33289 tokens, on two GPUs, one of them with the uneven
 // engines.  The plan they choose takes 0.8 % more than the best of all in the mean (24 % at most, a launch at the edge
-// of a second round); the kernels and the choice before took 13 % more (50 % at most).
+// of a second round); the kernels and the choice before took 13 % more (50 % at most).  The pieces' among them are fits to the
+// same layers at 16 to 1400 tokens since they read whole lines, 152 launches, times the 1.18 by which the tiles' constants
+// exceeded that GPU's times: 0.2 % more than the best of six plans in the mean, 5 % at most.
 // Linear operands whose rows end within a line have kernels and constants of their own: stages of 64 bytes, tiles of up to 128 x
 // 256, and constants fitted to launches by themselves before the other linear operands had stages of whole lines.  10 layers of
 // 96 to 3104 channels, 40 to 33289 tokens, FP16 and INT8, 240 launches: 6.5 % less in the mean than when all linear operands
@@ -1982,8 +2003,8 @@ constexpr TileCost kTileCosts[3][kLinearPlans] = {
     {{}, {}, {128, 128, 2, 4.64f, 0.00f, 0.231f, 0.60f, 0.61f, 1.02f, 0.40f, 0.25f}, {},
         {64, 64, 2, 3.82f, 0.29f, 0.082f, 0.23f, 0.70f, 0.89f, 0.63f, 0.34f},
         {128, 128, 1, 4.02f, 0.77f, 0.142f, 0.99f, 0.f, 1.30f, 0.77f, 0.51f, 0.10f}, {}, {},
-        {32, 64, 1, 2.77f, 0.86f, 0.064f, 0.27f, 0.f, 1.03f, 0.71f, 0.62f, 0.00f},
-        {32, 32, 1, 2.90f, 0.65f, 0.046f, 0.20f, 0.f, 1.12f, 0.71f, 0.32f, 0.08f},
+        {32, 64, 1, 1.77f, 1.47f, 0.058f, 0.16f, 0.f, 0.98f, 0.83f, 0.40f},
+        {32, 32, 2, 2.56f, 0.18f, 0.045f, 0.14f, 0.86f, 1.03f, 0.69f, 0.20f},
         {256, 256, 1, 0.00f, 4.48f, 0.440f, 1.88f, 0.f, 1.02f, 0.54f, 0.97f, 0.11f},
         {256, 192, 1, 5.13f, 0.01f, 0.388f, 1.26f, 0.f, 1.35f, 0.67f, 0.56f, 0.15f},
         {128, 192, 2, 4.47f, 0.10f, 0.289f, 0.70f, 0.78f, 0.99f, 0.47f, 0.38f},
@@ -2071,17 +2092,18 @@ int launch_tiles(hipStream_t stream, LinearArgs const& a, Kernel kernel, int thr
     return check_launch("int8_linear");
 }
 
-// The same for pieces of `channels` x `tokens`, in as many parts as a.parts says.
+// The same for pieces of `channels` x `tokens` by `threads` threads, stages of `stage` bytes of k dealt to them, in as many parts
+// as a.parts says.
 template <bool IL, typename Kernel>
-int launch_pieces(hipStream_t stream, LinearArgs a, Kernel kernel, int channels, int tokens)
+int launch_pieces(hipStream_t stream, LinearArgs a, Kernel kernel, int channels, int tokens, int threads, int stage)
 {
     uint32_t const nbm = (uint32_t) ceil_div(a.N, channels);
     a.tokMain = ceil_div(a.T, tokens);
     a.mainTiles = (int) nbm * a.tokMain * a.parts;
-    a.perPart = ceil_div(a.K / (IL ? 32 : 64), a.parts);
-    uint32_t const behind = IL ? prefetch_workgroups(a, 512) : 0u;
+    a.perPart = ceil_div(a.K / stage, a.parts);
+    uint32_t const behind = IL ? prefetch_workgroups(a, threads) : 0u;
     hipLaunchKernelGGL(kernel, dim3(nbm, (uint32_t) a.tokMain, (uint32_t) a.parts + ceil_div(behind, nbm * (uint32_t) a.tokMain)),
-        dim3(512), 0, stream, address(a.w), address(a.a), address(a.alpha), address(a.beta), a.K, a.T, a.N, a.parts,
+        dim3(threads), 0, stream, address(a.w), address(a.a), address(a.alpha), address(a.beta), a.K, a.T, a.N, a.parts,
         a.perPart, a);
     return check_launch("int8_linear");
 }
@@ -2123,18 +2145,10 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
         case kTile256x256: return run(linear_tile_kernel<IL, IL_OUT, EPI, 4, 2, 2, 4, 4, 2>, 512);
         case kTile256x192: return run(linear_tile_kernel<IL, IL_OUT, EPI, 4, 2, 2, 3, 5, 2>, 512);
         case kTile128x192: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 3, 4, 2>, 256);
-        case kPiece32x64: return launch_pieces<IL>(stream, a, linear_piece_kernel<IL_OUT, EPI, 1, 2, 4, 4>, 32, 64);
-        case kPiece32x32: return launch_pieces<IL>(stream, a, linear_piece_kernel<IL_OUT, EPI, 1, 1, 8, 4>, 32, 32);
+        case kPiece32x64: return launch_pieces<IL>(stream, a, linear_piece_kernel<IL_OUT, EPI, 1, 2, 4, 4>, 32, 64, 512, 32);
+        case kPiece32x32: return launch_pieces<IL>(stream, a, linear_piece_kernel<IL_OUT, EPI, 1, 1, 8, 4>, 32, 32, 512, 32);
         default: break;
         }
-    }
-    else if (plan == kPiece32x64)
-    {
-        return launch_pieces<IL>(stream, a, linear_piece_dma_kernel<IL_OUT, EPI, 1, 2, 3, 2>, 32, 64);
-    }
-    else if (plan == kPiece32x32)
-    {
-        return launch_pieces<IL>(stream, a, linear_piece_dma_kernel<IL_OUT, EPI, 1, 1, 4, 2>, 32, 32);
     }
     else if (a.K % 128 != 0)
     {
@@ -2145,6 +2159,8 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
         case kTile128x128: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 4, 2, 1, 4, 4>, 512);
         case kTile64x128: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 2, 4, 3>, 256);
         case kTile64x64: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 1, 1, 4, 4>, 256);
+        case kPiece32x64: return launch_pieces<IL>(stream, a, linear_piece_dma_kernel<IL_OUT, EPI, 1, 2, 3, 8, 2, 2>, 32, 64, 512, 64);
+        case kPiece32x32: return launch_pieces<IL>(stream, a, linear_piece_dma_kernel<IL_OUT, EPI, 1, 1, 4, 8, 2, 2>, 32, 32, 512, 64);
         default: break;
         }
     }
@@ -2152,6 +2168,8 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
     {
         switch (plan)
         {
+        case kPiece32x64: return launch_pieces<IL>(stream, a, linear_piece_dma_kernel<IL_OUT, EPI, 1, 2, 3, 4, 4, 1>, 32, 64, 256, 128);
+        case kPiece32x32: return launch_pieces<IL>(stream, a, linear_piece_dma_kernel<IL_OUT, EPI, 1, 1, 2, 4, 4, 2>, 32, 32, 256, 128);
         case kTile256x256: return run(linear_tile_kernel<IL, IL_OUT, EPI, 4, 2, 2, 4, 2, 2, 4>, 512);
         case kTile256x192: return run(linear_tile_kernel<IL, IL_OUT, EPI, 4, 2, 2, 3, 2, 2, 4>, 512);
         case kTile128x192: return run(linear_tile_kernel<IL, IL_OUT, EPI, 2, 2, 2, 3, 2, 2, 4>, 256);
@@ -2175,11 +2193,12 @@ int launch_partial(hipStream_t stream, LinearArgs a, int parts, void* partial, W
     a.prefetch = prefetch;
     if constexpr (IL)
     {
-        return launch_pieces<IL>(stream, a, linear_piece_kernel<false, EPI, 1, 1, 8, 4>, 32, 32);
+        return launch_pieces<IL>(stream, a, linear_piece_kernel<false, EPI, 1, 1, 8, 4>, 32, 32, 512, 32);
     }
     else
     {
-        return launch_pieces<IL>(stream, a, linear_piece_dma_kernel<false, EPI, 1, 1, 4, 2>, 32, 32);
+        return a.K % 128 == 0 ? launch_pieces<IL>(stream, a, linear_piece_dma_kernel<false, EPI, 1, 1, 4, 4, 4, 1>, 32, 32, 256, 128)
+                              : launch_pieces<IL>(stream, a, linear_piece_dma_kernel<false, EPI, 1, 1, 4, 8, 2, 2>, 32, 32, 512, 64);
     }
 }
 

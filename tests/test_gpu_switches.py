@@ -179,6 +179,33 @@ def test_linear_tiles_of_linear_operands(plan, T, K, N):
         assert np.array_equal(got, want)
 
 
+# pieces of linear operands: whole lines (K a multiple of 64 FP16 values; four wavefronts, rings of two and three stages) and
+# rows that end within a line (eight, rings of three and four).  Fewer stages than wavefronts, as many as their rings have and
+# one more, wavefronts with fewer than the others or none.
+@pytest.mark.parametrize("plan", [8, 9])
+@pytest.mark.parametrize("T,K,N", [(1, 64, 32), (33, 256, 96), (64, 512, 32), (65, 576, 160), (31, 832, 64), (70, 1600, 96),
+                                   (32, 3072, 128), (33, 32, 64), (63, 608, 96), (65, 1056, 32)])
+def test_pieces_of_linear_operands(plan, T, K, N):
+    """FP16 against binary64 and the oracle; INT8 byte for byte against the register-staged kernel."""
+    r = rng(92 + T)
+    x = r.standard_normal((T, K)).astype(np.float16)
+    w = (0.05 * r.standard_normal((N, K))).astype(np.float16)
+    alpha, beta = r.uniform(0.5, 1.5, N).astype(np.float32), (0.1 * r.standard_normal(N)).astype(np.float32)
+    with tuning("TRTAMD_LINEAR_PLAN", plan):
+        assert capi.api().test_linear_plan(0, T, 2 * K, N, 0) == plan
+        got = run_fp16(x, w, alpha, beta, False)
+        gelu = run_fp16(x, w, alpha, beta, True)
+    assert_fp_close(got, (x.astype(np.float64) @ w.astype(np.float64).T) * alpha + beta, what=f"plan {plan} against binary64")
+    assert_fp_close(gelu, oracle.fp16_linear(x, w, alpha, beta, gelu=True), what=f"plan {plan} GELU")
+    a, w8, al, be = problem(93 + T, T, 2 * K, N)
+    for out_il in (False, True):
+        with tuning("TRTAMD_LINEAR_DIRECT", 0):
+            want = run_gpu(a, w8, al, be, capi.LINEAR_AFFINE, out_il=out_il)
+        with tuning("TRTAMD_LINEAR_PLAN", plan):
+            got = run_gpu(a, w8, al, be, capi.LINEAR_AFFINE, out_il=out_il)
+        assert np.array_equal(got, want)
+
+
 # the same tiles of interleaved operands: stages of 64 bytes, rings of four and five
 @pytest.mark.parametrize("plan", [7, 10, 11, 12])
 @pytest.mark.parametrize("T,K,N", [(1, 64, 32), (191, 256, 128), (193, 320, 160), (257, 384, 288), (130, 1088, 224)])
