@@ -2552,11 +2552,17 @@ bool interleaved(trtamd_int8_linear_params const& p)
 
 } // namespace
 
+// Pieces, whose launches are as long as the trip of their weights; and layers with longer rows than they have of them, whose
+// workgroups walk a chain of stages that each wait for weights from memory (a model of 24 layers does not stay in the last-level
+// cache): a pass of 24 layers of 1024 channels with the second feed-forward layer's weights fetched by the projection, us: 316
+// tokens 707 -> 688, 531 811 -> 805, 1006 912 -> 905, 1509 1148 -> 1136, 2810 1632 -> 1592, 3775 1881 -> 1853, 6782 2830 -> 2806,
+// no difference where the projection leaves no CU idle.  The first feed-forward layer's weights ahead of their launch cost up to
+// 1 %, the other two's bring nothing.
 WeightPrefetch prefetch_of(trtamd_int8_linear_params const& next)
 {
     // N: the channel blocks have to come round to the same XCD in every k-slab
     if (!interleaved(next) || next.N % 256 != 0
-        || !is_piece(small_plan<true>(args_of(next), next.epilogue == TRTAMD_LINEAR_GELU)))
+        || (next.K <= next.N && !is_piece(small_plan<true>(args_of(next), next.epilogue == TRTAMD_LINEAR_GELU))))
     {
         return {nullptr, 0};
     }

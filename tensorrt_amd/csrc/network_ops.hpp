@@ -10,8 +10,8 @@
 namespace trtamd
 {
 
-// Weights that an INT8 linear launch should bring into the caches beside its own work, for a later launch of few tokens:
-// such a launch is bound by the latency of its weights, and the CUs that the launches before it leave idle can fetch them.
+// Weights that an INT8 linear launch should bring into the caches beside its own work, for a later launch that is bound by the
+// latency of its weights: few tokens, or long rows.  The CUs that the launches before it leave idle can fetch them.
 // `units` KB of a 32-interleaved matrix, each 32 output channels of one k-slab; the 32-channel block with number c is read
 // on XCD c % 8 and fetched there.  data == nullptr: nothing.
 struct WeightPrefetch

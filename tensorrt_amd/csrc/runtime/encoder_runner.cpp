@@ -465,8 +465,8 @@ private:
         int32_t* partial;
         trtamd_half_t* out;
         float lastScale;
-        // What few tokens ask for (network_ops.hpp), the same in every layer: the weights to fetch ahead, and the number of
-        // workgroups that share a piece of the second feed-forward layer.
+        // What the launches ask of each other (network_ops.hpp), the same in every layer: the weights to fetch ahead, and the
+        // number of workgroups that share a piece of the second feed-forward layer.
         WeightPrefetch qkvAhead, projAhead, ffn1Ahead, ffn2Ahead;
         int ffn2Parts;
 

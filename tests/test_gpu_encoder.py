@@ -217,6 +217,23 @@ def test_native_runner_with_few_tokens_of_1024_channels(large_model, lens):
         assert np.array_equal(got.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("lens", [[257], [300, 16], [384, 147], [384] * 4, [384] * 7 + [122], [384] * 14 + [1]])
+def test_native_runner_fetches_long_rows_ahead(large_model, lens):
+    """The second feed-forward layer's weights are fetched by the projection's launch where it leaves CUs idle, beside tiles of
+    each kind and beside pieces, up to launches that have nothing to spare: the bytes of the chain of single operations."""
+    import torch
+    cfg, enc = large_model
+    r = rng(33 + sum(lens))
+    c = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    t = int(c[-1])
+    i, s = r.integers(0, cfg.vocab, t).astype(np.int32), r.integers(0, 2, t).astype(np.int32)
+    want = enc.enqueue(i, s, c).cpu().numpy()
+    for _ in range(2):
+        got = enc.enqueue_native(i, s, c)
+        torch.cuda.synchronize()
+        assert np.array_equal(got.cpu().numpy(), want)
+
+
 def test_native_runner_replays_from_a_captured_graph(setup):
     """enqueue launches kernels only (no allocation, copy, memset or synchronisation), so a caller can record it
     into a graph.  Every replay is checked, with eager work on the same buffers between the replays."""
