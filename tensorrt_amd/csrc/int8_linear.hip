@@ -1945,7 +1945,8 @@ __global__ __launch_bounds__(NW * 64, PER_SIMD) void linear_piece_dma_kernel(uin
 // engines.  The plan they choose takes 0.8 % more than the best of all in the mean (24 % at most, a launch at the edge
 // of a second round); the kernels and the choice before took 13 % more (50 % at most).  The pieces' among them are fits to the
 // same layers at 16 to 1400 tokens since they read whole lines, 152 launches, times the 1.18 by which the tiles' constants
-// exceeded that GPU's times: 0.2 % more than the best of six plans in the mean, 5 % at most.
+// exceeded that GPU's times, and the wider pieces' a little more, for what they take in whole passes (102 tokens x 768 -> 2304:
+// the pass is 0.2 us a layer faster in the small ones): 0.01 % more than the best of six plans in the mean, 2 % at most.
 // Linear operands whose rows end within a line have kernels and constants of their own: stages of 64 bytes, tiles of up to 128 x
 // 256, and constants fitted to launches by themselves before the other linear operands had stages of whole lines.  10 layers of
 // 96 to 3104 channels, 40 to 33289 tokens, FP16 and INT8, 240 launches: 6.5 % less in the mean than when all linear operands
@@ -2003,7 +2004,7 @@ constexpr TileCost kTileCosts[3][kLinearPlans] = {
     {{}, {}, {128, 128, 2, 4.64f, 0.00f, 0.231f, 0.60f, 0.61f, 1.02f, 0.40f, 0.25f}, {},
         {64, 64, 2, 3.82f, 0.29f, 0.082f, 0.23f, 0.70f, 0.89f, 0.63f, 0.34f},
         {128, 128, 1, 4.02f, 0.77f, 0.142f, 0.99f, 0.f, 1.30f, 0.77f, 0.51f, 0.10f}, {}, {},
-        {32, 64, 1, 1.77f, 1.47f, 0.058f, 0.16f, 0.f, 0.98f, 0.83f, 0.40f},
+        {32, 64, 1, 1.77f, 1.65f, 0.058f, 0.16f, 0.f, 0.98f, 0.83f, 0.40f},
         {32, 32, 2, 2.56f, 0.18f, 0.045f, 0.14f, 0.86f, 1.03f, 0.69f, 0.20f},
         {256, 256, 1, 0.00f, 4.48f, 0.440f, 1.88f, 0.f, 1.02f, 0.54f, 0.97f, 0.11f},
         {256, 192, 1, 5.13f, 0.01f, 0.388f, 1.26f, 0.f, 1.35f, 0.67f, 0.56f, 0.15f},
