@@ -28,6 +28,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <atomic>
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -1547,6 +1548,7 @@ __global__ __launch_bounds__(kWavesF16* kWaveSize) void fmha_f16_kernel(FmhaArgs
 // to the length, that kernel / this one, us per plugin call: 32 x 128 keys 12.5 / 5.8, 128 x 256 41.7 / 37.5, 32 x 384
 // 19.8 / 19.6, 128 x 384 71.7 / 64.6, 16 x 512 22.8 / 19.5.  What is left is the L2: K and V of a unit are read once for every
 // 64 queries, 133 MB for the 35.8 MB of 32 x 384.
+// WHOLE: launches so small that a CU has room for all of it (kWholeWorkgroups); K, V and Q are requested together then.
 // ------------------------------------------------------------------------------------------
 constexpr int kQueriesF16 = kWavesF16T * kQPerWave;
 __device__ u32x4 const kZeroRow[8] = {}; // 64 binary16 zeros, in memory
@@ -1561,7 +1563,7 @@ __device__ __forceinline__ void for_each_block(F&& f)
     }
 }
 
-template <int NKB, bool DEBUG>
+template <int NKB, bool DEBUG, bool WHOLE>
 __device__ __forceinline__ void attend_f16_turns(
     FmhaArgs const& a, SeqInfo const& sq, int const b, int const n, int const q0, uint8_t* const lds,
     uint64_t const* const masks, bool const holes)
@@ -1601,19 +1603,30 @@ __device__ __forceinline__ void attend_f16_turns(
             load_to_lds16_sbase(src, off, dst);
         }
     };
-    auto request_block = [&](int mat, int kb) { request(mat, kb * 64 + wave * 16, sq.nk, kb * 64 + wave * 16, kb < NKB - 1); };
+    constexpr int kRowV = WHOLE ? NKB * 64 : 0; // V's first row in LDS
+    auto request_block = [&](int mat, int kb) {
+        request(mat, kb * 64 + wave * 16, sq.nk, (mat == 2 ? kRowV : 0) + kb * 64 + wave * 16, kb < NKB - 1);
+    };
 
     int const qw = q0 + wave * kQPerWave; // this wavefront's first query
     bool const active = qw < sq.nq;       // if not, it only brings in its rows
-    // Q passes through the place of this wavefront's rows of the last block
-    int const qRow = (NKB - 1) * 64 + wave * 16;
+    // Q passes through the place of this wavefront's rows of the last block; WHOLE: it has one of its own
+    int const qRow = (WHOLE ? 2 * NKB : NKB - 1) * 64 + wave * 16;
     request(0, qw, sq.nq, qRow, false);
 #pragma unroll
-    for (int kb = 0; kb < NKB - 1; ++kb)
+    for (int kb = 0; kb < (WHOLE ? NKB : NKB - 1); ++kb)
     {
         request_block(1, kb);
     }
-    wait_vmcnt<2 * (NKB - 1)>();
+    if constexpr (WHOLE)
+    {
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb)
+        {
+            request_block(2, kb);
+        }
+    }
+    wait_vmcnt<WHOLE ? 4 * NKB : 2 * (NKB - 1)>();
     f16x8 qreg[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -1621,7 +1634,10 @@ __device__ __forceinline__ void attend_f16_turns(
         qreg[h] = *reinterpret_cast<f16x8 const*>(lds + (qRow + lq) * kRow + swz<2>(lq, h * 4 + g) * 16);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(qreg[0]), "+v"(qreg[1])::"memory"); // read before it is overwritten
-    request_block(1, NKB - 1);
+    if constexpr (!WHOLE)
+    {
+        request_block(1, NKB - 1);
+    }
 
     int const lastKeys = sq.nk - (NKB - 1) * 64;
     int const lastHalves = (lastKeys + 31) >> 5;   // 32-key halves of the last block that hold keys
@@ -1631,10 +1647,10 @@ __device__ __forceinline__ void attend_f16_turns(
     f32x4 acc[NT];
     auto scores = [&](auto block) {
         constexpr int kb = decltype(block)::value;
-        // in flight behind block kb: the later blocks of K and V of the blocks before kb - 1
-        wait_vmcnt<2 * (NKB - 1 - kb + (kb > 0 ? kb - 1 : 0))>();
+        // in flight behind block kb: the later blocks of K and V of the blocks before kb - 1; WHOLE: and all of V
+        wait_vmcnt<2 * (NKB - 1 - kb + (WHOLE ? NKB : kb > 0 ? kb - 1 : 0))>();
         __syncthreads(); // everybody's rows of block kb have landed, and everybody has read block kb - 1
-        if constexpr (kb > 0)
+        if constexpr (kb > 0 && !WHOLE)
         {
             request_block(2, kb - 1);
         }
@@ -1678,8 +1694,11 @@ __device__ __forceinline__ void attend_f16_turns(
         __builtin_amdgcn_sched_barrier(0);
     };
     for_each_block<NKB>(scores);
-    __syncthreads();
-    request_block(2, NKB - 1);
+    if constexpr (!WHOLE)
+    {
+        __syncthreads();
+        request_block(2, NKB - 1);
+    }
 
     int const q = qw + lq;
     bool const qValid = q < sq.nq;
@@ -1764,7 +1783,7 @@ __device__ __forceinline__ void attend_f16_turns(
                 preg[w * 4 + 2] = p23[0];
                 preg[w * 4 + 3] = p23[1];
             }
-            int const vrow = kb * 64 + hb * 32 + 4 * g + (lq >> 2);
+            int const vrow = kRowV + kb * 64 + hb * 32 + 4 * g + (lq >> 2);
             uint8_t const* vbase = lds + vrow * kRow + 8 * (lq & 1);
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt)
@@ -1815,7 +1834,7 @@ __device__ __forceinline__ void attend_f16_turns(
     }
 }
 
-template <int KT, bool DEBUG>
+template <int KT, bool DEBUG, bool WHOLE>
 __global__ __launch_bounds__(kWavesF16T* kWaveSize)
     __attribute__((amdgpu_waves_per_eu(KT <= 4 ? 4 : KT <= 6 ? 3 : 2))) void fmha_f16_turns_kernel(
     TRTAMD_FMHA_LEADING_PARAMS, FmhaArgs const rest)
@@ -1863,7 +1882,7 @@ __global__ __launch_bounds__(kWavesF16T* kWaveSize)
     {
 #define TRTAMD_BLOCKS(NKB)                                                                                             \
     case NKB:                                                                                                          \
-        if constexpr (KT >= NKB) attend_f16_turns<NKB, DEBUG>(a, sq, b, n, q0, smem, masks, holes);                                        \
+        if constexpr (KT >= NKB) attend_f16_turns<NKB, DEBUG, WHOLE>(a, sq, b, n, q0, smem, masks, holes);             \
         break
         TRTAMD_BLOCKS(1);
         TRTAMD_BLOCKS(2);
@@ -2235,22 +2254,27 @@ int ensure_lds(void const* key, char const* name, int ldsBytes)
     return TRTAMD_STATUS_SUCCESS;
 }
 
-template <typename K>
-int launch_fmha(K kernel, char const* name, hipStream_t stream, FmhaArgs const& args, int ldsBytes, int waves)
+template <auto KERNEL>
+int launch_fmha(char const* name, hipStream_t stream, FmhaArgs const& args, int ldsBytes, int waves)
 {
-    int const st = ensure_lds(reinterpret_cast<void const*>(kernel), name, ldsBytes);
-    if (st != TRTAMD_STATUS_SUCCESS)
+    static std::atomic<bool> reserved{false}; // known without the lock from the second launch on
+    if (!reserved.load(std::memory_order_acquire))
     {
-        return st;
+        int const st = ensure_lds(reinterpret_cast<void const*>(KERNEL), name, ldsBytes);
+        if (st != TRTAMD_STATUS_SUCCESS)
+        {
+            return st;
+        }
+        reserved.store(true, std::memory_order_release);
     }
     unsigned const blocks = (unsigned) args.B * args.N * args.qSplit;
-    if constexpr (std::is_invocable_v<K, FmhaArgs>)
+    if constexpr (std::is_invocable_v<decltype(KERNEL), FmhaArgs>)
     {
-        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(waves * kWaveSize), ldsBytes, stream, args);
+        hipLaunchKernelGGL(KERNEL, dim3(blocks), dim3(waves * kWaveSize), ldsBytes, stream, args);
     }
     else
     {
-        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(waves * kWaveSize), ldsBytes, stream, TRTAMD_FMHA_LEADING_ARGS(args), args);
+        hipLaunchKernelGGL(KERNEL, dim3(blocks), dim3(waves * kWaveSize), ldsBytes, stream, TRTAMD_FMHA_LEADING_ARGS(args), args);
     }
     return check_launch(name);
 }
@@ -2277,11 +2301,11 @@ int run_i8(hipStream_t stream, FmhaArgs const& a, bool interleaved)
     {
 #define TRTAMD_I8P(KT)                                                                                                 \
     case KT:                                                                                                           \
-        return a.packedMask ? launch_fmha(fmha_i8_prefix_kernel<KT, false, DEBUG, true>, "fmha_i8_masked", stream, a,  \
+        return a.packedMask ? launch_fmha<fmha_i8_prefix_kernel<KT, false, DEBUG, true>>("fmha_i8_masked", stream, a,  \
                    Lds<1>::total(KT), kWavesI8)                                                                        \
-            : interleaved ? launch_fmha(fmha_i8_prefix_kernel<KT, true, DEBUG>, "fmha_i8_prefix_interleaved", stream, \
+            : interleaved ? launch_fmha<fmha_i8_prefix_kernel<KT, true, DEBUG>>("fmha_i8_prefix_interleaved", stream, \
                    a, Lds<1>::total(KT), kWavesI8)                                                                     \
-                           : launch_fmha(fmha_i8_prefix_kernel<KT, false, DEBUG>, "fmha_i8_prefix", stream, a,         \
+                           : launch_fmha<fmha_i8_prefix_kernel<KT, false, DEBUG>>("fmha_i8_prefix", stream, a,         \
                                Lds<1>::total(KT), kWavesI8)
         switch (kt)
         {
@@ -2297,9 +2321,9 @@ int run_i8(hipStream_t stream, FmhaArgs const& a, bool interleaved)
     }
 #define TRTAMD_I8(KT)                                                                                                  \
     case KT:                                                                                                           \
-        return interleaved ? launch_fmha(fmha_i8_kernel<KT, true, DEBUG>, "fmha_i8_interleaved", stream, a,           \
+        return interleaved ? launch_fmha<fmha_i8_kernel<KT, true, DEBUG>>("fmha_i8_interleaved", stream, a,           \
                    Lds<1>::total(KT), kWavesI8)                                                                        \
-                           : launch_fmha(fmha_i8_kernel<KT, false, DEBUG>, "fmha_i8", stream, a, Lds<1>::total(KT),    \
+                           : launch_fmha<fmha_i8_kernel<KT, false, DEBUG>>("fmha_i8", stream, a, Lds<1>::total(KT),    \
                                kWavesI8)
     switch (kt)
     {
@@ -2323,6 +2347,32 @@ enum class F16Kernel
     kSTREAM
 };
 
+// Launches of no more workgroups than CUs, each with a CU's LDS to itself, have K, V and 64 queries there at once: nothing waits for
+// a place, which takes one or two trips to the L2 out of the chain.  Sequences of a third of the length to the length, 12 heads,
+// in turns / so, us: 2 x 128 keys 3.96 / 3.84, 2 x 180 4.36 / 4.27, 2 x 256 4.91 / 4.84, 2 x 384 5.62 / 5.57 (an FP16 pass of one
+// request 337.9 / 333.5); with more workgroups, which it would keep off the CU, 8 x 180 5.08 / 5.25, 4 x 384 6.66 / 8.95; and at
+// 512 keys, whose 136 KB a CU takes longer to bring in than it waits otherwise, 2 x 512 6.15 / 6.35.
+constexpr int64_t kWholeWorkgroups = 256;
+constexpr int kWholeBlocks = 6;
+constexpr int whole_lds(int kt)
+{
+    return 2 * Lds<2>::matBytes(kt) + kQueriesF16 * Lds<2>::kRow;
+}
+
+template <int KT, bool DEBUG>
+int launch_turns(hipStream_t stream, FmhaArgs const& a)
+{
+    if constexpr (KT <= kWholeBlocks)
+    {
+        if ((int64_t) a.B * a.N * a.qSplit <= kWholeWorkgroups)
+        {
+            return launch_fmha<fmha_f16_turns_kernel<KT, DEBUG, true>>("fmha_f16_whole", stream, a, whole_lds(KT), kWavesF16T);
+        }
+    }
+    return launch_fmha<fmha_f16_turns_kernel<KT, DEBUG, false>>("fmha_f16_turns", stream, a, Lds<2>::matBytes(KT), kWavesF16T);
+}
+
+
 template <bool DEBUG>
 int run_f16(hipStream_t stream, FmhaArgs const& a, F16Kernel which)
 {
@@ -2341,9 +2391,7 @@ int run_f16(hipStream_t stream, FmhaArgs const& a, F16Kernel which)
     if (which == F16Kernel::kTURNS)
     {
 #define TRTAMD_F16T(KT)                                                                                                \
-    case KT:                                                                                                           \
-        return launch_fmha(                                                                                            \
-            fmha_f16_turns_kernel<KT, DEBUG>, "fmha_f16_turns", stream, a, Lds<2>::matBytes(KT), kWavesF16T)
+    case KT: return launch_turns<KT, DEBUG>(stream, a)
         switch (kt)
         {
             TRTAMD_F16T(1);
@@ -2357,7 +2405,7 @@ int run_f16(hipStream_t stream, FmhaArgs const& a, F16Kernel which)
 #undef TRTAMD_F16T
     }
 #define TRTAMD_F16(KT)                                                                                                 \
-    case KT: return launch_fmha(fmha_f16_kernel<KT, DEBUG>, "fmha_f16", stream, a, Lds<2>::total(KT), kWavesF16)
+    case KT: return launch_fmha<fmha_f16_kernel<KT, DEBUG>>("fmha_f16", stream, a, Lds<2>::total(KT), kWavesF16)
     switch (kt)
     {
         TRTAMD_F16(1);
@@ -2386,8 +2434,12 @@ int prepare_kt()
     st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_i8_kernel<KT, true, false>), "fmha_i8_interleaved",
                       Lds<1>::total(KT));
     st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_i8_kernel<KT, false, false>), "fmha_i8", Lds<1>::total(KT));
-    st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_f16_turns_kernel<KT, false>), "fmha_f16_turns",
+    st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_f16_turns_kernel<KT, false, false>), "fmha_f16_turns",
                       Lds<2>::matBytes(KT));
+    if constexpr (KT <= kWholeBlocks)
+    {
+        st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_f16_turns_kernel<KT, false, true>), "fmha_f16_whole", whole_lds(KT));
+    }
     st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_f16_kernel<KT, false>), "fmha_f16", Lds<2>::total(KT));
     return st;
 }

@@ -247,6 +247,29 @@ def test_fmha_fp16_packed_tile_edges(api, B, N, S):
     assert_fp_close(host(out), oracle.mha_fused_f16_packed(qkv, cu, N, D), what="FP16 packed, tile edges")
 
 
+@pytest.mark.parametrize("S,lens", [(64, [1, 64, 63, 17]), (128, [65, 128, 1, 64]), (192, [129, 192, 191, 64]),
+                                    (256, [193, 256, 255, 128]), (384, [257, 384, 321, 320, 64]), (512, [385, 512, 449])])
+def test_fmha_fp16_few_workgroups(api, S, lens):
+    """Launches of no more workgroups than CUs have all of K and V in LDS at once, larger ones in turns: the same bytes for the
+    same sequences, lengths either side of the blocks of 64 keys; and the oracle's result."""
+    from tensorrt_amd import capi
+    N = 2
+    once = rng(33).standard_normal((sum(lens), 3 * N * D)).astype(np.float16)
+    parts = {64: 1, 128: 2, 192: 3, 256: 4, 384: 6, 512: 8}[S]
+    copies = 256 // (len(lens) * N * parts) + 1 # one launch on each side of 256 workgroups
+    got = []
+    for n in (1, copies):
+        cu = _cu(lens * n)
+        d_qkv, d_cu, out = dev(np.tile(once, (n, 1))), dev(cu), dev_empty((int(cu[-1]), N * D), np.float16, fill=0)
+        p = _params(capi, qkv_ptr=ptr(d_qkv), o_ptr=ptr(out), b=len(lens) * n, h=N, s=S, d=D, qkv_stride_in_bytes=2 * 3 * N * D,
+                    o_stride_in_bytes=2 * N * D, scale_bmm1=half2_bits(0.125), cu_seqlens=ptr(d_cu))
+        api.check(api.fused_mha_run(stream(), 1, C.byref(p)))
+        sync()
+        got.append(host(out))
+    assert_fp_close(got[0], oracle.mha_fused_f16_packed(once, _cu(lens), N, D), what="FP16 packed, few workgroups")
+    assert np.array_equal(np.tile(got[0], (copies, 1)), got[1])
+
+
 @pytest.mark.parametrize("s,longest", [(40, 64), (250, 256), (257, 384), (300, 384), (400, 512)])
 def test_fmha_fp16_sequences_longer_than_s(api, s, longest):
     """s chooses the kernel; sequences up to the 64, 128, 192, 256, 384 or 512 keys that it holds are served whole."""
