@@ -114,6 +114,22 @@ __device__ inline void rows_transpose(uint32_t (&x)[4])
     x[3] = t23[1];
 }
 
+// The order in which a launch's workgroups take its units: bit 0 says the longest sequences first instead of the sequences as
+// they come, the rest is the number of ids, a multiple of 512, of which every other round of 256 goes backwards.
+constexpr uint32_t kRanked = 1;
+constexpr uint32_t kTwoRounds = 512;
+
+// Ids are dealt to the 8 XCDs in turn and there to the 32 CUs, so a round of 256 of them puts a workgroup on every CU, and the
+// next round, in the same order, would give the CU of the longest unit the longest again, and the CU of a unit's first part,
+// which is always full, a first part again: 32 is a multiple of 2 and of 4 parts, and the last part of a short sequence is
+// empty.  Backwards, within each XCD, a round evens out what the one before it left uneven.  (What the hardware does beyond the
+// first rounds, or with another number of CUs, only costs evenness: the ids of a whole round change places among themselves.)
+__device__ __forceinline__ uint32_t id_of_workgroup(uint32_t bid, uint32_t order)
+{
+    uint32_t const odd = 0u - ((bid >> 8) & 1u);
+    return bid ^ (odd & (bid < order ? 0xf8u : 0u)); // an id of an odd round is not a multiple of 512: bit 0 makes no difference
+}
+
 struct FmhaArgs
 {
     void const* qkv;
@@ -136,7 +152,7 @@ struct FmhaArgs
     int32_t clampP;              // scale_softmax may push p beyond 127
     int32_t* dbgAcc1;            // optional [B][N][S][S] int32 (INT8) / float bits (FP16)
     int8_t* dbgP8;               // optional [B][N][S][S]
-    int32_t ranked;              // serve the longest sequences first (pointless when one round holds every workgroup)
+    uint32_t order;              // see kRanked
     FastDiv partDiv, headDiv;    // by qSplit and N
 };
 
@@ -145,14 +161,14 @@ struct FmhaArgs
 #define TRTAMD_FMHA_LEADING_PARAMS                                                                                     \
     uint64_t const qkv, uint64_t const cuSeqlens, uint32_t const qSplit, uint32_t const qSplitMul,                      \
         uint32_t const qSplitShifts, uint32_t const N, uint32_t const headMul, uint32_t const headShifts, int const B, \
-        int const S, int const ranked, int const total
+        int const S, uint32_t const order, int const total
 #define TRTAMD_FMHA_LEADING_ARGS(a)                                                                                    \
     address((a).qkv), address((a).cuSeqlens), (a).partDiv.d, (a).partDiv.mul, (a).partDiv.shifts, (a).headDiv.d,       \
-        (a).headDiv.mul, (a).headDiv.shifts, (a).B, (a).S, (a).ranked, (a).total
+        (a).headDiv.mul, (a).headDiv.shifts, (a).B, (a).S, (a).order, (a).total
 #define TRTAMD_FMHA_ARGS_OF(rest)                                                                                      \
-    fmha_args(qkv, cuSeqlens, {qSplit, qSplitMul, qSplitShifts}, {N, headMul, headShifts}, B, S, ranked, total, rest)
+    fmha_args(qkv, cuSeqlens, {qSplit, qSplitMul, qSplitShifts}, {N, headMul, headShifts}, B, S, order, total, rest)
 __device__ __forceinline__ FmhaArgs fmha_args(uint64_t qkv, uint64_t cuSeqlens, FastDiv const& partDiv,
-    FastDiv const& headDiv, int B, int S, int ranked, int total, FmhaArgs const& rest)
+    FastDiv const& headDiv, int B, int S, uint32_t order, int total, FmhaArgs const& rest)
 {
     FmhaArgs a = rest;
     a.qkv = global_ptr<void const>(qkv);
@@ -163,7 +179,7 @@ __device__ __forceinline__ FmhaArgs fmha_args(uint64_t qkv, uint64_t cuSeqlens, 
     a.N = (int) headDiv.d;
     a.B = B;
     a.S = S;
-    a.ranked = ranked;
+    a.order = order;
     a.total = total;
     return a;
 }
@@ -794,7 +810,7 @@ __device__ inline SeqInfo pick_sequence_in_registers(FmhaArgs const& a, int rank
 template <int THREADS>
 __device__ inline SeqInfo pick_sequence_info(FmhaArgs const& a, int rank, int capacity, PickLds& l, int& bOut)
 {
-    if (a.cuSeqlens == nullptr || a.B > kMaxRanked || !a.ranked)
+    if (a.cuSeqlens == nullptr || a.B > kMaxRanked || !(a.order & kRanked))
     {
         bOut = rank; // fixed layout (equal lengths), too many sequences, or a launch of a single round: natural order
         return seq_info(a, rank, capacity);
@@ -1235,12 +1251,13 @@ __global__ __launch_bounds__(kWavesI8* kWaveSize) __attribute__((amdgpu_waves_pe
     uint8_t* sV = smem + Lds<1>::matBytes(KT);
     __shared__ PickLds sPick;
     FmhaArgs const a = TRTAMD_FMHA_ARGS_OF(rest);
-    UnitPart up = unit_of_workgroup(blockIdx.x, B * N * qSplit, a.partDiv);
+    uint32_t const bid = id_of_workgroup(blockIdx.x, order);
+    UnitPart up = unit_of_workgroup(bid, B * N * qSplit, a.partDiv);
     if (!INTERLEAVED && a.qSplit == 1 && (a.N & 1) == 0)
     {
         // Linear layout ([token][head][Q K V][64 bytes]): V of head n and Q of head n + 1 lie in one 128-byte line, so
         // the two heads of a pair go to one XCD (18239 tokens x 16 heads: 36.2 -> 35.2 us)
-        UnitPart const pair = unit_of_workgroup(blockIdx.x, B * N * qSplit, 2);
+        UnitPart const pair = unit_of_workgroup(bid, B * N * qSplit, 2);
         up.unit = pair.unit * 2u + (uint32_t) pair.part;
     }
     int const part = up.part;
@@ -1842,7 +1859,8 @@ __global__ __launch_bounds__(kWavesF16T* kWaveSize)
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     __shared__ PickLds sPick;
     FmhaArgs const a = TRTAMD_FMHA_ARGS_OF(rest);
-    UnitPart const up = unit_of_workgroup(blockIdx.x, B * N * qSplit, a.partDiv);
+    uint32_t const bid = id_of_workgroup(blockIdx.x, order);
+    UnitPart const up = unit_of_workgroup(bid, B * N * qSplit, a.partDiv);
     uint32_t const rank = up.unit / a.headDiv;
     int const n = __builtin_amdgcn_readfirstlane((int) (up.unit - rank * a.headDiv.d));
     int const q0 = __builtin_amdgcn_readfirstlane(up.part) * kQueriesF16;
@@ -1926,7 +1944,8 @@ __global__ __launch_bounds__(kWavesStream* kWaveSize) __attribute__((amdgpu_wave
     __shared__ PickLds sPick;
     __shared__ uint64_t sMask[8];
     FmhaArgs const a = TRTAMD_FMHA_ARGS_OF(rest);
-    UnitPart const up = unit_of_workgroup(blockIdx.x, B * N * qSplit, a.partDiv);
+    uint32_t const bid = id_of_workgroup(blockIdx.x, order);
+    UnitPart const up = unit_of_workgroup(bid, B * N * qSplit, a.partDiv);
     uint32_t const rank = up.unit / a.headDiv;
     int const n = __builtin_amdgcn_readfirstlane((int) (up.unit - rank * a.headDiv.d));
     int b;
@@ -2568,31 +2587,54 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
     a.dbgAcc1 = dbgAcc1;
     a.dbgP8 = dbgP8;
     {
-        // The order in which sequences are served matters when workgroups run in several rounds (the long ones
-        // first, so that the short ones fill the tail).  When every workgroup of the launch is resident at once it
-        // changes nothing, and the workgroups skip the ranking (a trip to LDS and two barriers before their loads).
-        // Workgroups of 64 queries are short enough to even out by themselves (12 heads x 128 sequences of 67-200 keys:
-        // 29.1 us in natural order, 36.8 ranked); those of 128 queries are all resident at once up to four per CU, and the
-        // order then spreads the long ones over the CUs (12 heads, ranked / not: 16 x 512 18.0 / 21.2 us, 32 x 384 19.0 / 20.4,
-        // 64 x 384 32.8 / 33.6), until there are several rounds of them (16 heads, 128 x 384: 85.6 / 82.4).
+        // The order in which sequences are served: the longest first costs a workgroup the ranking (0.25 us: a trip to LDS or a
+        // few across the lanes before its loads) and evens out the CUs, or fills the tail of a launch of several rounds with
+        // short ones.  Every other round backwards (id_of_workgroup) costs nothing.  12 or 16 heads, sequences of a third of
+        // the length to the length:
+        // - FP16, 128 queries per workgroup: all resident at once up to four per CU; longest first below 3072 of them
+        //   (16 x 512 18.0 us against 21.2 in natural order, 32 x 384 19.0 / 20.4; 128 x 384, 16 heads, 85.6 / 82.4), and every
+        //   other round backwards always: 32 x 384 15.3 -> 14.8, 32 x 180 9.3 -> 8.2, 96 x 180 19.2 -> 17.0, and in natural order
+        //   128 x 180 31.9 -> 27.0, 128 x 256 40.0 -> 37.2 (16 heads).
+        // - FP16, 64 queries: short enough to even out by themselves, natural order with rounds backwards (22 x 180 8.0 -> 6.7,
+        //   21 x 250 10.6 -> 10.0, 16 x 250 8.3 -> 8.6, mean of 45 launches 1.04x); of 321 keys and more longest first as well
+        //   (8 x 384 8.3 -> 7.2, 12 x 384 9.1 -> 8.4; mean of 27 launches 1.06x, 1.04x without it).
+        // - INT8, two or three workgroups per CU at a time: longest first beyond one round of all CUs' places, and before that
+        //   where the units are long enough for the ranking to pay, from 768 of them with three blocks of keys
+        //   (32 x 180 7.3 -> 6.9), 512 with five (14 x 310 9.5 -> 8.7), 256 with more (16 x 384 12.2 -> 9.9).  Rounds go backwards
+        //   where a unit has an even number of parts (32 x 384 16.4 -> 11.7, longest first alone 12.7; 24 x 512, 16 heads,
+        //   25.4 -> 23.0); three parts are spread by themselves (24 x 180 5.6 -> 6.1), and units that are not shared have
+        //   enough rounds to even out (64 x 256, 16 heads, 18.2 -> 18.7).
         int64_t const workgroups = (int64_t) a.B * a.N * a.qSplit;
+        bool ranked, back;
         if (f16 == F16Kernel::kSTREAM)
         {
-            a.ranked = workgroups < 3072 ? 1 : 0;
+            ranked = workgroups < 3072;
+            back = true;
+        }
+        else if (f16 == F16Kernel::kTURNS)
+        {
+            ranked = kt >= 6 && workgroups >= 512;
+            back = true;
         }
         else
         {
             int64_t const lds = dataType == 2 ? Lds<1>::total(kt) : Lds<2>::total(kt);
             int64_t const perCu
                 = std::max<int64_t>(1, std::min<int64_t>(dataType == 2 ? 3 : 2, (160 * 1024) / std::max<int64_t>(lds, 1)));
-            a.ranked = f16 == F16Kernel::kGENERAL && workgroups > perCu * 256 ? 1 : 0;
+            int64_t const without = dataType != 2 || kt <= 2 ? perCu * 256 : kt >= 6 ? 256 : kt == 5 ? 512 : 767;
+            ranked = workgroups > std::min(perCu * 256, without);
+            back = dataType == 2 && ranked && a.qSplit % 2 == 0;
         }
-        // tuning override: TRTAMD_FMHA_RANKED=0 / 1 forces natural order / the longest-first order
+        // tuning override: TRTAMD_FMHA_RANKED=0 forces natural order with every round forwards, 1 the longest-first order
         int const forcedRank = tuning(Tuning::kFmhaRanked);
         if (forcedRank >= 0)
         {
-            a.ranked = forcedRank ? 1 : 0;
+            ranked = forcedRank != 0;
+            back = back && ranked;
         }
+        // sequences of one length (24.0 us forwards, 24.1 backwards, 32 x 384) have nothing to even out
+        uint32_t const paired = back && a.cuSeqlens ? (uint32_t) std::min<int64_t>(workgroups, INT32_MAX) / kTwoRounds * kTwoRounds : 0;
+        a.order = paired | (ranked ? kRanked : 0);
     }
     if (interleaved)
     {

@@ -327,6 +327,49 @@ def test_longest_first_order_reaches_every_sequence(B):
     assert all((outs[0][:, cu[b]:cu[b + 1]] != 55).any() for b in range(B) if lens[b])
 
 
+# (data type, sequences, heads, longest): workgroups of 64 and of 128 queries and shared INT8 units, one workgroup short of two,
+# three and four rounds of 256, as many and one more, in natural order and the longest first
+@pytest.mark.parametrize("dtype,B,N,S", [(1, 511, 1, 64), (1, 512, 1, 64), (1, 513, 1, 64), (1, 128, 2, 192), (1, 43, 2, 321),
+                                         (1, 1023, 1, 128), (1, 1024, 1, 128), (1, 1025, 1, 128), (1, 192, 2, 200),
+                                         (1, 3329, 1, 64), (2, 128, 1, 384), (2, 129, 1, 330), (2, 192, 2, 190),
+                                         (2, 511, 1, 128), (2, 512, 1, 128), (2, 257, 2, 65)])
+def test_rounds_that_go_backwards_reach_every_unit(dtype, B, N, S):
+    """The order that the launcher chooses writes the bytes of the sequences' own order, and of every unit."""
+    r = rng(1800 + B + S)
+    lens = r.integers(1, S + 1, B)
+    lens[0], lens[B // 2], lens[-1] = S, 0, 1
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T = int(cu[-1])
+    qkv = r.standard_normal((T, 3 * N * 64)).astype(np.float32)
+    bits = lambda x: int(np.float32(x).view(np.uint32))
+    p = capi.FmhaParams()
+    if dtype == 2:
+        q, s_q = quantize_amax(qkv)
+        d_qkv = dev(interleave(q))
+        p.qkv_stride_in_bytes = p.o_stride_in_bytes = T
+        p.interleaved = 1
+        p.scale_bmm1, p.scale_softmax, p.scale_bmm2 = bits(s_q * s_q * 0.125), bits(127.0), bits(s_q / 127.0 / 0.02)
+    else:
+        d_qkv = dev(qkv.astype(np.float16))
+        p.qkv_stride_in_bytes, p.o_stride_in_bytes = 2 * 3 * N * 64, 2 * N * 64
+        p.scale_bmm1, p.scale_softmax, p.scale_bmm2 = half2_bits(0.125), half2_bits(1.0), half2_bits(1.0)
+    d_cu = dev(cu)
+    p.qkv_ptr, p.cu_seqlens = ptr(d_qkv), ptr(d_cu)
+    p.b, p.h, p.s, p.d = B, N, S, 64
+    api = capi.api()
+    outs = []
+    for order in (None, 0):
+        out = dev_empty((N * 2, T, 32), np.int8, fill=55) if dtype == 2 else dev_empty((T, N * 64), np.float16, fill=-7)
+        p.o_ptr = ptr(out)
+        with tuning("TRTAMD_FMHA_RANKED", -1 if order is None else order):
+            api.check(api.fused_mha_run(stream(), dtype, C.byref(p)))
+            sync()
+        outs.append(host(out))
+    assert np.array_equal(outs[0], outs[1])
+    units = outs[0].reshape(N, 2, T, 32).transpose(2, 0, 1, 3).reshape(T, N, 64) if dtype == 2 else outs[0].reshape(T, N, 64)
+    assert (units != (55 if dtype == 2 else -7)).any(axis=2).all()
+
+
 # launches that fill the chip (768 workgroups of 128 queries): lengths on either side of a wavefront's 32 queries, a
 # workgroup's 128, half a block and a block of keys; scores whose maximum grows from block to block and scores of one size
 @pytest.mark.parametrize("S,B,N", [(64, 192, 4), (384, 64, 4), (512, 48, 4)])
