@@ -1859,7 +1859,7 @@ __global__ __launch_bounds__(kWavesF16T* kWaveSize)
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     __shared__ PickLds sPick;
     FmhaArgs const a = TRTAMD_FMHA_ARGS_OF(rest);
-    uint32_t const bid = id_of_workgroup(blockIdx.x, order);
+    uint32_t const bid = KT <= 2 ? blockIdx.x : id_of_workgroup(blockIdx.x, order);
     UnitPart const up = unit_of_workgroup(bid, B * N * qSplit, a.partDiv);
     uint32_t const rank = up.unit / a.headDiv;
     int const n = __builtin_amdgcn_readfirstlane((int) (up.unit - rank * a.headDiv.d));
@@ -2533,24 +2533,36 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
     a.N = p->h;
     a.S = p->s;
     int const kt = pick_kt(p->s);
-    // FP16: 128 queries per workgroup where that makes three workgroups and more for each of the 256 CUs,
-    // 64 of them and the scores of all their keys in registers where it does not (12 heads: 16 x 256 keys, 384 workgroups of
-    // 128, 7.9 against 8.8 us; 32 x 256, 768 of them, 13.9 against 13.1; 16 heads, 8 x 384, 384: 9.6 against 10.2).
+    int const blocks = ceil_div(p->s, 64);
+    // FP16: 128 queries per workgroup from so many of these workgroups on, by blocks of 64 keys; 64 of them and the scores of all
+    // their keys in registers below.  The latter run in one round up to four, three or two of them per CU, as their LDS leaves
+    // room (longer sequences need more of it each), and a second round costs more than the wider workgroups that leave some CUs
+    // with two of them, others with three.  12 or 16 heads, sequences of a third of the length to the length, us with 64 / with
+    // 128 queries: 64 x 128 keys 8.1 / 7.7, 48 x 128 7.8 / 8.1; 27 x 180 8.0 / 7.1, 21 x 180 6.7 / 6.9; 27 x 230 10.1 / 7.9,
+    // 21 x 230 7.8 / 7.9; 20 x 310 11.7 / 10.1, 14 x 310 8.2 / 8.8; 16 x 384 12.0 / 9.8, 10 x 384 8.2 / 9.1; 12 x 440 12.9 / 9.8,
+    // 6 x 440 7.8 / 9.2; 10 x 512 14.3 / 10.8 (16 heads), 6 x 512 7.5 / 9.5.
+    // With one or two blocks of keys a second round of the wide ones is no better: 110 x 128 13.0 / 14.4, 225 x 128 24.8 / 29.9;
+    // and a row of at most 64 keys leaves half of them idle: 64 x 64 4.5 / 5.3, 600 x 64 25.6 / 28.3.
+    constexpr int kStreamFrom[] = {INT32_MAX, 768, 600, 544, 540, 432, 384, 360};
     constexpr int kStreamTile = kWavesStream * kStreamQueries;
     int const streamParts = ceil_div(kt * 64, kStreamTile);
     F16Kernel f16 = F16Kernel::kGENERAL;
     if (dataType == 1 && !tuning(Tuning::kFmhaGeneric)
         && p->qkv_stride_in_bytes < (1LL << 29)) // eight tokens within a 32-bit offset
     {
-        f16 = (int64_t) p->b * p->h * streamParts >= 768 ? F16Kernel::kSTREAM : F16Kernel::kTURNS;
+        int64_t const wide = (int64_t) p->b * p->h * streamParts;
+        f16 = wide >= kStreamFrom[blocks - 1] && (blocks > 2 || wide <= 1024) ? F16Kernel::kSTREAM : F16Kernel::kTURNS;
     }
     {
         // Workgroups per (sequence, head).  Every extra workgroup stages K and V again, so a unit is only shared
-        // while the launch would otherwise leave the chip partly idle or badly balanced.  INT8 (three workgroups per
-        // CU, 768 places): below 896 units two workgroups per unit, which also evens out a single round of units of
-        // very different lengths (768 units of 128-384 keys: 24.9 against 27.8 us; 512 units: 18.7 against 23.1 us;
-        // 896 units: 29.1 against 28.1 us), and more of them only to reach one round (256 units: three, 12.6 us
-        // against 13.1 with two and 17.4 with one; at most four).  The general FP16 kernel (its K and V take most of a
+        // while the launch would otherwise leave the chip partly idle or badly balanced.  INT8, three workgroups per CU of up to
+        // six blocks of keys and two of more: two per unit even out a round or two of units of very different lengths, and
+        // more of them fill one round, 768 workgroups or, from six blocks on, 512 (240 units of 256 keys: three 7.0 us, four
+        // 7.6; 144 units of 384: four 8.1, three 8.8; 336 units: two 11.2, three 12.4).  One per unit once rounds that go
+        // forwards and backwards are even with it: from 640 units of one or two blocks (672 units: one 6.7, two 7.4; 600: 6.4 /
+        // 6.0), 768 of three or four (192 keys: 9.0 / 10.0; 720 units: 10.9 / 9.9), 640 of five (752 units: 15.8 / 18.3, 600 of
+        // one length: 25.9 / 23.8), 1040 of six (900: 28.5 / 26.2; 1152: 31.5 / 32.6), 720 of more (440 keys: 26.9 / 29.2).
+        // The general FP16 kernel (its K and V take most of a
         // CU's LDS, one workgroup per CU, and staging them is 40 % of a workgroup's time): only below 160 units (192 units
         // of 192-384 keys: 15.3 us alone, 17.5 us shared by two; 144 units: 14.9 against 12.9 us).  The other FP16 kernels
         // take 64 or 128 queries each, of as many as the kernel has room for: a sequence longer than s that still fits
@@ -2561,7 +2573,11 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         int split = 1;
         if (dataType == 2)
         {
-            split = heads >= 896 ? 1 : (int) std::max<int64_t>(2, std::min<int64_t>(4, ceil_div<int64_t>(768, heads)));
+            constexpr int kAloneFrom[] = {640, 640, 768, 768, 640, 1040, 720, 720}; // by blocks of keys
+            int const most = blocks <= 5 && heads > 192 ? 3 : 4;
+            split = heads >= kAloneFrom[blocks - 1]
+                ? 1
+                : (int) std::max<int64_t>(2, std::min<int64_t>(most, ceil_div<int64_t>(blocks <= 5 ? 768 : 512, heads)));
         }
         else if (f16 != F16Kernel::kGENERAL)
         {
@@ -2595,15 +2611,15 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         //   (16 x 512 18.0 us against 21.2 in natural order, 32 x 384 19.0 / 20.4; 128 x 384, 16 heads, 85.6 / 82.4), and every
         //   other round backwards always: 32 x 384 15.3 -> 14.8, 32 x 180 9.3 -> 8.2, 96 x 180 19.2 -> 17.0, and in natural order
         //   128 x 180 31.9 -> 27.0, 128 x 256 40.0 -> 37.2 (16 heads).
-        // - FP16, 64 queries: short enough to even out by themselves, natural order with rounds backwards (22 x 180 8.0 -> 6.7,
-        //   21 x 250 10.6 -> 10.0, 16 x 250 8.3 -> 8.6, mean of 45 launches 1.04x); of 321 keys and more longest first as well
-        //   (8 x 384 8.3 -> 7.2, 12 x 384 9.1 -> 8.4; mean of 27 launches 1.06x, 1.04x without it).
+        // - FP16, 64 queries: short enough to even out by themselves, natural order, from three blocks of keys on with rounds
+        //   backwards (22 x 180 8.0 -> 6.7, 21 x 250 10.6 -> 10.0, 16 x 250 8.3 -> 8.6, mean of 45 launches 1.04x; 20 x 100,
+        //   16 heads, 5.26 -> 5.32); of 321 keys and more longest first as well (8 x 384 8.3 -> 7.2, 12 x 384 9.1 -> 8.4; mean of 27 launches 1.06x, 1.04x without it).
         // - INT8, two or three workgroups per CU at a time: longest first beyond one round of all CUs' places, and before that
         //   where the units are long enough for the ranking to pay, from 768 of them with three blocks of keys
-        //   (32 x 180 7.3 -> 6.9), 512 with five (14 x 310 9.5 -> 8.7), 256 with more (16 x 384 12.2 -> 9.9).  Rounds go backwards
+        //   (32 x 180 7.3 -> 6.9), beyond 512 with five and more (14 x 310 9.5 -> 8.7, 16 x 384 12.2 -> 9.9).  Rounds go backwards
         //   where a unit has an even number of parts (32 x 384 16.4 -> 11.7, longest first alone 12.7; 24 x 512, 16 heads,
-        //   25.4 -> 23.0); three parts are spread by themselves (24 x 180 5.6 -> 6.1), and units that are not shared have
-        //   enough rounds to even out (64 x 256, 16 heads, 18.2 -> 18.7).
+        //   25.4 -> 23.0) or one, up to four of them per CU or with one or two blocks of keys (70 x 100 6.1 -> 5.7, 64 x 160
+        //   8.6 -> 8.0; beyond, 86 x 256 17.5 -> 18.8); three parts are spread by themselves (24 x 180 5.6 -> 6.1).
         int64_t const workgroups = (int64_t) a.B * a.N * a.qSplit;
         bool ranked, back;
         if (f16 == F16Kernel::kSTREAM)
@@ -2613,17 +2629,17 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         }
         else if (f16 == F16Kernel::kTURNS)
         {
-            ranked = kt >= 6 && workgroups >= 512;
-            back = true;
+            ranked = blocks >= 6 && workgroups >= 512;
+            back = blocks > 2;
         }
         else
         {
             int64_t const lds = dataType == 2 ? Lds<1>::total(kt) : Lds<2>::total(kt);
             int64_t const perCu
                 = std::max<int64_t>(1, std::min<int64_t>(dataType == 2 ? 3 : 2, (160 * 1024) / std::max<int64_t>(lds, 1)));
-            int64_t const without = dataType != 2 || kt <= 2 ? perCu * 256 : kt >= 6 ? 256 : kt == 5 ? 512 : 767;
+            int64_t const without = dataType != 2 || blocks <= 2 ? perCu * 256 : blocks >= 5 ? 512 : 767;
             ranked = workgroups > std::min(perCu * 256, without);
-            back = dataType == 2 && ranked && a.qSplit % 2 == 0;
+            back = dataType == 2 && ranked && (a.qSplit == 1 ? blocks <= 2 || workgroups <= 1024 : a.qSplit % 2 == 0);
         }
         // tuning override: TRTAMD_FMHA_RANKED=0 forces natural order with every round forwards, 1 the longest-first order
         int const forcedRank = tuning(Tuning::kFmhaRanked);

@@ -53,9 +53,12 @@ INT8_PACKED = [
     # B, N, S (max), lens rule
     (3, 2, 128, "rand"), (2, 16, 384, "c4"), (5, 3, 64, "rand"), (4, 2, 192, "rand"), (3, 2, 256, "full"),
     (2, 2, 512, "rand"), (6, 1, 96, "edge"),
-    # unit counts either side of where the launcher stops sharing a (sequence, head) unit between workgroups (896),
-    # a count that takes three workgroups per unit, and one whose ids do not fill whole spans of 8 x parts
+    # unit counts of one workgroup each, one that takes three workgroups per unit, and one whose ids do not fill whole spans
+    # of 8 x parts
     (55, 16, 128, "rand"), (56, 16, 128, "rand"), (17, 16, 256, "c4"), (13, 3, 384, "rand"),
+    # either side of where the launcher stops sharing a (sequence, head) unit between workgroups, by blocks of keys
+    (213, 3, 128, "rand"), (40, 16, 128, "rand"), (767, 1, 130, "edge"), (256, 3, 130, "rand"), (64, 3, 256, "rand"),
+    (193, 1, 256, "rand"), (16, 8, 321, "c4"), (43, 3, 321, "rand"),
 ]
 
 

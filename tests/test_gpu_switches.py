@@ -332,7 +332,8 @@ def test_longest_first_order_reaches_every_sequence(B):
 @pytest.mark.parametrize("dtype,B,N,S", [(1, 511, 1, 64), (1, 512, 1, 64), (1, 513, 1, 64), (1, 128, 2, 192), (1, 43, 2, 321),
                                          (1, 1023, 1, 128), (1, 1024, 1, 128), (1, 1025, 1, 128), (1, 192, 2, 200),
                                          (1, 3329, 1, 64), (2, 128, 1, 384), (2, 129, 1, 330), (2, 192, 2, 190),
-                                         (2, 511, 1, 128), (2, 512, 1, 128), (2, 257, 2, 65)])
+                                         (2, 511, 1, 128), (2, 512, 1, 128), (2, 257, 2, 65), (2, 320, 2, 128),
+                                         (2, 512, 2, 190), (2, 205, 5, 190), (2, 193, 1, 250)])
 def test_rounds_that_go_backwards_reach_every_unit(dtype, B, N, S):
     """The order that the launcher chooses writes the bytes of the sequences' own order, and of every unit."""
     r = rng(1800 + B + S)
@@ -410,6 +411,40 @@ def test_fp16_attention_of_full_launches(S, B, N, growing, ranked):
         assert_fp_close(got[lo:hi, n * 64:(n + 1) * 64], want, what=f"sequence {b} of {hi - lo}, head {n}")
 
 
+# one workgroup of 128 queries short of the lines between the two FP16 kernels, by blocks of keys, and on them; past one round
+# of four per CU with two blocks
+@pytest.mark.parametrize("B,N,S", [(1024, 1, 64), (767, 1, 128), (768, 1, 128), (1024, 1, 100), (205, 5, 100), (299, 1, 192),
+                                   (300, 1, 192), (271, 1, 200), (272, 1, 200), (179, 1, 260), (180, 1, 260), (143, 1, 384),
+                                   (144, 1, 321), (95, 1, 400), (96, 1, 448), (89, 1, 512), (90, 1, 449)])
+def test_fp16_attention_on_either_side_of_its_kernels_lines(B, N, S):
+    api = capi.api()
+    r = rng(1900 + B + S)
+    edges = [n for n in (S, 1, 16, 63, 64, 65, 127, 128, 129, S - 1, 193, 257, 385) if n <= S]
+    lens = np.array([edges[i % len(edges)] for i in range(B)])
+    lens[7] = 0
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T = int(cu[-1])
+    qkv = r.standard_normal((T, N, 3, 64)).astype(np.float16)
+    d_qkv, d_cu = dev(qkv), dev(cu)
+    out = dev_empty((T + 64, N * 64), np.float16, fill=-7)
+    p = capi.FmhaParams()
+    p.qkv_ptr, p.o_ptr, p.cu_seqlens = ptr(d_qkv), ptr(out), ptr(d_cu)
+    p.qkv_stride_in_bytes, p.o_stride_in_bytes = 2 * 3 * N * 64, 2 * N * 64
+    p.b, p.h, p.s, p.d = B, N, S, 64
+    p.scale_bmm1, p.scale_softmax, p.scale_bmm2 = half2_bits(0.125), half2_bits(1.0), half2_bits(1.0)
+    api.check(api.fused_mha_run(stream(), 1, C.byref(p)))
+    sync()
+    got = host(out)
+    assert (got[T:] == -7).all()
+    for b in [*range(2 * len(edges)), *range(B - len(edges), B)]:
+        lo, hi = int(cu[b]), int(cu[b + 1])
+        if lo == hi:
+            continue
+        n = b % N
+        want = attention_f64(qkv[lo:hi, n, 0], qkv[lo:hi, n, 1], qkv[lo:hi, n, 2], 0.125)
+        assert_fp_close(got[lo:hi, n * 64:(n + 1) * 64], want, what=f"sequence {b} of {hi - lo}, head {n}")
+
+
 @pytest.mark.parametrize("scale", [0.125, 1.0])
 def test_fp16_attention_of_full_launches_keeps_infinite_scores_apart(scale):
     """Keys with a score of -infinity weigh nothing, also where they are a whole block or the first one; an infinite V
@@ -447,7 +482,7 @@ def test_fp16_attention_of_full_launches_keeps_infinite_scores_apart(scale):
     assert np.isinf(own).all() if scale == 0.125 else not np.isfinite(own).any()
 
 
-# packed masks: launches of either FP16 kernel (768 workgroups of 128 queries and fewer) and INT8
+# packed masks: launches of either FP16 kernel and INT8
 @pytest.mark.parametrize("dtype,scale", [(1, 0.125), (1, 1.0), (2, 0.125)])
 @pytest.mark.parametrize("S,B,N", [(64, 9, 2), (96, 9, 2), (128, 9, 2), (384, 9, 2), (128, 200, 4), (384, 70, 4)])
 def test_attention_with_packed_masks(dtype, scale, S, B, N):
