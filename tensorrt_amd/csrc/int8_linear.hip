@@ -90,7 +90,7 @@ struct LinearArgs
     int persist;   // persistent kernel: workgroups that loop over the 256 x 256 tiles
     int pieces;    // large tiles: the tokens behind them go in 64 x 64 pieces (see linear_piece64)
     int parts;     // pieces: workgroups that share the k range of a piece, each with an output of its own
-    int perPart;   // pieces: 32-byte k-slabs (interleaved operands) or 64-byte stages of each
+    int perPart;   // pieces: 32-byte k-slabs (interleaved operands) or stages of 64 or 128 bytes of each
     FastDiv panelDiv, perPanelDiv; // tiles: by panel and tokMain * panel
     WeightPrefetch prefetch; // by the workgroups behind mainTiles of the interleaved tile and piece kernels
 };
