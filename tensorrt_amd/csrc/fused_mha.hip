@@ -2391,7 +2391,6 @@ int launch_turns(hipStream_t stream, FmhaArgs const& a)
     return launch_fmha<fmha_f16_turns_kernel<KT, DEBUG, false>>("fmha_f16_turns", stream, a, Lds<2>::matBytes(KT), kWavesF16T);
 }
 
-
 template <bool DEBUG>
 int run_f16(hipStream_t stream, FmhaArgs const& a, F16Kernel which)
 {
@@ -2561,7 +2560,9 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         // 7.6; 144 units of 384: four 8.1, three 8.8; 336 units: two 11.2, three 12.4).  One per unit once rounds that go
         // forwards and backwards are even with it: from 640 units of one or two blocks (672 units: one 6.7, two 7.4; 600: 6.4 /
         // 6.0), 768 of three or four (192 keys: 9.0 / 10.0; 720 units: 10.9 / 9.9), 640 of five (752 units: 15.8 / 18.3, 600 of
-        // one length: 25.9 / 23.8), 1040 of six (900: 28.5 / 26.2; 1152: 31.5 / 32.6), 720 of more (440 keys: 26.9 / 29.2).
+        // one length: 25.9 / 23.8), 896 of six, 720 of more (440 keys: 26.9 / 29.2).  (Six by themselves: 900 units 28.5 / 26.2,
+        // 1152 31.5 / 32.6; but such launches are also halves of a pass on two streams, whose other half fills the idle CUs:
+        // 1008 and 1040 units side by side, 24 layers, 11.94 ms a pass with one workgroup per unit, 12.05 with two for 1008.)
         // The general FP16 kernel (its K and V take most of a
         // CU's LDS, one workgroup per CU, and staging them is 40 % of a workgroup's time): only below 160 units (192 units
         // of 192-384 keys: 15.3 us alone, 17.5 us shared by two; 144 units: 14.9 against 12.9 us).  The other FP16 kernels
@@ -2573,7 +2574,7 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
         int split = 1;
         if (dataType == 2)
         {
-            constexpr int kAloneFrom[] = {640, 640, 768, 768, 640, 1040, 720, 720}; // by blocks of keys
+            constexpr int kAloneFrom[] = {640, 640, 768, 768, 640, 896, 720, 720}; // by blocks of keys
             int const most = blocks <= 5 && heads > 192 ? 3 : 4;
             split = heads >= kAloneFrom[blocks - 1]
                 ? 1
