@@ -2538,11 +2538,11 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
     // room (longer sequences need more of it each), and a second round costs more than the wider workgroups that leave some CUs
     // with two of them, others with three.  12 or 16 heads, sequences of a third of the length to the length, us with 64 / with
     // 128 queries: 64 x 128 keys 8.1 / 7.7, 48 x 128 7.8 / 8.1; 27 x 180 8.0 / 7.1, 21 x 180 6.7 / 6.9; 27 x 230 10.1 / 7.9,
-    // 21 x 230 7.8 / 7.9; 20 x 310 11.7 / 10.1, 14 x 310 8.2 / 8.8; 16 x 384 12.0 / 9.8, 10 x 384 8.2 / 9.1; 12 x 440 12.9 / 9.8,
-    // 6 x 440 7.8 / 9.2; 10 x 512 14.3 / 10.8 (16 heads), 6 x 512 7.5 / 9.5.
+    // 21 x 230 7.8 / 7.9; 20 x 310 11.7 / 10.1, 14 x 310 8.2 / 8.8; 16 x 384 12.0 / 9.8, 13 x 345 9.4 / 9.8, 10 x 384 8.2 / 9.1;
+    // 12 x 440 12.9 / 9.8, 6 x 440 7.8 / 9.2; 10 x 512 14.3 / 10.8 (16 heads), 6 x 512 7.5 / 9.5.
     // With one or two blocks of keys a second round of the wide ones is no better: 110 x 128 13.0 / 14.4, 225 x 128 24.8 / 29.9;
     // and a row of at most 64 keys leaves half of them idle: 64 x 64 4.5 / 5.3, 600 x 64 25.6 / 28.3.
-    constexpr int kStreamFrom[] = {INT32_MAX, 768, 600, 544, 540, 432, 384, 360};
+    constexpr int kStreamFrom[] = {INT32_MAX, 768, 600, 544, 540, 504, 384, 360};
     constexpr int kStreamTile = kWavesStream * kStreamQueries;
     int const streamParts = ceil_div(kt * 64, kStreamTile);
     F16Kernel f16 = F16Kernel::kGENERAL;
