@@ -1938,15 +1938,18 @@ __global__ __launch_bounds__(NW * 64, PER_SIMD) void linear_piece_dma_kernel(uin
 // workgroups are dealt to the engines evenly, so on some GPUs a launch of one workgroup per CU runs a second round from
 // 3/4 of the CUs on (7765 tokens x 768 -> 768, 246 workgroups: 12.3 us on one GPU, 16.8 us on another).  Small tiles fill the
 // chip where the problem has few of them, large ones move fewer bytes per multiplication where it has many, and the pieces
-// cut the chain of stages by eight where neither fills it.
+// cut the chain of stages by eight, or by four where they read whole lines, where neither fills it.
 //
 // The constants are fits.  Linear operands: to launches by themselves on the four layers of 768- and 1024-channel FP16
 // encoders (graph replays, weights in the last-level cache), 16 to 33289 tokens, on two GPUs, one of them with the uneven
 // engines.  The plan they choose takes 0.8 % more than the best of all in the mean (24 % at most, a launch at the edge
-// of a second round); the kernels and the choice before took 13 % more (50 % at most).  The pieces' among them are fits to the
-// same layers at 16 to 1400 tokens since they read whole lines, 152 launches, times the 1.18 by which the tiles' constants
-// exceeded that GPU's times, and the wider pieces' a little more, for what they take in whole passes (102 tokens x 768 -> 2304:
-// the pass is 0.2 us a layer faster in the small ones): 0.01 % more than the best of six plans in the mean, 2 % at most.
+// of a second round); the kernels and the choice before took 13 % more (50 % at most).  The pieces' among them, which read whole
+// lines, are fits to 30 layers of 64 to 4096 FP16 values or twice as many INT8 ones, 32 to 4096 channels, 1 to 4000 tokens, 1800
+// launches, each piece's time multiplied by what the estimate of 64 x 64 tiles exceeds theirs by at the same sizes: tiles are
+// estimated 1.0 times what they take at rows of 8 KB and 1.4 times at 128 bytes, and the choice is between the two.  0.6 % more
+// than the best of ten plans in the mean, 1.8 % at most more than with the pieces of half lines.  (Fitted to the encoders' layers
+// only, the pieces were taken for short rows where tiles are faster, us: 2100 tokens x 128 -> 512, FP16, 5.3 against 3.7 in tiles;
+// 1700 x 384 -> 384 4.9 / 4.2; 600 x 384 -> 1152 5.0 / 4.4; 384 x 512 -> 2048 5.6 / 5.2.)
 // Linear operands whose rows end within a line have kernels and constants of their own: stages of 64 bytes, tiles of up to 128 x
 // 256, and constants fitted to launches by themselves before the other linear operands had stages of whole lines.  10 layers of
 // 96 to 3104 channels, 40 to 33289 tokens, FP16 and INT8, 240 launches: 6.5 % less in the mean than when all linear operands
@@ -2004,8 +2007,8 @@ constexpr TileCost kTileCosts[3][kLinearPlans] = {
     {{}, {}, {128, 128, 2, 4.64f, 0.00f, 0.231f, 0.60f, 0.61f, 1.02f, 0.40f, 0.25f}, {},
         {64, 64, 2, 3.82f, 0.29f, 0.082f, 0.23f, 0.70f, 0.89f, 0.63f, 0.34f},
         {128, 128, 1, 4.02f, 0.77f, 0.142f, 0.99f, 0.f, 1.30f, 0.77f, 0.51f, 0.10f}, {}, {},
-        {32, 64, 1, 1.77f, 1.65f, 0.058f, 0.16f, 0.f, 0.98f, 0.83f, 0.40f},
-        {32, 32, 2, 2.56f, 0.18f, 0.045f, 0.14f, 0.86f, 1.03f, 0.69f, 0.20f},
+        {32, 64, 1, 3.12f, 1.14f, 0.038f, 0.02f, 0.f, 1.08f, 0.89f, 0.56f},
+        {32, 32, 2, 3.73f, 0.13f, 0.018f, 0.f, 1.78f, 1.72f, 0.61f, 0.54f},
         {256, 256, 1, 0.00f, 4.48f, 0.440f, 1.88f, 0.f, 1.02f, 0.54f, 0.97f, 0.11f},
         {256, 192, 1, 5.13f, 0.01f, 0.388f, 1.26f, 0.f, 1.35f, 0.67f, 0.56f, 0.15f},
         {128, 192, 2, 4.47f, 0.10f, 0.289f, 0.70f, 0.78f, 0.99f, 0.47f, 0.38f},

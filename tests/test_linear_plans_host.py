@@ -42,6 +42,21 @@ def test_many_tokens_with_rows_that_end_within_a_line(T, row_bytes, N, gelu):
     assert plan(LINEAR, T, row_bytes, N, gelu) in ({1} if T > 2048 else {1, 3})
 
 
+@pytest.mark.parametrize("T,row_bytes,N,gelu", [(1200, 256, 512, 0), (2600, 256, 384, 0), (4000, 128, 256, 0), (1700, 384, 576, 0),
+                                                (2100, 512, 256, 0), (800, 640, 960, 0), (600, 768, 1152, 0), (1400, 768, 384, 0),
+                                                (384, 768, 1536, 1), (512, 1024, 1536, 0), (1200, 1024, 512, 0),
+                                                (384, 1024, 2048, 1), (256, 1280, 2560, 0), (700, 1536, 768, 0)])
+def test_short_rows_go_in_tiles(T, row_bytes, N, gelu):
+    """Layers with short rows of whole lines, where 64 x 64 tiles take 5 to 30 % less than the pieces."""
+    assert plan(LINEAR, T, row_bytes, N, gelu) in (4, 14)
+
+
+@pytest.mark.parametrize("T,row_bytes,N,want", [(1, 128, 256, 9), (65, 256, 512, 9), (102, 1536, 2304, 9),
+                                                (448, 6144, 768, 8), (96, 8192, 1024, 9), (2100, 256, 32, 9)])
+def test_few_tokens_go_in_pieces(T, row_bytes, N, want):
+    assert plan(LINEAR, T, row_bytes, N) == want
+
+
 def layers(layout, size, hidden, ffn):
     """The four linear layers of an encoder layer: row bytes, channels, GELU."""
     return [(layout, size * hidden, 3 * hidden, 0), (layout, size * hidden, hidden, 0), (layout, size * hidden, ffn, 1),
