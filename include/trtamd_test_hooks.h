@@ -38,6 +38,12 @@ TRTAMD_API int trtamd_test_linear_plan(int32_t interleaved, int32_t T, int32_t r
 /* How often the calling thread has worked such a number out, rather than remembered it. */
 TRTAMD_API int64_t trtamd_test_linear_estimates(void);
 
+/* What trtamd_fused_mha_run launches for these parameters under the switches as they are; of the pointers only counts which are
+ * NULL.  Bits 0-3: the kernel, 0 INT8 or the general FP16 one, FP16 with 64 queries per workgroup (1; 3: with all of K and V in
+ * LDS at once) or with 128 (2); bits 4-7: workgroups per (sequence, head); bit 8: the longest sequences first; from bit 17 on:
+ * how many times two rounds of 256 workgroups, the second of them backwards.  -1: parameters that have no kernel. */
+TRTAMD_API int64_t trtamd_test_fmha_route(int32_t data_type, trtamd_fmha_params const* params);
+
 #ifdef __cplusplus
 }
 #endif

@@ -136,6 +136,7 @@ _SIGS = {
     "trtamd_test_reset_tuning": (C.c_int, [C.c_char_p]),
     "trtamd_test_linear_plan": (C.c_int, [i32, i32, i32, i32, i32]),
     "trtamd_test_linear_estimates": (C.c_int64, []),
+    "trtamd_test_fmha_route": (C.c_int64, [i32, C.POINTER(FmhaParams)]),
     "trtamd_unfused_mha_static": (C.c_int, [c_p, i32, i32, i32, i32, i32, c_p, c_p, c_p]),
     "trtamd_fused_mha_run": (C.c_int, [c_p, i32, C.POINTER(FmhaParams)]),
     "trtamd_fused_mha_run_debug": (C.c_int, [c_p, i32, C.POINTER(FmhaParams), c_p, c_p]),
@@ -162,7 +163,7 @@ _SIGS = {
 
 # Entry points declared in include/trtamd_test_hooks.h (test-only).
 TEST_HOOK_SYMBOLS = ["trtamd_fused_mha_run_debug", "trtamd_test_set_tuning", "trtamd_test_reset_tuning",
-                     "trtamd_test_linear_plan", "trtamd_test_linear_estimates"]
+                     "trtamd_test_linear_plan", "trtamd_test_linear_estimates", "trtamd_test_fmha_route"]
 # Entry points declared in include/trtamd_bert_kernels.h are the rest of the table.
 # Entry points declared in include/trtamd_encoder_ops.h.
 ENCODER_OPS_SYMBOLS = ["trtamd_int8_linear", "trtamd_fp16_linear", "trtamd_int8_linear_to_interleaved", "trtamd_int8_interleaved_to_linear",

@@ -2373,6 +2373,10 @@ enum class F16Kernel
 // 512 keys, whose 136 KB a CU takes longer to bring in than it waits otherwise, 2 x 512 6.15 / 6.35.
 constexpr int64_t kWholeWorkgroups = 256;
 constexpr int kWholeBlocks = 6;
+bool is_whole(int kt, int64_t workgroups)
+{
+    return kt <= kWholeBlocks && workgroups <= kWholeWorkgroups;
+}
 constexpr int whole_lds(int kt)
 {
     return 2 * Lds<2>::matBytes(kt) + kQueriesF16 * Lds<2>::kRow;
@@ -2383,7 +2387,7 @@ int launch_turns(hipStream_t stream, FmhaArgs const& a)
 {
     if constexpr (KT <= kWholeBlocks)
     {
-        if ((int64_t) a.B * a.N * a.qSplit <= kWholeWorkgroups)
+        if (is_whole(KT, (int64_t) a.B * a.N * a.qSplit))
         {
             return launch_fmha<fmha_f16_turns_kernel<KT, DEBUG, true>>("fmha_f16_whole", stream, a, whole_lds(KT), kWavesF16T);
         }
@@ -2484,6 +2488,134 @@ float half_bits_to_float(uint16_t h)
     return bits_to_float(bits);
 }
 
+// What a launch runs.
+struct FmhaRoute
+{
+    F16Kernel f16;
+    int parts;      // workgroups per (sequence, head) unit
+    uint32_t order; // FmhaArgs.order
+};
+
+FmhaRoute route_of(int32_t dataType, trtamd_fmha_params const& p)
+{
+    int const kt = pick_kt(p.s);
+    int const blocks = ceil_div(p.s, 64);
+    // FP16: 128 queries per workgroup from so many of these workgroups on, by blocks of 64 keys; 64 of them and the scores of all
+    // their keys in registers below.  The latter run in one round up to four, three or two of them per CU, as their LDS leaves
+    // room (longer sequences need more of it each), and a second round costs more than the wider workgroups that leave some CUs
+    // with two of them, others with three.  12 or 16 heads, sequences of a third of the length to the length, us with 64 / with
+    // 128 queries: 64 x 128 keys 8.1 / 7.7, 48 x 128 7.8 / 8.1; 27 x 180 8.0 / 7.1, 21 x 180 6.7 / 6.9; 27 x 230 10.1 / 7.9,
+    // 21 x 230 7.8 / 7.9; 20 x 310 11.7 / 10.1, 14 x 310 8.2 / 8.8; 16 x 384 12.0 / 9.8, 13 x 345 9.4 / 9.8, 10 x 384 8.2 / 9.1;
+    // 12 x 440 12.9 / 9.8, 6 x 440 7.8 / 9.2; 10 x 512 14.3 / 10.8 (16 heads), 6 x 512 7.5 / 9.5.
+    // With one or two blocks of keys a second round of the wide ones is no better: 110 x 128 13.0 / 14.4, 225 x 128 24.8 / 29.9;
+    // and a row of at most 64 keys leaves half of them idle: 64 x 64 4.5 / 5.3, 600 x 64 25.6 / 28.3.
+    constexpr int kStreamFrom[] = {INT32_MAX, 768, 600, 544, 540, 504, 384, 360};
+    constexpr int kStreamTile = kWavesStream * kStreamQueries;
+    int const streamParts = ceil_div(kt * 64, kStreamTile);
+    FmhaRoute r{F16Kernel::kGENERAL, 1, 0};
+    F16Kernel& f16 = r.f16;
+    if (dataType == 1 && !tuning(Tuning::kFmhaGeneric)
+        && p.qkv_stride_in_bytes < (1LL << 29)) // eight tokens within a 32-bit offset
+    {
+        int64_t const wide = (int64_t) p.b * p.h * streamParts;
+        f16 = wide >= kStreamFrom[blocks - 1] && (blocks > 2 || wide <= 1024) ? F16Kernel::kSTREAM : F16Kernel::kTURNS;
+    }
+    // Workgroups per (sequence, head).  Every extra workgroup stages K and V again, so a unit is only shared
+    // while the launch would otherwise leave the chip partly idle or badly balanced.  INT8, three workgroups per CU of up to
+    // six blocks of keys and two of more: two per unit even out a round or two of units of very different lengths, and
+    // more of them fill one round, 768 workgroups or, from six blocks on, 512 (240 units of 256 keys: three 7.0 us, four
+    // 7.6; 144 units of 384: four 8.1, three 8.8; 336 units: two 11.2, three 12.4).  One per unit once rounds that go
+    // forwards and backwards are even with it: from 640 units of one or two blocks (672 units: one 6.7, two 7.4; 600: 6.4 /
+    // 6.0), 768 of three or four (192 keys: 9.0 / 10.0; 720 units: 10.9 / 9.9), 640 of five (752 units: 15.8 / 18.3, 600 of
+    // one length: 25.9 / 23.8), 896 of six, 720 of more (440 keys: 26.9 / 29.2).  (Six by themselves: 900 units 28.5 / 26.2,
+    // 1152 31.5 / 32.6; but such launches are also halves of a pass on two streams, whose other half fills the idle CUs:
+    // 1008 and 1040 units side by side, 24 layers, 11.94 ms a pass with one workgroup per unit, 12.05 with two for 1008.)
+    // The general FP16 kernel (its K and V take most of a
+    // CU's LDS, one workgroup per CU, and staging them is 40 % of a workgroup's time): only below 160 units (192 units
+    // of 192-384 keys: 15.3 us alone, 17.5 us shared by two; 144 units: 14.9 against 12.9 us).  The other FP16 kernels
+    // take 64 or 128 queries each, of as many as the kernel has room for: a sequence longer than s that still fits
+    // is served whole, as by the kernels that walk the queries.
+    int const waves = dataType == 2 ? kWavesI8 : kWavesF16;
+    int const maxSplit = std::max(1, ceil_div(ceil_div(p.s, kQPerWave), waves));
+    int64_t const heads = (int64_t) p.b * p.h;
+    int split = 1;
+    if (dataType == 2)
+    {
+        constexpr int kAloneFrom[] = {640, 640, 768, 768, 640, 896, 720, 720}; // by blocks of keys
+        int const most = blocks <= 5 && heads > 192 ? 3 : 4;
+        split = heads >= kAloneFrom[blocks - 1]
+            ? 1
+            : (int) std::max<int64_t>(2, std::min<int64_t>(most, ceil_div<int64_t>(blocks <= 5 ? 768 : 512, heads)));
+    }
+    else if (f16 != F16Kernel::kGENERAL)
+    {
+        split = f16 == F16Kernel::kTURNS ? kt : streamParts;
+    }
+    else
+    {
+        while (split < maxSplit && heads * split < 160)
+        {
+            split *= 2;
+        }
+    }
+    r.parts = f16 != F16Kernel::kGENERAL ? split : std::min(split, maxSplit);
+    // tuning override: TRTAMD_FMHA_QSPLIT=<n> forces the number of workgroups per head
+    int const forced = tuning(Tuning::kFmhaQsplit);
+    if (forced > 0 && f16 == F16Kernel::kGENERAL)
+    {
+        r.parts = std::min(forced, maxSplit);
+    }
+    // The order in which sequences are served: the longest first costs a workgroup the ranking (0.25 us: a trip to LDS or a
+    // few across the lanes before its loads) and evens out the CUs, or fills the tail of a launch of several rounds with
+    // short ones.  Every other round backwards (id_of_workgroup) costs nothing.  12 or 16 heads, sequences of a third of
+    // the length to the length:
+    // - FP16, 128 queries per workgroup: all resident at once up to four per CU; longest first below 3072 of them
+    //   (16 x 512 18.0 us against 21.2 in natural order, 32 x 384 19.0 / 20.4; 128 x 384, 16 heads, 85.6 / 82.4), and every
+    //   other round backwards always: 32 x 384 15.3 -> 14.8, 32 x 180 9.3 -> 8.2, 96 x 180 19.2 -> 17.0, and in natural order
+    //   128 x 180 31.9 -> 27.0, 128 x 256 40.0 -> 37.2 (16 heads).
+    // - FP16, 64 queries: short enough to even out by themselves, natural order, from three blocks of keys on with rounds
+    //   backwards (22 x 180 8.0 -> 6.7, 21 x 250 10.6 -> 10.0, 16 x 250 8.3 -> 8.6, mean of 45 launches 1.04x; 20 x 100,
+    //   16 heads, 5.26 -> 5.32); of 321 keys and more longest first as well (8 x 384 8.3 -> 7.2, 12 x 384 9.1 -> 8.4; mean of 27 launches 1.06x, 1.04x without it).
+    // - INT8, two or three workgroups per CU at a time: longest first beyond one round of all CUs' places, and before that
+    //   where the units are long enough for the ranking to pay, from 768 of them with three blocks of keys
+    //   (32 x 180 7.3 -> 6.9), beyond 512 with five and more (14 x 310 9.5 -> 8.7, 16 x 384 12.2 -> 9.9).  Rounds go backwards
+    //   where a unit has an even number of parts (32 x 384 16.4 -> 11.7, longest first alone 12.7; 24 x 512, 16 heads,
+    //   25.4 -> 23.0) or one, up to four of them per CU or with one or two blocks of keys (70 x 100 6.1 -> 5.7, 64 x 160
+    //   8.6 -> 8.0; beyond, 86 x 256 17.5 -> 18.8); three parts are spread by themselves (24 x 180 5.6 -> 6.1).
+    int64_t const workgroups = (int64_t) p.b * p.h * r.parts;
+    bool ranked, back;
+    if (f16 == F16Kernel::kSTREAM)
+    {
+        ranked = workgroups < 3072;
+        back = true;
+    }
+    else if (f16 == F16Kernel::kTURNS)
+    {
+        ranked = blocks >= 6 && workgroups >= 512;
+        back = blocks > 2;
+    }
+    else
+    {
+        int64_t const lds = dataType == 2 ? Lds<1>::total(kt) : Lds<2>::total(kt);
+        int64_t const perCu
+            = std::max<int64_t>(1, std::min<int64_t>(dataType == 2 ? 3 : 2, (160 * 1024) / std::max<int64_t>(lds, 1)));
+        int64_t const without = dataType != 2 || blocks <= 2 ? perCu * 256 : blocks >= 5 ? 512 : 767;
+        ranked = workgroups > std::min(perCu * 256, without);
+        back = dataType == 2 && ranked && (r.parts == 1 ? blocks <= 2 || workgroups <= 1024 : r.parts % 2 == 0);
+    }
+    // tuning override: TRTAMD_FMHA_RANKED=0 forces natural order with every round forwards, 1 the longest-first order
+    int const forcedRank = tuning(Tuning::kFmhaRanked);
+    if (forcedRank >= 0)
+    {
+        ranked = forcedRank != 0;
+        back = back && ranked;
+    }
+    // sequences of one length (24.0 us forwards, 24.1 backwards, 32 x 384) have nothing to even out
+    uint32_t const paired = back && p.cu_seqlens ? (uint32_t) std::min<int64_t>(workgroups, INT32_MAX) / kTwoRounds * kTwoRounds : 0;
+    r.order = paired | (ranked ? kRanked : 0);
+    return r;
+}
+
 int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const* p, int32_t* dbgAcc1, int8_t* dbgP8)
 {
     if (!p)
@@ -2531,128 +2663,13 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
     a.B = p->b;
     a.N = p->h;
     a.S = p->s;
-    int const kt = pick_kt(p->s);
-    int const blocks = ceil_div(p->s, 64);
-    // FP16: 128 queries per workgroup from so many of these workgroups on, by blocks of 64 keys; 64 of them and the scores of all
-    // their keys in registers below.  The latter run in one round up to four, three or two of them per CU, as their LDS leaves
-    // room (longer sequences need more of it each), and a second round costs more than the wider workgroups that leave some CUs
-    // with two of them, others with three.  12 or 16 heads, sequences of a third of the length to the length, us with 64 / with
-    // 128 queries: 64 x 128 keys 8.1 / 7.7, 48 x 128 7.8 / 8.1; 27 x 180 8.0 / 7.1, 21 x 180 6.7 / 6.9; 27 x 230 10.1 / 7.9,
-    // 21 x 230 7.8 / 7.9; 20 x 310 11.7 / 10.1, 14 x 310 8.2 / 8.8; 16 x 384 12.0 / 9.8, 13 x 345 9.4 / 9.8, 10 x 384 8.2 / 9.1;
-    // 12 x 440 12.9 / 9.8, 6 x 440 7.8 / 9.2; 10 x 512 14.3 / 10.8 (16 heads), 6 x 512 7.5 / 9.5.
-    // With one or two blocks of keys a second round of the wide ones is no better: 110 x 128 13.0 / 14.4, 225 x 128 24.8 / 29.9;
-    // and a row of at most 64 keys leaves half of them idle: 64 x 64 4.5 / 5.3, 600 x 64 25.6 / 28.3.
-    constexpr int kStreamFrom[] = {INT32_MAX, 768, 600, 544, 540, 504, 384, 360};
-    constexpr int kStreamTile = kWavesStream * kStreamQueries;
-    int const streamParts = ceil_div(kt * 64, kStreamTile);
-    F16Kernel f16 = F16Kernel::kGENERAL;
-    if (dataType == 1 && !tuning(Tuning::kFmhaGeneric)
-        && p->qkv_stride_in_bytes < (1LL << 29)) // eight tokens within a 32-bit offset
-    {
-        int64_t const wide = (int64_t) p->b * p->h * streamParts;
-        f16 = wide >= kStreamFrom[blocks - 1] && (blocks > 2 || wide <= 1024) ? F16Kernel::kSTREAM : F16Kernel::kTURNS;
-    }
-    {
-        // Workgroups per (sequence, head).  Every extra workgroup stages K and V again, so a unit is only shared
-        // while the launch would otherwise leave the chip partly idle or badly balanced.  INT8, three workgroups per CU of up to
-        // six blocks of keys and two of more: two per unit even out a round or two of units of very different lengths, and
-        // more of them fill one round, 768 workgroups or, from six blocks on, 512 (240 units of 256 keys: three 7.0 us, four
-        // 7.6; 144 units of 384: four 8.1, three 8.8; 336 units: two 11.2, three 12.4).  One per unit once rounds that go
-        // forwards and backwards are even with it: from 640 units of one or two blocks (672 units: one 6.7, two 7.4; 600: 6.4 /
-        // 6.0), 768 of three or four (192 keys: 9.0 / 10.0; 720 units: 10.9 / 9.9), 640 of five (752 units: 15.8 / 18.3, 600 of
-        // one length: 25.9 / 23.8), 896 of six, 720 of more (440 keys: 26.9 / 29.2).  (Six by themselves: 900 units 28.5 / 26.2,
-        // 1152 31.5 / 32.6; but such launches are also halves of a pass on two streams, whose other half fills the idle CUs:
-        // 1008 and 1040 units side by side, 24 layers, 11.94 ms a pass with one workgroup per unit, 12.05 with two for 1008.)
-        // The general FP16 kernel (its K and V take most of a
-        // CU's LDS, one workgroup per CU, and staging them is 40 % of a workgroup's time): only below 160 units (192 units
-        // of 192-384 keys: 15.3 us alone, 17.5 us shared by two; 144 units: 14.9 against 12.9 us).  The other FP16 kernels
-        // take 64 or 128 queries each, of as many as the kernel has room for: a sequence longer than s that still fits
-        // is served whole, as by the kernels that walk the queries.
-        int const waves = dataType == 2 ? kWavesI8 : kWavesF16;
-        int const maxSplit = std::max(1, ceil_div(ceil_div(p->s, kQPerWave), waves));
-        int64_t const heads = (int64_t) p->b * p->h;
-        int split = 1;
-        if (dataType == 2)
-        {
-            constexpr int kAloneFrom[] = {640, 640, 768, 768, 640, 896, 720, 720}; // by blocks of keys
-            int const most = blocks <= 5 && heads > 192 ? 3 : 4;
-            split = heads >= kAloneFrom[blocks - 1]
-                ? 1
-                : (int) std::max<int64_t>(2, std::min<int64_t>(most, ceil_div<int64_t>(blocks <= 5 ? 768 : 512, heads)));
-        }
-        else if (f16 != F16Kernel::kGENERAL)
-        {
-            split = f16 == F16Kernel::kTURNS ? kt : streamParts;
-        }
-        else
-        {
-            while (split < maxSplit && heads * split < 160)
-            {
-                split *= 2;
-            }
-        }
-        a.qSplit = f16 != F16Kernel::kGENERAL ? split : std::min(split, maxSplit);
-        // tuning override: TRTAMD_FMHA_QSPLIT=<n> forces the number of workgroups per head
-        int const forced = tuning(Tuning::kFmhaQsplit);
-        if (forced > 0 && f16 == F16Kernel::kGENERAL)
-        {
-            a.qSplit = std::min(forced, maxSplit);
-        }
-    }
+    FmhaRoute const route = route_of(dataType, *p);
+    a.qSplit = route.parts;
+    a.order = route.order;
     a.partDiv = fast_div((uint32_t) a.qSplit);
     a.headDiv = fast_div((uint32_t) a.N);
     a.dbgAcc1 = dbgAcc1;
     a.dbgP8 = dbgP8;
-    {
-        // The order in which sequences are served: the longest first costs a workgroup the ranking (0.25 us: a trip to LDS or a
-        // few across the lanes before its loads) and evens out the CUs, or fills the tail of a launch of several rounds with
-        // short ones.  Every other round backwards (id_of_workgroup) costs nothing.  12 or 16 heads, sequences of a third of
-        // the length to the length:
-        // - FP16, 128 queries per workgroup: all resident at once up to four per CU; longest first below 3072 of them
-        //   (16 x 512 18.0 us against 21.2 in natural order, 32 x 384 19.0 / 20.4; 128 x 384, 16 heads, 85.6 / 82.4), and every
-        //   other round backwards always: 32 x 384 15.3 -> 14.8, 32 x 180 9.3 -> 8.2, 96 x 180 19.2 -> 17.0, and in natural order
-        //   128 x 180 31.9 -> 27.0, 128 x 256 40.0 -> 37.2 (16 heads).
-        // - FP16, 64 queries: short enough to even out by themselves, natural order, from three blocks of keys on with rounds
-        //   backwards (22 x 180 8.0 -> 6.7, 21 x 250 10.6 -> 10.0, 16 x 250 8.3 -> 8.6, mean of 45 launches 1.04x; 20 x 100,
-        //   16 heads, 5.26 -> 5.32); of 321 keys and more longest first as well (8 x 384 8.3 -> 7.2, 12 x 384 9.1 -> 8.4; mean of 27 launches 1.06x, 1.04x without it).
-        // - INT8, two or three workgroups per CU at a time: longest first beyond one round of all CUs' places, and before that
-        //   where the units are long enough for the ranking to pay, from 768 of them with three blocks of keys
-        //   (32 x 180 7.3 -> 6.9), beyond 512 with five and more (14 x 310 9.5 -> 8.7, 16 x 384 12.2 -> 9.9).  Rounds go backwards
-        //   where a unit has an even number of parts (32 x 384 16.4 -> 11.7, longest first alone 12.7; 24 x 512, 16 heads,
-        //   25.4 -> 23.0) or one, up to four of them per CU or with one or two blocks of keys (70 x 100 6.1 -> 5.7, 64 x 160
-        //   8.6 -> 8.0; beyond, 86 x 256 17.5 -> 18.8); three parts are spread by themselves (24 x 180 5.6 -> 6.1).
-        int64_t const workgroups = (int64_t) a.B * a.N * a.qSplit;
-        bool ranked, back;
-        if (f16 == F16Kernel::kSTREAM)
-        {
-            ranked = workgroups < 3072;
-            back = true;
-        }
-        else if (f16 == F16Kernel::kTURNS)
-        {
-            ranked = blocks >= 6 && workgroups >= 512;
-            back = blocks > 2;
-        }
-        else
-        {
-            int64_t const lds = dataType == 2 ? Lds<1>::total(kt) : Lds<2>::total(kt);
-            int64_t const perCu
-                = std::max<int64_t>(1, std::min<int64_t>(dataType == 2 ? 3 : 2, (160 * 1024) / std::max<int64_t>(lds, 1)));
-            int64_t const without = dataType != 2 || blocks <= 2 ? perCu * 256 : blocks >= 5 ? 512 : 767;
-            ranked = workgroups > std::min(perCu * 256, without);
-            back = dataType == 2 && ranked && (a.qSplit == 1 ? blocks <= 2 || workgroups <= 1024 : a.qSplit % 2 == 0);
-        }
-        // tuning override: TRTAMD_FMHA_RANKED=0 forces natural order with every round forwards, 1 the longest-first order
-        int const forcedRank = tuning(Tuning::kFmhaRanked);
-        if (forcedRank >= 0)
-        {
-            ranked = forcedRank != 0;
-            back = back && ranked;
-        }
-        // sequences of one length (24.0 us forwards, 24.1 backwards, 32 x 384) have nothing to even out
-        uint32_t const paired = back && a.cuSeqlens ? (uint32_t) std::min<int64_t>(workgroups, INT32_MAX) / kTwoRounds * kTwoRounds : 0;
-        a.order = paired | (ranked ? kRanked : 0);
-    }
     if (interleaved)
     {
         // strides carry the total token count (qkvToContextInt8InterleavedPlugin.cpp:280-281)
@@ -2741,7 +2758,7 @@ int fused_mha_run(hipStream_t stream, int32_t dataType, trtamd_fmha_params const
     a.c = s1 * kLog2e;
     a.scaleSoftmax = 1.f;
     a.scaleBmm2 = 1.f;
-    return dbgAcc1 ? run_f16<true>(stream, a, f16) : run_f16<false>(stream, a, f16);
+    return dbgAcc1 ? run_f16<true>(stream, a, route.f16) : run_f16<false>(stream, a, route.f16);
 }
 
 } // namespace
@@ -2760,6 +2777,17 @@ extern "C" int trtamd_fused_mha_run_debug(trtamd_stream_t stream, int32_t data_t
     trtamd_fmha_params const* params, int32_t* acc1, int8_t* p8)
 {
     return fused_mha_run(as_stream(stream), data_type, params, acc1, p8);
+}
+
+extern "C" int64_t trtamd_test_fmha_route(int32_t data_type, trtamd_fmha_params const* p)
+{
+    if (!p || (data_type != 1 && data_type != 2) || p->b <= 0 || p->h <= 0 || !trtamd_fused_mha_is_valid(data_type, p->d, p->s))
+    {
+        return -1;
+    }
+    FmhaRoute const r = route_of(data_type, *p);
+    bool const whole = r.f16 == F16Kernel::kTURNS && is_whole(pick_kt(p->s), (int64_t) p->b * p->h * r.parts);
+    return (int64_t) (whole ? 3 : (int) r.f16) | r.parts << 4 | (int64_t) r.order << 8;
 }
 
 extern "C" int trtamd_fused_mha_prepare(void)
