@@ -1565,7 +1565,8 @@ __global__ __launch_bounds__(kWavesF16* kWaveSize) void fmha_f16_kernel(FmhaArgs
 // to the length, that kernel / this one, us per plugin call: 32 x 128 keys 12.5 / 5.8, 128 x 256 41.7 / 37.5, 32 x 384
 // 19.8 / 19.6, 128 x 384 71.7 / 64.6, 16 x 512 22.8 / 19.5.  What is left is the L2: K and V of a unit are read once for every
 // 64 queries, 133 MB for the 35.8 MB of 32 x 384.
-// WHOLE: launches so small that a CU has room for all of it (kWholeWorkgroups); K, V and Q are requested together then.
+// WHOLE: launches so small that a CU has room for all of it (kWholeWorkgroups); K, V and Q of sequences of up to kWholeBlocks
+// blocks are requested together then.
 // ------------------------------------------------------------------------------------------
 constexpr int kQueriesF16 = kWavesF16T * kQPerWave;
 __device__ u32x4 const kZeroRow[8] = {}; // 64 binary16 zeros, in memory
@@ -1579,6 +1580,16 @@ __device__ __forceinline__ void for_each_block(F&& f)
         for_each_block<N, I + 1>(f);
     }
 }
+
+// Launches of no more workgroups than CUs, each with a CU's LDS to itself, have K, V and 64 queries of a sequence there at once:
+// nothing waits for a place, which takes one or two trips to the L2 out of the chain.  With five blocks of keys and more a CU takes
+// longer to bring it all in than it waits otherwise, so longer sequences of such a launch go in turns.  In turns / so, graph
+// replays, us, means over 1 to 250 sequences and 1 to 16 heads: all of 64 keys 3.75 / 3.59, of 128 4.23 / 4.24, of 192 4.78 / 4.74,
+// of 256 5.24 / 5.23, of 320 5.93 / 6.00, of 384 6.55 / 6.76; up to 64 of the 384 keys that the kernel has room for 3.77 / 3.65.
+// With more workgroups than CUs it would keep others off them: 8 x 180 5.08 / 5.25, 4 x 384 6.66 / 8.95.
+constexpr int64_t kWholeWorkgroups = 256;
+constexpr int kWholeBlocks = 4;
+constexpr int kWholeCapacity = 6; // blocks that the kernels of such launches have room for at most
 
 template <int NKB, bool DEBUG, bool WHOLE>
 __device__ __forceinline__ void attend_f16_turns(
@@ -1900,7 +1911,8 @@ __global__ __launch_bounds__(kWavesF16T* kWaveSize)
     {
 #define TRTAMD_BLOCKS(NKB)                                                                                             \
     case NKB:                                                                                                          \
-        if constexpr (KT >= NKB) attend_f16_turns<NKB, DEBUG, WHOLE>(a, sq, b, n, q0, smem, masks, holes);             \
+        if constexpr (KT >= NKB)                                                                                       \
+            attend_f16_turns<NKB, DEBUG, WHOLE && NKB <= kWholeBlocks>(a, sq, b, n, q0, smem, masks, holes);           \
         break
         TRTAMD_BLOCKS(1);
         TRTAMD_BLOCKS(2);
@@ -2366,26 +2378,20 @@ enum class F16Kernel
     kSTREAM
 };
 
-// Launches of no more workgroups than CUs, each with a CU's LDS to itself, have K, V and 64 queries there at once: nothing waits for
-// a place, which takes one or two trips to the L2 out of the chain.  Sequences of a third of the length to the length, 12 heads,
-// in turns / so, us: 2 x 128 keys 3.96 / 3.84, 2 x 180 4.36 / 4.27, 2 x 256 4.91 / 4.84, 2 x 384 5.62 / 5.57 (an FP16 pass of one
-// request 337.9 / 333.5); with more workgroups, which it would keep off the CU, 8 x 180 5.08 / 5.25, 4 x 384 6.66 / 8.95; and at
-// 512 keys, whose 136 KB a CU takes longer to bring in than it waits otherwise, 2 x 512 6.15 / 6.35.
-constexpr int64_t kWholeWorkgroups = 256;
-constexpr int kWholeBlocks = 6;
 bool is_whole(int kt, int64_t workgroups)
 {
-    return kt <= kWholeBlocks && workgroups <= kWholeWorkgroups;
+    return kt <= kWholeCapacity && workgroups <= kWholeWorkgroups;
 }
 constexpr int whole_lds(int kt)
 {
-    return 2 * Lds<2>::matBytes(kt) + kQueriesF16 * Lds<2>::kRow;
+    int const whole = std::min(kt, kWholeBlocks);
+    return std::max(Lds<2>::matBytes(kt), 2 * Lds<2>::matBytes(whole) + kQueriesF16 * Lds<2>::kRow);
 }
 
 template <int KT, bool DEBUG>
 int launch_turns(hipStream_t stream, FmhaArgs const& a)
 {
-    if constexpr (KT <= kWholeBlocks)
+    if constexpr (KT <= kWholeCapacity)
     {
         if (is_whole(KT, (int64_t) a.B * a.N * a.qSplit))
         {
@@ -2458,7 +2464,7 @@ int prepare_kt()
     st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_i8_kernel<KT, false, false>), "fmha_i8", Lds<1>::total(KT));
     st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_f16_turns_kernel<KT, false, false>), "fmha_f16_turns",
                       Lds<2>::matBytes(KT));
-    if constexpr (KT <= kWholeBlocks)
+    if constexpr (KT <= kWholeCapacity)
     {
         st = st ? st : ensure_lds(reinterpret_cast<void const*>(fmha_f16_turns_kernel<KT, false, true>), "fmha_f16_whole", whole_lds(KT));
     }

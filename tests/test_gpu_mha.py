@@ -251,10 +251,11 @@ def test_fmha_fp16_packed_tile_edges(api, B, N, S):
 
 
 @pytest.mark.parametrize("S,lens", [(64, [1, 64, 63, 17]), (128, [65, 128, 1, 64]), (192, [129, 192, 191, 64]),
-                                    (256, [193, 256, 255, 128]), (384, [257, 384, 321, 320, 64]), (512, [385, 512, 449])])
+                                    (256, [193, 256, 255, 128]), (384, [257, 384, 321, 320, 64]), (384, [256, 257, 193, 65]),
+                                    (512, [385, 512, 449])])
 def test_fmha_fp16_few_workgroups(api, S, lens):
-    """Launches of no more workgroups than CUs have all of K and V in LDS at once, larger ones in turns: the same bytes for the
-    same sequences, lengths either side of the blocks of 64 keys; and the oracle's result."""
+    """Launches of no more workgroups than CUs have all of K and V of up to four blocks of 64 keys in LDS at once, larger ones and
+    longer sequences in turns: the same bytes for the same sequences, lengths either side of the blocks; and the oracle's result."""
     from tensorrt_amd import capi
     N = 2
     once = rng(33).standard_normal((sum(lens), 3 * N * D)).astype(np.float16)
