@@ -2494,6 +2494,32 @@ float half_bits_to_float(uint16_t h)
     return bits_to_float(bits);
 }
 
+// INT8: workgroups per (sequence, head) unit of the padded layout, where every query row is computed and units differ by their
+// masks only.  Three workgroups of up to six blocks of keys have room on a CU, two of more.  Units that do not come in even halves,
+// an odd number of tiles of 64 queries or 96 queries, go to one workgroup each from 641 on: one round up to 768 units, and hardly
+// worse than halves beyond (alone / in two, us: 700 units of 96 keys 6.9 / 7.9, of 192 14.9 / 15.7, of 320 28.4 / 30.6; 800 of 96
+// 7.8 / 8.8, of 320 35.1 / 34.6).  128 keys are even halves, but masks leave some units shorter: alone with them (700 units 1.06 to
+// 1.10 of the speed, 800 1.02 to 1.10), in two without (800 units 10.3 / 9.9).  Even halves stay together up to 895 units (800 of
+// 256 keys: alone 0.82 to 0.86 of the speed, of 384 0.87, of 512 0.88), beyond which the line is not at its best: halves are still
+// 1.07 to 1.14 times as fast at 1152 units.  Below, as many as fill a round of 768: two, three or four, but of five and six blocks three
+// from 193 units on (in three / in four, 240 units: 320 keys 1.29 of the speed, 384 15.5 / 18.4 us, 512 27.2 / 24.9) and of six
+// blocks two from 342 (in two / in three: 300 units of 384 keys 20.6 / 19.1, 352 21.1 / 22.0).
+int padded_int8_parts(trtamd_fmha_params const& p, int blocks)
+{
+    int64_t const units = (int64_t) p.b * p.h;
+    bool const uneven = blocks % 2 == 1 || p.s <= 96 || (blocks == 2 && p.packed_mask_ptr);
+    if (units >= (uneven ? 641 : 896))
+    {
+        return 1;
+    }
+    if (blocks == 6 && units >= 342)
+    {
+        return 2;
+    }
+    int64_t const most = (blocks == 5 || blocks == 6) && units >= 193 ? 3 : 4;
+    return (int) std::max<int64_t>(2, std::min(most, ceil_div<int64_t>(768, units)));
+}
+
 // What a launch runs.
 struct FmhaRoute
 {
@@ -2545,7 +2571,11 @@ FmhaRoute route_of(int32_t dataType, trtamd_fmha_params const& p)
     int const maxSplit = std::max(1, ceil_div(ceil_div(p.s, kQPerWave), waves));
     int64_t const heads = (int64_t) p.b * p.h;
     int split = 1;
-    if (dataType == 2)
+    if (dataType == 2 && !p.cu_seqlens)
+    {
+        split = padded_int8_parts(p, blocks);
+    }
+    else if (dataType == 2)
     {
         constexpr int kAloneFrom[] = {640, 640, 768, 768, 640, 896, 720, 720}; // by blocks of keys
         int const most = blocks <= 5 && heads > 192 ? 3 : 4;

@@ -60,3 +60,18 @@ def test_every_part_has_queries_and_every_round_is_whole(dtype, s, layout):
         if dtype == FP16:
             assert r.parts == {TURNS: blocks, WHOLE: blocks, STREAM: -(-blocks // 2)}[r.kernel]
             assert (r.kernel == WHOLE) == (r.kernel != STREAM and units * blocks <= 256 and s <= 384)
+
+
+# either side of each line between the numbers of parts
+@pytest.mark.parametrize("s,masked,parts", [
+    (64, True, {200: 1, 1000: 1}),
+    (96, True, {300: 2, 640: 2, 641: 1, 800: 1, 896: 1}), (96, False, {640: 2, 641: 1, 800: 1}),
+    (128, True, {640: 2, 641: 1, 800: 1}), (128, False, {640: 2, 800: 2, 895: 2, 896: 1}),
+    (192, False, {255: 3, 383: 3, 384: 2, 640: 2, 641: 1, 768: 1}),
+    (256, False, {192: 4, 193: 4, 255: 4, 256: 3, 383: 3, 384: 2, 768: 2, 895: 2, 896: 1}),
+    (320, False, {192: 4, 193: 3, 383: 3, 384: 2, 640: 2, 641: 1}),
+    (384, True, {170: 4, 171: 4, 192: 4, 193: 3, 256: 3, 341: 3, 342: 2, 895: 2, 896: 1}), (384, False, {192: 4, 256: 3, 896: 1}),
+    (448, False, {171: 4, 255: 4, 256: 3, 383: 3, 384: 2, 640: 2, 641: 1}),
+    (512, False, {171: 4, 255: 4, 256: 3, 383: 3, 384: 2, 720: 2, 895: 2, 896: 1})])
+def test_parts_of_padded_int8_units(s, masked, parts):
+    assert {u: route(INT8, u, s, packed=False, masked=masked).parts for u in parts} == parts
