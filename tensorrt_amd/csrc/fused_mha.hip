@@ -2494,30 +2494,66 @@ float half_bits_to_float(uint16_t h)
     return bits_to_float(bits);
 }
 
-// INT8: workgroups per (sequence, head) unit of the padded layout, where every query row is computed and units differ by their
-// masks only.  Three workgroups of up to six blocks of keys have room on a CU, two of more.  Units that do not come in even halves,
-// an odd number of tiles of 64 queries or 96 queries, go to one workgroup each from 641 on: one round up to 768 units, and hardly
-// worse than halves beyond (alone / in two, us: 700 units of 96 keys 6.9 / 7.9, of 192 14.9 / 15.7, of 320 28.4 / 30.6; 800 of 96
-// 7.8 / 8.8, of 320 35.1 / 34.6).  128 keys are even halves, but masks leave some units shorter: alone with them (700 units 1.06 to
-// 1.10 of the speed, 800 1.02 to 1.10), in two without (800 units 10.3 / 9.9).  Even halves stay together up to 895 units (800 of
-// 256 keys: alone 0.82 to 0.86 of the speed, of 384 0.87, of 512 0.88), beyond which the line is not at its best: halves are still
-// 1.07 to 1.14 times as fast at 1152 units.  Below, as many as fill a round of 768: two, three or four, but of five and six blocks three
-// from 193 units on (in three / in four, 240 units: 320 keys 1.29 of the speed, 384 15.5 / 18.4 us, 512 27.2 / 24.9) and of six
-// blocks two from 342 (in two / in three: 300 units of 384 keys 20.6 / 19.1, 352 21.1 / 22.0).
-int padded_int8_parts(trtamd_fmha_params const& p, int blocks)
+// INT8 units that are alike: of the padded layout, where every query row is computed and units differ by their masks only, and of a
+// packed batch that is as good as padded, which the interleaved layout's strides show, since they are its number of tokens.
+bool alike(trtamd_fmha_params const& p)
+{
+    return !p.cu_seqlens || (p.interleaved && p.qkv_stride_in_bytes >= ceil_div<int64_t>((int64_t) p.b * p.s * 15, 16));
+}
+
+// INT8: from how many (sequence, head) units on each has a workgroup of its own, by blocks of keys.  Three workgroups of up to six
+// blocks have room on a CU, two of more; every extra workgroup of a unit stages K and V again.
+// Packed sequences: once rounds that go forwards and backwards even out units of different lengths, from 640 units of one or two
+// blocks (672 units: one 6.7, two 7.4 us; 600: 6.4 / 6.0), 768 of three or four (192 keys: 9.0 / 10.0; 720 units: 10.9 / 9.9), 640
+// of five (752 units: 15.8 / 18.3), 896 of six, 720 of more (440 keys: 26.9 / 29.2).  (Six by themselves: 900 units 28.5 / 26.2,
+// 1152 31.5 / 32.6; but such launches are also halves of a pass on two streams, whose other half fills the idle CUs: 1008 and 1040
+// units side by side, 24 layers, 11.94 ms a pass with one workgroup per unit, 12.05 with two for 1008.)
+// Units that are alike: those that do not come in even halves, an odd number of tiles of 64 queries or 96 queries, from 641 on: one
+// round up to 768 units, and hardly worse than halves beyond (alone / in two, us: 700 units of 96 keys 6.9 / 7.9, of 192 14.9 /
+// 15.7, of 320 28.4 / 30.6; 800 of 96 7.8 / 8.8, of 320 35.1 / 34.6).  128 keys are even halves, but masks leave some units shorter:
+// alone with them (700 units 1.06 to 1.10 of the speed, 800 1.02 to 1.10), in two without (800 units 10.3 / 9.9).  Even halves stay
+// together up to 895 units (800 of 256 keys: alone 0.82 to 0.86 of the speed, of 384 0.87, of 512 0.88), beyond which the line is
+// not at its best: halves are still 1.07 to 1.14 times as fast at 1152 units.
+int64_t int8_alone_from(trtamd_fmha_params const& p, int blocks)
+{
+    if (!alike(p))
+    {
+        constexpr int kUnlike[] = {640, 640, 768, 768, 640, 896, 720, 720};
+        return kUnlike[blocks - 1];
+    }
+    bool const uneven = blocks % 2 == 1 || p.s <= 96 || (blocks == 2 && p.packed_mask_ptr && !p.cu_seqlens);
+    return uneven ? 641 : 896;
+}
+
+// INT8: workgroups per unit.  Below that line as many as fill a round of 768, two to four, but for five and six blocks of keys and
+// more, whose workgroups are longer.
+// Alike, padded, us: three from 193 units on (240 units, in three / in four: 320 keys 1.29 of the speed, 384 15.5 / 18.4; of 256 keys,
+// padded, 0.95 to 0.98, packed 8.8 / 9.5; of 512 27.2 / 24.9), of six blocks two from 342 on, where three would be more than four
+// workgroups per CU (300 units, in two / in three, 20.6 / 19.1, 352 21.1 / 22.0).
+// Others, geometric means over lengths of a third of s to s, of less than a sixth of s, from one on and between: of five blocks three
+// from 193 units on (226 units 1.09 times as fast as in four; of 256 keys 0.99), of more from 171 (206 units of 384 keys 1.10 times
+// as fast, of 448 1.15, of 512 1.11).  Two of six blocks from 288 on (268 units 0.95 times as fast as in three, 288 0.99, 316 1.00,
+// 356 1.06), of more from 320 (288 units of 448 keys 0.93, of 512 0.99; 316 0.98 and 0.99, 356 1.00 and 0.98; where lengths spread
+// from a third of s, 288 and 316 units 1.06).
+int int8_parts(trtamd_fmha_params const& p, int blocks)
 {
     int64_t const units = (int64_t) p.b * p.h;
-    bool const uneven = blocks % 2 == 1 || p.s <= 96 || (blocks == 2 && p.packed_mask_ptr);
-    if (units >= (uneven ? 641 : 896))
+    if (units >= int8_alone_from(p, blocks))
     {
         return 1;
     }
-    if (blocks == 6 && units >= 342)
+    int three = 256, two = 384;
+    if (alike(p))
     {
-        return 2;
+        three = blocks == 5 || blocks == 6 || (blocks == 4 && p.cu_seqlens) ? 193 : three;
+        two = blocks == 6 ? 342 : two;
     }
-    int64_t const most = (blocks == 5 || blocks == 6) && units >= 193 ? 3 : 4;
-    return (int) std::max<int64_t>(2, std::min(most, ceil_div<int64_t>(768, units)));
+    else if (blocks >= 5)
+    {
+        three = blocks == 5 ? 193 : 171;
+        two = blocks == 5 ? two : blocks == 6 ? 288 : 320;
+    }
+    return units >= two ? 2 : units >= three ? 3 : 4;
 }
 
 // What a launch runs.
@@ -2552,36 +2588,17 @@ FmhaRoute route_of(int32_t dataType, trtamd_fmha_params const& p)
         int64_t const wide = (int64_t) p.b * p.h * streamParts;
         f16 = wide >= kStreamFrom[blocks - 1] && (blocks > 2 || wide <= 1024) ? F16Kernel::kSTREAM : F16Kernel::kTURNS;
     }
-    // Workgroups per (sequence, head).  Every extra workgroup stages K and V again, so a unit is only shared
-    // while the launch would otherwise leave the chip partly idle or badly balanced.  INT8, three workgroups per CU of up to
-    // six blocks of keys and two of more: two per unit even out a round or two of units of very different lengths, and
-    // more of them fill one round, 768 workgroups or, from six blocks on, 512 (240 units of 256 keys: three 7.0 us, four
-    // 7.6; 144 units of 384: four 8.1, three 8.8; 336 units: two 11.2, three 12.4).  One per unit once rounds that go
-    // forwards and backwards are even with it: from 640 units of one or two blocks (672 units: one 6.7, two 7.4; 600: 6.4 /
-    // 6.0), 768 of three or four (192 keys: 9.0 / 10.0; 720 units: 10.9 / 9.9), 640 of five (752 units: 15.8 / 18.3, 600 of
-    // one length: 25.9 / 23.8), 896 of six, 720 of more (440 keys: 26.9 / 29.2).  (Six by themselves: 900 units 28.5 / 26.2,
-    // 1152 31.5 / 32.6; but such launches are also halves of a pass on two streams, whose other half fills the idle CUs:
-    // 1008 and 1040 units side by side, 24 layers, 11.94 ms a pass with one workgroup per unit, 12.05 with two for 1008.)
-    // The general FP16 kernel (its K and V take most of a
-    // CU's LDS, one workgroup per CU, and staging them is 40 % of a workgroup's time): only below 160 units (192 units
-    // of 192-384 keys: 15.3 us alone, 17.5 us shared by two; 144 units: 14.9 against 12.9 us).  The other FP16 kernels
-    // take 64 or 128 queries each, of as many as the kernel has room for: a sequence longer than s that still fits
-    // is served whole, as by the kernels that walk the queries.
+    // Workgroups per (sequence, head).  The general FP16 kernel (its K and V take most of a CU's LDS, one workgroup per CU, and
+    // staging them is 40 % of a workgroup's time) shares a unit only below 160 of them (192 units of 192-384 keys: 15.3 us alone,
+    // 17.5 us shared by two; 144 units: 14.9 against 12.9 us).  The other FP16 kernels take 64 or 128 queries each, of as many as
+    // the kernel has room for: a sequence longer than s that still fits is served whole, as by the kernels that walk the queries.
     int const waves = dataType == 2 ? kWavesI8 : kWavesF16;
     int const maxSplit = std::max(1, ceil_div(ceil_div(p.s, kQPerWave), waves));
     int64_t const heads = (int64_t) p.b * p.h;
     int split = 1;
-    if (dataType == 2 && !p.cu_seqlens)
+    if (dataType == 2)
     {
-        split = padded_int8_parts(p, blocks);
-    }
-    else if (dataType == 2)
-    {
-        constexpr int kAloneFrom[] = {640, 640, 768, 768, 640, 896, 720, 720}; // by blocks of keys
-        int const most = blocks <= 5 && heads > 192 ? 3 : 4;
-        split = heads >= kAloneFrom[blocks - 1]
-            ? 1
-            : (int) std::max<int64_t>(2, std::min<int64_t>(most, ceil_div<int64_t>(blocks <= 5 ? 768 : 512, heads)));
+        split = int8_parts(p, blocks);
     }
     else if (f16 != F16Kernel::kGENERAL)
     {
@@ -2613,11 +2630,14 @@ FmhaRoute route_of(int32_t dataType, trtamd_fmha_params const& p)
     //   backwards (22 x 180 8.0 -> 6.7, 21 x 250 10.6 -> 10.0, 16 x 250 8.3 -> 8.6, mean of 45 launches 1.04x; 20 x 100,
     //   16 heads, 5.26 -> 5.32); of 321 keys and more longest first as well (8 x 384 8.3 -> 7.2, 12 x 384 9.1 -> 8.4; mean of 27 launches 1.06x, 1.04x without it).
     // - INT8, two or three workgroups per CU at a time: longest first beyond one round of all CUs' places, and before that
-    //   where the units are long enough for the ranking to pay, from 768 of them with three blocks of keys
+    //   where the units are long enough for the ranking to pay, from 768 of them with three and four blocks of keys
     //   (32 x 180 7.3 -> 6.9), beyond 512 with five and more (14 x 310 9.5 -> 8.7, 16 x 384 12.2 -> 9.9).  Rounds go backwards
     //   where a unit has an even number of parts (32 x 384 16.4 -> 11.7, longest first alone 12.7; 24 x 512, 16 heads,
     //   25.4 -> 23.0) or one, up to four of them per CU or with one or two blocks of keys (70 x 100 6.1 -> 5.7, 64 x 160
-    //   8.6 -> 8.0; beyond, 86 x 256 17.5 -> 18.8); three parts are spread by themselves (24 x 180 5.6 -> 6.1).
+    //   8.6 -> 8.0; beyond, 86 x 256 17.5 -> 18.8); three parts are spread by themselves (24 x 180 5.6 -> 6.1).  Beyond
+    //   768, four parts of four blocks, a tile of queries each, are short enough without the ranking (13 x 256, 16 heads, 8.0 ->
+    //   7.2), and units that are alike have nothing to rank, but parts of different lengths (34 x 192 of one length, 16 heads,
+    //   1.06 times as fast backwards).
     int64_t const workgroups = (int64_t) p.b * p.h * r.parts;
     bool ranked, back;
     if (f16 == F16Kernel::kSTREAM)
@@ -2636,8 +2656,10 @@ FmhaRoute route_of(int32_t dataType, trtamd_fmha_params const& p)
         int64_t const perCu
             = std::max<int64_t>(1, std::min<int64_t>(dataType == 2 ? 3 : 2, (160 * 1024) / std::max<int64_t>(lds, 1)));
         int64_t const without = dataType != 2 || blocks <= 2 ? perCu * 256 : blocks >= 5 ? 512 : 767;
-        ranked = workgroups > std::min(perCu * 256, without);
-        back = dataType == 2 && ranked && (r.parts == 1 ? blocks <= 2 || workgroups <= 1024 : r.parts % 2 == 0);
+        bool const beyond = workgroups > without;
+        bool const level = dataType == 2 && (alike(p) || (blocks == 4 && r.parts == 4 && workgroups > 768));
+        ranked = beyond && !level;
+        back = dataType == 2 && beyond && (r.parts == 1 ? !level && (blocks <= 2 || workgroups <= 1024) : r.parts % 2 == 0);
     }
     // tuning override: TRTAMD_FMHA_RANKED=0 forces natural order with every round forwards, 1 the longest-first order
     int const forcedRank = tuning(Tuning::kFmhaRanked);

@@ -28,11 +28,14 @@ def params(dtype, units, s, packed=True, masked=False, heads=1):
     return p
 
 
-def route(dtype, units, s, **layout):
+def decode(r):
     """backwards: the number of workgroups whose every other round of 256 goes backwards."""
-    r = capi.api().test_fmha_route(dtype, C.byref(params(dtype, units, s, **layout)))
     assert r >= 0
     return Route(r & 15, r >> 4 & 15, bool(r >> 8 & 1), (r >> 17) * 512)
+
+
+def route(dtype, units, s, **layout):
+    return decode(capi.api().test_fmha_route(dtype, C.byref(params(dtype, units, s, **layout))))
 
 
 def test_parameters_without_a_kernel():
@@ -75,3 +78,38 @@ def test_every_part_has_queries_and_every_round_is_whole(dtype, s, layout):
     (512, False, {171: 4, 255: 4, 256: 3, 383: 3, 384: 2, 720: 2, 895: 2, 896: 1})])
 def test_parts_of_padded_int8_units(s, masked, parts):
     assert {u: route(INT8, u, s, packed=False, masked=masked).parts for u in parts} == parts
+
+
+@pytest.mark.parametrize("s,parts", [
+    (128, {200: 2, 639: 2, 640: 1}), (192, {200: 3, 383: 3, 384: 2, 767: 2, 768: 1}),
+    (256, {192: 4, 193: 4, 255: 4, 256: 3, 383: 3, 384: 2, 767: 2, 768: 1}), (320, {192: 4, 193: 3, 383: 3, 384: 2, 639: 2, 640: 1}),
+    (384, {170: 4, 171: 3, 256: 3, 287: 3, 288: 2, 895: 2, 896: 1}),
+    (448, {170: 4, 171: 3, 256: 3, 319: 3, 320: 2, 719: 2, 720: 1}), (512, {170: 4, 171: 3, 256: 3, 319: 3, 320: 2, 719: 2, 720: 1})])
+def test_parts_of_packed_int8_units(s, parts):
+    assert {u: route(INT8, u, s).parts for u in parts} == parts
+
+
+# units, s: longest first, whether every other round goes backwards
+@pytest.mark.parametrize("units,s,ranked,backwards", [
+    (255, 192, False, False), (256, 192, True, False), (384, 192, True, True),
+    (191, 256, False, False), (192, 256, True, True), (193, 256, False, True), (255, 256, False, True), (256, 256, True, False), (384, 256, True, True),
+    (128, 384, False, False), (129, 384, True, True), (256, 384, True, False), (288, 384, True, True),
+    (1024, 384, True, True), (1025, 384, True, False), (1200, 128, True, True)])
+def test_order_of_packed_int8_units(units, s, ranked, backwards):
+    r = route(INT8, units, s)
+    assert (r.ranked, r.backwards) == (ranked, units * r.parts // 512 * 512 if backwards else 0)
+
+
+@pytest.mark.parametrize("s", [128, 192, 256, 320, 384, 448, 512])
+def test_packed_int8_units_that_fill_their_length_go_as_padded_ones(s):
+    """The interleaved layout's strides are the number of tokens: from 15/16 of what the length allows on the split of the padded
+    layout (of four blocks of keys one part less from 193 to 255 units), in natural order."""
+    for units in (100, 200, 240, 256, 300, 352, 512, 700, 800, 1000, 1200):
+        parts = 3 if s == 256 and 193 <= units <= 255 else route(INT8, units, s, packed=False).parts
+        packed = route(INT8, units, s)
+        most = units * s
+        for tokens, full in ((most, True), (-(-most * 15 // 16), True), (-(-most * 15 // 16) - 1, False), (units, False)):
+            p = params(INT8, units, s)
+            p.interleaved, p.qkv_stride_in_bytes, p.o_stride_in_bytes = 1, tokens, tokens
+            r = decode(capi.api().test_fmha_route(INT8, C.byref(p)))
+            assert (r.parts == parts and not r.ranked) if full else r == packed, (units, tokens)
