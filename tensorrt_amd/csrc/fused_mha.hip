@@ -2623,12 +2623,17 @@ FmhaRoute route_of(int32_t dataType, trtamd_fmha_params const& p)
     // short ones.  Every other round backwards (id_of_workgroup) costs nothing.  12 or 16 heads, sequences of a third of
     // the length to the length:
     // - FP16, 128 queries per workgroup: all resident at once up to four per CU; longest first below 3072 of them
-    //   (16 x 512 18.0 us against 21.2 in natural order, 32 x 384 19.0 / 20.4; 128 x 384, 16 heads, 85.6 / 82.4), and every
-    //   other round backwards always: 32 x 384 15.3 -> 14.8, 32 x 180 9.3 -> 8.2, 96 x 180 19.2 -> 17.0, and in natural order
-    //   128 x 180 31.9 -> 27.0, 128 x 256 40.0 -> 37.2 (16 heads).
-    // - FP16, 64 queries: short enough to even out by themselves, natural order, from three blocks of keys on with rounds
-    //   backwards (22 x 180 8.0 -> 6.7, 21 x 250 10.6 -> 10.0, 16 x 250 8.3 -> 8.6, mean of 45 launches 1.04x; 20 x 100,
-    //   16 heads, 5.26 -> 5.32); of 321 keys and more longest first as well (8 x 384 8.3 -> 7.2, 12 x 384 9.1 -> 8.4; mean of 27 launches 1.06x, 1.04x without it).
+    //   (16 x 512 18.0 us against 21.2 in natural order, 32 x 384 19.0 / 20.4; 128 x 384, 16 heads, 85.6 / 82.4).  Every other
+    //   round backwards where a unit has an even number of parts (32 x 180 9.3 -> 8.2, 96 x 180 19.2 -> 17.0, and in natural order
+    //   128 x 180 31.9 -> 27.0, 128 x 256 40.0 -> 37.2, 16 heads).  Three parts are spread by themselves, but for launches of up
+    //   to three workgroups per CU (13 x 384, 16 heads, 12.5 -> 12.1) or beyond one round (32 x 384 15.3 -> 14.8); between 768 and
+    //   1024 of them lengths of up to 276 of 384 keys lose up to 9 % (19 x 276, 16 heads, 11.9 -> 13.0), short ones 7 %, and in
+    //   natural order any lose 1 to 3 %.
+    // - FP16, 64 queries: short enough to even out by themselves, natural order.  Rounds backwards with four blocks of keys
+    //   (lengths from one on, 10 x 256, 16 heads, 6.8 -> 6.4) and with more than six (8 x 448, 12.4 -> 10.6), not with three or
+    //   five (23 x 192 of up to 140 keys 6.5 -> 7.0; 10 x 320 of up to 230 6.7 -> 7.4).  Six blocks: longest first and backwards up
+    //   to 767 workgroups, three per CU, all resident (8 x 384 9.8 -> 8.9, of one length 10.25 -> 10.54); beyond, a second round of
+    //   long ones waits for the first (11 x 384 of 256 keys and more 12.1 -> 13.6, of less than 64 4.36 -> 4.64).
     // - INT8, two or three workgroups per CU at a time: longest first beyond one round of all CUs' places, and before that
     //   where the units are long enough for the ranking to pay, from 768 of them with three and four blocks of keys
     //   (32 x 180 7.3 -> 6.9), beyond 512 with five and more (14 x 310 9.5 -> 8.7, 16 x 384 12.2 -> 9.9).  Rounds go backwards
@@ -2643,12 +2648,12 @@ FmhaRoute route_of(int32_t dataType, trtamd_fmha_params const& p)
     if (f16 == F16Kernel::kSTREAM)
     {
         ranked = workgroups < 3072;
-        back = true;
+        back = r.parts % 2 == 0 || workgroups < 768 || (ranked && workgroups > 1024);
     }
     else if (f16 == F16Kernel::kTURNS)
     {
-        ranked = blocks >= 6 && workgroups >= 512;
-        back = blocks > 2;
+        ranked = blocks == 6 && workgroups >= 512 && workgroups < 768;
+        back = ranked || blocks == 4 || blocks > 6;
     }
     else
     {
