@@ -2577,7 +2577,11 @@ FmhaRoute route_of(int32_t dataType, trtamd_fmha_params const& p)
     // 12 x 440 12.9 / 9.8, 6 x 440 7.8 / 9.2; 10 x 512 14.3 / 10.8 (16 heads), 6 x 512 7.5 / 9.5.
     // With one or two blocks of keys a second round of the wide ones is no better: 110 x 128 13.0 / 14.4, 225 x 128 24.8 / 29.9;
     // and a row of at most 64 keys leaves half of them idle: 64 x 64 4.5 / 5.3, 600 x 64 25.6 / 28.3.
-    constexpr int kStreamFrom[] = {INT32_MAX, 768, 600, 544, 540, 504, 384, 360};
+    // Padded sequences, whose workgroups are alike but for masks, with 64 / with 128 queries: 20 x 192, 16 heads, 9.6 / 10.6; 20 x 256
+    // 13.5 / 13.9, 28 x 256, 12 heads, 14.5 / 14.1; 9 x 384, 16 heads, 14.3 / 12.5, 10 x 384 11.0 / 11.6; 8 x 448 14.9 / 12.2; 8 x 512
+    // 15.6 / 13.7.
+    constexpr int kStreamFrom[2][8] = {{INT32_MAX, 768, 600, 544, 540, 504, 384, 360}, // packed
+        {INT32_MAX, 768, 768, 768, 540, 432, 384, 360}};
     constexpr int kStreamTile = kWavesStream * kStreamQueries;
     int const streamParts = ceil_div(kt * 64, kStreamTile);
     FmhaRoute r{F16Kernel::kGENERAL, 1, 0};
@@ -2586,7 +2590,7 @@ FmhaRoute route_of(int32_t dataType, trtamd_fmha_params const& p)
         && p.qkv_stride_in_bytes < (1LL << 29)) // eight tokens within a 32-bit offset
     {
         int64_t const wide = (int64_t) p.b * p.h * streamParts;
-        f16 = wide >= kStreamFrom[blocks - 1] && (blocks > 2 || wide <= 1024) ? F16Kernel::kSTREAM : F16Kernel::kTURNS;
+        f16 = wide >= kStreamFrom[p.cu_seqlens ? 0 : 1][blocks - 1] && (blocks > 2 || wide <= 1024) ? F16Kernel::kSTREAM : F16Kernel::kTURNS;
     }
     // Workgroups per (sequence, head).  The general FP16 kernel (its K and V take most of a CU's LDS, one workgroup per CU, and
     // staging them is 40 % of a workgroup's time) shares a unit only below 160 of them (192 units of 192-384 keys: 15.3 us alone,

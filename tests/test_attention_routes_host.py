@@ -128,3 +128,12 @@ def test_packed_int8_units_that_fill_their_length_go_as_padded_ones(s):
 def test_order_of_packed_fp16_workgroups(units, s, kernel, ranked, backwards):
     r = route(FP16, units, s)
     assert (r.kernel, r.ranked, r.backwards) == (kernel, ranked, units * r.parts // 512 * 512 if backwards else 0)
+
+
+@pytest.mark.parametrize("s,stream_from", [(64, None), (128, 768), (192, 384), (256, 384), (320, 180), (384, 144), (448, 96), (512, 90)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_padded_fp16_sequences_change_kernels_where_they_are_faster(s, stream_from, masked):
+    line = stream_from or 5000
+    for units, kernel in ((line - 1, TURNS), (line, TURNS if stream_from is None else STREAM)):
+        r = route(FP16, units, s, packed=False, masked=masked)
+        assert (r.kernel, r.backwards) == (kernel, 0), units
