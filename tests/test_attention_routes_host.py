@@ -117,14 +117,14 @@ def test_packed_int8_units_that_fill_their_length_go_as_padded_ones(s):
 
 # units, s: kernel, longest first, whether every other round goes backwards
 @pytest.mark.parametrize("units,s,kernel,ranked,backwards", [
-    (299, 192, TURNS, False, False), (767, 192, STREAM, True, True), (1600, 192, STREAM, False, True),   # two parts of three
+    (383, 192, TURNS, False, False), (384, 192, STREAM, True, True), (767, 192, STREAM, True, True), (1600, 192, STREAM, False, True),   # two parts of three
     (128, 256, TURNS, False, True), (271, 256, TURNS, False, True), (272, 256, STREAM, True, True), (1536, 256, STREAM, False, True),
     (100, 320, TURNS, False, False), (200, 320, STREAM, True, True),
     (85, 384, TURNS, False, False), (86, 384, TURNS, True, True), (127, 384, TURNS, True, True), (128, 384, TURNS, False, False),
     (167, 384, TURNS, False, False), (168, 384, STREAM, True, False), (171, 384, STREAM, True, True), (255, 384, STREAM, True, True),
     (256, 384, STREAM, True, False), (341, 384, STREAM, True, False), (342, 384, STREAM, True, True), (1023, 384, STREAM, True, True),
     (1024, 384, STREAM, False, False),
-    (64, 448, TURNS, False, True), (89, 512, TURNS, False, True), (128, 448, STREAM, True, True), (768, 512, STREAM, False, True)])
+    (64, 448, TURNS, False, True), (107, 448, TURNS, False, True), (108, 448, STREAM, True, False), (89, 512, TURNS, False, True), (128, 448, STREAM, True, True), (768, 512, STREAM, False, True)])
 def test_order_of_packed_fp16_workgroups(units, s, kernel, ranked, backwards):
     r = route(FP16, units, s)
     assert (r.kernel, r.ranked, r.backwards) == (kernel, ranked, units * r.parts // 512 * 512 if backwards else 0)
