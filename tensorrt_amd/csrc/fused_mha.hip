@@ -2575,7 +2575,7 @@ FmhaRoute route_of(int32_t dataType, trtamd_fmha_params const& p)
     // of s to s, of less than a sixth of s, from one on and between turn over.  12 or 16 heads, sequences of a third of the length to
     // the length, us with 64 / with 128 queries: 64 x 128 keys 8.1 / 7.7, 48 x 128 7.8 / 8.1; 27 x 180 in the capacity of 256 8.0 /
     // 7.1, 21 x 180 6.7 / 6.9; 27 x 230 10.1 / 7.9, 21 x 230 7.8 / 7.9; 16 x 384 12.0 / 9.8, 13 x 345 9.4 / 9.8, 10 x 384 8.2 / 9.1;
-    // 9 x 448 15.8 / 12.6, 6 x 448, 16 heads, 11.2 / 10.0, but from one key on 7.9 / 9.4; 10 x 512 14.3 / 10.8 (16 heads), 6 x 512
+    // 8 x 448 12.4 / 10.0, of one length 14.8 / 12.8, of up to 74 keys 4.6 / 5.0, from one on, 6 x 448, 16 heads, 7.9 / 9.4; 10 x 512 14.3 / 10.8 (16 heads), 6 x 512
     // 7.5 / 9.5.  Three blocks: 28 x 192, all of them, 9.9 / 11.0; up to 32 keys 4.3 / 4.7.
     // With one or two blocks of keys a second round of the wide ones is no better: 110 x 128 13.0 / 14.4, 225 x 128 24.8 / 29.9 (only
     // sequences of up to 21 of 128 keys are slower so, 126 x 128 8.8 / 7.8);
@@ -2583,7 +2583,7 @@ FmhaRoute route_of(int32_t dataType, trtamd_fmha_params const& p)
     // Padded sequences, whose workgroups are alike but for masks, with 64 / with 128 queries: 20 x 192, 16 heads, 9.6 / 10.6; 20 x 256
     // 13.5 / 13.9, 28 x 256, 12 heads, 14.5 / 14.1; 9 x 384, 16 heads, 14.3 / 12.5, 10 x 384 11.0 / 11.6; 8 x 448 14.9 / 12.2; 8 x 512
     // 15.6 / 13.7.
-    constexpr int kStreamFrom[2][8] = {{INT32_MAX, 768, 768, 544, 540, 504, 432, 360}, // packed
+    constexpr int kStreamFrom[2][8] = {{INT32_MAX, 768, 768, 544, 540, 504, 384, 360}, // packed
         {INT32_MAX, 768, 768, 768, 540, 432, 384, 360}};
     constexpr int kStreamTile = kWavesStream * kStreamQueries;
     int const streamParts = ceil_div(kt * 64, kStreamTile);

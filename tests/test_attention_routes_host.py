@@ -124,7 +124,7 @@ def test_packed_int8_units_that_fill_their_length_go_as_padded_ones(s):
     (167, 384, TURNS, False, False), (168, 384, STREAM, True, False), (171, 384, STREAM, True, True), (255, 384, STREAM, True, True),
     (256, 384, STREAM, True, False), (341, 384, STREAM, True, False), (342, 384, STREAM, True, True), (1023, 384, STREAM, True, True),
     (1024, 384, STREAM, False, False),
-    (64, 448, TURNS, False, True), (107, 448, TURNS, False, True), (108, 448, STREAM, True, False), (89, 512, TURNS, False, True), (128, 448, STREAM, True, True), (768, 512, STREAM, False, True)])
+    (64, 448, TURNS, False, True), (95, 448, TURNS, False, True), (96, 448, STREAM, True, False), (89, 512, TURNS, False, True), (128, 448, STREAM, True, True), (768, 512, STREAM, False, True)])
 def test_order_of_packed_fp16_workgroups(units, s, kernel, ranked, backwards):
     r = route(FP16, units, s)
     assert (r.kernel, r.ranked, r.backwards) == (kernel, ranked, units * r.parts // 512 * 512 if backwards else 0)
