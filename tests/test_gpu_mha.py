@@ -53,10 +53,10 @@ INT8_PACKED = [
     # B, N, S (max), lens rule
     (3, 2, 128, "rand"), (2, 16, 384, "c4"), (5, 3, 64, "rand"), (4, 2, 192, "rand"), (3, 2, 256, "full"),
     (2, 2, 512, "rand"), (6, 1, 96, "edge"),
-    # unit counts of one workgroup each, one that takes three workgroups per unit, and one whose ids do not fill whole spans
-    # of 8 x parts
+    # units of one workgroup each, of three and of four, of which the last do not fill whole spans of 8 x 4 ids
     (55, 16, 128, "rand"), (56, 16, 128, "rand"), (17, 16, 256, "c4"), (13, 3, 384, "rand"),
-    # either side of where the launcher stops sharing a (sequence, head) unit between workgroups, by blocks of keys
+    # either side of some of the lines between the launcher's splits and orders: two workgroups per unit and one of two and of
+    # three blocks of keys; four with the longest first and in natural order of four blocks; the order of six
     (213, 3, 128, "rand"), (40, 16, 128, "rand"), (767, 1, 130, "edge"), (256, 3, 130, "rand"), (64, 3, 256, "rand"),
     (193, 1, 256, "rand"), (16, 8, 321, "c4"), (43, 3, 321, "rand"),
 ]
@@ -69,7 +69,7 @@ def _lens(r, B, S, rule):
         return np.full(B, S)
     if rule == "edge":
         base = [1, 0, 15, 16, 17, 64, 65, S]
-        return np.array([min(v, S) for v in base][:B])
+        return np.resize(np.minimum(base, S), B)
     return r.integers(1, S + 1, B)
 
 

@@ -12,6 +12,7 @@ import oracle
 from helpers import (assert_fp_close, assert_int8_close, attention_f64, dev, dev_empty, half2_bits, host,
                      int8_attention_parity, ptr, quantize_amax, rng, stream, sync)
 from tensorrt_amd import capi
+from test_attention_routes_host import STREAM, TURNS, WHOLE, decode
 from test_gpu_linear import interleave, problem, run_fp16, run_gpu
 
 pytestmark = pytest.mark.gpu
@@ -25,6 +26,11 @@ def tuning(name, value):
         yield
     finally:
         api.check(api.test_reset_tuning(name.encode()))
+
+
+def route(dtype, p):
+    """What the launcher makes of a call's parameters."""
+    return decode(capi.api().test_fmha_route(dtype, C.byref(p)))
 
 
 def test_unknown_switch_is_refused():
@@ -327,18 +333,28 @@ def test_longest_first_order_reaches_every_sequence(B):
     assert all((outs[0][:, cu[b]:cu[b + 1]] != 55).any() for b in range(B) if lens[b])
 
 
-# (data type, sequences, heads, longest): workgroups of 64 and of 128 queries and shared INT8 units, one workgroup short of two,
-# three and four rounds of 256, as many and one more, in natural order and the longest first
-@pytest.mark.parametrize("dtype,B,N,S", [(1, 511, 1, 64), (1, 512, 1, 64), (1, 513, 1, 64), (1, 128, 2, 192), (1, 43, 2, 321),
-                                         (1, 1023, 1, 128), (1, 1024, 1, 128), (1, 1025, 1, 128), (1, 192, 2, 200),
-                                         (1, 3329, 1, 64), (2, 128, 1, 384), (2, 129, 1, 330), (2, 192, 2, 190),
-                                         (2, 511, 1, 128), (2, 512, 1, 128), (2, 257, 2, 65), (2, 320, 2, 128),
-                                         (2, 512, 2, 190), (2, 205, 5, 190), (2, 193, 1, 250)])
-def test_rounds_that_go_backwards_reach_every_unit(dtype, B, N, S):
+# (data type, sequences, heads, longest), the workgroups whose rounds change places, longest first: whole pairs of rounds, some
+# workgroups more and one pair short, FP16 with 64 and with 128 queries per workgroup, INT8 units in one, two and four parts; INT8
+# sequences that all have the length in natural order; and launches without any such rounds.
+@pytest.mark.parametrize("dtype,B,N,S,backwards,ranked", [
+    (1, 128, 1, 256, 512, False), (1, 255, 1, 200, 512, False), (1, 257, 1, 256, 1024, False), (1, 65, 1, 450, 512, False),
+    (1, 43, 2, 321, 512, True), (1, 127, 1, 384, 512, True), (1, 192, 2, 190, 512, True), (1, 511, 1, 192, 512, True),
+    (1, 513, 1, 192, 1024, True), (1, 128, 1, 512, 512, True), (1, 171, 1, 384, 512, True), (1, 342, 1, 384, 1024, True),
+    (1, 1537, 1, 192, 3072, False), (1, 769, 1, 448, 3072, False),
+    (2, 129, 1, 384, 512, True), (2, 192, 2, 190, 512, True), (2, 400, 1, 190, 512, True), (2, 144, 2, 330, 512, True),
+    (2, 160, 5, 128, 512, True), (2, 1025, 1, 128, 1024, True), (2, 768, 1, 192, 512, True), (2, 193, 1, 256, 512, False),
+    (2, 255, 1, 250, 512, False), (2, 400, 1, -192, 512, False), (2, 200, 3, -384, 1024, False),
+    (1, 513, 1, 64, 0, False), (1, 240, 1, 320, 512, True), (1, 256, 1, 384, 0, True), (1, 1024, 1, 384, 0, False),
+    (2, 100, 1, 384, 0, False), (2, 257, 1, 190, 0, True), (2, 800, 1, -192, 0, False)])
+def test_rounds_that_go_backwards_reach_every_unit(dtype, B, N, S, backwards, ranked):
     """The order that the launcher chooses writes the bytes of the sequences' own order, and of every unit."""
-    r = rng(1800 + B + S)
-    lens = r.integers(1, S + 1, B)
-    lens[0], lens[B // 2], lens[-1] = S, 0, 1
+    r = rng(1800 + B + abs(S))
+    if S < 0: # all of this length
+        S = -S
+        lens = np.full(B, S)
+    else:
+        lens = r.integers(1, min(S, 40 if B > 600 else S) + 1, B)
+        lens[0], lens[B // 2], lens[-1] = S, 0, 1
     cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     T = int(cu[-1])
     qkv = r.standard_normal((T, 3 * N * 64)).astype(np.float32)
@@ -357,6 +373,7 @@ def test_rounds_that_go_backwards_reach_every_unit(dtype, B, N, S):
     d_cu = dev(cu)
     p.qkv_ptr, p.cu_seqlens = ptr(d_qkv), ptr(d_cu)
     p.b, p.h, p.s, p.d = B, N, S, 64
+    assert (route(dtype, p).backwards, route(dtype, p).ranked) == (backwards, ranked)
     api = capi.api()
     outs = []
     for order in (None, 0):
@@ -371,12 +388,13 @@ def test_rounds_that_go_backwards_reach_every_unit(dtype, B, N, S):
     assert (units != (55 if dtype == 2 else -7)).any(axis=2).all()
 
 
-# launches that fill the chip (768 workgroups of 128 queries): lengths on either side of a wavefront's 32 queries, a
-# workgroup's 128, half a block and a block of keys; scores whose maximum grows from block to block and scores of one size
-@pytest.mark.parametrize("S,B,N", [(64, 192, 4), (384, 64, 4), (512, 48, 4)])
+# launches that fill the chip: 768 workgroups of 128 queries, or of 64 with at most 64 keys; lengths on either side of a
+# wavefront's 32 queries, a workgroup's 128, half a block and a block of keys; scores whose maximum grows from block to block and
+# scores of one size
+@pytest.mark.parametrize("S,B,N,kernel", [(64, 192, 4, TURNS), (128, 192, 4, STREAM), (384, 64, 4, STREAM), (512, 48, 4, STREAM)])
 @pytest.mark.parametrize("growing", [False, True])
 @pytest.mark.parametrize("ranked", [0, 1])
-def test_fp16_attention_of_full_launches(S, B, N, growing, ranked):
+def test_fp16_attention_of_full_launches(S, B, N, kernel, growing, ranked):
     api = capi.api()
     r = rng(1600 + S)
     edges = [n for n in (1, 31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129, 161, 255, 257, 383, 384, 449, 511, 512) if n <= S]
@@ -397,6 +415,7 @@ def test_fp16_attention_of_full_launches(S, B, N, growing, ranked):
     p.qkv_stride_in_bytes, p.o_stride_in_bytes = 2 * 3 * N * 64, 2 * N * 64
     p.b, p.h, p.s, p.d = B, N, S, 64
     p.scale_bmm1, p.scale_softmax, p.scale_bmm2 = half2_bits(0.125), half2_bits(1.0), half2_bits(1.0)
+    assert route(1, p).kernel == kernel and route(1, p).parts * B * N == 768
     with tuning("TRTAMD_FMHA_RANKED", ranked):
         api.check(api.fused_mha_run(stream(), 1, C.byref(p)))
         sync()
@@ -413,10 +432,12 @@ def test_fp16_attention_of_full_launches(S, B, N, growing, ranked):
 
 # one workgroup of 128 queries short of the lines between the two FP16 kernels, by blocks of keys, and on them; past one round
 # of four per CU with two blocks
-@pytest.mark.parametrize("B,N,S", [(1024, 1, 64), (767, 1, 128), (768, 1, 128), (1024, 1, 100), (205, 5, 100), (299, 1, 192),
-                                   (300, 1, 192), (271, 1, 200), (272, 1, 200), (179, 1, 260), (180, 1, 260), (143, 1, 384),
-                                   (144, 1, 321), (95, 1, 400), (96, 1, 448), (89, 1, 512), (90, 1, 449)])
-def test_fp16_attention_on_either_side_of_its_kernels_lines(B, N, S):
+@pytest.mark.parametrize("B,N,S,kernel", [
+    (1024, 1, 64, TURNS), (767, 1, 128, TURNS), (768, 1, 128, STREAM), (1024, 1, 100, STREAM), (205, 5, 100, TURNS),
+    (383, 1, 192, TURNS), (384, 1, 192, STREAM), (271, 1, 200, TURNS), (272, 1, 200, STREAM), (179, 1, 260, TURNS),
+    (180, 1, 260, STREAM), (167, 1, 384, TURNS), (168, 1, 321, STREAM), (95, 1, 400, TURNS), (96, 1, 448, STREAM),
+    (89, 1, 512, TURNS), (90, 1, 449, STREAM)])
+def test_fp16_attention_on_either_side_of_its_kernels_lines(B, N, S, kernel):
     api = capi.api()
     r = rng(1900 + B + S)
     edges = [n for n in (S, 1, 16, 63, 64, 65, 127, 128, 129, S - 1, 193, 257, 385) if n <= S]
@@ -432,6 +453,7 @@ def test_fp16_attention_on_either_side_of_its_kernels_lines(B, N, S):
     p.qkv_stride_in_bytes, p.o_stride_in_bytes = 2 * 3 * N * 64, 2 * N * 64
     p.b, p.h, p.s, p.d = B, N, S, 64
     p.scale_bmm1, p.scale_softmax, p.scale_bmm2 = half2_bits(0.125), half2_bits(1.0), half2_bits(1.0)
+    assert route(1, p).kernel == kernel
     api.check(api.fused_mha_run(stream(), 1, C.byref(p)))
     sync()
     got = host(out)
@@ -443,6 +465,60 @@ def test_fp16_attention_on_either_side_of_its_kernels_lines(B, N, S):
         n = b % N
         want = attention_f64(qkv[lo:hi, n, 0], qkv[lo:hi, n, 1], qkv[lo:hi, n, 2], 0.125)
         assert_fp_close(got[lo:hi, n * 64:(n + 1) * 64], want, what=f"sequence {b} of {hi - lo}, head {n}")
+
+
+# one unit short of the lines between the numbers of INT8 workgroups per unit, by blocks of keys, and on them
+@pytest.mark.parametrize("layout,units,S,parts", [
+    ("packed", 639, 128, 2), ("packed", 640, 128, 1), ("packed", 383, 192, 3), ("packed", 384, 192, 2), ("packed", 767, 130, 2),
+    ("packed", 768, 192, 1), ("packed", 255, 256, 4), ("packed", 256, 256, 3), ("packed", 767, 256, 2), ("packed", 768, 200, 1),
+    ("packed", 192, 260, 4), ("packed", 193, 320, 3), ("packed", 639, 320, 2), ("packed", 640, 260, 1), ("packed", 170, 384, 4),
+    ("packed", 171, 330, 3), ("packed", 287, 330, 3), ("packed", 288, 384, 2), ("packed", 895, 384, 2), ("packed", 896, 330, 1),
+    ("packed", 319, 400, 3), ("packed", 320, 512, 2), ("packed", 719, 448, 2), ("packed", 720, 400, 1), ("packed", 719, 512, 2),
+    ("packed", 720, 460, 1),
+    ("full", 193, 256, 3), ("full", 192, 384, 4), ("full", 193, 384, 3), ("full", 341, 384, 3), ("full", 342, 384, 2),
+    ("full", 641, 192, 1), ("full", 800, 128, 2),
+    ("padded", 640, 96, 2), ("padded", 641, 96, 1), ("padded", 641, 128, 2), ("padded", 255, 256, 4), ("padded", 256, 256, 3),
+    ("padded", 192, 320, 4), ("padded", 193, 320, 3), ("padded", 341, 384, 3), ("padded", 342, 384, 2), ("padded", 256, 512, 3),
+    ("masked", 640, 128, 2), ("masked", 641, 128, 1), ("masked", 192, 384, 4), ("masked", 193, 384, 3)])
+def test_int8_attention_on_either_side_of_its_lines(layout, units, S, parts):
+    """The bytes of one workgroup per unit, and of every unit."""
+    r = rng(2000 + units + S)
+    full = layout != "packed"
+    lens = np.full(units, S) if full else np.concatenate([[S, S - 1, 0, 1, 64, 65], r.integers(1, 40, units - 6)])
+    T = int(lens.sum())
+    bits = lambda x: int(np.float32(x).view(np.uint32))
+    p = capi.FmhaParams()
+    p.b, p.h, p.s, p.d = units, 1, S, 64
+    p.scale_bmm1, p.scale_softmax, p.scale_bmm2 = bits(0.0009 * 0.125), bits(127.0), bits(0.75 / 127)
+    q = np.clip(np.rint(33 * r.standard_normal((T, 192), np.float32)), -127, 127).astype(np.int8)
+    if layout in ("packed", "full"):
+        d_qkv, d_cu = dev(interleave(q)), dev(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32))
+        p.cu_seqlens, p.interleaved = ptr(d_cu), 1
+        p.qkv_stride_in_bytes = p.o_stride_in_bytes = T
+        shape = (2, T, 32)
+    else:
+        d_qkv = dev(q.reshape(S, units, 192))
+        p.qkv_stride_in_bytes, p.o_stride_in_bytes = 192 * units, 64 * units
+        shape = (S, units, 64)
+        if layout == "masked":
+            mask = (np.arange(S)[:, None] < r.integers(1, S + 1, units)[None, :]).astype(np.int32)
+            packed, _ = oracle.convert_mask(mask, *((1, 8) if S == 384 else (2, 2)))
+            d_mask = dev(packed)
+            p.packed_mask_ptr, p.packed_mask_stride_in_bytes = ptr(d_mask), packed.shape[1] * 4
+    p.qkv_ptr = ptr(d_qkv)
+    assert route(2, p).parts == parts
+    api = capi.api()
+    outs = []
+    for forced in (-1, 1):
+        out = dev_empty(shape, np.int8, fill=-128)
+        p.o_ptr = ptr(out)
+        with tuning("TRTAMD_FMHA_QSPLIT", forced):
+            assert route(2, p).parts == (parts if forced < 0 else 1)
+            api.check(api.fused_mha_run(stream(), 2, C.byref(p)))
+            sync()
+        outs.append(host(out))
+    assert np.array_equal(outs[0], outs[1])
+    assert (outs[0] != -128).all() # a result is a mean of values of at most 127, times 0.75
 
 
 @pytest.mark.parametrize("scale", [0.125, 1.0])
@@ -482,10 +558,12 @@ def test_fp16_attention_of_full_launches_keeps_infinite_scores_apart(scale):
     assert np.isinf(own).all() if scale == 0.125 else not np.isfinite(own).any()
 
 
-# packed masks: launches of either FP16 kernel and INT8
+# packed masks: FP16 launches of few workgroups, of more of them with 64 queries, and with 128; and INT8
 @pytest.mark.parametrize("dtype,scale", [(1, 0.125), (1, 1.0), (2, 0.125)])
-@pytest.mark.parametrize("S,B,N", [(64, 9, 2), (96, 9, 2), (128, 9, 2), (384, 9, 2), (128, 200, 4), (384, 70, 4)])
-def test_attention_with_packed_masks(dtype, scale, S, B, N):
+@pytest.mark.parametrize("S,B,N,kernel", [(64, 9, 2, WHOLE), (96, 9, 2, WHOLE), (128, 9, 2, WHOLE), (384, 9, 2, WHOLE),
+                                          (64, 150, 2, TURNS), (96, 72, 2, TURNS), (128, 99, 2, TURNS), (384, 30, 2, TURNS),
+                                          (128, 200, 4, STREAM), (384, 70, 4, STREAM)])
+def test_attention_with_packed_masks(dtype, scale, S, B, N, kernel):
     """Masks that are a prefix of every kind of length, that have holes in the first, a middle and the last block, that
     leave one key or none: the general kernel's results to the bar, zeros where no key is left.  FP16 scales on either side of
     ln 2, from where on the scale times the largest binary32 value is infinite."""
@@ -518,6 +596,7 @@ def test_attention_with_packed_masks(dtype, scale, S, B, N):
         p.packed_mask_stride_in_bytes = packed.shape[1] * 4
         p.b, p.h, p.s, p.d = B, N, S, 64
         p.scale_bmm1, p.scale_softmax, p.scale_bmm2 = scales
+        assert dtype == 2 or route(1, p).kernel in (kernel, 0) # 0: the general kernel, asked for
         api.check(api.fused_mha_run(stream(), dtype, C.byref(p)))
         sync()
         return host(out)
@@ -539,3 +618,35 @@ def test_attention_with_packed_masks(dtype, scale, S, B, N):
             if keep.any():
                 ref = attention_f64(qkv[:, b, 1, 0], qkv[keep, b, 1, 1], qkv[keep, b, 1, 2], scale)
                 assert_fp_close(got[:, b, 64:128], ref, what=f"sequence {b}")
+
+
+@pytest.mark.parametrize("S,copies", [(64, 15), (96, 8), (128, 8), (384, 3)])
+def test_masked_fp16_launches_of_few_workgroups_give_the_bytes_of_larger_ones(S, copies):
+    """With all of K and V in LDS at once and in turns: masks that are a prefix, that have holes in the first, a middle and the
+    last block, that leave one key or none."""
+    api = capi.api()
+    B, N = 9, 2
+    r = rng(2100 + S)
+    mask = np.ones((S, B), np.int32)
+    for b in range(1, B):
+        mask[:, b] = r.integers(0, 2, S) if b >= 5 else np.arange(S) < [S, 1, S - 1, min(65, S - 1), S // 2 + 3][b]
+    mask[:min(64, S), 6] = 0
+    mask[:, 7] = 0
+    mask[S - 1, 8] = 1
+    qkv = r.standard_normal((S, B, N, 3, 64)).astype(np.float16)
+    got = []
+    for n, kernel in ((1, WHOLE), (copies, TURNS)):
+        packed, _ = oracle.convert_mask(np.tile(mask, (1, n)), *((1, 8) if S == 384 else (2, 2)))
+        d_qkv, d_mask, out = dev(np.tile(qkv, (1, n, 1, 1, 1))), dev(packed), dev_empty((S, B * n, N * 64), np.float16, fill=55)
+        p = capi.FmhaParams()
+        p.qkv_ptr, p.o_ptr, p.packed_mask_ptr = ptr(d_qkv), ptr(out), ptr(d_mask)
+        p.qkv_stride_in_bytes, p.o_stride_in_bytes = 2 * 3 * B * n * N * 64, 2 * B * n * N * 64
+        p.packed_mask_stride_in_bytes = packed.shape[1] * 4
+        p.b, p.h, p.s, p.d = B * n, N, S, 64
+        p.scale_bmm1, p.scale_softmax, p.scale_bmm2 = half2_bits(0.125), half2_bits(1.0), half2_bits(1.0)
+        assert route(1, p).kernel == kernel
+        api.check(api.fused_mha_run(stream(), 1, C.byref(p)))
+        sync()
+        got.append(host(out))
+    assert (got[0][:, 7] == 0).all()
+    assert np.array_equal(np.tile(got[0], (1, copies, 1)), got[1])
