@@ -1556,9 +1556,9 @@ __global__ __launch_bounds__(kWavesF16* kWaveSize) void fmha_f16_kernel(FmhaArgs
 }
 
 // ------------------------------------------------------------------------------------------
-// FP16, launches that leave CUs idle, on cu_seqlens or a packed mask (with holes too): the same specialisation, but K and V
-// take turns in LDS, one block of V in the place of each block of K as soon as every wavefront has multiplied it.  48 KB for 384 keys instead of
-// 96 KB: three workgroups of four wavefronts share a CU, so that one computes while another waits for its sequence, its K
+// FP16, launches with too few workgroups for 128 queries each (route_of), and any with at most 64 keys, on cu_seqlens or a packed
+// mask (with holes too): the same specialisation, but K and V take turns in LDS, one block of V in the place of each block of K as
+// soon as every wavefront has multiplied it.  48 KB for 384 keys instead of 96 KB: three workgroups of four wavefronts share a CU, so that one computes while another waits for its sequence, its K
 // or its V, and a unit's queries are shared out 64 at a time over as many workgroups.  What bounds either kernel is that
 // wait; with one workgroup per CU nothing covered it.  All of Q, K and V come by direct-to-LDS loads, whose number in
 // flight the waits below count; a wavefront requests 16 rows of every block.  12 heads, sequences of a third of the length

@@ -1946,8 +1946,10 @@ __global__ __launch_bounds__(NW * 64, PER_SIMD) void linear_piece_dma_kernel(uin
 // of a second round); the kernels and the choice before took 13 % more (50 % at most).  The pieces' among them, which read whole
 // lines, are fits to 30 layers of 64 to 4096 FP16 values or twice as many INT8 ones, 32 to 4096 channels, 1 to 4000 tokens, 1800
 // launches, each piece's time multiplied by what the estimate of 64 x 64 tiles exceeds theirs by at the same sizes: tiles are
-// estimated 1.0 times what they take at rows of 8 KB and 1.4 times at 128 bytes, and the choice is between the two.  0.6 % more
-// than the best of ten plans in the mean, 1.8 % at most more than with the pieces of half lines.  (Fitted to the encoders' layers
+// estimated 1.0 times what they take at rows of 8 KB and 1.4 times at 128 bytes, and the choice is between the two; the wider pieces'
+// tile a tenth more than fitted, since where the two pieces are even the small ones are (102 tokens x 768 -> 3072: 4.85 us, 4.93 in
+// the wide ones).  0.6 % more than the best of ten plans in the mean; one launch takes 4 % more than with the pieces of half lines, no
+// other more than 3 %.  (Fitted to the encoders' layers
 // only, the pieces were taken for short rows where tiles are faster, us: 2100 tokens x 128 -> 512, FP16, 5.3 against 3.7 in tiles;
 // 1700 x 384 -> 384 4.9 / 4.2; 600 x 384 -> 1152 5.0 / 4.4; 384 x 512 -> 2048 5.6 / 5.2.)
 // Linear operands whose rows end within a line have kernels and constants of their own: stages of 64 bytes, tiles of up to 128 x
@@ -2007,7 +2009,7 @@ constexpr TileCost kTileCosts[3][kLinearPlans] = {
     {{}, {}, {128, 128, 2, 4.64f, 0.00f, 0.231f, 0.60f, 0.61f, 1.02f, 0.40f, 0.25f}, {},
         {64, 64, 2, 3.82f, 0.29f, 0.082f, 0.23f, 0.70f, 0.89f, 0.63f, 0.34f},
         {128, 128, 1, 4.02f, 0.77f, 0.142f, 0.99f, 0.f, 1.30f, 0.77f, 0.51f, 0.10f}, {}, {},
-        {32, 64, 1, 3.12f, 1.14f, 0.038f, 0.02f, 0.f, 1.08f, 0.89f, 0.56f},
+        {32, 64, 1, 3.12f, 1.25f, 0.038f, 0.02f, 0.f, 1.08f, 0.89f, 0.56f},
         {32, 32, 2, 3.73f, 0.13f, 0.018f, 0.f, 1.78f, 1.72f, 0.61f, 0.54f},
         {256, 256, 1, 0.00f, 4.48f, 0.440f, 1.88f, 0.f, 1.02f, 0.54f, 0.97f, 0.11f},
         {256, 192, 1, 5.13f, 0.01f, 0.388f, 1.26f, 0.f, 1.35f, 0.67f, 0.56f, 0.15f},
@@ -2188,7 +2190,9 @@ int launch_plan(hipStream_t stream, LinearArgs a, int plan)
     return set_error(TRTAMD_STATUS_BAD_PARAM, "int8_linear: no such plan for this layout: %d", plan);
 }
 
-// Partial sums of `parts` workgroups per piece, in pieces of 32 x 32.
+// Partial sums of `parts` workgroups per piece, in pieces of 32 x 32.  Parts are no more than bring the workgroups to one per CU, so
+// linear operands have the LDS of a second one for rings of four stages of whole lines (up to 128 tokens x 3072 -> 768, FP16: 4.29 us
+// in traced passes, 4.40 with rings of two).
 template <bool IL, int EPI>
 int launch_partial(hipStream_t stream, LinearArgs a, int parts, void* partial, WeightPrefetch const& prefetch = {nullptr, 0})
 {
@@ -2293,7 +2297,8 @@ int small_plan(LinearArgs a, bool gelu)
 }
 
 // Parts of a layer whose launch is `plan`: as many as bring its workgroups to one per CU, and no less than 1 KB of k for
-// each (two k-slabs per wavefront).  The wider pieces are chosen where the smaller ones no longer fit on the CUs at once, so
+// each (two stages for each wavefront of linear operands, eight with 64 bytes or four with 128; four slabs of 32 bytes of interleaved
+// ones).  The wider pieces are chosen where the smaller ones no longer fit on the CUs at once, so
 // there is nothing left to share them between.
 int parts_of(int plan, LinearArgs const& a)
 {
@@ -2558,10 +2563,10 @@ bool interleaved(trtamd_int8_linear_params const& p)
 
 // Pieces, whose launches are as long as the trip of their weights; and layers with longer rows than they have of them, whose
 // workgroups walk a chain of stages that each wait for weights from memory (a model of 24 layers does not stay in the last-level
-// cache): a pass of 24 layers of 1024 channels with the second feed-forward layer's weights fetched by the projection, us: 316
-// tokens 707 -> 688, 531 811 -> 805, 1006 912 -> 905, 1509 1148 -> 1136, 2810 1632 -> 1592, 3775 1881 -> 1853, 6782 2830 -> 2806,
-// no difference where the projection leaves no CU idle.  The first feed-forward layer's weights ahead of their launch cost up to
-// 1 %, the other two's bring nothing.
+// cache): a pass of 24 layers of 1024 channels without / with the second feed-forward layer's weights fetched by the projection, us,
+// processes in turn: 464 tokens 737 / 730, 531 847 / 833, 795 916 / 903, 837 921 / 908, 1144 1074 / 1044, 1781 1253 / 1232, 3268
+// 1758 / 1747, no difference where the projection leaves no CU idle.  The first feed-forward layer's weights ahead of their launch
+// cost up to 1 %, the other two's bring nothing.
 WeightPrefetch prefetch_of(trtamd_int8_linear_params const& next)
 {
     // N: the channel blocks have to come round to the same XCD in every k-slab

@@ -51,6 +51,12 @@ def test_short_rows_go_in_tiles(T, row_bytes, N, gelu):
     assert plan(LINEAR, T, row_bytes, N, gelu) in (4, 14)
 
 
+@pytest.mark.parametrize("T", [97, 102, 128])
+def test_the_smaller_pieces_where_both_are_even(T):
+    """The first layers of a 768-channel FP16 encoder."""
+    assert plan(LINEAR, T, 1536, 2304) == plan(LINEAR, T, 1536, 3072, 1) == 9
+
+
 @pytest.mark.parametrize("T,row_bytes,N,want", [(1, 128, 256, 9), (65, 256, 512, 9), (102, 1536, 2304, 9),
                                                 (448, 6144, 768, 8), (96, 8192, 1024, 9), (2100, 256, 32, 9)])
 def test_few_tokens_go_in_pieces(T, row_bytes, N, want):
