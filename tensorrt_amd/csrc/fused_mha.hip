@@ -1558,8 +1558,8 @@ __global__ __launch_bounds__(kWavesF16* kWaveSize) void fmha_f16_kernel(FmhaArgs
 // ------------------------------------------------------------------------------------------
 // FP16, launches with too few workgroups for 128 queries each (route_of), and any with at most 64 keys, on cu_seqlens or a packed
 // mask (with holes too): the same specialisation, but K and V take turns in LDS, one block of V in the place of each block of K as
-// soon as every wavefront has multiplied it.  48 KB for 384 keys instead of 96 KB: three workgroups of four wavefronts share a CU, so that one computes while another waits for its sequence, its K
-// or its V, and a unit's queries are shared out 64 at a time over as many workgroups.  What bounds either kernel is that
+// soon as every wavefront has multiplied it.  48 KB for 384 keys instead of 96 KB: three workgroups of four wavefronts share a CU, so
+// that one computes while another waits for its sequence, its K or its V, and a unit's queries are shared out 64 at a time over as many workgroups.  What bounds either kernel is that
 // wait; with one workgroup per CU nothing covered it.  All of Q, K and V come by direct-to-LDS loads, whose number in
 // flight the waits below count; a wavefront requests 16 rows of every block.  12 heads, sequences of a third of the length
 // to the length, that kernel / this one, us per plugin call: 32 x 128 keys 12.5 / 5.8, 128 x 256 41.7 / 37.5, 32 x 384
@@ -2501,8 +2501,8 @@ bool alike(trtamd_fmha_params const& p)
     return !p.cu_seqlens || (p.interleaved && p.qkv_stride_in_bytes >= ceil_div<int64_t>((int64_t) p.b * p.s * 15, 16));
 }
 
-// INT8: from how many (sequence, head) units on each has a workgroup of its own, by blocks of keys.  Three workgroups of up to six
-// blocks have room on a CU, two of more; every extra workgroup of a unit stages K and V again.
+// INT8: from how many (sequence, head) units on each has a workgroup of its own, by blocks of keys (one block always has).  Three
+// workgroups of up to six blocks have room on a CU, two of more; every extra workgroup of a unit stages K and V again.
 // Packed sequences: once rounds that go forwards and backwards even out units of different lengths, from 640 units of one or two
 // blocks (672 units: one 6.7, two 7.4 us; 600: 6.4 / 6.0), 768 of three or four (192 keys: 9.0 / 10.0; 720 units: 10.9 / 9.9), 640
 // of five (752 units: 15.8 / 18.3), 896 of six, 720 of more (440 keys: 26.9 / 29.2).  (Six by themselves: 900 units 28.5 / 26.2,
@@ -2575,8 +2575,8 @@ FmhaRoute route_of(int32_t dataType, trtamd_fmha_params const& p)
     // of s to s, of less than a sixth of s, from one on and between turn over.  12 or 16 heads, sequences of a third of the length to
     // the length, us with 64 / with 128 queries: 64 x 128 keys 8.1 / 7.7, 48 x 128 7.8 / 8.1; 27 x 180 in the capacity of 256 8.0 /
     // 7.1, 21 x 180 6.7 / 6.9; 27 x 230 10.1 / 7.9, 21 x 230 7.8 / 7.9; 16 x 384 12.0 / 9.8, 13 x 345 9.4 / 9.8, 10 x 384 8.2 / 9.1;
-    // 8 x 448 12.4 / 10.0, of one length 14.8 / 12.8, of up to 74 keys 4.6 / 5.0, from one on, 6 x 448, 16 heads, 7.9 / 9.4; 10 x 512 14.3 / 10.8 (16 heads), 6 x 512
-    // 7.5 / 9.5.  Three blocks: 28 x 192, all of them, 9.9 / 11.0; up to 32 keys 4.3 / 4.7.
+    // 8 x 448 12.4 / 10.0, of one length 14.8 / 12.8, of up to 74 keys 4.6 / 5.0, from one on, 6 x 448, 16 heads, 7.9 / 9.4;
+    // 10 x 512 14.3 / 10.8 (16 heads), 6 x 512 7.5 / 9.5.  Three blocks: 28 x 192, all of them, 9.9 / 11.0; up to 32 keys 4.3 / 4.7.
     // With one or two blocks of keys a second round of the wide ones is no better: 110 x 128 13.0 / 14.4, 225 x 128 24.8 / 29.9 (only
     // sequences of up to 21 of 128 keys are slower so, 126 x 128 8.8 / 7.8);
     // and a row of at most 64 keys leaves half of them idle: 64 x 64 4.5 / 5.3, 600 x 64 25.6 / 28.3.
@@ -2680,7 +2680,8 @@ FmhaRoute route_of(int32_t dataType, trtamd_fmha_params const& p)
         ranked = forcedRank != 0;
         back = back && ranked;
     }
-    // sequences of one length (24.0 us forwards, 24.1 backwards, 32 x 384) have nothing to even out
+    // Padded sequences go in their own order, every round forwards: of one length they have nothing to even out (32 x 384 24.0 us
+    // forwards, 24.1 backwards); masks of different lengths were not tried backwards.
     uint32_t const paired = back && p.cu_seqlens ? (uint32_t) std::min<int64_t>(workgroups, INT32_MAX) / kTwoRounds * kTwoRounds : 0;
     r.order = paired | (ranked ? kRanked : 0);
     return r;
