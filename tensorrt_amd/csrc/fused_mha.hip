@@ -1559,11 +1559,11 @@ __global__ __launch_bounds__(kWavesF16* kWaveSize) void fmha_f16_kernel(FmhaArgs
 // FP16, launches with too few workgroups for 128 queries each (route_of), and any with at most 64 keys, on cu_seqlens or a packed
 // mask (with holes too): the same specialisation, but K and V take turns in LDS, one block of V in the place of each block of K as
 // soon as every wavefront has multiplied it.  48 KB for 384 keys instead of 96 KB: three workgroups of four wavefronts share a CU, so
-// that one computes while another waits for its sequence, its K or its V, and a unit's queries are shared out 64 at a time over as many workgroups.  What bounds either kernel is that
-// wait; with one workgroup per CU nothing covered it.  All of Q, K and V come by direct-to-LDS loads, whose number in
-// flight the waits below count; a wavefront requests 16 rows of every block.  12 heads, sequences of a third of the length
-// to the length, that kernel / this one, us per plugin call: 32 x 128 keys 12.5 / 5.8, 128 x 256 41.7 / 37.5, 32 x 384
-// 19.8 / 19.6, 128 x 384 71.7 / 64.6, 16 x 512 22.8 / 19.5.  What is left is the L2: K and V of a unit are read once for every
+// that one computes while another waits for its sequence, its K or its V, and a unit's queries are shared out 64 at a time over as
+// many workgroups.  What bounds either kernel is that wait; with one workgroup per CU nothing covered it.  All of Q, K and V come by
+// direct-to-LDS loads, whose number in flight the waits below count; a wavefront requests 16 rows of every block.  12 heads, sequences
+// of a third of the length to the length, that kernel / this one, us per plugin call: 32 x 128 keys 12.5 / 5.8, 128 x 256 41.7 / 37.5,
+// 32 x 384 19.8 / 19.6, 128 x 384 71.7 / 64.6, 16 x 512 22.8 / 19.5.  What is left is the L2: K and V of a unit are read once for every
 // 64 queries, 133 MB for the 35.8 MB of 32 x 384.
 // WHOLE: launches so small that a CU has room for all of it (kWholeWorkgroups); K, V and Q of sequences of up to kWholeBlocks
 // blocks are requested together then.
